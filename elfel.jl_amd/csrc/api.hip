@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <mutex>
 #include <new>
 
 #include "common.h"
@@ -104,6 +105,54 @@ void release(Buf &b)
     b.bytes = 0;
 }
 
+// ---- pinned words of the contexts ------------------------------------------
+// 64 bytes of pinned host memory a context, from one page shared by the first
+// TOLD_SLOTS contexts (a pinned allocation of its own takes 0.3 ms of
+// elfel_hip_init); the page is freed with the last context that holds a slot.
+namespace {
+constexpr int TOLD_SLOTS = 64;
+std::mutex told_mu;
+char *told_page = nullptr;
+uint64_t told_used = 0;
+}  // namespace
+
+static void *told_get()
+{
+    std::lock_guard<std::mutex> g(told_mu);
+    if (!told_page && hipHostMalloc((void **)&told_page, 64 * TOLD_SLOTS, hipHostMallocPortable) != hipSuccess) {
+        (void)hipGetLastError();
+        told_page = nullptr;
+        return nullptr;
+    }
+    if (~told_used) {
+        const int k = __builtin_ctzll(~told_used);
+        told_used |= 1ull << k;
+        return told_page + 64 * k;
+    }
+    void *p = nullptr;
+    if (hipHostMalloc(&p, 64, hipHostMallocPortable) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    return p;
+}
+
+static void told_put(void *p)
+{
+    if (!p) return;
+    std::lock_guard<std::mutex> g(told_mu);
+    const ptrdiff_t at = told_page ? (char *)p - told_page : -1;
+    if (at < 0 || at >= 64 * TOLD_SLOTS) {
+        hipHostFree(p);
+        return;
+    }
+    told_used &= ~(1ull << (at / 64));
+    if (!told_used) {
+        hipHostFree(told_page);
+        told_page = nullptr;
+    }
+}
+
 // ---- timing ----------------------------------------------------------------
 static hipEvent_t ev_get(elfel_hip_ctx *c)
 {
@@ -193,8 +242,15 @@ extern "C" int elfel_hip_init(int device, elfel_hip_ctx **out)
             delete c;
             return ELFEL_ENOMEM;
         }
+        if (!(c->told = told_get())) {
+            release(c->dscal);
+            hipStreamDestroy(c->stream);
+            delete c;
+            return ELFEL_ENOMEM;
+        }
         // this device's address of the allocation-free entry point's scratch
         if (int rc = noalloc_init_device(device)) {
+            told_put(c->told);
             release(c->dscal);
             hipStreamDestroy(c->stream);
             delete c;
@@ -220,6 +276,7 @@ extern "C" int elfel_hip_free(elfel_hip_ctx *c)
                    &c->fpat.ptr, &c->fpat.ind, &c->fpat.perm, &c->fpat.seg, &c->fpat.fperm, &c->fpat.fbeg,
                    &c->fpat.coo, &c->fpat.fcoo};
     for (Buf *b : bufs) release(*b);
+    told_put(c->told);
     batch_free(c);
     for (auto &p : c->tm.pending) { hipEventDestroy(p.a); hipEventDestroy(p.b); }
     if (c->tm.r0) hipEventDestroy(c->tm.r0);
@@ -319,9 +376,10 @@ extern "C" int elfel_hip_sparse(elfel_hip_ctx *c, int64_t nrow, int64_t ncol, in
         const int64_t nmaj = csc ? ncol : nrow, nmin = csc ? nrow : ncol;
         const int minor_bits = bits_for(nmin), major_bits = bits_for(nmaj);
         int rc;
-        if ((rc = ensure(c, c->keys[0], 8 * n)) || (rc = ensure(c, c->keys[1], 8 * n)) || (rc = ensure(c, c->vals[0], 8 * n)) ||
-            (rc = ensure(c, c->vals[1], 8 * n)) || (rc = ensure(c, c->stage64, 16 * n)) ||
-            (rc = ensure(c, c->ptr, 4 * (nmaj + 1))) || (rc = ensure(c, c->ind, 4 * n)) || (rc = ensure(c, c->val, 8 * n)))
+        const bool buckets = bucket_takes(n, nmaj, nmin);
+        if ((rc = ensure(c, c->vals[0], 8 * n)) || (rc = ensure(c, c->stage64, 16 * n)) ||
+            (rc = ensure(c, c->ptr, 4 * (nmaj + 1))) || (rc = ensure(c, c->ind, 4 * n)) || (rc = ensure(c, c->val, 8 * n)) ||
+            (buckets && (rc = ensure(c, c->keys[0], bucket_scratch_bytes(n, nmaj)))))
             return rc;
         c->has_result = false;
         int64_t *dI = (int64_t *)c->stage64.p, *dJ = dI + n;
@@ -330,19 +388,38 @@ extern "C" int elfel_hip_sparse(elfel_hip_ctx *c, int64_t nrow, int64_t ncol, in
             HIPCHK(c, hipMemcpyAsync(dJ, col, 8 * n, hipMemcpyHostToDevice, c->stream));
             HIPCHK(c, hipMemcpyAsync(c->vals[0].p, val, 8 * n, hipMemcpyHostToDevice, c->stream));
         }
-        uint64_t *k0 = (uint64_t *)c->keys[0].p, *k1 = (uint64_t *)c->keys[1].p;
-        uint64_t *v0 = (uint64_t *)c->vals[0].p, *v1 = (uint64_t *)c->vals[1].p;
-        if ((rc = plain_coo_keys(c, dI, dJ, n, nrow, ncol, minor_bits, csc, k0))) return rc;
-        int flags = 0;
-        if ((rc = take_flags(c, &flags))) return rc;
-        if (flags & DERR_RANGE) return set_err(c, ELFEL_ERANGE, "row or column index out of range");
-        if ((rc = radix_sort_pairs(c, k0, v0, k1, v1, n, major_bits + minor_bits))) return rc;
-        if ((rc = build_csr_from_sorted(c, k0, (const double *)v0, n, minor_bits, nmaj, (int32_t *)c->ptr.p,
-                                        (int32_t *)c->ind.p, (double *)c->val.p, (int32_t *)c->dscal.p, true)))
-            return rc;
-        int32_t h = 0;
-        HIPCHK(c, hipMemcpyAsync(&h, c->dscal.p, 4, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
+        int64_t h = 0;
+        bool done = false;
+        if (buckets) {
+            int flags = 0;
+            bool toolong = false;
+            if ((rc = bucket_coo(c, c->keys[0].p, n, dI, dJ, (const double *)c->vals[0].p, nrow, ncol, csc,
+                                 (int32_t *)c->ptr.p, (int32_t *)c->ind.p, (double *)c->val.p, &flags, &toolong, &h)))
+                return rc;
+            if (flags) {
+                HIPCHK(c, hipMemsetAsync((int *)c->dscal.p + 1, 0, sizeof(int), c->stream));
+                if (flags & DERR_RANGE) return set_err(c, ELFEL_ERANGE, "row or column index out of range");
+            }
+            done = !toolong;
+        }
+        if (!done) {
+            if ((rc = ensure(c, c->keys[0], 8 * n)) || (rc = ensure(c, c->keys[1], 8 * n)) || (rc = ensure(c, c->vals[1], 8 * n)))
+                return rc;
+            uint64_t *k0 = (uint64_t *)c->keys[0].p, *k1 = (uint64_t *)c->keys[1].p;
+            uint64_t *v0 = (uint64_t *)c->vals[0].p, *v1 = (uint64_t *)c->vals[1].p;
+            if ((rc = plain_coo_keys(c, dI, dJ, n, nrow, ncol, minor_bits, csc, k0))) return rc;
+            int flags = 0;
+            if ((rc = take_flags(c, &flags))) return rc;
+            if (flags & DERR_RANGE) return set_err(c, ELFEL_ERANGE, "row or column index out of range");
+            if ((rc = radix_sort_pairs(c, k0, v0, k1, v1, n, major_bits + minor_bits))) return rc;
+            if ((rc = build_csr_from_sorted(c, k0, (const double *)v0, n, minor_bits, nmaj, (int32_t *)c->ptr.p,
+                                            (int32_t *)c->ind.p, (double *)c->val.p, (int32_t *)c->dscal.p, true)))
+                return rc;
+            int32_t h32 = 0;
+            HIPCHK(c, hipMemcpyAsync(&h32, c->dscal.p, 4, hipMemcpyDeviceToHost, c->stream));
+            HIPCHK(c, hipStreamSynchronize(c->stream));
+            h = h32;
+        }
         c->nnz = h;
         c->nrow = nrow; c->ncol = ncol; c->nmaj = nmaj; c->nmin = nmin; c->layout = layout;
         c->has_result = true;

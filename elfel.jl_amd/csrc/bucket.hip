@@ -1,0 +1,477 @@
+// bucket.hip -- COO -> CSR/CSC build by row buckets: the entries of each major
+// row brought together by one counting pass, then every row ordered, summed
+// and written by one workgroup out of LDS.
+//
+// The result is that of the stable sort of sort.hip (SparseArrays.sparse,
+// src/Assemblers.jl:121-123): within a row the entries are ordered by (minor
+// index, stream position), and each run of equal minor indices is summed left
+// to right.  Stream positions are distinct, so the order does not depend on
+// where the counting pass happened to put an entry, and every run gives the
+// same bits.
+//
+//   k_bk_zero     the row counts, the look-back states and the counters
+//   k_bk_count    entries per major row; each entry's place in its row
+//   k_bk_scan     exclusive scan of the counts (one pass, decoupled look-back),
+//                 and the first row of every tile of BK_TILE entries
+//   k_bk_scatter  (minor, stream position) of every entry into its row
+//   k_bk_tile     per tile: rank every entry within its row, find the runs,
+//                 sum them, and write the row pointers, indices and values at
+//                 the place that a second look-back over the tiles gives
+//
+// Bytes per entry (n entries, u of them distinct): the two indices twice (32),
+// its place written and read (8), the packed entry written and read (16), the
+// value (8, gathered), and 12 u/n of output -- against 40 a pass of the radix
+// sort and five to six passes.  Measured against it (whole calls): 1 045 458
+// entries of a T3 mesh on the device 249 -> 91 us, 4608 entries 148 -> 40 us.
+#include <algorithm>
+
+#include "common.h"
+
+#define BK_BLOCK 256
+#define BK_TB 512                   // work-items of a tile
+#define BK_ROWMAX 512               // longest row that a tile holds; a longer one goes to the sort
+#define BK_TILE 1536                // entries that start in a tile, its last row's overhang beyond
+#define BK_CAP (BK_TILE + BK_ROWMAX)
+#define BK_CAP_LOG2 11
+#define BK_ROUNDS (BK_CAP / BK_TB)
+#define BK_COUNT_ITEMS 2            // entries per work-item of the counting pass
+#define BK_HASH_LOG2 10             // its LDS slots, twice its entries
+#define BK_HASH (1 << BK_HASH_LOG2)
+#define BK_SCAN_ITEMS 16
+#define BK_SCAN_CHUNK (BK_BLOCK * BK_SCAN_ITEMS)
+
+static_assert(BK_CAP == 1 << BK_CAP_LOG2 && BK_CAP % BK_TB == 0, "a tile is a whole number of rounds");
+static_assert(BK_HASH >= 2 * BK_BLOCK * BK_COUNT_ITEMS, "the hash of the counting pass is at most half full");
+
+// ---- decoupled look-back -------------------------------------------------------
+// One 64-bit word per block of the scan: the upper half says whether the lower
+// holds nothing yet, the block's own total or the total up to and including
+// it.  Blocks take their numbers from a counter when they start, so every
+// block that one waits for has started and waits only for earlier ones: the
+// wait ends.  The word carries its own flag, so relaxed agent-scope accesses
+// are enough.
+enum { LB_EMPTY = 0, LB_TOTAL = 1, LB_PREFIX = 2 };
+
+__device__ __forceinline__ void lb_store(uint64_t *st, uint32_t flag, uint32_t v)
+{
+    __hip_atomic_store(st, ((uint64_t)flag << 32) | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ void lb_publish(uint64_t *st, uint32_t t, uint32_t total)
+{
+    lb_store(st + t, t == 0 ? LB_PREFIX : LB_TOTAL, total);
+}
+
+// The sum of the totals of blocks 0 .. t - 1, for one whole wave (the same in
+// every lane); publishes the inclusive sum of block t.
+__device__ __forceinline__ uint32_t lb_wait(uint64_t *st, uint32_t t, uint32_t total)
+{
+    const int lane = threadIdx.x & 63;
+    uint32_t run = 0;
+    for (int64_t hi = (int64_t)t - 1; hi >= 0; hi -= 64) {
+        const int64_t j = hi - lane;
+        uint64_t w;
+        uint64_t have_prefix;
+        do {
+            w = j >= 0 ? __hip_atomic_load(st + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : (uint64_t)LB_TOTAL << 32;
+            have_prefix = __ballot((uint32_t)(w >> 32) == LB_PREFIX);
+            const uint64_t empty = __ballot((uint32_t)(w >> 32) == LB_EMPTY);
+            // lanes nearer than the first inclusive sum must all hold something
+            const uint64_t need = have_prefix ? (have_prefix & (~have_prefix + 1)) - 1 : ~0ull;
+            if (!(empty & need)) break;
+            __builtin_amdgcn_s_sleep(1);
+        } while (true);
+        const int first = have_prefix ? __builtin_ctzll(have_prefix) : 63;
+        uint32_t v = lane <= first ? (uint32_t)w : 0u;
+        for (int d = 32; d > 0; d >>= 1) v += (uint32_t)__shfl_xor((int)v, d, 64);
+        run += v;
+        if (have_prefix) break;
+    }
+    if (t != 0 && lane == 0) lb_store(st + t, LB_PREFIX, run + total);
+    return run;
+}
+
+// ---- control words ---------------------------------------------------------------
+// BK_LONG: a row longer than BK_ROWMAX exists and the tiles do not hold it; the
+// kernels after the scan then leave every output alone.
+enum { BK_T_SCAN = 0, BK_T_TILE = 1, BK_LONG = 2, BK_NCTL = 4 };
+
+__global__ void k_bk_zero(uint4 *__restrict__ p, int64_t n4)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n4) p[i] = make_uint4(0, 0, 0, 0);
+}
+
+// ---- the stream -------------------------------------------------------------------
+struct CooSource {
+    const int64_t *row, *col;
+    int64_t nrow, ncol;
+    int csc;
+    __device__ __forceinline__ bool get(int64_t k, uint32_t &major, uint32_t &minor) const
+    {
+        const int64_t r = row[k], q = col[k];
+        const bool ok = r >= 1 && r <= nrow && q >= 1 && q <= ncol;
+        major = ok ? (uint32_t)(csc ? q - 1 : r - 1) : 0u;
+        minor = ok ? (uint32_t)(csc ? r - 1 : q - 1) : 0u;
+        return ok;
+    }
+};
+
+// Entries per row and every entry's place in its row.  One atomic per entry on
+// the rows' counters is bound by atomics to the same address (a million
+// entries of a T3 mesh 42 us, all in one row 11 ms), so a workgroup first
+// counts the rows of its entries in an LDS hash and then adds each distinct
+// row once.  512 entries a workgroup: 2048 took 56 against 43 us for six million
+// entries and 12 against 4 us for 4608, where the chain of hash probes of one
+// work-item is the time.
+__global__ __launch_bounds__(BK_BLOCK) void k_bk_count(CooSource src, int64_t n, uint32_t *__restrict__ cnt,
+                                                       uint32_t *__restrict__ place, int *__restrict__ err)
+{
+    __shared__ int32_t key[BK_HASH];
+    __shared__ uint32_t num[BK_HASH];
+    for (int i = threadIdx.x; i < BK_HASH; i += BK_BLOCK) {
+        key[i] = -1;
+        num[i] = 0;
+    }
+    __syncthreads();
+    const int64_t base = (int64_t)blockIdx.x * (BK_BLOCK * BK_COUNT_ITEMS);
+    uint32_t slot[BK_COUNT_ITEMS], loc[BK_COUNT_ITEMS];
+    bool bad = false;
+#pragma unroll
+    for (int q = 0; q < BK_COUNT_ITEMS; q++) {
+        const int64_t k = base + q * BK_BLOCK + threadIdx.x;
+        uint32_t major = 0, minor;
+        if (k < n && !src.get(k, major, minor)) bad = true;
+        slot[q] = major;
+    }
+#pragma unroll
+    for (int q = 0; q < BK_COUNT_ITEMS; q++) {
+        if (base + q * BK_BLOCK + threadIdx.x < n) {
+            const int32_t r = (int32_t)slot[q];
+            uint32_t s = ((uint32_t)r * 2654435761u) >> (32 - BK_HASH_LOG2);
+            while (true) {
+                const int32_t old = atomicCAS(&key[s], -1, r);
+                if (old == -1 || old == r) break;
+                s = (s + 1) & (BK_HASH - 1);
+            }
+            slot[q] = s;
+            loc[q] = atomicAdd(&num[s], 1u);
+        }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < BK_HASH; i += BK_BLOCK)
+        if (key[i] >= 0) num[i] = atomicAdd(&cnt[key[i]], num[i]);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < BK_COUNT_ITEMS; q++) {
+        const int64_t k = base + q * BK_BLOCK + threadIdx.x;
+        if (k < n) place[k] = num[slot[q]] + loc[q];
+    }
+    if (bad) atomicOr(err, DERR_RANGE);
+}
+
+// cnt[0 .. nmaj] (cnt[nmaj] = 0) -> the rows' first entries, and for every tile
+// t the first row that starts at or after t * BK_TILE with that start (tile
+// nt: nmaj and n).  A row's interval (s, s + len] holds the tile boundaries
+// that the next row is the first to reach.
+__global__ __launch_bounds__(BK_BLOCK) void k_bk_scan(uint32_t *__restrict__ cnt, int64_t nmaj, uint32_t n, uint32_t nt,
+                                                      uint32_t *__restrict__ trow, uint32_t *__restrict__ tstart,
+                                                      uint64_t *__restrict__ st, uint32_t *__restrict__ ctl)
+{
+    __shared__ uint32_t wsum[BK_BLOCK / 64], sh_b, sh_base;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    if (tid == 0) sh_b = atomicAdd(&ctl[BK_T_SCAN], 1u);
+    __syncthreads();
+    const uint32_t b = sh_b;
+    const int64_t r0 = (int64_t)b * BK_SCAN_CHUNK + tid * BK_SCAN_ITEMS;
+    uint32_t v[BK_SCAN_ITEMS], sum = 0, most = 0;
+#pragma unroll
+    for (int i = 0; i < BK_SCAN_ITEMS; i += 4) {
+        uint4 q = make_uint4(0, 0, 0, 0);
+        if (r0 + i + 3 <= nmaj) q = *(const uint4 *)(cnt + r0 + i);
+        else {
+            if (r0 + i <= nmaj) q.x = cnt[r0 + i];
+            if (r0 + i + 1 <= nmaj) q.y = cnt[r0 + i + 1];
+            if (r0 + i + 2 <= nmaj) q.z = cnt[r0 + i + 2];
+        }
+        v[i] = q.x; v[i + 1] = q.y; v[i + 2] = q.z; v[i + 3] = q.w;
+    }
+#pragma unroll
+    for (int i = 0; i < BK_SCAN_ITEMS; i++) {
+        sum += v[i];
+        most = max(most, v[i]);
+    }
+    uint32_t inc = sum;
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t o = (uint32_t)__shfl_up((int)inc, d, 64);
+        if (lane >= d) inc += o;
+    }
+    if (lane == 63) wsum[w] = inc;
+    __syncthreads();
+    uint32_t woff = 0, total = 0;
+    for (int k = 0; k < BK_BLOCK / 64; k++) {
+        if (k < w) woff += wsum[k];
+        total += wsum[k];
+    }
+    if (w == 0) {
+        if (lane == 0) lb_publish(st, b, total);
+        const uint32_t base = lb_wait(st, b, total);
+        if (lane == 0) sh_base = base;
+    }
+    __syncthreads();
+    uint32_t s = sh_base + woff + inc - sum;
+    if (most > BK_ROWMAX) ctl[BK_LONG] = 1u;
+#pragma unroll
+    for (int i = 0; i < BK_SCAN_ITEMS; i++) {
+        const uint32_t c = v[i];
+        v[i] = s;
+        for (uint32_t t = s / BK_TILE + 1; t <= (s + c) / BK_TILE; t++) {  // c = 0 past the last row
+            trow[t] = (uint32_t)(r0 + i + 1);
+            tstart[t] = s + c;
+        }
+        s += c;
+    }
+#pragma unroll
+    for (int i = 0; i < BK_SCAN_ITEMS; i += 4) {
+        if (r0 + i + 3 <= nmaj) *(uint4 *)(cnt + r0 + i) = make_uint4(v[i], v[i + 1], v[i + 2], v[i + 3]);
+        else {
+            if (r0 + i <= nmaj) cnt[r0 + i] = v[i];
+            if (r0 + i + 1 <= nmaj) cnt[r0 + i + 1] = v[i + 1];
+            if (r0 + i + 2 <= nmaj) cnt[r0 + i + 2] = v[i + 2];
+        }
+    }
+    if (b == 0 && tid == 0) {
+        trow[0] = 0;
+        tstart[0] = 0;
+        trow[nt] = (uint32_t)nmaj;
+        tstart[nt] = n;
+    }
+}
+
+// The entries of a row side by side, each packed with its row's first entry in
+// the bits above `bits` = minor bits + kbits (those that overflow drop out: a
+// tile spans fewer than 2^11 entries), its minor index and its stream position.
+__global__ __launch_bounds__(BK_BLOCK) void k_bk_scatter(CooSource src, int64_t n, const uint32_t *__restrict__ start,
+                                                         const uint32_t *__restrict__ place, int bits, int kbits,
+                                                         uint64_t *__restrict__ packed)
+{
+    const int64_t k = (int64_t)blockIdx.x * BK_BLOCK + threadIdx.x;
+    if (k >= n) return;
+    uint32_t major, minor;
+    src.get(k, major, minor);
+    const uint32_t s = start[major];
+    packed[(int64_t)s + place[k]] = ((uint64_t)s << bits) | ((uint64_t)minor << kbits) | (uint64_t)k;
+}
+
+// One workgroup per tile of whole rows, at most BK_CAP entries of rows of at
+// most BK_ROWMAX.  An entry less the tile's first entry (in the row field) is
+// (row begin, minor, stream position), so entries of a tile compare as plain
+// integers.  Each work-item counts, for four neighbouring entries at once, how
+// many entries of their rows are smaller: broadcast reads from LDS, for the 20
+// to 100 entries of a finite-element row as many steps as a sorting network
+// would take, without its exchanges.  512 work-items and 36 KiB of LDS fill a
+// CU with four workgroups; 256 work-items of the same tile left it half empty
+// (six million entries 137 against 83 us).
+__global__ __launch_bounds__(BK_TB) void k_bk_tile(const uint64_t *__restrict__ packed, const double *__restrict__ vals,
+                                                   const uint32_t *__restrict__ start, const uint32_t *__restrict__ trow,
+                                                   const uint32_t *__restrict__ tstart, uint32_t nt, int64_t nmaj,
+                                                   int bits, int kbits, uint64_t *__restrict__ st,
+                                                   uint32_t *__restrict__ ctl, const int *__restrict__ err,
+                                                   int32_t *__restrict__ ptr, int32_t *__restrict__ ind,
+                                                   double *__restrict__ out, int32_t *__restrict__ nnz_dev,
+                                                   int32_t *__restrict__ told)
+{
+    __shared__ __align__(16) uint64_t sk[BK_CAP + 4];  // the entries by row; then the values in sorted order
+    __shared__ uint64_t ss[BK_CAP];                    // the entries, sorted
+    __shared__ uint16_t se[BK_CAP + 1];                // end of a row, at its begin; then the runs before an entry
+    __shared__ uint64_t hm[BK_CAP / 64];               // one bit per entry that starts a run
+    __shared__ uint32_t sh_t, sh_base;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    // nothing is written when an index was out of range or a row is too long
+    // (the flags were set by earlier kernels: the same for every workgroup)
+    if (*err != 0 || ctl[BK_LONG] != 0) {
+        if (blockIdx.x == 0 && tid == 0) {
+            told[0] = 0;
+            told[1] = *err;
+            told[2] = (int32_t)ctl[BK_LONG];
+        }
+        return;
+    }
+    if (tid == 0) sh_t = atomicAdd(&ctl[BK_T_TILE], 1u);
+    __syncthreads();
+    const uint32_t t = sh_t;
+    const int64_t row0 = trow[t], row1 = trow[t + 1];
+    const uint32_t s0 = tstart[t];
+    const int m = (int)(tstart[t + 1] - s0);  // <= BK_CAP
+    const uint64_t rebase = (uint64_t)s0 << bits;
+    uint64_t kr[BK_ROUNDS];
+#pragma unroll
+    for (int q = 0; q < BK_ROUNDS; q++) {
+        const int p = q * BK_TB + tid;
+        kr[q] = p < m ? packed[(int64_t)s0 + p] - rebase : ~0ull;
+    }
+#pragma unroll
+    for (int q = 0; q < BK_ROUNDS; q++) sk[q * BK_TB + tid] = kr[q];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < BK_ROUNDS; q++) {
+        const int p = q * BK_TB + tid;
+        const uint32_t b = (uint32_t)(kr[q] >> bits);
+        if (p < m && (p == m - 1 || (uint32_t)(sk[p + 1] >> bits) != b)) se[b] = (uint16_t)(p + 1);
+    }
+    __syncthreads();
+    for (int p = 4 * tid; p < m; p += 4 * BK_TB) {
+        const uint64_t k0 = sk[p], k1 = sk[p + 1], k2 = sk[p + 2], k3 = sk[p + 3];  // past m: larger than any entry
+        const int last = min(p + 3, m - 1);
+        const int b = (int)(k0 >> bits), e = se[(uint32_t)(sk[last] >> bits)];
+        int c0 = b, c1 = b, c2 = b, c3 = b, j = b;
+        for (; j + 4 <= e; j += 4) {
+            const uint64_t o0 = sk[j], o1 = sk[j + 1], o2 = sk[j + 2], o3 = sk[j + 3];
+            c0 += (o0 < k0) + (o1 < k0) + (o2 < k0) + (o3 < k0);
+            c1 += (o0 < k1) + (o1 < k1) + (o2 < k1) + (o3 < k1);
+            c2 += (o0 < k2) + (o1 < k2) + (o2 < k2) + (o3 < k2);
+            c3 += (o0 < k3) + (o1 < k3) + (o2 < k3) + (o3 < k3);
+        }
+        for (; j < e; j++) {
+            const uint64_t o = sk[j];
+            c0 += o < k0;
+            c1 += o < k1;
+            c2 += o < k2;
+            c3 += o < k3;
+        }
+        ss[c0] = k0;
+        if (p + 1 < m) ss[c1] = k1;
+        if (p + 2 < m) ss[c2] = k2;
+        if (p + 3 < m) ss[c3] = k3;
+    }
+    __syncthreads();
+    // runs: entries that differ in more than the stream position start one
+    const uint64_t kmask = (1ull << kbits) - 1;
+    const uint32_t mmask = (uint32_t)((1ull << (bits - kbits)) - 1);
+    double vr[BK_ROUNDS];
+#pragma unroll
+    for (int q = 0; q < BK_ROUNDS; q++) {
+        const int p = q * BK_TB + tid;
+        kr[q] = p < m ? ss[p] : 0;
+        vr[q] = p < m ? vals[kr[q] & kmask] : 0.0;
+    }
+#pragma unroll
+    for (int q = 0; q < BK_ROUNDS; q++) {
+        const int p = q * BK_TB + tid;
+        const uint64_t h = __ballot(p < m && (p == 0 || (ss[p - 1] >> kbits) != (kr[q] >> kbits)));
+        if (lane == 0) hm[q * (BK_TB / 64) + w] = h;
+    }
+    __syncthreads();
+    // runs before each word of hm (every wave computes them, lanes as words)
+    static_assert(BK_CAP / 64 == 32, "one lane per word of the run mask, twice");
+    const uint32_t pc = (uint32_t)__popcll(hm[lane & 31]);
+    uint32_t inc = pc;
+#pragma unroll
+    for (int d = 1; d < 32; d <<= 1) {
+        const uint32_t o = (uint32_t)__shfl_up((int)inc, d, 32);
+        if ((lane & 31) >= d) inc += o;
+    }
+    const uint32_t total = (uint32_t)__shfl((int)inc, 31, 64);
+    if (tid == 0) lb_publish(st, t, total);
+    double *sv = (double *)sk;
+    uint32_t un[BK_ROUNDS];
+    const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+#pragma unroll
+    for (int q = 0; q < BK_ROUNDS; q++) {
+        const int p = q * BK_TB + tid, word = q * (BK_TB / 64) + w;
+        un[q] = (uint32_t)__shfl((int)(inc - pc), word, 64) + (uint32_t)__popcll(hm[word] & lt);
+        if (p < m) {
+            sv[p] = vr[q];
+            se[p] = (uint16_t)un[q];
+        }
+    }
+    if (tid == 0) se[m] = (uint16_t)total;
+    if (w == 0) {
+        const uint32_t base = lb_wait(st, t, total);
+        if (lane == 0) sh_base = base;
+    }
+    __syncthreads();
+    const uint32_t base = sh_base;
+#pragma unroll
+    for (int q = 0; q < BK_ROUNDS; q++) {
+        const int p = q * BK_TB + tid, word = q * (BK_TB / 64) + w;
+        if (p >= m || !((hm[word] >> lane) & 1)) continue;
+        // the next run's start, or the tile's end
+        const uint64_t above = lane == 63 ? 0ull : hm[word] >> (lane + 1);
+        int e = above ? p + 1 + __builtin_ctzll(above) : -1;
+        for (int x = word + 1; e < 0; x++) {
+            if (x * 64 >= m) e = m;
+            else if (hm[x]) e = x * 64 + __builtin_ctzll(hm[x]);
+        }
+        double acc = vr[q];
+        for (int j = p + 1; j < e; j++) acc += sv[j];
+        const int64_t u = (int64_t)base + un[q];
+        ind[u] = (int32_t)((uint32_t)(kr[q] >> kbits) & mmask);
+        out[u] = acc;
+    }
+    for (int64_t r = row0 + tid; r < row1; r += BK_TB) ptr[r] = (int32_t)(base + se[start[r] - s0]);
+    if (t == nt - 1 && tid == 0) {
+        const int32_t nnz = (int32_t)(base + total);
+        ptr[nmaj] = nnz;
+        *nnz_dev = nnz;
+        told[0] = nnz;
+        told[1] = 0;
+        told[2] = 0;
+    }
+}
+
+// ---- host -------------------------------------------------------------------------
+static int64_t bk_tiles(int64_t n) { return n / BK_TILE + 1; }
+static int64_t bk_scan_blocks(int64_t nmaj) { return ceil_div(nmaj + 1, BK_SCAN_CHUNK); }
+// words zeroed before a build: control words, the look-back states, the counts
+static int64_t bk_zero_words(int64_t n, int64_t nmaj)
+{
+    return (BK_NCTL + 2 * bk_scan_blocks(nmaj) + 2 * bk_tiles(n) + nmaj + 1 + 7) & ~(int64_t)3;
+}
+
+size_t bucket_scratch_bytes(int64_t n, int64_t nmaj)
+{
+    return 8 * (size_t)n + 4 * (size_t)n + 16 + 4 * (size_t)bk_zero_words(n, nmaj) + 8 * (size_t)(bk_tiles(n) + 1) + 64;
+}
+
+// Where the buckets apply: the counts are zeroed, scanned and read over all
+// rows, so a matrix of far more rows than entries keeps the sort; and a minor
+// index, a stream position and a place in a tile have to fit one 64-bit word.
+bool bucket_takes(int64_t n, int64_t nmaj, int64_t nmin)
+{
+    return n > 0 && n < INT32_MAX && nmaj <= 16 * n + 65536 && bits_for(nmin) + bits_for(n) + BK_CAP_LOG2 <= 64;
+}
+
+int bucket_coo(elfel_hip_ctx *c, void *scratch, int64_t n, const int64_t *row, const int64_t *col, const double *val,
+               int64_t nrow, int64_t ncol, int csc, int32_t *ptr, int32_t *ind, double *out, int *flags, bool *toolong,
+               int64_t *nnz)
+{
+    const int64_t nmaj = csc ? ncol : nrow, nt = bk_tiles(n), nsb = bk_scan_blocks(nmaj);
+    const CooSource src{row, col, nrow, ncol, csc};
+    uint64_t *packed = (uint64_t *)scratch;
+    uint32_t *ctl = (uint32_t *)(packed + n);
+    ctl += ((16 - ((uintptr_t)ctl & 15)) & 15) / 4;  // 16-byte words
+    uint64_t *st_scan = (uint64_t *)(ctl + BK_NCTL), *st_tile = st_scan + nsb;
+    uint32_t *cnt = (uint32_t *)(st_tile + nt);
+    cnt += ((16 - ((uintptr_t)cnt & 15)) & 15) / 4;
+    const int64_t zw = bk_zero_words(n, nmaj);
+    uint32_t *trow = ctl + zw, *tstart = trow + nt + 1, *place = tstart + nt + 1;
+    const int kbits = bits_for(n), bits = kbits + bits_for(csc ? nrow : ncol);
+    int *err = (int *)c->dscal.p + 1;
+    int32_t *told = (int32_t *)c->told;
+    hipLaunchKernelGGL(k_bk_zero, dim3(ceil_div(zw / 4, 256)), dim3(256), 0, c->stream, (uint4 *)ctl, zw / 4);
+    hipLaunchKernelGGL(k_bk_count, dim3(ceil_div(n, BK_BLOCK * BK_COUNT_ITEMS)), dim3(BK_BLOCK), 0, c->stream, src, n, cnt,
+                       place, err);
+    hipLaunchKernelGGL(k_bk_scan, dim3((unsigned)nsb), dim3(BK_BLOCK), 0, c->stream, cnt, nmaj, (uint32_t)n, (uint32_t)nt,
+                       trow, tstart, st_scan, ctl);
+    hipLaunchKernelGGL(k_bk_scatter, dim3(ceil_div(n, BK_BLOCK)), dim3(BK_BLOCK), 0, c->stream, src, n, cnt, place, bits, kbits,
+                       packed);
+    hipLaunchKernelGGL(k_bk_tile, dim3((unsigned)nt), dim3(BK_TB), 0, c->stream, packed, val, cnt, trow, tstart,
+                       (uint32_t)nt, nmaj, bits, kbits, st_tile, ctl, err, ptr, ind, out, (int32_t *)c->dscal.p, told);
+    HIPCHK(c, hipGetLastError());
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    *nnz = told[0];
+    *flags = told[1];
+    *toolong = told[2] != 0;
+    return 0;
+}

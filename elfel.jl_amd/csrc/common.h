@@ -186,6 +186,9 @@ struct elfel_hip_ctx {
     // of elements with det J <= 0 (byte 32)
     Buf dscal;
     Timing tm;
+    // pinned host words that a kernel leaves its counts in (entry count, error
+    // flags, rows too long): read after a wait, without a copy of their own
+    void *told = nullptr;
     // solver scratch: vectors, then the SELL-64 copy of the free block
     Buf pcg, pcg_sell;
     // batched problems (batch.hip)
@@ -302,6 +305,16 @@ int build_csr_from_sorted(elfel_hip_ctx *c, const uint64_t *keys, const double *
 // Sorted (row, value) pairs -> dense vector (rows without entries = 0).
 int build_dense_from_sorted(elfel_hip_ctx *c, const uint64_t *keys, const double *vals, int64_t n,
                             int64_t ndofs, double *out);
+
+// ---- bucket.hip ---------------------------------------------------------------
+// COO stream (device arrays, 1-based indices) -> CSR/CSC by row buckets; waits.
+// flags: the range errors found (nothing is written then); toolong: a row is
+// longer than the tiles hold (nothing is written: use the sort).
+bool bucket_takes(int64_t n, int64_t nmaj, int64_t nmin);
+size_t bucket_scratch_bytes(int64_t n, int64_t nmaj);
+int bucket_coo(elfel_hip_ctx *c, void *scratch, int64_t n, const int64_t *row, const int64_t *col, const double *val,
+               int64_t nrow, int64_t ncol, int csc, int32_t *ptr, int32_t *ind, double *out, int *flags, bool *toolong,
+               int64_t *nnz);
 
 // ---- plain.hip (FP64, unfused arithmetic) -------------------------------------
 int plain_assemble(elfel_hip_ctx *c, const elfel_hip_problem *pb, const QTable &tab, const Coef &cf);

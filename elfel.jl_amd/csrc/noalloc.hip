@@ -21,7 +21,8 @@ constexpr int64_t NMAX = ELFEL_NOALLOC_MAX_COO;
 constexpr size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 // the layout of the scratch: keys and values twice (the radix sort's
 // ping-pong), the digit histogram, the scan's block sums, the segment-head
-// flags and positions, and the entry count
+// flags and positions, and the entry count.  The row buckets lay their own
+// scratch over the whole of it.
 constexpr int64_t RS_TILE_KEYS = 4096;  // keys per radix tile (sort.hip)
 constexpr size_t B_KEYS = align256(8 * (size_t)NMAX);
 constexpr size_t B_HIST = align256(4 * (size_t)(256 * ((NMAX + RS_TILE_KEYS - 1) / RS_TILE_KEYS)));
@@ -102,6 +103,18 @@ extern "C" int elfel_hip_sparse_noalloc(elfel_hip_ctx *c, int64_t nrow, int64_t 
         s.n_cap = NMAX;
         int32_t *nnz_dev = (int32_t *)(base + O_NNZ);
         int rc;
+        // row buckets where their scratch fits in the array (up to some seven
+        // million rows at the largest n); the sort for the rest and for long rows
+        if (bucket_takes(n, nmaj, nmin) && bucket_scratch_bytes(n, nmaj) <= SCRATCH_BYTES) {
+            int bad = 0;
+            bool toolong = false;
+            if ((rc = bucket_coo(c, base, n, row, col, val, nrow, ncol, csc, ptr, ind, out, &bad, &toolong, nnz))) return rc;
+            if (bad) {
+                HIPCHK(c, hipMemsetAsync((int *)c->dscal.p + 1, 0, sizeof(int), c->stream));
+                if (bad & DERR_RANGE) return set_err(c, ELFEL_ERANGE, "row or column index out of range");
+            }
+            if (!toolong) return ELFEL_OK;
+        }
         if (n > 0) HIPCHK(c, hipMemcpyAsync(v0, val, 8 * (size_t)n, hipMemcpyDeviceToDevice, c->stream));
         if ((rc = plain_coo_keys(c, row, col, n, nrow, ncol, minor_bits, csc, k0))) return rc;
         // the range flags live in the context's device scalars (set at init)

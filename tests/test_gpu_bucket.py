@@ -1,0 +1,97 @@
+"""The row-bucket COO build (elfel_hip_sparse, elfel_hip_sparse_noalloc) at the
+edges of its tiles, against the oracle's sparse(): pattern and values bit for
+bit (tolerance 0, the same sums in the same order).  1536 entries start in a
+tile, rows of up to 512 are held, longer ones and matrices of far more rows
+than entries take the sort."""
+import numpy as np
+import pytest
+
+import oracle as O
+from elfel_hip import _lib as L
+from test_zz_no_alloc import Hip, _noalloc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def hip():
+    h = Hip()
+    yield h
+    h.free()
+
+
+def _rows(lengths, ncol, rng):
+    """A stream with the given entries per row, rows interleaved, columns repeating."""
+    I = rng.permutation(np.repeat(np.arange(1, len(lengths) + 1), lengths))
+    return I, rng.integers(1, ncol + 1, I.size)
+
+
+def _case(name, rng):
+    if name.startswith("n="):
+        n = int(name[2:])
+        return (*_rows(rng.multinomial(n, np.full(40, 1 / 40)), 23, rng), 40, 23)
+    if name.startswith("row="):  # one long row between short ones, and a tile that it straddles
+        k = int(name[4:])
+        return (*_rows([3] * 500 + [k] + [0] * 7 + [5] * 300, max(k // 2, 1), rng), 808, max(k // 2, 1))
+    if name == "long rows side by side":  # every tile at its largest
+        return (*_rows([511, 1024, 1, 512, 512, 512, 512, 511, 1][2:], 600, rng), 7, 600)
+    if name == "empty ends":
+        return (*_rows([0] * 9000 + [2] * 50 + [0] * 9000, 60, rng), 18050, 60)
+    if name == "one entry":
+        return np.array([7]), np.array([3]), 9, 4
+    if name == "one row":
+        return (*_rows([400], 1, rng), 1, 1)
+    if name == "two rows, all duplicates":
+        return (*_rows([300, 300], 1, rng), 2, 1)
+    if name == "more rows than entries":
+        return (*_rows([1] * 30 + [0] * 69970, 30, rng), 70000, 30)
+    if name == "last columns":  # indices next to the limit of int32
+        n = 3000
+        return rng.integers(1, 50, n), 2 ** 31 - 2 - rng.integers(0, 40, n), 50, 2 ** 31 - 2
+    raise ValueError(name)
+
+
+CASES = ["n=1535", "n=1536", "n=1537", "n=2048", "n=3072", "n=9001", "row=511", "row=512", "row=513", "row=1600",
+         "long rows side by side", "empty ends", "one entry", "one row", "two rows, all duplicates",
+         "more rows than entries", "last columns"]
+
+
+@pytest.mark.parametrize("csc", [False, True])
+@pytest.mark.parametrize("name", CASES)
+def test_bucket_build_equals_oracle(name, csc, ctx, hip):
+    rng = np.random.default_rng(5)
+    I, J, nrow, ncol = _case(name, rng)
+    I, J = I.astype(np.int64), J.astype(np.int64)
+    if csc:  # the cases describe the major rows
+        I, J, nrow, ncol = J, I, ncol, nrow
+    V = rng.standard_normal(I.size)
+    V[::7] = -0.0
+    V[3::31] = np.inf
+    if csc is False and nrow >= 2 ** 31 - 2:
+        pytest.skip("the oracle's pointers over 2^31 rows")
+    ref = O.sparse(I, J, V, nrow, ncol, csc=csc)
+    lay = L.CSC if csc else L.CSR
+    for _ in range(2):
+        nnz = ctx.sparse(I, J, V, nrow, ncol, layout=lay)
+        got = ctx.copy_sparse(base=0)[:3]
+        assert nnz == ref[0][-1]
+        for a, b in zip(got, ref):
+            assert np.array_equal(a, b, equal_nan=True) and np.array_equal(np.signbit(a), np.signbit(b)), name
+        got = _noalloc(ctx, hip, I, J, V, nrow, ncol, lay)
+        for a, b in zip(got[1:], ref):
+            assert np.array_equal(a, b, equal_nan=True), name
+
+
+def test_bucket_build_refuses_then_works(ctx):
+    rng = np.random.default_rng(6)
+    I, J = rng.integers(1, 31, 5000), rng.integers(1, 31, 5000)
+    V = rng.standard_normal(5000)
+    for bad in (0, 31, -5, 2 ** 40):
+        K = J.copy()
+        K[4321] = bad
+        with pytest.raises(L.ElfelRangeError):
+            ctx.sparse(I, K, V, 30, 30, layout=L.CSR)
+    ctx.sparse(I, J, V, 30, 30, layout=L.CSR)
+    ref = O.sparse(I, J, V, 30, 30, csc=False)
+    for a, b in zip(ctx.copy_sparse(base=0)[:3], ref):
+        assert np.array_equal(a, b)
