@@ -441,6 +441,11 @@ __global__ void k_i32_to_i64(const int32_t *__restrict__ s, int64_t *__restrict_
 static int fetch_nnz(elfel_hip_ctx *c)
 {
     if (c->nnz >= 0) return 0;
+    if (c->nnz_told) {  // the kernel leaves it in pinned memory
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        c->nnz = ((const int32_t *)c->told)[0];
+        return 0;
+    }
     int32_t h = 0;
     HIPCHK(c, hipMemcpyAsync(&h, c->dscal.p, 4, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -712,6 +717,7 @@ extern "C" int elfel_hip_assemble(elfel_hip_ctx *c, const elfel_hip_problem *pb,
             }
         }
         c->has_result = false;
+        c->nnz_told = false;
         c->used_method = pb->method;
         c->used_precision = pb->precision;
         c->used_note.clear();

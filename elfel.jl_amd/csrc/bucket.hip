@@ -103,6 +103,7 @@ __global__ void k_bk_zero(uint4 *__restrict__ p, int64_t n4)
 }
 
 // ---- the stream -------------------------------------------------------------------
+// A COO stream: every entry is an item of the counting pass, one entry wide.
 struct CooSource {
     const int64_t *row, *col;
     int64_t nrow, ncol;
@@ -115,16 +116,38 @@ struct CooSource {
         minor = ok ? (uint32_t)(csc ? r - 1 : q - 1) : 0u;
         return ok;
     }
+    __device__ __forceinline__ bool item(int64_t k, uint32_t &major, uint32_t &wide) const
+    {
+        uint32_t minor;
+        wide = 1;
+        return get(k, major, minor);
+    }
 };
 
-// Entries per row and every entry's place in its row.  One atomic per entry on
+// The stream of an element loop: a local dof of an element is one item, as wide
+// as its row of the element block.
+template <int ND>
+struct FormSource {
+    const int32_t *edof;
+    uint32_t wide[2];  // entries of the first `nfull` local rows, and of the others
+    int nfull;
+    __device__ __forceinline__ bool item(int64_t k, uint32_t &major, uint32_t &w) const
+    {
+        major = (uint32_t)edof[k];
+        w = (int)((uint32_t)k % ND) < nfull ? wide[0] : wide[1];
+        return true;
+    }
+};
+
+// Entries per row and every item's place in its row (n items).  One atomic per entry on
 // the rows' counters is bound by atomics to the same address (a million
 // entries of a T3 mesh 42 us, all in one row 11 ms), so a workgroup first
 // counts the rows of its entries in an LDS hash and then adds each distinct
 // row once.  512 entries a workgroup: 2048 took 56 against 43 us for six million
 // entries and 12 against 4 us for 4608, where the chain of hash probes of one
 // work-item is the time.
-__global__ __launch_bounds__(BK_BLOCK) void k_bk_count(CooSource src, int64_t n, uint32_t *__restrict__ cnt,
+template <typename Source>
+__global__ __launch_bounds__(BK_BLOCK) void k_bk_count(Source src, int64_t n, uint32_t *__restrict__ cnt,
                                                        uint32_t *__restrict__ place, int *__restrict__ err)
 {
     __shared__ int32_t key[BK_HASH];
@@ -135,13 +158,14 @@ __global__ __launch_bounds__(BK_BLOCK) void k_bk_count(CooSource src, int64_t n,
     }
     __syncthreads();
     const int64_t base = (int64_t)blockIdx.x * (BK_BLOCK * BK_COUNT_ITEMS);
-    uint32_t slot[BK_COUNT_ITEMS], loc[BK_COUNT_ITEMS];
+    uint32_t slot[BK_COUNT_ITEMS], loc[BK_COUNT_ITEMS], wide[BK_COUNT_ITEMS];
     bool bad = false;
 #pragma unroll
     for (int q = 0; q < BK_COUNT_ITEMS; q++) {
         const int64_t k = base + q * BK_BLOCK + threadIdx.x;
-        uint32_t major = 0, minor;
-        if (k < n && !src.get(k, major, minor)) bad = true;
+        uint32_t major = 0;
+        wide[q] = 0;
+        if (k < n && !src.item(k, major, wide[q])) bad = true;
         slot[q] = major;
     }
 #pragma unroll
@@ -155,7 +179,7 @@ __global__ __launch_bounds__(BK_BLOCK) void k_bk_count(CooSource src, int64_t n,
                 s = (s + 1) & (BK_HASH - 1);
             }
             slot[q] = s;
-            loc[q] = atomicAdd(&num[s], 1u);
+            loc[q] = atomicAdd(&num[s], wide[q]);
         }
     }
     __syncthreads();
@@ -263,6 +287,24 @@ __global__ __launch_bounds__(BK_BLOCK) void k_bk_scatter(CooSource src, int64_t 
     packed[(int64_t)s + place[k]] = ((uint64_t)s << bits) | ((uint64_t)minor << kbits) | (uint64_t)k;
 }
 
+// The same for the stream of an element loop: work-item x is the entry of local
+// row a and local column b of an element.
+template <int ND>
+__global__ __launch_bounds__(BK_BLOCK) void k_bk_scatter_form(FormMap map, int64_t n2, const int32_t *__restrict__ edof,
+                                                              const uint32_t *__restrict__ start,
+                                                              const uint32_t *__restrict__ place, int bits, int kbits,
+                                                              uint64_t *__restrict__ packed)
+{
+    const int64_t x = (int64_t)blockIdx.x * BK_BLOCK + threadIdx.x;
+    if (x >= n2) return;
+    const int64_t ea = x / ND, e = ea / ND;
+    const int b = (int)(x - ea * ND), a = (int)(ea - e * ND);
+    if (b >= map.ncol[a]) return;
+    const uint32_t s = start[edof[ea]];
+    const uint64_t k = (uint64_t)(e * map.nmat + map.pos[a * ND + b]);
+    packed[(int64_t)s + place[ea] + b] = ((uint64_t)s << bits) | ((uint64_t)(uint32_t)edof[e * ND + b] << kbits) | k;
+}
+
 // One workgroup per tile of whole rows, at most BK_CAP entries of rows of at
 // most BK_ROWMAX.  An entry less the tile's first entry (in the row field) is
 // (row begin, minor, stream position), so entries of a tile compare as plain
@@ -272,14 +314,19 @@ __global__ __launch_bounds__(BK_BLOCK) void k_bk_scatter(CooSource src, int64_t 
 // would take, without its exchanges.  512 work-items and 36 KiB of LDS fill a
 // CU with four workgroups; 256 work-items of the same tile left it half empty
 // (six million entries 137 against 83 us).
+//
+// SUM: the values and (LOAD) the load vector; else the sort order.  LOAD: the
+// load-vector entries of a dof are those of the (element, local dof) pairs on
+// the diagonal of its row, which the run of the diagonal holds in stream
+// order.
+template <bool SUM, bool LOAD>
 __global__ __launch_bounds__(BK_TB) void k_bk_tile(const uint64_t *__restrict__ packed, const double *__restrict__ vals,
+                                                   const double *__restrict__ fvals, uint32_t nd,
                                                    const uint32_t *__restrict__ start, const uint32_t *__restrict__ trow,
                                                    const uint32_t *__restrict__ tstart, uint32_t nt, int64_t nmaj,
                                                    int bits, int kbits, uint64_t *__restrict__ st,
-                                                   uint32_t *__restrict__ ctl, const int *__restrict__ err,
-                                                   int32_t *__restrict__ ptr, int32_t *__restrict__ ind,
-                                                   double *__restrict__ out, int32_t *__restrict__ nnz_dev,
-                                                   int32_t *__restrict__ told)
+                                                   uint32_t *__restrict__ ctl, const int *__restrict__ err, BucketOut o,
+                                                   int32_t *__restrict__ nnz_dev, int32_t *__restrict__ told)
 {
     __shared__ __align__(16) uint64_t sk[BK_CAP + 4];  // the entries by row; then the values in sorted order
     __shared__ uint64_t ss[BK_CAP];                    // the entries, sorted
@@ -353,7 +400,8 @@ __global__ __launch_bounds__(BK_TB) void k_bk_tile(const uint64_t *__restrict__ 
     for (int q = 0; q < BK_ROUNDS; q++) {
         const int p = q * BK_TB + tid;
         kr[q] = p < m ? ss[p] : 0;
-        vr[q] = p < m ? vals[kr[q] & kmask] : 0.0;
+        if constexpr (SUM) vr[q] = p < m ? vals[kr[q] & kmask] : 0.0;
+        else if (p < m) o.perm[(int64_t)s0 + p] = (int32_t)(kr[q] & kmask);
     }
 #pragma unroll
     for (int q = 0; q < BK_ROUNDS; q++) {
@@ -381,7 +429,7 @@ __global__ __launch_bounds__(BK_TB) void k_bk_tile(const uint64_t *__restrict__ 
         const int p = q * BK_TB + tid, word = q * (BK_TB / 64) + w;
         un[q] = (uint32_t)__shfl((int)(inc - pc), word, 64) + (uint32_t)__popcll(hm[word] & lt);
         if (p < m) {
-            sv[p] = vr[q];
+            if constexpr (SUM) sv[p] = vr[q];
             se[p] = (uint16_t)un[q];
         }
     }
@@ -396,6 +444,12 @@ __global__ __launch_bounds__(BK_TB) void k_bk_tile(const uint64_t *__restrict__ 
     for (int q = 0; q < BK_ROUNDS; q++) {
         const int p = q * BK_TB + tid, word = q * (BK_TB / 64) + w;
         if (p >= m || !((hm[word] >> lane) & 1)) continue;
+        const int64_t u = (int64_t)base + un[q];
+        o.ind[u] = (int32_t)((uint32_t)(kr[q] >> kbits) & mmask);
+        if constexpr (!SUM) {
+            o.seg[u] = (int32_t)(s0 + p);
+            continue;
+        }
         // the next run's start, or the tile's end
         const uint64_t above = lane == 63 ? 0ull : hm[word] >> (lane + 1);
         int e = above ? p + 1 + __builtin_ctzll(above) : -1;
@@ -405,14 +459,44 @@ __global__ __launch_bounds__(BK_TB) void k_bk_tile(const uint64_t *__restrict__ 
         }
         double acc = vr[q];
         for (int j = p + 1; j < e; j++) acc += sv[j];
-        const int64_t u = (int64_t)base + un[q];
-        ind[u] = (int32_t)((uint32_t)(kr[q] >> kbits) & mmask);
-        out[u] = acc;
+        o.val[u] = acc;
     }
-    for (int64_t r = row0 + tid; r < row1; r += BK_TB) ptr[r] = (int32_t)(base + se[start[r] - s0]);
+    for (int64_t r = row0 + tid; r < row1; r += BK_TB) {
+        const int b = (int)(start[r] - s0);
+        o.ptr[r] = (int32_t)(base + se[b]);
+        if constexpr (LOAD) {
+            int lo = b, hi = (int)(start[r + 1] - s0);
+            const int e = hi;
+            const uint64_t diag = ((uint64_t)b << bits) | ((uint64_t)r << kbits);
+            while (lo < hi) {
+                const int mid = (lo + hi) >> 1;
+                if (ss[mid] < diag) lo = mid + 1;
+                else hi = mid;
+            }
+            double acc = 0.0;
+            int cnt = 0;
+            if constexpr (!SUM) o.fbeg[r] = (int32_t)(start[r] / nd);
+            for (int p = lo; p < e && ((ss[p] ^ diag) >> kbits) == 0; p++) {
+                const uint32_t k = (uint32_t)(ss[p] & kmask), el = k / (nd * nd), ab = k - el * (nd * nd), a = ab / nd;
+                if (ab - a * nd != a) continue;  // two local dofs of an element with one number
+                if constexpr (SUM) {
+                    const double x = fvals[(int64_t)el * nd + a];
+                    acc = cnt == 0 ? x : acc + x;
+                } else {
+                    o.fperm[start[r] / nd + cnt] = (int32_t)(el * nd + a);
+                }
+                cnt++;
+            }
+            if constexpr (SUM) o.F[r] = cnt ? 0.0 + acc : 0.0;  // start! zeros the vector, assemble! adds
+        }
+    }
     if (t == nt - 1 && tid == 0) {
         const int32_t nnz = (int32_t)(base + total);
-        ptr[nmaj] = nnz;
+        o.ptr[nmaj] = nnz;
+        if constexpr (!SUM) {
+            o.seg[nnz] = (int32_t)start[nmaj];
+            if constexpr (LOAD) o.fbeg[nmaj] = (int32_t)(start[nmaj] / nd);
+        }
         *nnz_dev = nnz;
         told[0] = nnz;
         told[1] = 0;
@@ -429,9 +513,44 @@ static int64_t bk_zero_words(int64_t n, int64_t nmaj)
     return (BK_NCTL + 2 * bk_scan_blocks(nmaj) + 2 * bk_tiles(n) + nmaj + 1 + 7) & ~(int64_t)3;
 }
 
-size_t bucket_scratch_bytes(int64_t n, int64_t nmaj)
+// The scratch: the packed entries, what is zeroed (control words, look-back
+// states, row counts), the tiles' first rows and entries, the items' places.
+namespace {
+struct Scratch {
+    uint64_t *packed, *st_scan, *st_tile;
+    uint32_t *ctl, *cnt, *trow, *tstart, *place;
+    int64_t zero_words, nt, nsb;
+};
+}  // namespace
+
+static size_t scratch_bytes(int64_t n, int64_t items, int64_t nmaj)
 {
-    return 8 * (size_t)n + 4 * (size_t)n + 16 + 4 * (size_t)bk_zero_words(n, nmaj) + 8 * (size_t)(bk_tiles(n) + 1) + 64;
+    return 8 * (size_t)n + 4 * (size_t)items + 4 * (size_t)bk_zero_words(n, nmaj) + 8 * (size_t)(bk_tiles(n) + 1) + 80;
+}
+
+static Scratch scratch_layout(void *p, int64_t n, int64_t nmaj)
+{
+    Scratch S;
+    S.nt = bk_tiles(n);
+    S.nsb = bk_scan_blocks(nmaj);
+    S.packed = (uint64_t *)p;
+    S.ctl = (uint32_t *)(S.packed + n);
+    S.ctl += ((16 - ((uintptr_t)S.ctl & 15)) & 15) / 4;  // 16-byte words
+    S.st_scan = (uint64_t *)(S.ctl + BK_NCTL);
+    S.st_tile = S.st_scan + S.nsb;
+    S.cnt = (uint32_t *)(S.st_tile + S.nt);
+    S.cnt += ((16 - ((uintptr_t)S.cnt & 15)) & 15) / 4;
+    S.zero_words = bk_zero_words(n, nmaj);
+    S.trow = S.ctl + S.zero_words;
+    S.tstart = S.trow + S.nt + 1;
+    S.place = S.tstart + S.nt + 1;
+    return S;
+}
+
+size_t bucket_scratch_bytes(int64_t n, int64_t nmaj) { return scratch_bytes(n, n, nmaj); }
+size_t bucket_form_bytes(const FormMap &m, int64_t E, int64_t ndofs)
+{
+    return scratch_bytes(E * m.nmat, E * m.nd, ndofs);
 }
 
 // Where the buckets apply: the counts are zeroed, scanned and read over all
@@ -441,37 +560,157 @@ bool bucket_takes(int64_t n, int64_t nmaj, int64_t nmin)
 {
     return n > 0 && n < INT32_MAX && nmaj <= 16 * n + 65536 && bits_for(nmin) + bits_for(n) + BK_CAP_LOG2 <= 64;
 }
+bool bucket_form_takes(const FormMap &m, int64_t E, int64_t ndofs)
+{
+    return E * m.nd < INT32_MAX && bucket_takes(E * m.nmat, ndofs, ndofs);
+}
+
+static void launch_zero_scan(elfel_hip_ctx *c, const Scratch &S, bool zero, int64_t n, int64_t nmaj)
+{
+    if (zero)
+        hipLaunchKernelGGL(k_bk_zero, dim3(ceil_div(S.zero_words / 4, 256)), dim3(256), 0, c->stream, (uint4 *)S.ctl,
+                           S.zero_words / 4);
+    else
+        hipLaunchKernelGGL(k_bk_scan, dim3((unsigned)S.nsb), dim3(BK_BLOCK), 0, c->stream, S.cnt, nmaj, (uint32_t)n,
+                           (uint32_t)S.nt, S.trow, S.tstart, S.st_scan, S.ctl);
+}
 
 int bucket_coo(elfel_hip_ctx *c, void *scratch, int64_t n, const int64_t *row, const int64_t *col, const double *val,
                int64_t nrow, int64_t ncol, int csc, int32_t *ptr, int32_t *ind, double *out, int *flags, bool *toolong,
                int64_t *nnz)
 {
-    const int64_t nmaj = csc ? ncol : nrow, nt = bk_tiles(n), nsb = bk_scan_blocks(nmaj);
+    const int64_t nmaj = csc ? ncol : nrow;
+    const Scratch S = scratch_layout(scratch, n, nmaj);
     const CooSource src{row, col, nrow, ncol, csc};
-    uint64_t *packed = (uint64_t *)scratch;
-    uint32_t *ctl = (uint32_t *)(packed + n);
-    ctl += ((16 - ((uintptr_t)ctl & 15)) & 15) / 4;  // 16-byte words
-    uint64_t *st_scan = (uint64_t *)(ctl + BK_NCTL), *st_tile = st_scan + nsb;
-    uint32_t *cnt = (uint32_t *)(st_tile + nt);
-    cnt += ((16 - ((uintptr_t)cnt & 15)) & 15) / 4;
-    const int64_t zw = bk_zero_words(n, nmaj);
-    uint32_t *trow = ctl + zw, *tstart = trow + nt + 1, *place = tstart + nt + 1;
     const int kbits = bits_for(n), bits = kbits + bits_for(csc ? nrow : ncol);
     int *err = (int *)c->dscal.p + 1;
-    int32_t *told = (int32_t *)c->told;
-    hipLaunchKernelGGL(k_bk_zero, dim3(ceil_div(zw / 4, 256)), dim3(256), 0, c->stream, (uint4 *)ctl, zw / 4);
-    hipLaunchKernelGGL(k_bk_count, dim3(ceil_div(n, BK_BLOCK * BK_COUNT_ITEMS)), dim3(BK_BLOCK), 0, c->stream, src, n, cnt,
-                       place, err);
-    hipLaunchKernelGGL(k_bk_scan, dim3((unsigned)nsb), dim3(BK_BLOCK), 0, c->stream, cnt, nmaj, (uint32_t)n, (uint32_t)nt,
-                       trow, tstart, st_scan, ctl);
-    hipLaunchKernelGGL(k_bk_scatter, dim3(ceil_div(n, BK_BLOCK)), dim3(BK_BLOCK), 0, c->stream, src, n, cnt, place, bits, kbits,
-                       packed);
-    hipLaunchKernelGGL(k_bk_tile, dim3((unsigned)nt), dim3(BK_TB), 0, c->stream, packed, val, cnt, trow, tstart,
-                       (uint32_t)nt, nmaj, bits, kbits, st_tile, ctl, err, ptr, ind, out, (int32_t *)c->dscal.p, told);
+    int32_t *told = (int32_t *)c->told + 4;  // words 0-3: the context's result
+    const BucketOut o{ptr, ind, out, nullptr, nullptr, nullptr, nullptr, nullptr};
+    launch_zero_scan(c, S, true, n, nmaj);
+    hipLaunchKernelGGL(k_bk_count<CooSource>, dim3(ceil_div(n, BK_BLOCK * BK_COUNT_ITEMS)), dim3(BK_BLOCK), 0, c->stream,
+                       src, n, S.cnt, S.place, err);
+    launch_zero_scan(c, S, false, n, nmaj);
+    hipLaunchKernelGGL(k_bk_scatter, dim3(ceil_div(n, BK_BLOCK)), dim3(BK_BLOCK), 0, c->stream, src, n, S.cnt, S.place,
+                       bits, kbits, S.packed);
+    hipLaunchKernelGGL((k_bk_tile<true, false>), dim3((unsigned)S.nt), dim3(BK_TB), 0, c->stream, S.packed, val,
+                       (const double *)nullptr, 1u, S.cnt, S.trow, S.tstart, (uint32_t)S.nt, nmaj, bits, kbits, S.st_tile,
+                       S.ctl, err, o, (int32_t *)c->dscal.p + 2, told);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipStreamSynchronize(c->stream));
     *nnz = told[0];
     *flags = told[1];
     *toolong = told[2] != 0;
+    return 0;
+}
+
+// ---- the stream of an element loop ------------------------------------------------
+void form_square(FormMap &m, int nd, int csc)
+{
+    m.nd = nd;
+    m.nmat = nd * nd;
+    for (int a = 0; a < nd; a++) {
+        m.ncol[a] = (uint8_t)nd;
+        for (int b = 0; b < nd; b++) m.pos[a * nd + b] = (int16_t)(csc ? b + nd * a : a + nd * b);
+    }
+}
+
+struct DofTables {
+    const int32_t *conn[2], *dof[2], *edof[2];
+    int nen[2], ncomp[2], encomp[2];
+};
+
+__global__ __launch_bounds__(256) void k_form_dofs(FormMap m, DofTables T, int64_t n, int32_t *__restrict__ edof)
+{
+    const int64_t x = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (x >= n) return;
+    const int64_t e = x / m.nd;
+    const FormMap::Src s = m.src[x - e * m.nd];
+    edof[x] = s.cell ? T.edof[s.field][e * T.encomp[s.field] + s.comp]
+                     : T.dof[s.field][(int64_t)T.conn[s.field][e * T.nen[s.field] + s.node] * T.ncomp[s.field] + s.comp];
+}
+
+int form_dofs(elfel_hip_ctx *c, const FormMap &m, int32_t *edof)
+{
+    DofTables T;
+    for (int f = 0; f < 2; f++) {
+        const Field &F = c->f[f];
+        T.conn[f] = (const int32_t *)F.conn.p;
+        T.dof[f] = (const int32_t *)F.dof.p;
+        T.edof[f] = (const int32_t *)F.edof.p;
+        T.nen[f] = F.nen;
+        T.ncomp[f] = F.ncomp;
+        T.encomp[f] = F.edof_ncomp;
+    }
+    const int64_t n = c->f[0].E * m.nd;
+    if (n == 0) return 0;
+    hipLaunchKernelGGL(k_form_dofs, dim3(ceil_div(n, 256)), dim3(256), 0, c->stream, m, T, n, edof);
+    HIPCHK(c, hipGetLastError());
+    return 0;
+}
+
+__global__ __launch_bounds__(256) void k_form_keys(FormMap m, int64_t n2, const int32_t *__restrict__ edof, int minor_bits,
+                                                   uint64_t *__restrict__ keys, uint64_t *__restrict__ fkeys)
+{
+    const int64_t x = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (x >= n2) return;
+    const int64_t ea = x / m.nd, e = ea / m.nd;
+    const int b = (int)(x - ea * m.nd), a = (int)(ea - e * m.nd);
+    const uint32_t major = (uint32_t)edof[ea];
+    if (b < m.ncol[a])
+        keys[e * m.nmat + m.pos[a * m.nd + b]] = ((uint64_t)major << minor_bits) | (uint64_t)(uint32_t)edof[e * m.nd + b];
+    if (fkeys && b == 0) fkeys[ea] = (uint64_t)major;
+}
+
+int form_keys(elfel_hip_ctx *c, const FormMap &m, int64_t E, const int32_t *edof, int minor_bits, uint64_t *keys,
+              uint64_t *fkeys)
+{
+    const int64_t n2 = E * m.nd * m.nd;
+    if (n2 == 0) return 0;
+    hipLaunchKernelGGL(k_form_keys, dim3((unsigned)((n2 + 255) / 256)), dim3(256), 0, c->stream, m, n2, edof, minor_bits,
+                       keys, fkeys);
+    HIPCHK(c, hipGetLastError());
+    return 0;
+}
+
+template <int ND>
+static void launch_form(elfel_hip_ctx *c, const Scratch &S, const FormMap &m, int64_t E, const int32_t *edof,
+                        int64_t ndofs, int bits, int kbits)
+{
+    FormSource<ND> src{edof, {m.ncol[0], m.ncol[ND - 1]}, ND};
+    for (int a = ND - 1; a > 0 && m.ncol[a] != m.ncol[0]; a--) src.nfull = a;
+    const int64_t items = E * ND, n2 = items * ND;
+    launch_zero_scan(c, S, true, E * m.nmat, ndofs);
+    hipLaunchKernelGGL(k_bk_count<FormSource<ND>>, dim3(ceil_div(items, BK_BLOCK * BK_COUNT_ITEMS)), dim3(BK_BLOCK), 0,
+                       c->stream, src, items, S.cnt, S.place, (int *)c->dscal.p + 1);
+    launch_zero_scan(c, S, false, E * m.nmat, ndofs);
+    hipLaunchKernelGGL(k_bk_scatter_form<ND>, dim3((unsigned)((n2 + BK_BLOCK - 1) / BK_BLOCK)), dim3(BK_BLOCK), 0,
+                       c->stream, m, n2, edof, S.cnt, S.place, bits, kbits, S.packed);
+}
+
+int bucket_form(elfel_hip_ctx *c, void *scratch, const FormMap &m, int64_t E, const int32_t *edof, int64_t ndofs,
+                const double *vals, const double *fvals, const BucketOut &o)
+{
+    const int64_t n = E * m.nmat;
+    const Scratch S = scratch_layout(scratch, n, ndofs);
+    const int kbits = bits_for(n), bits = kbits + bits_for(ndofs);
+    hipEvent_t ev = nullptr;
+    tm_begin(c, ELFEL_PH_SORT, &ev);
+    switch (m.nd) {
+#define F(N) case N: launch_form<N>(c, S, m, E, edof, ndofs, bits, kbits); break
+        F(2); F(3); F(4); F(6); F(8); F(9); F(11); F(12); F(15);
+#undef F
+    default: return set_err(c, ELFEL_ENOTSUP, "internal: element dof count without a bucket kernel");
+    }
+    HIPCHK(c, hipGetLastError());
+    tm_end(c, ELFEL_PH_SORT, ev);
+    tm_begin(c, ELFEL_PH_REDUCE, &ev);
+    const bool sum = vals != nullptr, load = m.nvec > 0;
+    auto kern = sum ? (load ? k_bk_tile<true, true> : k_bk_tile<true, false>)
+                    : (load ? k_bk_tile<false, true> : k_bk_tile<false, false>);
+    hipLaunchKernelGGL(kern, dim3((unsigned)S.nt), dim3(BK_TB), 0, c->stream, S.packed, vals, fvals, (uint32_t)m.nd, S.cnt,
+                       S.trow, S.tstart, (uint32_t)S.nt, ndofs, bits, kbits, S.st_tile, S.ctl, (int *)c->dscal.p + 1, o,
+                       (int32_t *)c->dscal.p, (int32_t *)c->told);
+    HIPCHK(c, hipGetLastError());
+    tm_end(c, ELFEL_PH_REDUCE, ev);
     return 0;
 }

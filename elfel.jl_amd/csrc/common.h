@@ -189,6 +189,15 @@ struct elfel_hip_ctx {
     // pinned host words that a kernel leaves its counts in (entry count, error
     // flags, rows too long): read after a wait, without a copy of their own
     void *told = nullptr;
+    bool nnz_told = false;        // nnz is -1 and will be in told[0] after a wait
+    // whether the rows of a problem's matrix fit the buckets' tiles: known after
+    // the first assembly on a mesh, dof map and weak form
+    struct {
+        bool valid = false, toolong = false;
+        int kind = -1, fe = -1, fe_p = -1;
+        int64_t ndofs = 0;
+        uint64_t key[6] = {0, 0, 0, 0, 0, 0};
+    } rows;
     // solver scratch: vectors, then the SELL-64 copy of the free block
     Buf pcg, pcg_sell;
     // batched problems (batch.hip)
@@ -307,6 +316,44 @@ int build_dense_from_sorted(elfel_hip_ctx *c, const uint64_t *keys, const double
                             int64_t ndofs, double *out);
 
 // ---- bucket.hip ---------------------------------------------------------------
+// The COO stream of an element loop, described instead of stored: `nd` dofs an
+// element, `nmat` entries an element in stream order; the entry of local major
+// index a and local minor index b is number pos[a * nd + b] of its element,
+// for b < ncol[a].  Where a local dof's number comes from: src[i] of the dof
+// table of field f (node k or the cell, component c).  nvec: load-vector
+// entries an element (nd, in the order of the dofs) or 0.
+#define FORM_MAXND 15
+struct FormMap {
+    struct Src { uint8_t field, cell, node, comp; };
+    int nd = 0, nmat = 0, nvec = 0;
+    Src src[FORM_MAXND];
+    uint8_t ncol[FORM_MAXND];
+    int16_t pos[FORM_MAXND * FORM_MAXND];
+};
+// a full nd x nd block, column-major (the entry of row i and column j is i + nd j)
+void form_square(FormMap &m, int nd, int csc);
+// The dofs of every element, edof[e * nd + i].
+int form_dofs(elfel_hip_ctx *c, const FormMap &m, int32_t *edof);
+// The stream's sort keys (major << minor_bits | minor) and, where fkeys is not
+// null, the load vector's.
+int form_keys(elfel_hip_ctx *c, const FormMap &m, int64_t E, const int32_t *edof, int minor_bits, uint64_t *keys,
+              uint64_t *fkeys);
+// What the tiles write: the matrix; its values and the load vector F (where
+// vals and, for F, fvals are given); the sort order of the stream: perm (the
+// stream position of every sorted position), seg (run starts, nnz + 1) and the
+// same of the load vector.  Null: not wanted.
+struct BucketOut {
+    int32_t *ptr, *ind;
+    double *val, *F;
+    int32_t *perm, *seg, *fperm, *fbeg;
+};
+size_t bucket_form_bytes(const FormMap &m, int64_t E, int64_t ndofs);
+bool bucket_form_takes(const FormMap &m, int64_t E, int64_t ndofs);
+// Does not wait.  c->told then receives the entry count [0] and whether a row
+// is longer than the tiles hold [2] (nothing is written then).
+int bucket_form(elfel_hip_ctx *c, void *scratch, const FormMap &m, int64_t E, const int32_t *edof, int64_t ndofs,
+                const double *vals, const double *fvals, const BucketOut &o);
+
 // COO stream (device arrays, 1-based indices) -> CSR/CSC by row buckets; waits.
 // flags: the range errors found (nothing is written then); toolong: a row is
 // longer than the tiles hold (nothing is written: use the sort).
@@ -318,31 +365,30 @@ int bucket_coo(elfel_hip_ctx *c, void *scratch, int64_t n, const int64_t *row, c
 
 // ---- plain.hip (FP64, unfused arithmetic) -------------------------------------
 int plain_assemble(elfel_hip_ctx *c, const elfel_hip_problem *pb, const QTable &tab, const Coef &cf);
-// COO buffers for n matrix entries and nv vector entries (plain method), and
-// the sort + reduce that turns the keys written into keys[0]/vals[0] (and
-// fkeys[0]/fvals[0]) into the CSR/CSC result and the load vector.
-// vec: the problem has a load vector (nv pairs, possibly none).
-int plain_buffers(elfel_hip_ctx *c, int64_t n, int64_t nv, int64_t ndofs, bool vec);
-// ---- families.hip: the REUSE method over a cached sort of the COO stream -----
-// What an element kernel writes: keys of the matrix and load-vector streams
-// (null: values only) and their values (FP64, or FP32 when asked for f32).
+// An element kernel's outputs: the values of the matrix stream and of the
+// load-vector stream (FP64, or FP32 when asked for f32).
 struct StreamOut {
-    uint64_t *keys, *fkeys;
     void *vals, *fvals;
 };
 typedef std::function<int(const StreamOut &, bool f32)> StreamElements;
+// The plain method on the stream of `m` (E elements, ndofs rows) whose values
+// `elements` writes: row buckets, or keys + sort + segmented reduce where the
+// buckets do not apply; the sparse matrix and load vector in the context.
+int plain_build(elfel_hip_ctx *c, const elfel_hip_problem *pb, const FormMap &m, int64_t E, int64_t ndofs,
+                const StreamElements &elements);
+// Buffers of the sort for n matrix entries and nv vector entries.
+int sort_buffers(elfel_hip_ctx *c, int64_t n, int64_t nv, bool vec);
+// ---- families.hip: the REUSE method over a cached sort of the COO stream -----
 // Assembles pb's problem by summing the runs of its stream through the cached
 // sort permutation (c->fpat; built on the first call for this mesh, dof map
-// and weak form): n matrix and nv load-vector stream entries (nv 0: no load
-// vector), ndofs rows, keys with minor_bits of minor index.  The result: the
-// sparse matrix (and load vector) in the context, FP64 values equal to the
-// plain method's bit for bit.
-int stream_reuse(elfel_hip_ctx *c, const elfel_hip_problem *pb, int64_t n, int64_t nv, int64_t ndofs, int minor_bits,
-                 bool f32, const StreamElements &elements);
+// and weak form) of the stream `m` describes.  The result: the sparse matrix
+// (and load vector) in the context, FP64 values equal to the plain method's
+// bit for bit.
+int stream_reuse(elfel_hip_ctx *c, const elfel_hip_problem *pb, const FormMap &m, int64_t E, int64_t ndofs, bool f32,
+                 const StreamElements &elements);
 // The 2D weak forms (plain.hip) on stream_reuse, FP64: the REUSE method's
 // path for meshes its tiles do not hold.
 int plain_stream_reuse(elfel_hip_ctx *c, const elfel_hip_problem *pb, const QTable &tab, const Coef &cf);
-int plain_finish(elfel_hip_ctx *c, int layout, int64_t n, int64_t nv, int64_t ndofs, int minor_bits, bool vec);
 
 // ---- families.hip (element families, plain FP64 method) -------------------------
 bool family_problem(const elfel_hip_problem *pb);

@@ -35,41 +35,45 @@ struct Geo {
     R gx[NQ][NEN], gy[NQ][NEN], jxw[NQ], det[NQ];
 };
 
-// Jacobian, determinant, spatial gradients and JxW at every quadrature point.
+// Jacobian, determinant, spatial gradients and JxW at quadrature point q.
+template <typename R, int NEN>
+__device__ __forceinline__ void geometry_at(const QTable &t, int q, const R *X, const R *Y, R *gx, R *gy, R &jxw, R &det)
+{
+    R j11 = X[0] * tab_g<R>(t, q, 0, 0), j21 = Y[0] * tab_g<R>(t, q, 0, 0);
+    R j12 = X[0] * tab_g<R>(t, q, 0, 1), j22 = Y[0] * tab_g<R>(t, q, 0, 1);
+#pragma unroll
+    for (int k = 1; k < NEN; k++) {
+        j11 += X[k] * tab_g<R>(t, q, k, 0);
+        j21 += Y[k] * tab_g<R>(t, q, k, 0);
+        j12 += X[k] * tab_g<R>(t, q, k, 1);
+        j22 += Y[k] * tab_g<R>(t, q, k, 1);
+    }
+    det = j11 * j22 - j21 * j12;
+    if constexpr (sizeof(R) == 8) {
+#pragma unroll
+        for (int k = 0; k < NEN; k++) {
+            const R a = tab_g<R>(t, q, k, 0), b = tab_g<R>(t, q, k, 1);
+            gx[k] = (j22 * a - j21 * b) / det;
+            gy[k] = (j11 * b - j12 * a) / det;
+        }
+    } else {
+        const R inv = R(1) / det;
+#pragma unroll
+        for (int k = 0; k < NEN; k++) {
+            const R a = tab_g<R>(t, q, k, 0), b = tab_g<R>(t, q, k, 1);
+            gx[k] = (j22 * a - j21 * b) * inv;
+            gy[k] = (j11 * b - j12 * a) * inv;
+        }
+    }
+    jxw = det * tab_w<R>(t, q);
+}
+
+// The same at every quadrature point.
 template <typename R, int NEN, int NQ>
 __device__ __forceinline__ void geometry(const QTable &t, const R *X, const R *Y, Geo<R, NEN, NQ> &g)
 {
 #pragma unroll
-    for (int q = 0; q < NQ; q++) {
-        R j11 = X[0] * tab_g<R>(t, q, 0, 0), j21 = Y[0] * tab_g<R>(t, q, 0, 0);
-        R j12 = X[0] * tab_g<R>(t, q, 0, 1), j22 = Y[0] * tab_g<R>(t, q, 0, 1);
-#pragma unroll
-        for (int k = 1; k < NEN; k++) {
-            j11 += X[k] * tab_g<R>(t, q, k, 0);
-            j21 += Y[k] * tab_g<R>(t, q, k, 0);
-            j12 += X[k] * tab_g<R>(t, q, k, 1);
-            j22 += Y[k] * tab_g<R>(t, q, k, 1);
-        }
-        const R det = j11 * j22 - j21 * j12;
-        g.det[q] = det;
-        if constexpr (sizeof(R) == 8) {
-#pragma unroll
-            for (int k = 0; k < NEN; k++) {
-                const R a = tab_g<R>(t, q, k, 0), b = tab_g<R>(t, q, k, 1);
-                g.gx[q][k] = (j22 * a - j21 * b) / det;
-                g.gy[q][k] = (j11 * b - j12 * a) / det;
-            }
-        } else {
-            const R inv = R(1) / det;
-#pragma unroll
-            for (int k = 0; k < NEN; k++) {
-                const R a = tab_g<R>(t, q, k, 0), b = tab_g<R>(t, q, k, 1);
-                g.gx[q][k] = (j22 * a - j21 * b) * inv;
-                g.gy[q][k] = (j11 * b - j12 * a) * inv;
-            }
-        }
-        g.jxw[q] = det * tab_w<R>(t, q);
-    }
+    for (int q = 0; q < NQ; q++) geometry_at<R, NEN>(t, q, X, Y, g.gx[q], g.gy[q], g.jxw[q], g.det[q]);
 }
 
 // Mixed-precision geometry.  An FP32 Jacobian loses up to ~1e-5 of the matrix

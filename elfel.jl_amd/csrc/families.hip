@@ -294,12 +294,6 @@ __device__ __forceinline__ void staged_store(VT *dst, int64_t e0, int64_t E, con
     __syncthreads();
 }
 
-__device__ __forceinline__ uint64_t coo_key(int32_t r, int32_t col, int minor_bits, int csc)
-{
-    const uint64_t mj = (uint64_t)(csc ? col : r), mn = (uint64_t)(csc ? r : col);
-    return (mj << minor_bits) | mn;
-}
-
 // ---- heat / mass on a nodal family --------------------------------------------
 // heat: ke[i,j] += dot(gradN_i, gradN_j) * (kappa JxW), fe[j] += N_j Q JxW
 //       (examples/heat/poisson/t4.jl:33-55, the loop of test/test_heat.jl:36-60);
@@ -308,14 +302,11 @@ __device__ __forceinline__ uint64_t coo_key(int32_t r, int32_t col, int minor_bi
 // VT double: the FP64 kernel (the reference's operation order).  VT float:
 // the REUSE method's MIXED kernel -- FP64 geometry (J, det J, one reciprocal
 // of det J in place of the divisions), FP32 gradients, products and sums over
-// the points, FP32 stored values.  keys / fkeys null: values only (the REUSE
-// method's numeric phase, whose sort order is cached).
+// the points, FP32 stored values.
 template <int KIND, int M, int NB, int NQ, typename VT>
 __global__ __launch_bounds__(256) void k_fam_scalar(int64_t E, const int32_t *__restrict__ conn,
-                                                    const double *__restrict__ x, const int32_t *__restrict__ dof,
-                                                    FamTab tab, double kappa, double Q, int minor_bits, int csc,
-                                                    uint64_t *__restrict__ keys, VT *__restrict__ vals,
-                                                    uint64_t *__restrict__ fkeys, VT *__restrict__ fvals)
+                                                    const double *__restrict__ x, FamTab tab, double kappa, double Q,
+                                                    VT *__restrict__ vals, VT *__restrict__ fvals)
 {
     constexpr bool F32 = sizeof(VT) == 4;
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -324,14 +315,11 @@ __global__ __launch_bounds__(256) void k_fam_scalar(int64_t E, const int32_t *__
     const bool valid = e < E;
     const int64_t ec = valid ? e : E - 1;
     double X[NB * M];
-    int32_t d[NB];
-    const bool want_keys = keys || fkeys;
 #pragma unroll
     for (int k = 0; k < NB; k++) {
         const int32_t n = conn[ec * NB + k];
 #pragma unroll
         for (int s = 0; s < M; s++) X[k * M + s] = x[(int64_t)n * M + s];
-        d[k] = want_keys ? dof[n] : 0;
     }
     VT ke[NB * NB], fe[NB];
 #pragma unroll
@@ -379,19 +367,6 @@ __global__ __launch_bounds__(256) void k_fam_scalar(int64_t E, const int32_t *__
             }
         }
     }
-    if (keys && valid) {
-        int64_t o = e * NB * NB;
-#pragma unroll
-        for (int j = 0; j < NB; j++)
-#pragma unroll
-            for (int i = 0; i < NB; i++) keys[o++] = coo_key(d[i], d[j], minor_bits, csc);
-    }
-    if constexpr (KIND == ELFEL_HEAT) {
-        if (fkeys && valid) {
-#pragma unroll
-            for (int j = 0; j < NB; j++) fkeys[e * NB + j] = (uint64_t)d[j];
-        }
-    }
     // values through LDS where the stage takes at most 40 KiB (heat T4 64^3
     // element kernel 51 -> 40 us); the larger blocks (FP64 T6 mass, 76 KiB)
     // keep direct stores and their occupancy
@@ -421,13 +396,8 @@ __global__ __launch_bounds__(256) void k_fam_scalar(int64_t E, const int32_t *__
 template <int VFE, int PFE, int NQ, typename VT>
 __global__ __launch_bounds__(256) void k_fam_reddy(int64_t E, const int32_t *__restrict__ conn_v,
                                                    const double2 *__restrict__ xy_v,
-                                                   const int32_t *__restrict__ dof_v,
-                                                   const int32_t *__restrict__ edof_v,
                                                    const int32_t *__restrict__ conn_p,
-                                                   const double2 *__restrict__ xy_p,
-                                                   const int32_t *__restrict__ dof_p,
-                                                   const int32_t *__restrict__ edof_p, FamTab tab, double mu,
-                                                   int minor_bits, int csc, uint64_t *__restrict__ keys,
+                                                   const double2 *__restrict__ xy_p, FamTab tab, double mu,
                                                    VT *__restrict__ vals)
 {
     constexpr bool F32 = sizeof(VT) == 4;  // the MIXED kernel (as k_fam_scalar)
@@ -460,30 +430,6 @@ __global__ __launch_bounds__(256) void k_fam_reddy(int64_t E, const int32_t *__r
             gx[q][k] = (VT)g[0]; gy[q][k] = (VT)g[1];
         }
     }
-    // dof numbers (for the keys only)
-    int32_t dx[NU], dy[NU], dp[NP];
-#pragma unroll
-    for (int k = 0; k < NU; k++) dx[k] = dy[k] = 0;
-#pragma unroll
-    for (int k = 0; k < NP; k++) dp[k] = 0;
-    if (keys) {
-#pragma unroll
-        for (int k = 0; k < NV; k++) {
-            const int32_t n = conn_v[e * NV + k];
-            dx[k] = dof_v[2 * (int64_t)n];
-            dy[k] = dof_v[2 * (int64_t)n + 1];
-        }
-        if constexpr (NU > NV) {  // the bubble's cell dofs
-            dx[NV] = edof_v[2 * e];
-            dy[NV] = edof_v[2 * e + 1];
-        }
-        if constexpr (PNODAL) {
-#pragma unroll
-            for (int k = 0; k < 3; k++) dp[k] = dof_p[conn_p[e * 3 + k]];
-        } else {
-            dp[0] = edof_p[e];
-        }
-    }
     // values in stream order, W at a time through a register word (cnt is a
     // constant at every call once the loops are unrolled)
     constexpr int NOUT = 4 * NU * NU + 4 * NU * NP, W = 16 / (int)sizeof(VT);
@@ -492,8 +438,7 @@ __global__ __launch_bounds__(256) void k_fam_reddy(int64_t E, const int32_t *__r
     VT *vout = vals + o0;
     VT wb[W];
     int cnt = 0;
-    auto put = [&](int32_t r, int32_t col, VT v) {
-        if (keys) keys[o0 + cnt] = coo_key(r, col, minor_bits, csc);
+    auto put = [&](VT v) {
         wb[cnt % W] = v;
         if (cnt % W == W - 1) {
             uint4 q;
@@ -516,7 +461,7 @@ __global__ __launch_bounds__(256) void k_fam_reddy(int64_t E, const int32_t *__r
 #pragma unroll
     for (int j = 0; j < NU; j++)
 #pragma unroll
-        for (int i = 0; i < NU; i++) put(dx[i], dx[j], k[i + NU * j]);
+        for (int i = 0; i < NU; i++) put(k[i + NU * j]);
     // kxy and its transpose
 #pragma unroll
     for (int i = 0; i < NU * NU; i++) k[i] = VT(0);
@@ -529,11 +474,11 @@ __global__ __launch_bounds__(256) void k_fam_reddy(int64_t E, const int32_t *__r
 #pragma unroll
     for (int j = 0; j < NU; j++)
 #pragma unroll
-        for (int i = 0; i < NU; i++) put(dx[i], dy[j], k[i + NU * j]);
+        for (int i = 0; i < NU; i++) put(k[i + NU * j]);
 #pragma unroll
     for (int b = 0; b < NU; b++)
 #pragma unroll
-        for (int a = 0; a < NU; a++) put(dy[a], dx[b], k[b + NU * a]);
+        for (int a = 0; a < NU; a++) put(k[b + NU * a]);
     // kyy
 #pragma unroll
     for (int i = 0; i < NU * NU; i++) k[i] = VT(0);
@@ -547,7 +492,7 @@ __global__ __launch_bounds__(256) void k_fam_reddy(int64_t E, const int32_t *__r
 #pragma unroll
     for (int j = 0; j < NU; j++)
 #pragma unroll
-        for (int i = 0; i < NU; i++) put(dy[i], dy[j], k[i + NU * j]);
+        for (int i = 0; i < NU; i++) put(k[i + NU * j]);
     // kxp, kyp and their transposes
 #pragma unroll
     for (int c = 0; c < 2; c++) {
@@ -563,11 +508,11 @@ __global__ __launch_bounds__(256) void k_fam_reddy(int64_t E, const int32_t *__r
 #pragma unroll
         for (int j = 0; j < NP; j++)
 #pragma unroll
-            for (int i = 0; i < NU; i++) put(c == 0 ? dx[i] : dy[i], dp[j], k[i + NU * j]);
+            for (int i = 0; i < NU; i++) put(k[i + NU * j]);
 #pragma unroll
         for (int b = 0; b < NU; b++)
 #pragma unroll
-            for (int a = 0; a < NP; a++) put(dp[a], c == 0 ? dx[b] : dy[b], k[b + NU * a]);
+            for (int a = 0; a < NP; a++) put(k[b + NU * a]);
     }
 }
 
@@ -577,13 +522,10 @@ bool reddy_pair(int vfe, int pfe)
            (vfe == ELFEL_Q4 && pfe == ELFEL_Q4L2);
 }
 
-// The element kernel's outputs: keys (or null) and values of the COO stream
-// and, for heat, of the load-vector stream.
 using FamOut = StreamOut;
 
 template <int KIND, int M, int NB, int NQ, typename VT>
-int launch_scalar(elfel_hip_ctx *c, const FamTab &tab, double kappa, double Q, int minor_bits, int csc,
-                  const FamOut &o)
+int launch_scalar(elfel_hip_ctx *c, const FamTab &tab, double kappa, double Q, const FamOut &o)
 {
     const Field &F = c->f[0];
     const bool heat = KIND == ELFEL_HEAT;
@@ -591,8 +533,7 @@ int launch_scalar(elfel_hip_ctx *c, const FamTab &tab, double kappa, double Q, i
     tm_begin(c, ELFEL_PH_ELEMENT, &ev);
     if (F.E > 0)
         hipLaunchKernelGGL((k_fam_scalar<KIND, M, NB, NQ, VT>), dim3(ceil_div(F.E, 256)), dim3(256), 0, c->stream, F.E,
-                           (const int32_t *)F.conn.p, (const double *)F.xy.p, (const int32_t *)F.dof.p, tab, kappa, Q,
-                           minor_bits, csc, o.keys, (VT *)o.vals, heat ? o.fkeys : nullptr,
+                           (const int32_t *)F.conn.p, (const double *)F.xy.p, tab, kappa, Q, (VT *)o.vals,
                            heat ? (VT *)o.fvals : nullptr);
     HIPCHK(c, hipGetLastError());
     tm_end(c, ELFEL_PH_ELEMENT, ev);
@@ -600,20 +541,16 @@ int launch_scalar(elfel_hip_ctx *c, const FamTab &tab, double kappa, double Q, i
 }
 
 template <int VFE, int PFE, int NQ, typename VT>
-int launch_reddy(elfel_hip_ctx *c, const FamTab &tab, double mu, int minor_bits, int csc, const FamOut &o)
+int launch_reddy(elfel_hip_ctx *c, const FamTab &tab, double mu, const FamOut &o)
 {
     const Field &V = c->f[0], &P = c->f[1];
     hipEvent_t ev = nullptr;
     tm_begin(c, ELFEL_PH_ELEMENT, &ev);
     if (V.E > 0)
         hipLaunchKernelGGL((k_fam_reddy<VFE, PFE, NQ, VT>), dim3(ceil_div(V.E, 256)), dim3(256), 0, c->stream, V.E,
-                           (const int32_t *)V.conn.p, (const double2 *)V.xy.p, (const int32_t *)V.dof.p,
-                           VFE == ELFEL_T3B ? (const int32_t *)V.edof.p : nullptr,
+                           (const int32_t *)V.conn.p, (const double2 *)V.xy.p,
                            PFE == ELFEL_T3 ? (const int32_t *)P.conn.p : nullptr,
-                           PFE == ELFEL_T3 ? (const double2 *)P.xy.p : nullptr,
-                           PFE == ELFEL_T3 ? (const int32_t *)P.dof.p : nullptr,
-                           PFE == ELFEL_Q4L2 ? (const int32_t *)P.edof.p : nullptr, tab, mu, minor_bits, csc,
-                           o.keys, (VT *)o.vals);
+                           PFE == ELFEL_T3 ? (const double2 *)P.xy.p : nullptr, tab, mu, (VT *)o.vals);
     HIPCHK(c, hipGetLastError());
     tm_end(c, ELFEL_PH_ELEMENT, ev);
     return 0;
@@ -758,8 +695,7 @@ __global__ __launch_bounds__(256) void k_fam_runs(const int32_t *__restrict__ pe
 
 // The element kernel of the problem (its weak form, element and rule) with
 // FP64 or FP32 stored values.
-int fam_elements(elfel_hip_ctx *c, const elfel_hip_problem *pb, const FamTab &tab, int minor_bits, int csc,
-                 const FamOut &o, bool f32)
+int fam_elements(elfel_hip_ctx *c, const elfel_hip_problem *pb, const FamTab &tab, const FamOut &o, bool f32)
 {
     const int fe = pb->fe;
     const bool heat = pb->kind == ELFEL_HEAT;
@@ -767,11 +703,11 @@ int fam_elements(elfel_hip_ctx *c, const elfel_hip_problem *pb, const FamTab &ta
     const int nq = tab.nq;
     int rc = 1;  // stays 1 when no kernel instance fits
 #define S(K_, M_, NB_, NQ_)                                                                          \
-    rc = f32 ? launch_scalar<K_, M_, NB_, NQ_, float>(c, tab, pb->kappa, pb->Q, minor_bits, csc, o) \
-             : launch_scalar<K_, M_, NB_, NQ_, double>(c, tab, pb->kappa, pb->Q, minor_bits, csc, o)
+    rc = f32 ? launch_scalar<K_, M_, NB_, NQ_, float>(c, tab, pb->kappa, pb->Q, o) \
+             : launch_scalar<K_, M_, NB_, NQ_, double>(c, tab, pb->kappa, pb->Q, o)
 #define R(V_, P_, NQ_)                                                                 \
-    rc = f32 ? launch_reddy<V_, P_, NQ_, float>(c, tab, pb->mu, minor_bits, csc, o) \
-             : launch_reddy<V_, P_, NQ_, double>(c, tab, pb->mu, minor_bits, csc, o)
+    rc = f32 ? launch_reddy<V_, P_, NQ_, float>(c, tab, pb->mu, o) \
+             : launch_reddy<V_, P_, NQ_, double>(c, tab, pb->mu, o)
     if (heat || pb->kind == ELFEL_MASS) {
         const bool h = heat;
         if (fe == ELFEL_L2) {
@@ -810,12 +746,13 @@ int fam_elements(elfel_hip_ctx *c, const elfel_hip_problem *pb, const FamTab &ta
     } while (0)
 
 // Symbolic phase of the stream REUSE method (c->fpat), when the cached one
-// does not describe this mesh, dof map and weak form.
-int stream_symbolic(elfel_hip_ctx *c, const elfel_hip_problem *pb, int64_t n, int64_t nv, int64_t ndofs,
-                    int minor_bits, const StreamElements &elements)
+// does not describe this mesh, dof map and weak form: the stream ordered by row
+// buckets, or sorted where they do not apply.
+int stream_symbolic(elfel_hip_ctx *c, const elfel_hip_problem *pb, const FormMap &m, int64_t E, int64_t ndofs)
 {
     FamPattern &P = c->fpat;
-    const bool heat = pb->kind == ELFEL_HEAT;
+    const int64_t n = E * m.nmat, nv = E * m.nvec;
+    const bool heat = m.nvec > 0;
     const Field &F0 = c->f[0], &F1 = c->f[1];
     const bool reddy = pb->kind == ELFEL_STOKES_REDDY;
     const bool two = reddy || pb->kind == ELFEL_STOKES_GEN || pb->kind == ELFEL_STOKES_VECLAP;
@@ -828,44 +765,59 @@ int stream_symbolic(elfel_hip_ctx *c, const elfel_hip_problem *pb, int64_t n, in
     const auto t0 = std::chrono::steady_clock::now();
     P.valid = false;
     int rc;
-    if ((rc = plain_buffers(c, n, nv, ndofs, heat)) || (rc = ensure(c, P.coo, 8 * std::max<int64_t>(n, 1))) ||
-        (rc = ensure(c, P.fcoo, 8 * std::max<int64_t>(nv, 1))) || (rc = ensure(c, P.perm, 4 * std::max<int64_t>(n, 1))) ||
-        (rc = ensure(c, P.fperm, 4 * std::max<int64_t>(nv, 1))) || (rc = ensure(c, P.fbeg, 4 * (ndofs + 1))) ||
-        (rc = ensure(c, P.ptr, 4 * (ndofs + 1))) || (rc = ensure(c, P.ind, 4 * std::max<int64_t>(n, 1))))
+    bool buckets = bucket_form_takes(m, E, ndofs);
+    if ((rc = ensure(c, P.coo, 8 * std::max<int64_t>(n, 1))) || (rc = ensure(c, P.fcoo, 8 * std::max<int64_t>(nv, 1))) ||
+        (rc = ensure(c, P.perm, 4 * std::max<int64_t>(n, 1))) || (rc = ensure(c, P.fperm, 4 * std::max<int64_t>(nv, 1))) ||
+        (rc = ensure(c, P.fbeg, 4 * (ndofs + 1))) || (rc = ensure(c, P.ptr, 4 * (ndofs + 1))) ||
+        (rc = ensure(c, P.ind, 4 * std::max<int64_t>(n, 1))) || (rc = ensure(c, c->geom, 4 * E * m.nd)))
         return rc;
-    uint64_t *k0 = (uint64_t *)c->keys[0].p, *k1 = (uint64_t *)c->keys[1].p;
-    uint64_t *v0 = (uint64_t *)c->vals[0].p, *v1 = (uint64_t *)c->vals[1].p;
-    uint64_t *fk0 = (uint64_t *)c->fkeys[0].p, *fk1 = (uint64_t *)c->fkeys[1].p;
-    uint64_t *fv0 = (uint64_t *)c->fvals[0].p, *fv1 = (uint64_t *)c->fvals[1].p;
-    // the stream's keys (its values land in coo, unused here)
-    const StreamOut o{k0, heat ? fk0 : nullptr, P.coo.p, heat ? P.fcoo.p : nullptr};
-    if ((rc = elements(o, false))) return rc;
-    hipEvent_t ev = nullptr;
-    tm_begin(c, ELFEL_PH_SORT, &ev);
-    FAM_LAUNCH(k_fam_iota, n, v0, n);
-    if ((rc = radix_sort_pairs(c, k0, v0, k1, v1, n, bits_for(ndofs) + minor_bits))) return rc;
-    if (heat) {
-        FAM_LAUNCH(k_fam_iota, nv, fv0, nv);
-        if ((rc = radix_sort_pairs(c, fk0, fv0, fk1, fv1, nv, bits_for(ndofs)))) return rc;
+    int32_t *edof = (int32_t *)c->geom.p;
+    if ((rc = form_dofs(c, m, edof))) return rc;
+    int64_t nnz = 0;
+    if (buckets) {
+        if ((rc = ensure(c, P.seg, 4 * (n + 1))) || (rc = ensure(c, c->keys[0], bucket_form_bytes(m, E, ndofs)))) return rc;
+        const BucketOut o{(int32_t *)P.ptr.p, (int32_t *)P.ind.p, nullptr, nullptr, (int32_t *)P.perm.p,
+                          (int32_t *)P.seg.p, (int32_t *)P.fperm.p, (int32_t *)P.fbeg.p};
+        if ((rc = bucket_form(c, c->keys[0].p, m, E, edof, ndofs, nullptr, nullptr, o))) return rc;
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        nnz = ((const int32_t *)c->told)[0];
+        buckets = ((const int32_t *)c->told)[2] == 0;
     }
-    tm_end(c, ELFEL_PH_SORT, ev);
-    if ((rc = build_csr_from_sorted(c, k0, nullptr, n, minor_bits, ndofs, (int32_t *)P.ptr.p, (int32_t *)P.ind.p,
-                                    nullptr, (int32_t *)c->dscal.p, false)))
-        return rc;
-    int32_t hnnz = 0;
-    HIPCHK(c, hipMemcpyAsync(&hnnz, c->dscal.p, 4, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    const int64_t nnz = hnnz;
-    if ((rc = ensure(c, P.seg, 4 * (nnz + 1)))) return rc;
-    FAM_LAUNCH(k_fam_narrow, n, v0, (int32_t *)P.perm.p, n);
-    if (n > 0) FAM_LAUNCH(k_fam_seg, nnz + 1, (const uint32_t *)c->segpos.p, nnz, n, (int32_t *)P.seg.p);
-    else FAM_LAUNCH(k_fam_fill_i32, (int64_t)1, (int32_t *)P.seg.p, (int64_t)1, 0);
-    if (heat) {
-        FAM_LAUNCH(k_fam_narrow, nv, fv0, (int32_t *)P.fperm.p, nv);
-        if (nv > 0) FAM_LAUNCH(k_fam_dense_begin, nv, fk0, nv, ndofs, (int32_t *)P.fbeg.p);
-        else FAM_LAUNCH(k_fam_fill_i32, ndofs + 1, (int32_t *)P.fbeg.p, ndofs + 1, 0);
+    if (!buckets) {
+        if ((rc = sort_buffers(c, n, nv, heat))) return rc;
+        const int minor_bits = bits_for(ndofs);
+        uint64_t *k0 = (uint64_t *)c->keys[0].p, *k1 = (uint64_t *)c->keys[1].p;
+        uint64_t *v0 = (uint64_t *)c->vals[0].p, *v1 = (uint64_t *)c->vals[1].p;
+        uint64_t *fk0 = (uint64_t *)c->fkeys[0].p, *fk1 = (uint64_t *)c->fkeys[1].p;
+        uint64_t *fv0 = (uint64_t *)c->fvals[0].p, *fv1 = (uint64_t *)c->fvals[1].p;
+        hipEvent_t ev = nullptr;
+        tm_begin(c, ELFEL_PH_SORT, &ev);
+        if ((rc = form_keys(c, m, E, edof, minor_bits, k0, heat ? fk0 : nullptr))) return rc;
+        FAM_LAUNCH(k_fam_iota, n, v0, n);
+        if ((rc = radix_sort_pairs(c, k0, v0, k1, v1, n, bits_for(ndofs) + minor_bits))) return rc;
+        if (heat) {
+            FAM_LAUNCH(k_fam_iota, nv, fv0, nv);
+            if ((rc = radix_sort_pairs(c, fk0, fv0, fk1, fv1, nv, bits_for(ndofs)))) return rc;
+        }
+        tm_end(c, ELFEL_PH_SORT, ev);
+        if ((rc = build_csr_from_sorted(c, k0, nullptr, n, minor_bits, ndofs, (int32_t *)P.ptr.p, (int32_t *)P.ind.p,
+                                        nullptr, (int32_t *)c->dscal.p, false)))
+            return rc;
+        int32_t hnnz = 0;
+        HIPCHK(c, hipMemcpyAsync(&hnnz, c->dscal.p, 4, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        nnz = hnnz;
+        if ((rc = ensure(c, P.seg, 4 * (nnz + 1)))) return rc;
+        FAM_LAUNCH(k_fam_narrow, n, v0, (int32_t *)P.perm.p, n);
+        if (n > 0) FAM_LAUNCH(k_fam_seg, nnz + 1, (const uint32_t *)c->segpos.p, nnz, n, (int32_t *)P.seg.p);
+        else FAM_LAUNCH(k_fam_fill_i32, (int64_t)1, (int32_t *)P.seg.p, (int64_t)1, 0);
+        if (heat) {
+            FAM_LAUNCH(k_fam_narrow, nv, fv0, (int32_t *)P.fperm.p, nv);
+            if (nv > 0) FAM_LAUNCH(k_fam_dense_begin, nv, fk0, nv, ndofs, (int32_t *)P.fbeg.p);
+            else FAM_LAUNCH(k_fam_fill_i32, ndofs + 1, (int32_t *)P.fbeg.p, ndofs + 1, 0);
+        }
+        HIPCHK(c, hipStreamSynchronize(c->stream));
     }
-    HIPCHK(c, hipStreamSynchronize(c->stream));
     P.kind = pb->kind; P.fe = pb->fe; P.fe_p = pfe; P.layout = pb->layout;
     memcpy(P.key, key, sizeof key);
     P.n = n; P.nv = nv; P.nnz = nnz; P.ndofs = ndofs;
@@ -878,16 +830,16 @@ int stream_symbolic(elfel_hip_ctx *c, const elfel_hip_problem *pb, int64_t n, in
 
 // Numeric phase: element values only, then every run summed through the
 // cached permutation.
-int stream_reuse(elfel_hip_ctx *c, const elfel_hip_problem *pb, int64_t n, int64_t nv, int64_t ndofs, int minor_bits,
-                 bool f32, const StreamElements &elements)
+int stream_reuse(elfel_hip_ctx *c, const elfel_hip_problem *pb, const FormMap &m, int64_t E, int64_t ndofs, bool f32,
+                 const StreamElements &elements)
 {
-    const bool heat = pb->kind == ELFEL_HEAT;
-    int rc = stream_symbolic(c, pb, n, nv, ndofs, minor_bits, elements);
+    const bool heat = m.nvec > 0;
+    int rc = stream_symbolic(c, pb, m, E, ndofs);
     if (rc) return rc;
     const FamPattern &P = c->fpat;
     if ((rc = ensure(c, c->val, 8 * std::max<int64_t>(P.nnz, 1)))) return rc;
     if (heat && (rc = ensure(c, c->F, 8 * std::max<int64_t>(ndofs, 1)))) return rc;
-    const StreamOut o{nullptr, nullptr, P.coo.p, heat ? P.fcoo.p : nullptr};
+    const StreamOut o{P.coo.p, heat ? P.fcoo.p : nullptr};
     if ((rc = elements(o, f32))) return rc;
     hipEvent_t ev = nullptr;
     tm_begin(c, ELFEL_PH_REDUCE, &ev);
@@ -975,6 +927,32 @@ int family_validate(elfel_hip_ctx *c, const elfel_hip_problem *pb)
     return 0;
 }
 
+// The Reddy blocks in stream order: kxx, kxy, kxy', kyy, kxp, kxp', kyp, kyp'
+// (a transpose row-major of its parent); local dofs ux, uy, p.
+static void reddy_map(int fe, int nu, int np, int csc, FormMap &m)
+{
+    const int nd = 2 * nu + np;
+    m.nd = nd;
+    m.nmat = 4 * nu * nu + 4 * nu * np;
+    auto at = [&](int i, int j) {
+        const int ri = i < nu ? 0 : i < 2 * nu ? 1 : 2, rj = j < nu ? 0 : j < 2 * nu ? 1 : 2;
+        const int li = i - ri * nu, lj = j - rj * nu;
+        if (ri < 2 && rj < 2) return (2 * ri + rj) * nu * nu + li + nu * lj;
+        if (ri == 2 && rj == 2) return -1;
+        const int c = ri < 2 ? ri : rj;  // the velocity component of the coupling block
+        const int base = 4 * nu * nu + c * 2 * nu * np;
+        return ri < 2 ? base + li + nu * lj : base + nu * np + li + np * lj;
+    };
+    for (int a = 0; a < nd; a++) {
+        m.ncol[a] = (uint8_t)(a < 2 * nu ? nd : 2 * nu);
+        for (int b = 0; b < nd; b++) m.pos[a * nd + b] = (int16_t)(csc ? at(b, a) : at(a, b));
+    }
+    const int nv = fam_ngeo(fe);
+    for (int c = 0; c < 2; c++)
+        for (int k = 0; k < nu; k++) m.src[c * nu + k] = {0, (uint8_t)(k >= nv), (uint8_t)k, (uint8_t)c};
+    for (int k = 0; k < np; k++) m.src[2 * nu + k] = {1, (uint8_t)(np == 1), (uint8_t)k, 0};
+}
+
 int family_assemble(elfel_hip_ctx *c, const elfel_hip_problem *pb)
 {
     const Field &F = c->f[0];
@@ -985,26 +963,24 @@ int family_assemble(elfel_hip_ctx *c, const elfel_hip_problem *pb)
     if (fam_table(fe, pfe, pfe == ELFEL_T3 ? ELFEL_T3 : fe, pb->rule, &tab))
         return set_err(c, ELFEL_ENOTSUP, "unsupported quadrature rule");
     const int nu = fam_nbf(fe), np = reddy ? fam_nbf(pfe) : 0;
-    const int64_t n = F.E * (reddy ? 4 * nu * nu + 4 * nu * np : nu * nu);
-    const bool heat = pb->kind == ELFEL_HEAT;
-    const int64_t nv = heat ? F.E * nu : 0;
-    const int64_t ndofs = c->nrow;
-    const int minor_bits = bits_for(ndofs);
     const int csc = pb->layout == ELFEL_CSC ? 1 : 0;
+    FormMap m;
+    if (reddy) {
+        reddy_map(fe, nu, np, csc, m);
+    } else {
+        form_square(m, nu, csc);
+        m.nvec = pb->kind == ELFEL_HEAT ? nu : 0;
+        for (int i = 0; i < nu; i++) m.src[i] = {0, 0, (uint8_t)i, 0};
+    }
+    auto elements = [&](const StreamOut &o, bool f32) { return fam_elements(c, pb, tab, o, f32); };
     // the cached permutation and run starts are int32: a longer stream runs the
     // plain FP64 method (its sort carries 64-bit positions)
-    if (pb->method == ELFEL_REUSE && n < INT32_MAX && nv < INT32_MAX)
-        return stream_reuse(c, pb, n, nv, ndofs, minor_bits, pb->precision == ELFEL_MIXED,
-                            [&](const StreamOut &o, bool f32) { return fam_elements(c, pb, tab, minor_bits, csc, o, f32); });
+    if (pb->method == ELFEL_REUSE && F.E * m.nmat < INT32_MAX && F.E * m.nvec < INT32_MAX)
+        return stream_reuse(c, pb, m, F.E, c->nrow, pb->precision == ELFEL_MIXED, elements);
     if (pb->method == ELFEL_REUSE) {
         c->used_method = ELFEL_SORT;
         c->used_precision = ELFEL_FP64;
         c->used_note = "plain FP64 method: a COO stream of 2^31 entries or more";
     }
-    int rc = plain_buffers(c, n, nv, ndofs, heat);
-    if (rc) return rc;
-    const FamOut o{(uint64_t *)c->keys[0].p, heat ? (uint64_t *)c->fkeys[0].p : nullptr, c->vals[0].p,
-                   heat ? c->fvals[0].p : nullptr};
-    if ((rc = fam_elements(c, pb, tab, minor_bits, csc, o, false))) return rc;
-    return plain_finish(c, pb->layout, n, nv, ndofs, minor_bits, heat);
+    return plain_build(c, pb, m, F.E, c->nrow, elements);
 }

@@ -1,7 +1,8 @@
-// plain.hip -- the plain FP64 method: gather, per-element kernels that write
-// the COO stream in Elfel's order, stable radix sort, in-order segmented
-// reduce.  Compiled with -ffp-contract=off so every product and sum rounds
-// exactly like the reference's unfused Julia arithmetic.
+// plain.hip -- the plain FP64 method: element kernels that write the values of
+// the COO stream in Elfel's order, and the matrix built from it by row buckets
+// (bucket.hip), or by the stable sort and in-order segmented reduce (sort.hip)
+// where those do not apply.  Compiled with -ffp-contract=off so every product
+// and sum rounds exactly like the reference's unfused Julia arithmetic.
 //
 // COO stream order (what SysmatAssemblerSparse's append! produces):
 //   per element, in element order (for el in elit, src/FEIterators.jl:92-98),
@@ -9,6 +10,8 @@
 //   src/LocalAssemblers.jl:68-83; assemble!, src/Assemblers.jl:97-102);
 //   Stokes adds kup column-major and transpose(kup) row-major of kup
 //   (src/Assemblers.jl:109-114), as test/test_stokes.jl:654-656 does.
+#include <string.h>
+
 #include "elem.h"
 
 // ---- index conversion: 1-based int64 -> 0-based int32 with range check ----
@@ -34,106 +37,162 @@ int convert_indices(elfel_hip_ctx *c, const int64_t *src_dev, int32_t *dst, int6
     return 0;
 }
 
-// ---- gather: element-major SoA copies of coordinates and dofs -------------
-// gxy[k*E + e] = xy[conn[e][k]], gd[j*E + e] = dof of element dof j, so the
-// element kernels read every operand with unit stride across a wavefront.
-template <int NEN, int NC>
-__global__ __launch_bounds__(256) void k_gather(int64_t E, const int32_t *__restrict__ conn,
-                                                const double2 *__restrict__ xy, const int32_t *__restrict__ dof,
-                                                const int32_t *__restrict__ connp, const int32_t *__restrict__ dofp,
-                                                double2 *__restrict__ gxy, int32_t *__restrict__ gd)
-{
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= E) return;
-#pragma unroll
-    for (int k = 0; k < NEN; k++) {
-        const int32_t n = conn[e * NEN + k];
-        gxy[k * E + e] = xy[n];
-#pragma unroll
-        for (int c = 0; c < NC; c++) gd[(k * NC + c) * E + e] = dof[(int64_t)n * NC + c];
-    }
-    if (connp) {
-#pragma unroll
-        for (int k = 0; k < 3; k++) gd[(NEN * NC + k) * E + e] = dofp[connp[e * 3 + k]];
-    }
-}
-
-// ---- element kernel: one work-item per element, COO in stream order -------
+// ---- element kernel: the values of the COO stream, in stream order ----------
+// A workgroup takes EB elements.  First a work-item per (element, point) leaves
+// the spatial gradients and JxW in LDS; then a work-item per (element, column of
+// the block) forms the column's ND values and stores them side by side, so that
+// a wavefront writes one contiguous range and the L2 lines are full before they
+// leave it.  (One work-item per element, its whole block and the sort keys
+// stored a value at a time 1152 bytes apart: elasticity T6 200^2 199 us, 0.9 TB/s
+// written; this kernel writes no keys and takes 41 us, 2.2 TB/s.)  The last items of an
+// element are the load vector (heat) or the coupling block and its transpose
+// (Stokes, ND values each).
 template <int KIND, int NEN, int NC, int NQ>
-__global__ __launch_bounds__(256) void k_elem_coo(int64_t E, const double2 *__restrict__ gxy,
-                                                  const int32_t *__restrict__ gd, Coef cf, QTable tab,
-                                                  int minor_bits, int csc, uint64_t *__restrict__ keys,
-                                                  double *__restrict__ vals, uint64_t *__restrict__ fkeys,
-                                                  double *__restrict__ fvals)
+struct ElemVals {
+    static constexpr int ND = NEN * NC;
+    static constexpr bool STOKES = KIND == ELFEL_STOKES_GEN || KIND == ELFEL_STOKES_VECLAP;
+    static constexpr bool HEAT = KIND == ELFEL_HEAT;
+    static constexpr int NBLK = ND * ND + (STOKES ? 2 * ND * 3 : 0);
+    static constexpr int ITEMS = ND + (STOKES ? 6 : 0) + (HEAT ? 1 : 0);
+    static constexpr int EB = NQ == 1 ? 256 : 64;
+    static constexpr int GS = (2 * NEN * NQ + NQ) | 1;  // words an element, odd against bank conflicts
+};
+
+template <int KIND, int NEN, int NC, int NQ>
+__global__ __launch_bounds__(256) void k_elem_vals(int64_t E, const int32_t *__restrict__ conn,
+                                                   const double2 *__restrict__ xy, Coef cf, QTable tab,
+                                                   double *__restrict__ vals, double *__restrict__ fvals)
 {
-    constexpr int ND = NEN * NC;
-    constexpr bool STOKES = (KIND == ELFEL_STOKES_GEN || KIND == ELFEL_STOKES_VECLAP);
-    constexpr int NBLK = ND * ND + (STOKES ? 2 * ND * 3 : 0);
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= E) return;
-    double X[NEN], Y[NEN];
+    using V = ElemVals<KIND, NEN, NC, NQ>;
+    constexpr int ND = V::ND, EB = V::EB, GS = V::GS;
+    __shared__ double sg[EB * GS];  // per element: gx[q][k], gy[q][k], jxw[q]
+    const int64_t e0 = (int64_t)blockIdx.x * EB;
+    for (int x = threadIdx.x; x < EB * NQ; x += 256) {
+        const int el = x % EB, q = __builtin_amdgcn_readfirstlane(x / EB);  // EB is a multiple of the wave
+        const int64_t e = e0 + el;
+        if (e >= E) continue;
+        double X[NEN], Y[NEN], gx[NEN], gy[NEN], jxw, det;
 #pragma unroll
-    for (int k = 0; k < NEN; k++) {
-        const double2 p = gxy[k * E + e];
-        X[k] = p.x; Y[k] = p.y;
-    }
-    int32_t d[ND + (STOKES ? 3 : 0)];
-#pragma unroll
-    for (int j = 0; j < ND + (STOKES ? 3 : 0); j++) d[j] = gd[j * E + e];
-    Geo<double, NEN, NQ> g;
-    geometry<double, NEN, NQ>(tab, X, Y, g);
-    double D[9];
-    const double sc = cf.scale_e ? cf.scale_e[padded(e, cf.cgap)] : 1.0;
-#pragma unroll
-    for (int i = 0; i < 9; i++) D[i] = cf.scale_e ? sc * cf.D[i] : cf.D[i];
-    const double kap = cf.kappa_e ? cf.kappa_e[padded(e, cf.cgap)] : cf.kappa;
-    auto key = [&](int32_t r, int32_t col) -> uint64_t {
-        const uint64_t mj = (uint64_t)(csc ? col : r), mn = (uint64_t)(csc ? r : col);
-        return (mj << minor_bits) | mn;
-    };
-    int64_t o = e * NBLK;
-    Entry<KIND, double, NEN, NC, NQ> ent;
-#pragma unroll
-    for (int j = 0; j < ND; j++) {
-        ent.column(g, D, j);
-#pragma unroll
-        for (int i = 0; i < ND; i++) {
-            if (keys) keys[o] = key(d[i], d[j]);
-            vals[o] = ent.value(g, kap, cf.mu, i, j);
-            o++;
+        for (int k = 0; k < NEN; k++) {
+            const double2 p = xy[conn[e * NEN + k]];
+            X[k] = p.x; Y[k] = p.y;
         }
+        geometry_at<double, NEN>(tab, q, X, Y, gx, gy, jxw, det);
+        double *g = sg + el * GS;
+#pragma unroll
+        for (int k = 0; k < NEN; k++) {
+            g[q * NEN + k] = gx[k];
+            g[(NQ + q) * NEN + k] = gy[k];
+        }
+        g[2 * NQ * NEN + q] = jxw;
     }
-    if constexpr (STOKES) {
-        double kup[ND][3];
+    __syncthreads();
+    for (int x = threadIdx.x; x < EB * V::ITEMS; x += 256) {
+        const int el = x / V::ITEMS, it = x - el * V::ITEMS;
+        const int64_t e = e0 + el;
+        if (e >= E) break;
+        const double *sge = sg + el * GS;
+        Geo<double, NEN, NQ> g;
 #pragma unroll
-        for (int jp = 0; jp < 3; jp++)
+        for (int q = 0; q < NQ; q++) {
 #pragma unroll
-            for (int i = 0; i < ND; i++) kup[i][jp] = kup_value<double, NEN, NC, NQ>(tab, g, i, jp);
-#pragma unroll
-        for (int jp = 0; jp < 3; jp++)
-#pragma unroll
-            for (int i = 0; i < ND; i++) {
-                if (keys) keys[o] = key(d[i], d[ND + jp]);
-                vals[o] = kup[i][jp];
-                o++;
+            for (int k = 0; k < NEN; k++) {
+                g.gx[q][k] = sge[q * NEN + k];
+                g.gy[q][k] = sge[(NQ + q) * NEN + k];
             }
+            g.jxw[q] = sge[2 * NQ * NEN + q];
+        }
+        double v[ND];
+        double *dst = vals + e * V::NBLK + it * ND;
+        if (it < ND) {
+            const int bj = it / NC, cj = it - bj * NC;
+            double gxj[NQ], gyj[NQ];
 #pragma unroll
-        for (int b = 0; b < ND; b++)
-#pragma unroll
-            for (int a = 0; a < 3; a++) {
-                if (keys) keys[o] = key(d[ND + a], d[b]);
-                vals[o] = kup[b][a];
-                o++;
+            for (int q = 0; q < NQ; q++) {
+                gxj[q] = sge[q * NEN + bj];
+                gyj[q] = sge[(NQ + q) * NEN + bj];
             }
-    }
-    if constexpr (KIND == ELFEL_HEAT) {
-        if (fvals) {
+            if constexpr (KIND == ELFEL_HEAT) {
+                const double kap = cf.kappa_e ? cf.kappa_e[padded(e, cf.cgap)] : cf.kappa;
+#pragma unroll
+                for (int i = 0; i < ND; i++) {
+                    double acc = 0.0;
+#pragma unroll
+                    for (int q = 0; q < NQ; q++)
+                        acc += (g.gx[q][i] * gxj[q] + g.gy[q][i] * gyj[q]) * (kap * g.jxw[q]);
+                    v[i] = acc;
+                }
+            } else if constexpr (KIND == ELFEL_ELAST || KIND == ELFEL_STOKES_GEN) {
+                const double sc = cf.scale_e ? cf.scale_e[padded(e, cf.cgap)] : 1.0;
+                double D[9], db[NQ][3];
+#pragma unroll
+                for (int i = 0; i < 9; i++) D[i] = cf.scale_e ? sc * cf.D[i] : cf.D[i];
+#pragma unroll
+                for (int q = 0; q < NQ; q++) dmul_b<double>(D, gxj[q], gyj[q], cj, db[q]);
+#pragma unroll
+                for (int i = 0; i < ND; i++) {
+                    double acc = 0.0;
+#pragma unroll
+                    for (int q = 0; q < NQ; q++)
+                        acc += dot_b<double>(db[q], g.gx[q][i / NC], g.gy[q][i / NC], i % NC) * g.jxw[q];
+                    v[i] = acc;
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < ND; i++) {
+                    double acc = 0.0;
+#pragma unroll
+                    for (int q = 0; q < NQ; q++)
+                        acc += (cf.mu * g.jxw[q]) * (g.gx[q][i / NC] * gxj[q] + g.gy[q][i / NC] * gyj[q]);
+                    v[i] = (i % NC) == cj ? acc : 0.0;
+                }
+            }
+        } else if constexpr (V::HEAT) {
+            if (!fvals) continue;
             const double Qe = cf.Q_e ? cf.Q_e[padded(e, cf.cgap)] : cf.Q;
 #pragma unroll
-            for (int j = 0; j < ND; j++) {
-                if (fkeys) fkeys[e * ND + j] = (uint64_t)d[j];
-                fvals[e * ND + j] = fe_value<double, NEN, NQ>(tab, g, Qe, j);
+            for (int j = 0; j < ND; j++) v[j] = fe_value<double, NEN, NQ>(tab, g, Qe, j);
+            dst = fvals + e * ND;
+        } else if constexpr (V::STOKES) {
+            if (it < ND + 3) {  // kup, column jp
+                const int jp = it - ND;
+                double np[NQ];
+#pragma unroll
+                for (int q = 0; q < NQ; q++) np[q] = jp == 0 ? tab.Np[q][0] : jp == 1 ? tab.Np[q][1] : tab.Np[q][2];
+#pragma unroll
+                for (int i = 0; i < ND; i++) {
+                    double acc = 0.0;
+#pragma unroll
+                    for (int q = 0; q < NQ; q++) {
+                        const double gi = (i % NC) == 0 ? g.gx[q][i / NC] : g.gy[q][i / NC];
+                        acc += (-g.jxw[q] * np[q]) * gi;
+                    }
+                    v[i] = acc;
+                }
+            } else {  // its transpose: rows b of kup, ND / 3 of them
+                const int b0 = (it - ND - 3) * (ND / 3);
+#pragma unroll
+                for (int bb = 0; bb < ND / 3; bb++) {
+                    const int b = b0 + bb;
+#pragma unroll
+                    for (int a = 0; a < 3; a++) {
+                        double acc = 0.0;
+#pragma unroll
+                        for (int q = 0; q < NQ; q++) {
+                            const double gi = (b % NC) == 0 ? sge[q * NEN + b / NC] : sge[(NQ + q) * NEN + b / NC];
+                            acc += (-g.jxw[q] * tab.Np[q][a]) * gi;
+                        }
+                        v[bb * 3 + a] = acc;
+                    }
+                }
             }
+        }
+        if constexpr (ND % 2 == 0) {
+#pragma unroll
+            for (int i = 0; i < ND; i += 2) *(double2 *)(dst + i) = make_double2(v[i], v[i + 1]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < ND; i++) dst[i] = v[i];
         }
     }
 }
@@ -188,36 +247,21 @@ int plain_vec_keys(elfel_hip_ctx *c, const int64_t *I, int64_t n, int64_t ndofs,
 
 // ---- orchestration --------------------------------------------------------
 template <int KIND, int NEN, int NC, int NQ>
-static int launch_plain(elfel_hip_ctx *c, const QTable &tab, const Coef &cf, int minor_bits, int csc,
-                        uint64_t *keys, double *vals, uint64_t *fkeys, double *fvals)
+static int launch_plain(elfel_hip_ctx *c, const QTable &tab, const Coef &cf, double *vals, double *fvals)
 {
     const Field &F = c->f[0];
     const int64_t E = F.E;
-    constexpr bool STOKES = (KIND == ELFEL_STOKES_GEN || KIND == ELFEL_STOKES_VECLAP);
-    const int nd = NEN * NC + (STOKES ? 3 : 0);
-    int rc = ensure(c, c->geom, (size_t)E * (NEN * sizeof(double2) + nd * sizeof(int32_t)));
-    if (rc) return rc;
-    double2 *gxy = (double2 *)c->geom.p;
-    int32_t *gd = (int32_t *)(gxy + (size_t)NEN * E);
     if (E == 0) return 0;  // no elements: an empty stream
     hipEvent_t ev = nullptr;
-    tm_begin(c, ELFEL_PH_GATHER, &ev);
-    hipLaunchKernelGGL((k_gather<NEN, NC>), dim3(ceil_div(E, 256)), dim3(256), 0, c->stream, E,
-                       (const int32_t *)F.conn.p, (const double2 *)F.xy.p, (const int32_t *)F.dof.p,
-                       STOKES ? (const int32_t *)c->f[1].conn.p : nullptr,
-                       STOKES ? (const int32_t *)c->f[1].dof.p : nullptr, gxy, gd);
-    HIPCHK(c, hipGetLastError());
-    tm_end(c, ELFEL_PH_GATHER, ev);
     tm_begin(c, ELFEL_PH_ELEMENT, &ev);
-    hipLaunchKernelGGL((k_elem_coo<KIND, NEN, NC, NQ>), dim3(ceil_div(E, 256)), dim3(256), 0, c->stream, E, gxy, gd,
-                       cf, tab, minor_bits, csc, keys, vals, fkeys, fvals);
+    hipLaunchKernelGGL((k_elem_vals<KIND, NEN, NC, NQ>), dim3(ceil_div(E, ElemVals<KIND, NEN, NC, NQ>::EB)), dim3(256), 0,
+                       c->stream, E, (const int32_t *)F.conn.p, (const double2 *)F.xy.p, cf, tab, vals, fvals);
     HIPCHK(c, hipGetLastError());
     tm_end(c, ELFEL_PH_ELEMENT, ev);
     return 0;
 }
 
-typedef int (*plain_fn)(elfel_hip_ctx *, const QTable &, const Coef &, int, int, uint64_t *, double *, uint64_t *,
-                        double *);
+typedef int (*plain_fn)(elfel_hip_ctx *, const QTable &, const Coef &, double *, double *);
 
 static plain_fn pick_plain(int kind, int fe, int nq)
 {
@@ -242,7 +286,7 @@ static plain_fn pick_plain(int kind, int fe, int nq)
     return nullptr;
 }
 
-int plain_buffers(elfel_hip_ctx *c, int64_t n, int64_t nv, int64_t ndofs, bool vec)
+int sort_buffers(elfel_hip_ctx *c, int64_t n, int64_t nv, bool vec)
 {
     int rc;
     if ((rc = ensure(c, c->keys[0], sizeof(uint64_t) * n)) || (rc = ensure(c, c->keys[1], sizeof(uint64_t) * n)) ||
@@ -250,98 +294,152 @@ int plain_buffers(elfel_hip_ctx *c, int64_t n, int64_t nv, int64_t ndofs, bool v
         return rc;
     if (vec) {
         if ((rc = ensure(c, c->fkeys[0], sizeof(uint64_t) * nv)) || (rc = ensure(c, c->fkeys[1], sizeof(uint64_t) * nv)) ||
-            (rc = ensure(c, c->fvals[0], sizeof(double) * nv)) || (rc = ensure(c, c->fvals[1], sizeof(double) * nv)) ||
-            (rc = ensure(c, c->F, sizeof(double) * ndofs)))
+            (rc = ensure(c, c->fvals[0], sizeof(double) * nv)) || (rc = ensure(c, c->fvals[1], sizeof(double) * nv)))
             return rc;
     }
-    if ((rc = ensure(c, c->ptr, sizeof(int32_t) * (ndofs + 1))) || (rc = ensure(c, c->ind, sizeof(int32_t) * n)) ||
-        (rc = ensure(c, c->val, sizeof(double) * n)))
-        return rc;
     return 0;
 }
 
-int plain_finish(elfel_hip_ctx *c, int layout, int64_t n, int64_t nv, int64_t ndofs, int minor_bits, bool vec)
+// The sort of the stream whose values are in vals[0] (and fvals[0]).
+static int build_by_sort(elfel_hip_ctx *c, const FormMap &m, int64_t E, const int32_t *edof, int64_t ndofs)
 {
+    const int64_t n = E * m.nmat, nv = E * m.nvec;
+    const int minor_bits = bits_for(ndofs);
+    const bool vec = m.nvec > 0;
+    int rc = sort_buffers(c, n, nv, vec);
+    if (rc) return rc;
     uint64_t *k0 = (uint64_t *)c->keys[0].p, *k1 = (uint64_t *)c->keys[1].p;
     uint64_t *v0 = (uint64_t *)c->vals[0].p, *v1 = (uint64_t *)c->vals[1].p;
     uint64_t *fk0 = vec ? (uint64_t *)c->fkeys[0].p : nullptr, *fk1 = vec ? (uint64_t *)c->fkeys[1].p : nullptr;
     uint64_t *fv0 = vec ? (uint64_t *)c->fvals[0].p : nullptr, *fv1 = vec ? (uint64_t *)c->fvals[1].p : nullptr;
     hipEvent_t ev = nullptr;
     tm_begin(c, ELFEL_PH_SORT, &ev);
-    int rc = radix_sort_pairs(c, k0, v0, k1, v1, n, bits_for(ndofs) + minor_bits);
-    if (rc) return rc;
-    if (vec) {
-        rc = radix_sort_pairs(c, fk0, fv0, fk1, fv1, nv, bits_for(ndofs));
-        if (rc) return rc;
-    }
+    if ((rc = form_keys(c, m, E, edof, minor_bits, k0, fk0))) return rc;
+    if ((rc = radix_sort_pairs(c, k0, v0, k1, v1, n, bits_for(ndofs) + minor_bits))) return rc;
+    if (vec && (rc = radix_sort_pairs(c, fk0, fv0, fk1, fv1, nv, bits_for(ndofs)))) return rc;
     tm_end(c, ELFEL_PH_SORT, ev);
     tm_begin(c, ELFEL_PH_REDUCE, &ev);
     rc = build_csr_from_sorted(c, k0, (const double *)v0, n, minor_bits, ndofs, (int32_t *)c->ptr.p,
                                (int32_t *)c->ind.p, (double *)c->val.p, (int32_t *)c->dscal.p, true);
     if (rc) return rc;
-    if (vec) {
-        rc = build_dense_from_sorted(c, fk0, (const double *)fv0, nv, ndofs, (double *)c->F.p);
-        if (rc) return rc;
-    }
+    if (vec && (rc = build_dense_from_sorted(c, fk0, (const double *)fv0, nv, ndofs, (double *)c->F.p))) return rc;
     tm_end(c, ELFEL_PH_REDUCE, ev);
+    return 0;
+}
+
+// Whether the rows of this problem's matrix fit the buckets' tiles depends on
+// the mesh, the dof map and the weak form alone.  The first assembly on them
+// waits for the answer and keeps it; later ones take the one way or the other
+// without a wait.
+int plain_build(elfel_hip_ctx *c, const elfel_hip_problem *pb, const FormMap &m, int64_t E, int64_t ndofs,
+                const StreamElements &elements)
+{
+    const int64_t n = E * m.nmat, nv = E * m.nvec;
+    const bool vec = m.nvec > 0;
+    const uint64_t key[6] = {c->f[0].mesh_version, c->f[0].dof_version, c->f[0].edof_version,
+                             c->f[1].mesh_version, c->f[1].dof_version, c->f[1].edof_version};
+    auto &R = c->rows;
+    const bool known = R.valid && R.kind == pb->kind && R.fe == pb->fe && R.fe_p == pb->fe_p && R.ndofs == ndofs &&
+                       memcmp(R.key, key, sizeof key) == 0;
+    bool buckets = bucket_form_takes(m, E, ndofs) && !(known && R.toolong);
+    int rc;
+    if ((rc = ensure(c, c->vals[0], 8 * n)) || (vec && (rc = ensure(c, c->fvals[0], 8 * nv))) ||
+        (vec && (rc = ensure(c, c->F, 8 * ndofs))) || (rc = ensure(c, c->ptr, 4 * (ndofs + 1))) ||
+        (rc = ensure(c, c->ind, 4 * n)) || (rc = ensure(c, c->val, 8 * n)) || (rc = ensure(c, c->geom, 4 * E * m.nd)) ||
+        (buckets && (rc = ensure(c, c->keys[0], bucket_form_bytes(m, E, ndofs)))))
+        return rc;
+    int32_t *edof = (int32_t *)c->geom.p;
+    hipEvent_t ev = nullptr;
+    tm_begin(c, ELFEL_PH_GATHER, &ev);
+    if ((rc = form_dofs(c, m, edof))) return rc;
+    tm_end(c, ELFEL_PH_GATHER, ev);
+    const StreamOut so{c->vals[0].p, vec ? c->fvals[0].p : nullptr};
+    if ((rc = elements(so, false))) return rc;
+    if (buckets) {
+        const BucketOut o{(int32_t *)c->ptr.p, (int32_t *)c->ind.p, (double *)c->val.p, vec ? (double *)c->F.p : nullptr,
+                          nullptr, nullptr, nullptr, nullptr};
+        if ((rc = bucket_form(c, c->keys[0].p, m, E, edof, ndofs, (const double *)so.vals, (const double *)so.fvals, o)))
+            return rc;
+        if (!known) {
+            HIPCHK(c, hipStreamSynchronize(c->stream));
+            R.toolong = ((const int32_t *)c->told)[2] != 0;
+            R.kind = pb->kind; R.fe = pb->fe; R.fe_p = pb->fe_p; R.ndofs = ndofs;
+            memcpy(R.key, key, sizeof key);
+            R.valid = true;
+            buckets = !R.toolong;
+        }
+        c->nnz_told = buckets;
+    }
+    if (!buckets && (rc = build_by_sort(c, m, E, edof, ndofs))) return rc;
     c->has_F = vec;
     c->nF = vec ? ndofs : 0;
     c->nmaj = ndofs;
     c->nmin = ndofs;
-    c->layout = layout;
+    c->layout = pb->layout;
     c->result_src = RES_PLAIN;
     return 0;
 }
 
-// The 2D weak forms on the stream REUSE method (FP64): the element kernel of
-// the plain method writes keys on the first call, values only afterwards, and
-// every entry is the sum of its run in the cached sort order.
+// The stream of a 2D weak form: the block column-major; Stokes then kup
+// column-major and transpose(kup) row-major of kup.
+static void plain_map(const Field &F, const elfel_hip_problem *pb, FormMap &m)
+{
+    const bool stokes = pb->kind == ELFEL_STOKES_GEN || pb->kind == ELFEL_STOKES_VECLAP;
+    const int csc = pb->layout == ELFEL_CSC ? 1 : 0;
+    const int nu = F.nen * F.ncomp;
+    if (!stokes) {
+        form_square(m, nu, csc);
+        m.nvec = pb->kind == ELFEL_HEAT ? nu : 0;
+    } else {
+        const int nd = nu + 3;
+        m.nd = nd;
+        m.nmat = nu * nu + 6 * nu;
+        // entry (row i, column j) of the element block in stream order, -1: none
+        auto at = [&](int i, int j) {
+            if (i < nu && j < nu) return i + nu * j;
+            if (i < nu) return nu * nu + (j - nu) * nu + i;
+            if (j < nu) return nu * nu + 3 * nu + j * 3 + (i - nu);
+            return -1;
+        };
+        for (int a = 0; a < nd; a++) {
+            m.ncol[a] = (uint8_t)(a < nu ? nd : nu);
+            for (int b = 0; b < nd; b++) m.pos[a * nd + b] = (int16_t)(csc ? at(b, a) : at(a, b));
+        }
+        for (int k = 0; k < 3; k++) m.src[nu + k] = {1, 0, (uint8_t)k, 0};
+    }
+    for (int i = 0; i < nu; i++) m.src[i] = {0, 0, (uint8_t)(i / F.ncomp), (uint8_t)(i % F.ncomp)};
+}
+
+// The 2D weak forms on the stream REUSE method (FP64): every entry is the sum
+// of its run in the cached sort order.
 int plain_stream_reuse(elfel_hip_ctx *c, const elfel_hip_problem *pb, const QTable &tab, const Coef &cf)
 {
     const Field &F = c->f[0];
-    const bool stokes = pb->kind == ELFEL_STOKES_GEN || pb->kind == ELFEL_STOKES_VECLAP;
     plain_fn fn = pick_plain(pb->kind, pb->fe, tab.nq);
     if (!fn) return set_err(c, ELFEL_ENOTSUP, "unsupported (kind, element, rule) for the plain method");
-    const int64_t nd = (int64_t)F.nen * F.ncomp;
-    const int64_t n = F.E * (nd * nd + (stokes ? 2 * nd * 3 : 0));
-    const bool heat = pb->kind == ELFEL_HEAT;
-    const int64_t nv = heat ? F.E * nd : 0;
-    const int64_t ndofs = c->nrow;
-    const int minor_bits = bits_for(ndofs);
-    const int csc = pb->layout == ELFEL_CSC ? 1 : 0;
+    FormMap m;
+    plain_map(F, pb, m);
     elfel_hip_problem p = *pb;
     p.precision = ELFEL_FP64;
-    if (n >= INT32_MAX || nv >= INT32_MAX) {  // the cached permutation is int32
+    if (F.E * m.nmat >= INT32_MAX || F.E * m.nvec >= INT32_MAX) {  // the cached permutation is int32
         p.method = ELFEL_SORT;
         c->used_method = ELFEL_SORT;
         c->used_note += " (a COO stream of 2^31 entries or more: the plain FP64 method)";
         c->nnz = -1;
         return plain_assemble(c, &p, tab, cf);
     }
-    return stream_reuse(c, &p, n, nv, ndofs, minor_bits, false, [&](const StreamOut &o, bool) {
-        return fn(c, tab, cf, minor_bits, csc, o.keys, (double *)o.vals, o.fkeys, (double *)o.fvals);
+    return stream_reuse(c, &p, m, F.E, c->nrow, false, [&](const StreamOut &o, bool) {
+        return fn(c, tab, cf, (double *)o.vals, (double *)o.fvals);
     });
 }
 
 int plain_assemble(elfel_hip_ctx *c, const elfel_hip_problem *pb, const QTable &tab, const Coef &cf)
 {
-    const Field &F = c->f[0];
-    const bool stokes = pb->kind == ELFEL_STOKES_GEN || pb->kind == ELFEL_STOKES_VECLAP;
     plain_fn fn = pick_plain(pb->kind, pb->fe, tab.nq);
     if (!fn) return set_err(c, ELFEL_ENOTSUP, "unsupported (kind, element, rule) for the plain method");
-    const int nc = F.ncomp, nen = F.nen;
-    const int64_t nd = (int64_t)nen * nc;
-    const int64_t nblk = nd * nd + (stokes ? 2 * nd * 3 : 0);
-    const int64_t n = F.E * nblk;
-    const int64_t ndofs = c->nrow;
-    const int csc = pb->layout == ELFEL_CSC ? 1 : 0;
-    const int minor_bits = bits_for(ndofs);
-    const bool heat = pb->kind == ELFEL_HEAT;
-    const int64_t nv = heat ? F.E * nd : 0;
-    int rc = plain_buffers(c, n, nv, ndofs, heat);
-    if (rc) return rc;
-    rc = fn(c, tab, cf, minor_bits, csc, (uint64_t *)c->keys[0].p, (double *)c->vals[0].p,
-            heat ? (uint64_t *)c->fkeys[0].p : nullptr, heat ? (double *)c->fvals[0].p : nullptr);
-    if (rc) return rc;
-    return plain_finish(c, pb->layout, n, nv, ndofs, minor_bits, heat);
+    FormMap m;
+    plain_map(c->f[0], pb, m);
+    return plain_build(c, pb, m, c->f[0].E, c->nrow, [&](const StreamOut &o, bool) {
+        return fn(c, tab, cf, (double *)o.vals, (double *)o.fvals);
+    });
 }

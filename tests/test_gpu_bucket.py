@@ -8,6 +8,7 @@ import pytest
 
 import oracle as O
 from elfel_hip import _lib as L
+from test_gpu_general_meshes import _oracle_heat, _same, fan_mesh
 from test_zz_no_alloc import Hip, _noalloc
 
 pytestmark = pytest.mark.gpu
@@ -95,3 +96,26 @@ def test_bucket_build_refuses_then_works(ctx):
     ref = O.sparse(I, J, V, 30, 30, csc=False)
     for a, b in zip(ctx.copy_sparse(base=0)[:3], ref):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("method", [L.SORT, L.REUSE])
+@pytest.mark.parametrize("layout", [L.CSR, L.CSC])
+def test_element_stream_at_the_longest_row(ctx, method, layout):
+    """A T3 fan's centre row has 3 K entries: 170 and 171 elements lie either
+    side of the 512 that a tile holds.  One context, so that the answer for one
+    mesh must not outlive it, with and without a wait, and a dof that two nodes
+    (hence an element's two local dofs) share."""
+    for K, tie in ((170, False), (171, False), (40, True), (170, False), (171, True), (30, False)):
+        conn, xy = fan_mesh(K, rings=2)
+        dn = np.random.default_rng(K).permutation(xy.shape[0]) + 1
+        if tie:
+            dn[2] = dn[1]  # neighbours on the first ring: one dof twice in an element
+        n = xy.shape[0]
+        ref = _oracle_heat(conn, xy, dn, n, layout)
+        ctx.set_mesh(0, conn, xy)
+        ctx.set_dofs(0, dn, n)
+        ctx.set_coefficients(conn.shape[0])
+        for wait in (True, False, False):
+            ctx.assemble(L.HEAT, L.T3, 1, method=method, layout=layout, kappa=1.3, Q=-2.0, wait=wait)
+            _same(ctx.copy_sparse(base=0), ref)
+            assert np.array_equal(ctx.copy_vector(n), ref[3])
