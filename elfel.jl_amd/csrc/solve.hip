@@ -30,13 +30,13 @@
 // the CSR matrix).  When every free column lies within a 16-bit offset of its
 // row (banded numberings: structured grids, RCM-ordered meshes) the columns
 // are stored as int16 offsets, 2 bytes per entry instead of 4.
-// Per iteration three kernels on a fixed grid of 4 workgroups per CU
-// (grid-stride loops): q = A p with one partial of p.q per workgroup; the
-// x / r / z update (every workgroup first sums the p.q and previous r.z
-// partials itself, in the same order) with partials of r.z and r.r; and
-// p = z + beta p.  No atomics and no extra reduction launches; every run gives
-// the same bits.  The CG scalars stay on the device and the host reads the
-// residual every CHECK iterations.
+// Per iteration two kernels on a fixed grid of 4 workgroups per CU (grid-stride
+// loops): q = A p with the new direction formed on the way, one partial of p.q
+// per workgroup; and the r / z update (every workgroup first sums the p.q
+// partials itself, in the same order) with partials of r.z and r.r.  No atomics
+// and no extra reduction launches; every run gives the same bits.  The CG
+// scalars stay on the device and the host reads the residual every CHECK
+// iterations.
 #include <math.h>
 
 #include <algorithm>
@@ -49,6 +49,9 @@ int env_int(const char *name, int dflt);  // reuse.hip
 #define SV_BLOCK 256
 #define CHECK 8
 #define SELL_UNROLL 12  // slices at most this wide are read with every load in flight at once
+#ifndef UP_ROWS
+#define UP_ROWS 4       // rows of the update likewise
+#endif
 #ifndef RU_DROP
 #define RU_DROP 1e-2   // reliable update when the recurrence residual has dropped by this factor
 #endif
@@ -59,7 +62,7 @@ int env_int(const char *name, int dflt);  // reuse.hip
 namespace {
 
 // Scalars (double) on the device, for the host's convergence checks.
-enum { S_RZ = 0, S_RR = 1, S_BB = 2, S_RR64 = 3, S_NS = 8 };
+enum { S_RZ = 0, S_RR = 1, S_BB = 2, S_RR64 = 3, S_ALPHA = 4, S_RZS = 5 /* two words */, S_NS = 8 };
 
 __device__ __forceinline__ double block_sum(double v, double *sh)
 {
@@ -71,6 +74,16 @@ __device__ __forceinline__ double block_sum(double v, double *sh)
     double s = 0.0;
     for (int k = 0; k < (int)(blockDim.x >> 6); k++) s += sh[k];
     return s;  // the same value in every thread
+}
+
+// The block of rows that a workgroup takes: workgroups go to the XCDs in turn, so
+// XCD x (of 8) takes the x-th eighth of the blocks, and the neighbouring rows
+// that a product gathers are read into one L2 instead of three (the solve on
+// 1500x1300 quads 240 -> 227 ms).
+__device__ __forceinline__ uint32_t row_block()
+{
+    const uint32_t g = gridDim.x, b = blockIdx.x;
+    return (g & 7) == 0 ? (b & 7) * (g >> 3) + (b >> 3) : b;
 }
 
 // Fixed-order sum of the g partials of the previous kernel (every block of
@@ -184,166 +197,275 @@ struct SellU {
 // A slice's start, width and uniform flag (the first loads of its row).
 struct SliceMeta {
     uint32_t o, w;
-    bool uni;
+    uint32_t uni;
 };
 __device__ __forceinline__ SliceMeta slice_meta(int64_t i, const uint32_t *__restrict__ off, SellU U)
 {
     // one wave holds one slice: s is the same on every lane
     const int64_t s = __builtin_amdgcn_readfirstlane((int)(i >> 6));
     const uint32_t o = off[s];
-    return SliceMeta{o, (off[s + 1] - o) >> 6, U.uflag[s] != 0u};
+    return SliceMeta{o, (off[s + 1] - o) >> 6, U.uflag[s]};
 }
 
-template <typename T, typename C>
-__device__ __forceinline__ T sell_row(int64_t i, const uint32_t *__restrict__ off, const C *__restrict__ col,
-                                      const T *__restrict__ val, const T *__restrict__ x, SellU U,
-                                      SliceMeta m)
-{
-    const int lane = (int)(i & 63);
-    const uint32_t o = m.o, w = m.w;
-    T acc = T(0);
-    const T *v = val + o + lane;
-    const C *c = col + o + lane;
-    const bool uni = m.uni;
-    const int32_t *d = U.uoff + (o >> 6);
-    const int32_t ri = (int32_t)i;
-    if (w <= SELL_UNROLL) {
-        // every load of the slice is issued before the first product: the
-        // values and (uniform slices) the gathers at once, else the columns,
-        // then the gathers.  Slots past w read slot 0 again (in bounds) and
-        // add nothing; in uniform slices they are skipped (w is the same on
-        // every lane), and the values, read once per product, bypass the
-        // caches that hold the vector
-        T vv[SELL_UNROLL], xx[SELL_UNROLL];
-        if (uni) {
+// What a product gathers: a vector, or the search direction z + beta p formed
+// on the way (the new direction of a neighbour's row is not written yet).
+template <typename T>
+struct VecGather {
+    const T *__restrict__ x;
+    struct Part { T a; };
+    __device__ __forceinline__ Part load(int32_t j) const { return Part{x[j]}; }
+    __device__ __forceinline__ T value(Part v) const { return v.a; }
+};
+template <typename T>
+struct DirGather {
+    const T *__restrict__ z, *__restrict__ p;
+    T beta;
+    struct Part { T a, b; };
+    __device__ __forceinline__ Part load(int32_t j) const { return Part{z[j], p[j]}; }
+    __device__ __forceinline__ T value(Part v) const { return v.a + beta * v.b; }
+};
+
+// A row's loads (slices of at most SELL_UNROLL entries), issued together ahead
+// of the sums: the values and (uniform slices) the gathers at once, else the
+// columns, then the gathers.  In uniform slices the slots past w are skipped
+// (w is the same on every lane), else they read slot 0 again (in bounds) and
+// add nothing; the values, read once per product, bypass the caches that hold
+// the vectors.
+template <typename T, typename C, typename V>
+struct RowLoads {
+    T v[SELL_UNROLL];
+    typename V::Part x[SELL_UNROLL];
+
+    __device__ __forceinline__ void load(int64_t i, const C *__restrict__ col, const T *__restrict__ val,
+                                         const V &g, SellU U, SliceMeta m)
+    {
+        const int lane = (int)(i & 63);
+        const T *vp = val + m.o + lane;
+        const C *c = col + m.o + lane;
+        const int32_t *d = U.uoff + (m.o >> 6);
+        const int32_t ri = (int32_t)i;
+        if (m.uni) {
+            // all offsets at once (the array is as much longer than its slots):
+            // read slot by slot behind k < w they came one scalar load after
+            // another, 0.2 us each
+            int32_t dk[SELL_UNROLL];
+#pragma unroll
+            for (int k = 0; k < SELL_UNROLL; k++) dk[k] = d[k];
 #pragma unroll
             for (int k = 0; k < SELL_UNROLL; k++) {
-                vv[k] = T(0);
-                xx[k] = T(0);
-                if (k < (int)w) {
-                    vv[k] = __builtin_nontemporal_load(v + (size_t)k * 64);
-                    xx[k] = x[ri + d[k]];
+                if (k < (int)m.w) {
+                    v[k] = __builtin_nontemporal_load(vp + (size_t)k * 64);
+                    x[k] = g.load(ri + dk[k]);
                 }
             }
         } else {
             int32_t cj[SELL_UNROLL];
 #pragma unroll
             for (int k = 0; k < SELL_UNROLL; k++) {
-                const int kk = k < (int)w ? k : 0;
-                vv[k] = v[(size_t)kk * 64];
+                const int kk = k < (int)m.w ? k : 0;
+                v[k] = vp[(size_t)kk * 64];
                 cj[k] = sell_col<C>(c[(size_t)kk * 64], i);
             }
 #pragma unroll
-            for (int k = 0; k < SELL_UNROLL; k++) xx[k] = x[cj[k]];
+            for (int k = 0; k < SELL_UNROLL; k++) x[k] = g.load(cj[k]);
         }
+    }
+    __device__ __forceinline__ T sum(const V &g, SliceMeta m) const
+    {
+        T acc = T(0);
 #pragma unroll
         for (int k = 0; k < SELL_UNROLL; k++)
-            if (k < (int)w) acc += vv[k] * xx[k];
+            if (k < (int)m.w) acc += v[k] * g.value(x[k]);
         return acc;
     }
-    if (uni) {
+};
+
+template <typename T, typename C, typename V>
+__device__ __forceinline__ T sell_row(int64_t i, const C *__restrict__ col, const T *__restrict__ val, const V &g, SellU U,
+                                      SliceMeta m)
+{
+    if (m.w <= SELL_UNROLL) {
+        RowLoads<T, C, V> R;
+        R.load(i, col, val, g, U, m);
+        return R.sum(g, m);
+    }
+    const int lane = (int)(i & 63);
+    const T *v = val + m.o + lane;
+    const C *c = col + m.o + lane;
+    const int32_t *d = U.uoff + (m.o >> 6);
+    const int32_t ri = (int32_t)i;
+    T acc = T(0);
+    if (m.uni) {
 #pragma unroll 4
-        for (uint32_t k = 0; k < w; k++) acc += v[(size_t)k * 64] * x[ri + d[k]];
+        for (uint32_t k = 0; k < m.w; k++) acc += v[(size_t)k * 64] * g.value(g.load(ri + d[k]));
     } else {
 #pragma unroll 4
-        for (uint32_t k = 0; k < w; k++) acc += v[(size_t)k * 64] * x[sell_col<C>(c[(size_t)k * 64], i)];
+        for (uint32_t k = 0; k < m.w; k++) acc += v[(size_t)k * 64] * g.value(g.load(sell_col<C>(c[(size_t)k * 64], i)));
     }
     return acc;
 }
 
 // The CG kernels run on a fixed grid of G workgroups with grid-stride loops
 // over the rows; each writes one partial per workgroup per dot product.
-//   parts layout: pq[G], rz[2][G] (by iteration parity), rr[G], aux[G]
+//   parts layout: pq[G], rz[G], rr[G], aux[G]
+//
+// Two kernels an iteration.  The product forms the new direction itself,
+// p = z + beta p, for its own row (stored, in the other of two buffers) and for
+// each entry it gathers, and adds the previous step to the iterate while it
+// holds the previous direction: a pass over z, p and p' and a launch less than
+// a direction kernel, and the update does not read p.  k_cg_fin closes a group
+// of CHECK iterations.  The dot products are summed as ever, so the bits are
+// those of the three-kernel iteration.  Mixed heat Q4 1500x1300, an iteration:
+// 55.7 -> 44.8 us (rows of the neighbouring blocks on one XCD: 5 us of it);
+// bytes a row (nine entries) 88 -> 80.  Two rows of loads in flight per
+// work-item measured slower than one (57 us: 144 registers, three waves a SIMD
+// where the grid has four), and so did taking the grid neighbours' values from
+// the next lane in place of two thirds of the gathers (46.6 us: L1 is not the
+// bound).
 
-// q = A p; partial p.q
-template <typename T, typename C>
-__global__ __launch_bounds__(SV_BLOCK) void k_cg_spmv(int64_t n, const uint32_t *__restrict__ off,
+// The iterate's last step, x += alpha p: the FP64 solve updates its FP64
+// iterate (TX = double).  The mixed solve adds alpha p to an FP32 accumulator
+// of the last few iterations' steps (TX = float), which k_cg_fin folds into the
+// FP64 iterate every CHECK iterations: an FP32 iterate itself absorbs the late,
+// small corrections (x + alpha p rounds back to x; the mixed solve then needed
+// 69 % more iterations than FP64 PCG on heat Q4 1024^2 against 9 % with an FP64
+// iterate, numpy emulation of this code), while the accumulator holds only
+// corrections, so each keeps its FP32 relative precision.
+//
+// DIR: p = z + beta p_old into p, x += alpha p_old; else the product with p_old
+// as it is (the first iteration of a group).  q = A p; partial p.q.  Workgroup 0
+// leaves this iteration's r.z in rzs[par].
+template <typename T, typename TX, typename C, bool DIR>
+__global__ __launch_bounds__(SV_BLOCK, 4) void k_cg_spmv(int64_t n, const uint32_t *__restrict__ off,
                                                       const C *__restrict__ col, const T *__restrict__ val,
-                                                      SellU U, const T *__restrict__ p, T *__restrict__ q,
+                                                      SellU U, const T *__restrict__ z, const T *__restrict__ p_old,
+                                                      T *__restrict__ p, T *__restrict__ q, TX *__restrict__ x,
+                                                      const double *__restrict__ part_rz, double *__restrict__ sc, int par,
                                                       double *__restrict__ part_pq)
 {
     __shared__ double sh[SV_BLOCK / 64];
+    using V = typename std::conditional<DIR, DirGather<T>, VecGather<T>>::type;
+    const int64_t stride = (int64_t)gridDim.x * SV_BLOCK;
+    const uint32_t blk = row_block();
+    int64_t i = (int64_t)blk * SV_BLOCK + threadIdx.x;
+    V g;
+    if constexpr (DIR) { g.z = z; g.p = p_old; } else g.x = p_old;
+    RowLoads<T, C, V> R0;
+    SliceMeta m0{0, 0, 0};
+    if (i < n) {
+        m0 = slice_meta(i, off, U);
+        if (m0.w <= SELL_UNROLL) R0.load(i, col, val, g, U, m0);
+    }
+    const double rz = sum_partials(part_rz, gridDim.x, sh);
+    if (blockIdx.x == 0 && threadIdx.x == 0) sc[S_RZS + par] = rz;
+    TX alphax = TX(0);
+    if constexpr (DIR) {
+        const double rz_old = sc[S_RZS + (par ^ 1)];
+        g.beta = (T)(rz_old != 0.0 ? rz / rz_old : 0.0);
+        alphax = (TX)sc[S_ALPHA];
+    }
     double d = 0.0;
-    // (Loading the next slice's start, width and flag while this slice's row
-    // is summed measured slower: 544 against 373 us per mixed iteration on
-    // heat Q4 4096^2.)
-    for (int64_t i = (int64_t)blockIdx.x * SV_BLOCK + threadIdx.x; i < n; i += (int64_t)gridDim.x * SV_BLOCK) {
-        const T y = sell_row<T, C>(i, off, col, val, p, U, slice_meta(i, off, U));
-        q[i] = y;
-        d += (double)p[i] * (double)y;
+    auto finish = [&](int64_t r, T y) {
+        T pr = p_old[r];
+        if constexpr (DIR) {
+            x[r] += alphax * (TX)pr;
+            pr = z[r] + g.beta * pr;
+            p[r] = pr;
+        }
+        q[r] = y;
+        d += (double)pr * (double)y;
+    };
+    while (i < n) {
+        finish(i, m0.w <= SELL_UNROLL ? R0.sum(g, m0) : sell_row<T, C, V>(i, col, val, g, U, m0));
+        i += stride;
+        if (i < n) {
+            m0 = slice_meta(i, off, U);
+            if (m0.w <= SELL_UNROLL) R0.load(i, col, val, g, U, m0);
+        }
     }
     const double s = block_sum(d, sh);
-    if (threadIdx.x == 0) part_pq[blockIdx.x] = s;
+    if (threadIdx.x == 0) part_pq[blk] = s;
 }
 
-// alpha = rz_old / pq; x += alpha p; r -= alpha q; z = M r; partials r.z (into
-// rz_new) and r.r
-// The FP64 solve updates its FP64 iterate here (TX = double).  The mixed
-// solve adds alpha p to an FP32 accumulator of the last few iterations' steps
-// (TX = float), which k_cg_flush folds into the FP64 iterate every CHECK
-// iterations: an FP32 iterate itself absorbs the late, small corrections
-// (x + alpha p rounds back to x; the mixed solve then needed 69 % more
-// iterations than FP64 PCG on heat Q4 1024^2 against 9 % with an FP64
-// iterate, numpy emulation of this code), while the accumulator holds only
-// corrections, so each keeps its FP32 relative precision.
-template <typename T, typename TX>
-__global__ __launch_bounds__(SV_BLOCK) void k_cg_update(int64_t n, const T *__restrict__ dinv, TX *__restrict__ x,
-                                                        T *__restrict__ r, T *__restrict__ z,
-                                                        const T *__restrict__ p, const T *__restrict__ q,
-                                                        const double *__restrict__ part_pq,
-                                                        const double *__restrict__ rz_old,
-                                                        double *__restrict__ rz_new, double *__restrict__ part_rr)
+// alpha = rz / pq; r -= alpha q; z = M r; partials r.z and r.r
+template <typename T>
+__global__ __launch_bounds__(SV_BLOCK) void k_cg_update(int64_t n, const T *__restrict__ dinv, T *__restrict__ r,
+                                                        T *__restrict__ z, const T *__restrict__ q,
+                                                        const double *__restrict__ part_pq, double *__restrict__ sc,
+                                                        int par, double *__restrict__ part_rz,
+                                                        double *__restrict__ part_rr)
 {
     __shared__ double sh[SV_BLOCK / 64];
     const int G = gridDim.x;
+    const int64_t stride = (int64_t)G * SV_BLOCK;
+    int64_t i = (int64_t)blockIdx.x * SV_BLOCK + threadIdx.x;
+    // the first rows' loads are in flight while alpha is formed
+    T rr[UP_ROWS], qq[UP_ROWS], dd[UP_ROWS];
+    auto load = [&]() {
+#pragma unroll
+        for (int u = 0; u < UP_ROWS; u++) {
+            const int64_t j = i + u * stride < n ? i + u * stride : n - 1;
+            rr[u] = r[j];
+            qq[u] = q[j];
+            dd[u] = dinv[j];
+        }
+    };
+    load();
+    const double rz = sc[S_RZS + par];
     const double pq = sum_partials(part_pq, G, sh);
-    const double rz = sum_partials(rz_old, G, sh);
     const double alpha64 = pq != 0.0 ? rz / pq : 0.0;
     const T alpha = (T)alpha64;
-    const TX alphax = (TX)alpha64;
+    if (blockIdx.x == 0 && threadIdx.x == 0) sc[S_ALPHA] = alpha64;
     double a = 0.0, b = 0.0;
-    for (int64_t i = (int64_t)blockIdx.x * SV_BLOCK + threadIdx.x; i < n; i += (int64_t)G * SV_BLOCK) {
-        x[i] += alphax * (TX)p[i];
-        const T ri = r[i] - alpha * q[i];
-        const T zi = dinv[i] * ri;
-        r[i] = ri;
-        z[i] = zi;
-        a += (double)ri * (double)zi;
-        b += (double)ri * (double)ri;
+    while (i < n) {
+#pragma unroll
+        for (int u = 0; u < UP_ROWS; u++) {
+            if (i + u * stride >= n) break;
+            const T ri = rr[u] - alpha * qq[u];
+            const T zi = dd[u] * ri;
+            r[i + u * stride] = ri;
+            z[i + u * stride] = zi;
+            a += (double)ri * (double)zi;
+            b += (double)ri * (double)ri;
+        }
+        i += UP_ROWS * stride;
+        if (i < n) load();
     }
     a = block_sum(a, sh);
     b = block_sum(b, sh);
-    if (threadIdx.x == 0) { rz_new[blockIdx.x] = a; part_rr[blockIdx.x] = b; }
+    if (threadIdx.x == 0) { part_rz[blockIdx.x] = a; part_rr[blockIdx.x] = b; }
 }
 
-// x += xlo, xlo = 0: the mixed solve's accumulated steps into its FP64 iterate
-__global__ void k_cg_flush(int64_t n, double *__restrict__ x, float *__restrict__ xlo)
-{
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) {
-        x[i] += (double)xlo[i];
-        xlo[i] = 0.f;
-    }
-}
-
-// beta = rz_new / rz_old; p = z + beta p.  Workgroup 0 also leaves rz and
-// ||r||^2 for the host.
-template <typename T>
-__global__ __launch_bounds__(SV_BLOCK) void k_cg_dir(int64_t n, const double *__restrict__ rz_new,
-                                                     const double *__restrict__ rz_old,
+// The end of a group of iterations: x += alpha p (and, mixed, the accumulated
+// steps xlo into the FP64 iterate), p = z + beta p.  Workgroup 0 also leaves rz
+// and ||r||^2 for the host.
+template <typename T, typename TX>
+__global__ __launch_bounds__(SV_BLOCK) void k_cg_fin(int64_t n, const double *__restrict__ part_rz,
                                                      const double *__restrict__ part_rr, const T *__restrict__ z,
-                                                     T *__restrict__ p, double *__restrict__ sc)
+                                                     T *__restrict__ p, TX *__restrict__ xs, double *__restrict__ x,
+                                                     double *__restrict__ sc, int par)
 {
     __shared__ double sh[SV_BLOCK / 64];
     const int G = gridDim.x;
-    const double a = sum_partials(rz_new, G, sh);
-    const double b = sum_partials(rz_old, G, sh);
-    const T beta = (T)(b != 0.0 ? a / b : 0.0);
-    for (int64_t i = (int64_t)blockIdx.x * SV_BLOCK + threadIdx.x; i < n; i += (int64_t)G * SV_BLOCK)
-        p[i] = z[i] + beta * p[i];
+    const double rz = sum_partials(part_rz, G, sh);
+    const double rz_old = sc[S_RZS + par];
+    const T beta = (T)(rz_old != 0.0 ? rz / rz_old : 0.0);
+    const TX alphax = (TX)sc[S_ALPHA];
+    for (int64_t i = (int64_t)blockIdx.x * SV_BLOCK + threadIdx.x; i < n; i += (int64_t)G * SV_BLOCK) {
+        const T pr = p[i];
+        TX t = xs[i];
+        t += alphax * (TX)pr;
+        if constexpr (sizeof(TX) == 4) {
+            x[i] += (double)t;
+            xs[i] = TX(0);
+        } else {
+            xs[i] = t;
+        }
+        p[i] = z[i] + beta * pr;
+    }
     if (blockIdx.x == 0) {
         const double rr = sum_partials(part_rr, G, sh);
-        if (threadIdx.x == 0) { sc[S_RZ] = a; sc[S_RR] = rr; }
+        if (threadIdx.x == 0) { sc[S_RZ] = rz; sc[S_RR] = rr; }
     }
 }
 
@@ -395,7 +517,7 @@ __global__ __launch_bounds__(SV_BLOCK) void k_sell_resid(int64_t n, const uint32
     __shared__ double sh[SV_BLOCK / 64];
     double rr = 0.0;
     for (int64_t i = (int64_t)blockIdx.x * SV_BLOCK + threadIdx.x; i < n; i += (int64_t)gridDim.x * SV_BLOCK) {
-        const double v = b[i] - sell_row<double, C>(i, off, col, val, x, U, slice_meta(i, off, U));
+        const double v = b[i] - sell_row<double, C>(i, col, val, VecGather<double>{x}, U, slice_meta(i, off, U));
         r[i] = v;
         rr += v * v;
     }
@@ -451,8 +573,8 @@ __global__ void k_fill(int64_t n, T *__restrict__ a, T v)
 template <typename T>
 struct Vecs {
     double *x;  // the iterate: FP64 in both solves
-    T *r, *z, *p, *q, *dinv;
-    float *xlo;  // mixed solve: the steps since the last k_cg_flush (null: x updated directly)
+    T *r, *z, *p, *p2, *q, *dinv;
+    float *xlo;  // mixed solve: the steps since the last k_cg_fin (null: x updated directly)
 };
 
 struct Sell {
@@ -472,29 +594,41 @@ template <>
 const float *sell_vals<float>(const Sell &S) { return S.v32; }
 
 struct Parts {
-    double *pq, *rz[2], *rr, *aux;
+    double *pq, *rz, *rr, *aux;
     int G;
 };
 
-// One PCG iteration on the stream; `par` is the iteration parity (the rz
-// partials of this iteration go to rz[par], the previous ones are rz[par ^ 1]).
-template <typename T>
-void cg_step(hipStream_t st, int64_t n, const Sell &S, const Vecs<T> &v, const Parts &P, int par, double *sc)
+template <typename T, typename TX, typename C>
+void cg_group_as(hipStream_t st, int64_t n, const Sell &S, Vecs<T> &v, TX *xs, const Parts &P, double *sc)
 {
     const dim3 g(P.G), b(SV_BLOCK);
-    if (S.c16)
-        hipLaunchKernelGGL((k_cg_spmv<T, int16_t>), g, b, 0, st, n, S.off, (const int16_t *)S.col, sell_vals<T>(S), S.U,
-                           v.p, v.q, P.pq);
-    else
-        hipLaunchKernelGGL((k_cg_spmv<T, int32_t>), g, b, 0, st, n, S.off, (const int32_t *)S.col, sell_vals<T>(S), S.U,
-                           v.p, v.q, P.pq);
-    if (v.xlo)
-        hipLaunchKernelGGL((k_cg_update<T, float>), g, b, 0, st, n, v.dinv, v.xlo, v.r, v.z, v.p, v.q, P.pq,
-                           P.rz[par ^ 1], P.rz[par], P.rr);
-    else
-        hipLaunchKernelGGL((k_cg_update<T, double>), g, b, 0, st, n, v.dinv, v.x, v.r, v.z, v.p, v.q, P.pq,
-                           P.rz[par ^ 1], P.rz[par], P.rr);
-    hipLaunchKernelGGL((k_cg_dir<T>), g, b, 0, st, n, P.rz[par], P.rz[par ^ 1], P.rr, v.z, v.p, sc);
+    const C *col = (const C *)S.col;
+    const T *val = sell_vals<T>(S);
+    for (int k = 0; k < CHECK; k++) {
+        if (k == 0) {
+            hipLaunchKernelGGL((k_cg_spmv<T, TX, C, false>), g, b, 0, st, n, S.off, col, val, S.U, (const T *)v.z,
+                               (const T *)v.p, v.p2, v.q, xs, P.rz, sc, k & 1, P.pq);
+        } else {
+            hipLaunchKernelGGL((k_cg_spmv<T, TX, C, true>), g, b, 0, st, n, S.off, col, val, S.U, (const T *)v.z,
+                               (const T *)v.p, v.p2, v.q, xs, P.rz, sc, k & 1, P.pq);
+            std::swap(v.p, v.p2);
+        }
+        hipLaunchKernelGGL((k_cg_update<T>), g, b, 0, st, n, (const T *)v.dinv, v.r, v.z, (const T *)v.q, P.pq, sc, k & 1,
+                           P.rz, P.rr);
+    }
+    hipLaunchKernelGGL((k_cg_fin<T, TX>), g, b, 0, st, n, P.rz, P.rr, (const T *)v.z, v.p, xs, v.x, sc, (CHECK - 1) & 1);
+}
+
+// CHECK PCG iterations on the stream.
+void cg_group(hipStream_t st, int64_t n, const Sell &S, Vecs<double> &v, const Parts &P, double *sc)
+{
+    if (S.c16) cg_group_as<double, double, int16_t>(st, n, S, v, v.x, P, sc);
+    else cg_group_as<double, double, int32_t>(st, n, S, v, v.x, P, sc);
+}
+void cg_group(hipStream_t st, int64_t n, const Sell &S, Vecs<float> &v, const Parts &P, double *sc)
+{
+    if (S.c16) cg_group_as<float, float, int16_t>(st, n, S, v, v.xlo, P, sc);
+    else cg_group_as<float, float, int32_t>(st, n, S, v, v.xlo, P, sc);
 }
 
 }  // namespace
@@ -524,12 +658,12 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
     const int G = (int)std::max<int64_t>(1, std::min<int64_t>(ceil_div(n, SV_BLOCK), 4 * (int64_t)prop.multiProcessorCount));
 
     // ---- scratch layout (8-byte words first, then 4-byte) -----------------
-    // doubles: xfull[N], b[n], r64[n], dinv64[n], parts[5 G], sc[S_NS],
-    //          FP64 vectors r z p q [4n] (FP64 solve only)
-    // floats:  r z p q dinv xlo [6n] (mixed solve only; its iterate is the FP64 xfull + xlo)
+    // doubles: xfull[N], b[n], r64[n], dinv64[n], parts[4 G], sc[S_NS],
+    //          FP64 vectors r z p p2 q [5n] (FP64 solve only)
+    // floats:  r z p p2 q dinv xlo [7n] (mixed solve only; its iterate is the FP64 xfull + xlo)
     // uint32:  off[nslices + 1], len[max(n, nslices)], total[4]
-    const size_t nd = (size_t)N + 3 * (size_t)n + 5 * (size_t)G + S_NS + (mixed ? 0 : 4 * (size_t)n);
-    const size_t nf = mixed ? 6 * (size_t)n : 0;
+    const size_t nd = (size_t)N + 3 * (size_t)n + 4 * (size_t)G + S_NS + (mixed ? 0 : 5 * (size_t)n);
+    const size_t nf = mixed ? 7 * (size_t)n : 0;
     const size_t nu32 = (size_t)nslices + 1 + (size_t)std::max<int64_t>(n, nslices) + (size_t)n + 4;
     int rc = ensure(c, c->pcg, 8 * nd + 4 * nf + 4 * nu32 + 256);
     if (rc) return rc;
@@ -540,19 +674,19 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
     double *dinv64 = dp; dp += n;
     Parts P;
     P.G = G;
-    P.pq = dp; dp += G; P.rz[0] = dp; dp += G; P.rz[1] = dp; dp += G; P.rr = dp; dp += G; P.aux = dp; dp += G;
+    P.pq = dp; dp += G; P.rz = dp; dp += G; P.rr = dp; dp += G; P.aux = dp; dp += G;
     double *sc = dp; dp += S_NS;
     Vecs<double> v64{};
     if (!mixed) {
         v64.x = xfull;  // the free part of the full vector is the iterate
-        v64.r = dp; dp += n; v64.z = dp; dp += n; v64.p = dp; dp += n; v64.q = dp; dp += n;
+        v64.r = dp; dp += n; v64.z = dp; dp += n; v64.p = dp; dp += n; v64.p2 = dp; dp += n; v64.q = dp; dp += n;
         v64.dinv = dinv64;
     }
     float *fp = (float *)dp;
     Vecs<float> v32{};
     if (mixed) {
         v32.x = xfull;  // the free part of the full vector is the iterate (FP64)
-        v32.r = fp; fp += n; v32.z = fp; fp += n; v32.p = fp; fp += n; v32.q = fp; fp += n;
+        v32.r = fp; fp += n; v32.z = fp; fp += n; v32.p = fp; fp += n; v32.p2 = fp; fp += n; v32.q = fp; fp += n;
         v32.dinv = fp; fp += n;
         v32.xlo = fp; fp += n;
     }
@@ -580,7 +714,7 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
     const size_t cbytes = (size_t)nnzp * (c16 ? 2 : 4);
     const size_t nslots = (size_t)nnzp / 64;
     const size_t vbytes = (size_t)nnzp * (8 + (mixed ? 4 : 0));
-    const size_t sbytes = ((cbytes + 15) & ~(size_t)15) + vbytes + 4 * (size_t)(nslices + 1) + 4 * nslots + 256;
+    const size_t sbytes = ((cbytes + 15) & ~(size_t)15) + vbytes + 4 * (size_t)(nslices + 1) + 4 * (nslots + SELL_UNROLL) + 256;
     if ((rc = ensure(c, c->pcg_sell, sbytes))) return rc;
     void *scol = c->pcg_sell.p;
     double *sv64 = (double *)((char *)c->pcg_sell.p + ((cbytes + 15) & ~(size_t)15));
@@ -643,15 +777,13 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
         *out_norm = sqrt(std::max(hh[S_RR64], 0.0));
         return 0;
     };
-    // r = (T) r64, z = M r (p = z on restart); the rz partials go where the next
-    // step reads the previous ones (rz[par ^ 1]); sc gets rz and ||r||^2
-    int par = 0;
+    // r = (T) r64, z = M r (p = z on restart); sc gets rz and ||r||^2
     auto reset = [&](auto &v, int restart) {
         using T = typename std::remove_pointer<decltype(v.r)>::type;
         hipLaunchKernelGGL((k_cg_reset<T>), dim3(G), dim3(SV_BLOCK), 0, st, n, (const double *)r64,
-                           (const T *)v.dinv, v.r, v.z, v.p, restart, P.rz[par ^ 1], P.rr);
+                           (const T *)v.dinv, v.r, v.z, v.p, restart, P.rz, P.rr);
         hipLaunchKernelGGL(k_reduce, dim3(1), dim3(1024), 0, st, (const double *)P.rr, G, sc, (int)S_RR,
-                           (const double *)P.rz[par ^ 1], (int)S_RZ);
+                           (const double *)P.rz, (int)S_RZ);
     };
 
     int it = 0, nupd = 0;
@@ -667,7 +799,7 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
                 if ((rc = read_sc(h))) return rc;
                 rrec = h[S_RR];
                 if (!(rrec > target * target) || it >= maxit) break;
-                for (int k = 0; k < CHECK; k++, par ^= 1) cg_step<double>(st, n, S, v64, P, par, sc);
+                cg_group(st, n, S, v64, P, sc);
                 HIPCHK(c, hipGetLastError());
                 it += CHECK;
             }
@@ -689,8 +821,7 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
                 if ((rc = read_sc(h))) return rc;
                 rrec = h[S_RR];
                 if (!(rrec > goal * goal) || it >= maxit) break;
-                for (int k = 0; k < CHECK; k++, par ^= 1) cg_step<float>(st, n, S, v32, P, par, sc);
-                hipLaunchKernelGGL(k_cg_flush, dim3(ceil_div(n, 256)), dim3(256), 0, st, n, v32.x, v32.xlo);
+                cg_group(st, n, S, v32, P, sc);
                 HIPCHK(c, hipGetLastError());
                 it += CHECK;
             }
