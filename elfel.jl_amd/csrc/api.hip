@@ -106,11 +106,11 @@ void release(Buf &b)
 }
 
 // ---- pinned words of the contexts ------------------------------------------
-// 64 bytes of pinned host memory a context, from one page shared by the first
+// TOLD_BYTES of pinned host memory a context, from one page shared by the first
 // TOLD_SLOTS contexts (a pinned allocation of its own takes 0.3 ms of
 // elfel_hip_init); the page is freed with the last context that holds a slot.
 namespace {
-constexpr int TOLD_SLOTS = 64;
+constexpr int TOLD_SLOTS = 64, TOLD_BYTES = 256;
 std::mutex told_mu;
 char *told_page = nullptr;
 uint64_t told_used = 0;
@@ -119,7 +119,7 @@ uint64_t told_used = 0;
 static void *told_get()
 {
     std::lock_guard<std::mutex> g(told_mu);
-    if (!told_page && hipHostMalloc((void **)&told_page, 64 * TOLD_SLOTS, hipHostMallocPortable) != hipSuccess) {
+    if (!told_page && hipHostMalloc((void **)&told_page, TOLD_BYTES * TOLD_SLOTS, hipHostMallocPortable) != hipSuccess) {
         (void)hipGetLastError();
         told_page = nullptr;
         return nullptr;
@@ -127,10 +127,10 @@ static void *told_get()
     if (~told_used) {
         const int k = __builtin_ctzll(~told_used);
         told_used |= 1ull << k;
-        return told_page + 64 * k;
+        return told_page + TOLD_BYTES * k;
     }
     void *p = nullptr;
-    if (hipHostMalloc(&p, 64, hipHostMallocPortable) != hipSuccess) {
+    if (hipHostMalloc(&p, TOLD_BYTES, hipHostMallocPortable) != hipSuccess) {
         (void)hipGetLastError();
         return nullptr;
     }
@@ -142,11 +142,11 @@ static void told_put(void *p)
     if (!p) return;
     std::lock_guard<std::mutex> g(told_mu);
     const ptrdiff_t at = told_page ? (char *)p - told_page : -1;
-    if (at < 0 || at >= 64 * TOLD_SLOTS) {
+    if (at < 0 || at >= TOLD_BYTES * TOLD_SLOTS) {
         hipHostFree(p);
         return;
     }
-    told_used &= ~(1ull << (at / 64));
+    told_used &= ~(1ull << (at / TOLD_BYTES));
     if (!told_used) {
         hipHostFree(told_page);
         told_page = nullptr;

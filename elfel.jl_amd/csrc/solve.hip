@@ -62,7 +62,7 @@ int env_int(const char *name, int dflt);  // reuse.hip
 namespace {
 
 // Scalars (double) on the device, for the host's convergence checks.
-enum { S_RZ = 0, S_RR = 1, S_BB = 2, S_RR64 = 3, S_ALPHA = 4, S_RZS = 5 /* two words */, S_NS = 8 };
+enum { S_RZ = 0, S_RR = 1, S_BB = 2, S_RR64 = 3, S_ALPHA = 4, S_RZS = 5 /* two words */, S_IT = 7, S_RREC = 8, S_NS = 10 };
 
 __device__ __forceinline__ double block_sum(double v, double *sh)
 {
@@ -111,7 +111,7 @@ __global__ void k_sell_rowlen(int64_t nfree, const int32_t *__restrict__ ptr, co
         f |= (d < -32768 || d > 32767) ? 1u : 0u;
     }
     len[i] = k;
-    far[i] = f;
+    if (f) *far = 1u;
 }
 
 // Column of entry k of a SELL row: 32-bit index, or 16-bit offset from the row.
@@ -124,7 +124,7 @@ __device__ __forceinline__ int32_t sell_col<int16_t>(int16_t c, int64_t row) { r
 
 // One wave per slice: width = longest row; writes 64 * width (the slice size).
 __global__ void k_sell_width(int64_t nfree, int64_t nslices, const uint32_t *__restrict__ len,
-                             uint32_t *__restrict__ size)
+                             uint32_t *__restrict__ size, uint32_t *__restrict__ wide)
 {
     const int64_t s = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const int lane = threadIdx.x & 63;
@@ -132,7 +132,10 @@ __global__ void k_sell_width(int64_t nfree, int64_t nslices, const uint32_t *__r
     const int64_t row = s * 64 + lane;
     uint32_t w = row < nfree ? len[row] : 0u;
     for (int d = 32; d > 0; d >>= 1) w = max(w, (uint32_t)__shfl_down((int)w, d, 64));
-    if (lane == 0) size[s] = 64u * w;  // lane 0 holds the maximum
+    if (lane == 0) {  // it holds the maximum
+        size[s] = 64u * w;
+        if (w > SELL_UNROLL) *wide = 1u;
+    }
 }
 
 template <typename C>
@@ -443,7 +446,7 @@ template <typename T, typename TX>
 __global__ __launch_bounds__(SV_BLOCK) void k_cg_fin(int64_t n, const double *__restrict__ part_rz,
                                                      const double *__restrict__ part_rr, const T *__restrict__ z,
                                                      T *__restrict__ p, TX *__restrict__ xs, double *__restrict__ x,
-                                                     double *__restrict__ sc, int par)
+                                                     double *__restrict__ sc, int par, double *__restrict__ hsc)
 {
     __shared__ double sh[SV_BLOCK / 64];
     const int G = gridDim.x;
@@ -465,7 +468,245 @@ __global__ __launch_bounds__(SV_BLOCK) void k_cg_fin(int64_t n, const double *__
     }
     if (blockIdx.x == 0) {
         const double rr = sum_partials(part_rr, G, sh);
-        if (threadIdx.x == 0) { sc[S_RZ] = rz; sc[S_RR] = rr; }
+        if (threadIdx.x == 0) { sc[S_RZ] = rz; sc[S_RR] = rr; hsc[S_RR] = rr; }
+    }
+}
+
+// ---- small systems: the whole iteration in one launch ---------------------------
+// Where every row has a work-item of its own and the rows are narrow, a group
+// of iterations after the other runs in one cooperative launch: a row's entries,
+// its residual, direction and iterate stay in registers, and only z and p (for
+// the neighbours' gathers) and the dot products' partials go through memory.
+// A workgroup is VB blocks of SV_BLOCK rows, each with the partials that the
+// grid-wide kernels form for the same block, summed in the same order: the
+// same bits.  Heat T3 100^2 FP64, an iteration: 15 us in two launches (each
+// half launch and sums of partials) -> 7 us.
+//
+// An exchange of partials is also the barrier between an iteration's two halves:
+// a workgroup publishes after its stores of z and p are complete, and who has
+// seen all partials may read them.  A slot holds EX_NONE until it is published;
+// three sets of slots take turns, and a slot is emptied once the next exchange
+// is through (everybody has read it then, and nobody looks at it before the
+// exchange after the next, which waits for this workgroup's next partial).
+// The launch is cooperative, so that all workgroups run and every wait ends;
+// a wait that lasts for seconds ends the solve with an error instead.
+// VB: the registers of a row (its entries, the gathers in flight) leave 512
+// work-items of FP64 rows or 768 of FP32 rows; larger workgroups spill (1024
+// FP64: 14.9 us an iteration at 9801 rows), smaller ones are more pollers of the
+// same slots (256: 10.5 and 10.8 against 9.4 and 9.0 us at 62 000 rows).
+// SM_GRID: as many workgroups as measured faster than two launches (iteration
+// at 100^2, 250^2, 300^2 rows FP64 7.8, 9.4, 10.3 against 15.3, 15.2, 16.8 us;
+// mixed 100^2, 250^2, 400^2 8.8, 9.0, 11.3 against 15.5, 14.8, 17.0), with an
+// eighth of the CUs left free.
+#define SM_VB8 2
+#define SM_VB4 3
+#define SM_GRID 224
+#define EX_NONE 0xfff8dead5eedbeefull
+#define EX_LIMIT (1 << 23)
+
+// z and p are written and gathered, and the slots filled and polled, with
+// relaxed agent-scope accesses: they bypass the XCDs' L2 (the compiler's
+// agent-scope fences, which write back and empty the whole L2, cost 2 us an
+// iteration at 62 000 rows and 3 at 86 000).  Order comes from waiting for the
+// wave's stores before the barrier that the partial is published behind, and
+// from gathering only behind the barrier that follows the last poll.
+template <typename T>
+__device__ __forceinline__ T dev_load(const T *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+template <typename T>
+__device__ __forceinline__ void dev_store(T *p, T v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+#define STORES_OUT() asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory")
+
+struct Exchange {
+    uint64_t *slots;  // [3][2][G]
+    int G;
+};
+
+__device__ __forceinline__ uint64_t ex_bits(double v)
+{
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    return b == EX_NONE ? 0x7ff8000000000000ull : b;
+}
+
+// Publishes the sums of a (and, TWO, of b) over each block's work-items, waits
+// for everybody's and returns their sums, formed as block_sum and sum_partials
+// form them.  e: the exchange's number.  False: the wait went on for too long.
+// The first four waves poll for all; a wait by every wave took three times as
+// long at 243 blocks.
+template <int VB, bool TWO>
+__device__ __forceinline__ bool exchange(const Exchange &X, uint32_t e, double &a, double &b, double (*sh)[VB * SV_BLOCK / 64],
+                                         double (*sum)[SV_BLOCK / 64], uint32_t *quit)
+{
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    uint64_t *set = X.slots + (size_t)(e % 3) * 2 * X.G, *old = X.slots + (size_t)((e + 2) % 3) * 2 * X.G;
+    const int blk = blockIdx.x * VB + tid;  // of the first VB work-items
+    STORES_OUT();
+    for (int d = 32; d > 0; d >>= 1) {
+        a += __shfl_down(a, d, 64);
+        if (TWO) b += __shfl_down(b, d, 64);
+    }
+    if (lane == 0) {
+        sh[0][w] = a;
+        if (TWO) sh[1][w] = b;
+    }
+    __syncthreads();
+    if (w == 0) {
+        if (tid < VB && blk < X.G) {
+            double s = 0.0, s2 = 0.0;
+            for (int k = 0; k < SV_BLOCK / 64; k++) {
+                s += sh[0][tid * (SV_BLOCK / 64) + k];
+                if (TWO) s2 += sh[1][tid * (SV_BLOCK / 64) + k];
+            }
+            dev_store(set + blk, ex_bits(s));
+            if (TWO) dev_store(set + X.G + blk, ex_bits(s2));
+        }
+    }
+    if (tid < SV_BLOCK) {
+        a = 0.0;
+        b = 0.0;
+        for (int i = tid; i < X.G; i += SV_BLOCK) {
+            uint64_t u, v = 0;
+            int spin = 0;
+            do {
+                u = dev_load(set + i);
+                if (TWO) v = dev_load(set + X.G + i);
+                if (u != EX_NONE && v != EX_NONE) break;
+            } while (++spin < EX_LIMIT);
+            if (spin >= EX_LIMIT) *quit = 1u;
+            a += __builtin_bit_cast(double, u);
+            if (TWO) b += __builtin_bit_cast(double, v);
+        }
+        for (int d = 32; d > 0; d >>= 1) {
+            a += __shfl_down(a, d, 64);
+            if (TWO) b += __shfl_down(b, d, 64);
+        }
+        if (lane == 0) {
+            sum[0][w] = a;
+            if (TWO) sum[1][w] = b;
+        }
+    }
+    __syncthreads();
+    a = 0.0;
+    b = 0.0;
+    for (int k = 0; k < SV_BLOCK / 64; k++) {
+        a += sum[0][k];
+        if (TWO) b += sum[1][k];
+    }
+    if (tid < VB && blk < X.G) {
+        dev_store(old + blk, (uint64_t)EX_NONE);
+        dev_store(old + X.G + blk, (uint64_t)EX_NONE);
+    }
+    return *quit == 0u;  // set before the barrier by whoever gave up
+}
+
+__global__ void k_cg_slots(uint64_t *__restrict__ slots, int n)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) slots[i] = EX_NONE;
+}
+
+// Groups of CHECK iterations from the state that k_cg_reset or this kernel left
+// (r, z, p, r.z partials) until ||r||^2 <= goal2 or maxit; leaves the same state
+// as k_cg_fin, the iteration count in sc[S_IT] (-1 if a wait failed) and ||r||^2 in sc[S_RREC].
+template <typename T, typename TX, typename C, int VB>
+__global__ __launch_bounds__(VB * SV_BLOCK) void k_cg_small(int64_t n, const uint32_t *__restrict__ off,
+                                                       const C *__restrict__ col, const T *__restrict__ val,
+                                                       const T *__restrict__ dinv, T *r_, T *z_, T *pa, T *pb, TX *xs_,
+                                                       double *x_, const double *part_rz, Exchange X, double *sc,
+                                                       double goal2, int it, int maxit)
+{
+    __shared__ double sh[2][VB * SV_BLOCK / 64], sum[2][SV_BLOCK / 64];
+    __shared__ uint32_t quit;
+    if (threadIdx.x == 0) quit = 0;
+    const int64_t i = (int64_t)blockIdx.x * (VB * SV_BLOCK) + threadIdx.x;
+    const bool live = i < n;
+    const int64_t ic = live ? i : n - 1;
+    const uint32_t s = (uint32_t)__builtin_amdgcn_readfirstlane((int)(ic >> 6));
+    const uint32_t o = off[s], w = (off[s + 1] - o) >> 6;
+    T v[SELL_UNROLL];
+    int32_t cj[SELL_UNROLL];
+#pragma unroll
+    for (int k = 0; k < SELL_UNROLL; k++) {
+        const size_t at = (size_t)o + (size_t)(k < (int)w ? k : 0) * 64 + (size_t)(ic & 63);
+        v[k] = val[at];
+        cj[k] = sell_col<C>(col[at], ic);
+    }
+    const T di = dinv[ic];
+    T ri = r_[ic], zi = z_[ic], pi = pa[ic];
+    TX xs = xs_[ic];
+    double xd = sizeof(TX) == 4 ? x_[ic] : 0.0;
+    // r.z of the state, summed as sum_partials does
+    double rz = 0.0, rz_old = 0.0, rr = 0.0, none = 0.0;
+    if (threadIdx.x < SV_BLOCK) {
+        for (int k = threadIdx.x; k < X.G; k += SV_BLOCK) rz += part_rz[k];
+        for (int d = 32; d > 0; d >>= 1) rz += __shfl_down(rz, d, 64);
+        if ((threadIdx.x & 63) == 0) sum[0][threadIdx.x >> 6] = rz;
+    }
+    __syncthreads();
+    rz = 0.0;
+    for (int k = 0; k < SV_BLOCK / 64; k++) rz += sum[0][k];
+    T *p_old = pa, *p_new = pb;
+    uint32_t e = 0;
+    bool dir = false, ok = true;
+    rr = sc[S_RR];  // the state's
+    while (ok && rr > goal2 && it < maxit) {
+        for (int k = 0; k < CHECK && ok; k++) {
+            T y[SELL_UNROLL];
+            if (dir) {
+                const T beta = (T)(rz_old != 0.0 ? rz / rz_old : 0.0);
+#pragma unroll
+                for (int q = 0; q < SELL_UNROLL; q++) y[q] = dev_load(z_ + cj[q]) + beta * dev_load(p_old + cj[q]);
+                pi = zi + beta * pi;
+                if (live) dev_store(p_new + i, pi);
+                T *t = p_old;
+                p_old = p_new;
+                p_new = t;
+            } else {
+#pragma unroll
+                for (int q = 0; q < SELL_UNROLL; q++) y[q] = dev_load(p_old + cj[q]);
+                dir = true;
+            }
+            T qi = T(0);
+#pragma unroll
+            for (int q = 0; q < SELL_UNROLL; q++)
+                if (q < (int)w) qi += v[q] * y[q];
+            double pq = 0.0;
+            if (live) pq += (double)pi * (double)qi;
+            if (!(ok = exchange<VB, false>(X, e++, pq, none, sh, sum, &quit))) break;
+            const double alpha64 = pq != 0.0 ? rz / pq : 0.0;
+            const T alpha = (T)alpha64;
+            double a = 0.0, b = 0.0;
+            if (live) {
+                ri = ri - alpha * qi;
+                zi = di * ri;
+                dev_store(z_ + i, zi);
+                a += (double)ri * (double)zi;
+                b += (double)ri * (double)ri;
+                xs += (TX)alpha64 * (TX)pi;
+            }
+            if (!(ok = exchange<VB, true>(X, e++, a, b, sh, sum, &quit))) break;
+            rz_old = rz;
+            rz = a;
+            rr = b;
+        }
+        if constexpr (sizeof(TX) == 4) {
+            xd += (double)xs;
+            xs = TX(0);
+        }
+        it += CHECK;
+    }
+    // the state that the next reset continues from
+    const T beta = (T)(rz_old != 0.0 ? rz / rz_old : 0.0);
+    if (live && dir) {
+        r_[i] = ri;
+        p_old[i] = zi + beta * pi;
+        if (p_old != pa) pa[i] = zi + beta * pi;
+        xs_[i] = xs;
+        if constexpr (sizeof(TX) == 4) x_[i] = xd;
+    }
+    // (every workgroup reads S_RR at its start: the result has its own word)
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        sc[S_RREC] = rr;
+        sc[S_IT] = ok ? (double)it : -1.0;
     }
 }
 
@@ -492,9 +733,15 @@ __global__ __launch_bounds__(SV_BLOCK) void k_cg_reset(int64_t n, const double *
     if (threadIdx.x == 0) { rz_out[blockIdx.x] = a; part_rr[blockIdx.x] = b; }
 }
 
+// Words into pinned host memory (read after a wait, without a copy).
+__global__ void k_tell(const uint32_t *__restrict__ u, uint32_t *__restrict__ hu)
+{
+    if (threadIdx.x < 4) hu[threadIdx.x] = u[threadIdx.x];
+}
+
 // One workgroup: sc[slot] = sum of g partials (and sc[slot2] of a second set).
-__global__ void k_reduce(const double *__restrict__ p, int g, double *__restrict__ sc, int slot,
-                         const double *__restrict__ p2, int slot2)
+__global__ void k_reduce(const double *__restrict__ p, int g, double *sc, int slot,
+                         const double *__restrict__ p2, int slot2, double *__restrict__ hsc)
 {
     __shared__ double sh[1024 / 64];
     const double a = sum_partials(p, g, sh);
@@ -502,6 +749,8 @@ __global__ void k_reduce(const double *__restrict__ p, int g, double *__restrict
     if (threadIdx.x == 0) {
         sc[slot] = a;
         if (p2) sc[slot2] = b;
+        if (hsc)  // all scalars to pinned host memory
+            for (int k = 0; k < S_NS; k++) hsc[k] = k == slot ? a : p2 && k == slot2 ? b : sc[k];
     }
 }
 
@@ -599,7 +848,7 @@ struct Parts {
 };
 
 template <typename T, typename TX, typename C>
-void cg_group_as(hipStream_t st, int64_t n, const Sell &S, Vecs<T> &v, TX *xs, const Parts &P, double *sc)
+void cg_group_as(hipStream_t st, int64_t n, const Sell &S, Vecs<T> &v, TX *xs, const Parts &P, double *sc, double *hsc)
 {
     const dim3 g(P.G), b(SV_BLOCK);
     const C *col = (const C *)S.col;
@@ -616,19 +865,56 @@ void cg_group_as(hipStream_t st, int64_t n, const Sell &S, Vecs<T> &v, TX *xs, c
         hipLaunchKernelGGL((k_cg_update<T>), g, b, 0, st, n, (const T *)v.dinv, v.r, v.z, (const T *)v.q, P.pq, sc, k & 1,
                            P.rz, P.rr);
     }
-    hipLaunchKernelGGL((k_cg_fin<T, TX>), g, b, 0, st, n, P.rz, P.rr, (const T *)v.z, v.p, xs, v.x, sc, (CHECK - 1) & 1);
+    hipLaunchKernelGGL((k_cg_fin<T, TX>), g, b, 0, st, n, P.rz, P.rr, (const T *)v.z, v.p, xs, v.x, sc,
+                       (CHECK - 1) & 1, hsc);
 }
 
-// CHECK PCG iterations on the stream.
-void cg_group(hipStream_t st, int64_t n, const Sell &S, Vecs<double> &v, const Parts &P, double *sc)
+// CHECK PCG iterations on the stream; ||r||^2 goes to hsc[S_RR] (host) too.
+void cg_group(hipStream_t st, int64_t n, const Sell &S, Vecs<double> &v, const Parts &P, double *sc, double *hsc)
 {
-    if (S.c16) cg_group_as<double, double, int16_t>(st, n, S, v, v.x, P, sc);
-    else cg_group_as<double, double, int32_t>(st, n, S, v, v.x, P, sc);
+    if (S.c16) cg_group_as<double, double, int16_t>(st, n, S, v, v.x, P, sc, hsc);
+    else cg_group_as<double, double, int32_t>(st, n, S, v, v.x, P, sc, hsc);
 }
-void cg_group(hipStream_t st, int64_t n, const Sell &S, Vecs<float> &v, const Parts &P, double *sc)
+void cg_group(hipStream_t st, int64_t n, const Sell &S, Vecs<float> &v, const Parts &P, double *sc, double *hsc)
 {
-    if (S.c16) cg_group_as<float, float, int16_t>(st, n, S, v, v.xlo, P, sc);
-    else cg_group_as<float, float, int32_t>(st, n, S, v, v.xlo, P, sc);
+    if (S.c16) cg_group_as<float, float, int16_t>(st, n, S, v, v.xlo, P, sc, hsc);
+    else cg_group_as<float, float, int32_t>(st, n, S, v, v.xlo, P, sc, hsc);
+}
+
+// Groups of iterations until ||r||^2 <= goal2 or maxit, in one launch; *it is
+// carried on.  1: the device cannot run the launch (nothing has run).
+template <typename T, typename TX, typename C>
+int cg_small_as(hipStream_t st, int64_t n, const Sell &S, Vecs<T> &v, TX *xs, const Parts &P, uint64_t *slots, double *sc,
+                double goal2, int it, int maxit)
+{
+    constexpr int VB = sizeof(T) == 8 ? SM_VB8 : SM_VB4;
+    const int grid = (P.G + VB - 1) / VB;
+    hipLaunchKernelGGL(k_cg_slots, dim3(ceil_div(6 * P.G, 256)), dim3(256), 0, st, slots, 6 * P.G);
+    Exchange X{slots, P.G};
+    const uint32_t *off = S.off;
+    const C *col = (const C *)S.col;
+    const T *val = sell_vals<T>(S);
+    const T *dinv = v.dinv;
+    const double *prz = P.rz;
+    double *x = v.x;
+    void *args[] = {&n, &off, &col, &val, &dinv, &v.r, &v.z, &v.p, &v.p2, &xs, &x, &prz, &X, &sc, &goal2, &it, &maxit};
+    const hipError_t e = hipLaunchCooperativeKernel(reinterpret_cast<const void *>(&k_cg_small<T, TX, C, VB>), dim3(grid),
+                                                    dim3(VB * SV_BLOCK), args, 0, st);
+    if (e == hipSuccess) return 0;
+    (void)hipGetLastError();
+    return 1;
+}
+int cg_small(hipStream_t st, int64_t n, const Sell &S, Vecs<double> &v, const Parts &P, uint64_t *slots, double *sc,
+             double goal2, int it, int maxit)
+{
+    return S.c16 ? cg_small_as<double, double, int16_t>(st, n, S, v, v.x, P, slots, sc, goal2, it, maxit)
+                 : cg_small_as<double, double, int32_t>(st, n, S, v, v.x, P, slots, sc, goal2, it, maxit);
+}
+int cg_small(hipStream_t st, int64_t n, const Sell &S, Vecs<float> &v, const Parts &P, uint64_t *slots, double *sc,
+             double goal2, int it, int maxit)
+{
+    return S.c16 ? cg_small_as<float, float, int16_t>(st, n, S, v, v.xlo, P, slots, sc, goal2, it, maxit)
+                 : cg_small_as<float, float, int32_t>(st, n, S, v, v.xlo, P, slots, sc, goal2, it, maxit);
 }
 
 }  // namespace
@@ -649,22 +935,22 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
     const bool mixed = precision == ELFEL_MIXED;
     const int64_t nslices = (n + 63) / 64;
     hipStream_t st = c->stream;
-    hipDeviceProp_t prop;
-    HIPCHK(c, hipGetDeviceProperties(&prop, c->device));
+    int cus = 0;
+    HIPCHK(c, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
     // the CG grid: 4 workgroups per CU (grid-stride loops), fewer for small
     // systems (8 and 16 per CU measured slower on heat Q4 4096^2: 407 and 412
     // against 381 us per mixed iteration; every workgroup of the next kernel
     // sums G partials)
-    const int G = (int)std::max<int64_t>(1, std::min<int64_t>(ceil_div(n, SV_BLOCK), 4 * (int64_t)prop.multiProcessorCount));
+    const int G = (int)std::max<int64_t>(1, std::min<int64_t>(ceil_div(n, SV_BLOCK), 4 * (int64_t)cus));
 
     // ---- scratch layout (8-byte words first, then 4-byte) -----------------
-    // doubles: xfull[N], b[n], r64[n], dinv64[n], parts[4 G], sc[S_NS],
+    // doubles: xfull[N], b[n], r64[n], dinv64[n], parts[4 G], slots[6 G], sc[S_NS],
     //          FP64 vectors r z p p2 q [5n] (FP64 solve only)
     // floats:  r z p p2 q dinv xlo [7n] (mixed solve only; its iterate is the FP64 xfull + xlo)
     // uint32:  off[nslices + 1], len[max(n, nslices)], total[4]
-    const size_t nd = (size_t)N + 3 * (size_t)n + 4 * (size_t)G + S_NS + (mixed ? 0 : 5 * (size_t)n);
+    const size_t nd = (size_t)N + 3 * (size_t)n + 10 * (size_t)G + S_NS + (mixed ? 0 : 5 * (size_t)n);
     const size_t nf = mixed ? 7 * (size_t)n : 0;
-    const size_t nu32 = (size_t)nslices + 1 + (size_t)std::max<int64_t>(n, nslices) + (size_t)n + 4;
+    const size_t nu32 = (size_t)nslices + 1 + (size_t)std::max<int64_t>(n, nslices) + 4;
     int rc = ensure(c, c->pcg, 8 * nd + 4 * nf + 4 * nu32 + 256);
     if (rc) return rc;
     double *dp = (double *)c->pcg.p;
@@ -675,6 +961,7 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
     Parts P;
     P.G = G;
     P.pq = dp; dp += G; P.rz = dp; dp += G; P.rr = dp; dp += G; P.aux = dp; dp += G;
+    uint64_t *slots = (uint64_t *)dp; dp += 6 * G;
     double *sc = dp; dp += S_NS;
     Vecs<double> v64{};
     if (!mixed) {
@@ -693,20 +980,20 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
     uint32_t *up = (uint32_t *)fp;
     uint32_t *off = up; up += nslices + 1;
     uint32_t *len = up; up += std::max<int64_t>(n, nslices);
-    uint32_t *far = up; up += n;
     uint32_t *total = up;
 
     HIPCHK(c, hipMemcpyAsync(xfull, x, 8 * N, hipMemcpyHostToDevice, st));
     HIPCHK(c, hipMemcpyAsync(b, F, 8 * n, hipMemcpyHostToDevice, st));
 
     // ---- SELL-64 of the free block ------------------------------------------
-    hipLaunchKernelGGL(k_sell_rowlen, dim3(ceil_div(n, 256)), dim3(256), 0, st, n, ptr, ind, len, far);
-    hipLaunchKernelGGL(k_sell_width, dim3(ceil_div(nslices * 64, 256)), dim3(256), 0, st, n, nslices, len, off);
+    hipLaunchKernelGGL(k_fill<uint32_t>, dim3(1), dim3(64), 0, st, (int64_t)4, total, 0u);
+    hipLaunchKernelGGL(k_sell_rowlen, dim3(ceil_div(n, 256)), dim3(256), 0, st, n, ptr, ind, len, total + 1);
+    hipLaunchKernelGGL(k_sell_width, dim3(ceil_div(nslices * 64, 256)), dim3(256), 0, st, n, nslices, len, off, total + 2);
     if ((rc = exclusive_scan_u32(c, off, nslices, total))) return rc;
-    if ((rc = exclusive_scan_u32(c, far, n, total + 1))) return rc;
-    uint32_t tot[2] = {0, 0};
-    HIPCHK(c, hipMemcpyAsync(tot, total, 8, hipMemcpyDeviceToHost, st));
+    volatile const uint32_t *tot = (const uint32_t *)c->told + 8;
+    hipLaunchKernelGGL(k_tell, dim3(1), dim3(64), 0, st, (const uint32_t *)total, (uint32_t *)c->told + 8);
     HIPCHK(c, hipStreamSynchronize(st));
+    const bool narrow = tot[2] == 0;  // no row of more than SELL_UNROLL entries
     const uint32_t nnzp = tot[0];
     const bool c16 = tot[1] == 0;  // every free column within a 16-bit offset of its row
     HIPCHK(c, hipMemcpyAsync(off + nslices, total, 4, hipMemcpyDeviceToDevice, st));
@@ -743,22 +1030,14 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
     HIPCHK(c, hipGetLastError());
     const Sell S{off, scol, c16, sv64, sv32, SellU{uflag, uoff}};
 
-    auto read_sc = [&](double *h) -> int {
-        HIPCHK(c, hipMemcpyAsync(h, sc, sizeof(double) * S_NS, hipMemcpyDeviceToHost, st));
-        HIPCHK(c, hipStreamSynchronize(st));
-        return 0;
-    };
+    // the scalars as the last reduction left them, in pinned memory
+    double *hsc = (double *)c->told + 8;
     // b = F_f - K_fd x_d, ||b||
     hipLaunchKernelGGL(k_rhs, dim3(G), dim3(SV_BLOCK), 0, st, n, ptr, ind, val, (const double *)xfull,
                        (const double *)b, b, P.aux);
     hipLaunchKernelGGL(k_reduce, dim3(1), dim3(1024), 0, st, (const double *)P.aux, G, sc, (int)S_BB,
-                       (const double *)nullptr, 0);
-    HIPCHK(c, hipGetLastError());
-    double h[S_NS];
-    if ((rc = read_sc(h))) return rc;
-    const double bnorm = h[S_BB] > 0 ? sqrt(h[S_BB]) : 1.0;
-    const double target = tol * bnorm;
-    // r64 = b - A x (FP64), its norm
+                       (const double *)nullptr, 0, (double *)nullptr);
+    // r64 = b - A x (FP64), its norm; waits
     auto true_residual = [&](double *out_norm) -> int {
         if (S.c16)
             hipLaunchKernelGGL((k_sell_resid<int16_t>), dim3(G), dim3(SV_BLOCK), 0, st, n, S.off,
@@ -769,12 +1048,10 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
                                (const int32_t *)S.col, S.v64, S.U, (const double *)xfull, (const double *)b, r64,
                                P.aux);
         hipLaunchKernelGGL(k_reduce, dim3(1), dim3(1024), 0, st, (const double *)P.aux, G, sc, (int)S_RR64,
-                           (const double *)nullptr, 0);
+                           (const double *)nullptr, 0, hsc);
         HIPCHK(c, hipGetLastError());
-        double hh[S_NS];
-        int r2 = read_sc(hh);
-        if (r2) return r2;
-        *out_norm = sqrt(std::max(hh[S_RR64], 0.0));
+        HIPCHK(c, hipStreamSynchronize(st));
+        *out_norm = sqrt(std::max(hsc[S_RR64], 0.0));
         return 0;
     };
     // r = (T) r64, z = M r (p = z on restart); sc gets rz and ||r||^2
@@ -783,28 +1060,47 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
         hipLaunchKernelGGL((k_cg_reset<T>), dim3(G), dim3(SV_BLOCK), 0, st, n, (const double *)r64,
                            (const T *)v.dinv, v.r, v.z, v.p, restart, P.rz, P.rr);
         hipLaunchKernelGGL(k_reduce, dim3(1), dim3(1024), 0, st, (const double *)P.rr, G, sc, (int)S_RR,
-                           (const double *)P.rz, (int)S_RZ);
+                           (const double *)P.rz, (int)S_RZ, hsc);
     };
 
     int it = 0, nupd = 0;
     double rn = 0.0;
     if ((rc = true_residual(&rn))) return rc;
+    const double bnorm = hsc[S_BB] > 0 ? sqrt(hsc[S_BB]) : 1.0;
+    const double target = tol * bnorm;
+    // Iterations until ||r||^2 <= goal2 or maxit from the state of the last reset,
+    // then the true residual (waits): *rrec the recurrence's ||r||^2, *norm the
+    // true residual's norm.  One launch where every row has its own work-item,
+    // the rows fit its registers and there are few enough workgroups.
+    auto solve_to = [&](auto &v, double goal2, double *rrec, double *norm) -> int {
+        using T = typename std::remove_pointer<decltype(v.r)>::type;
+        constexpr int VB = sizeof(T) == 8 ? SM_VB8 : SM_VB4;
+        if (narrow && n <= (int64_t)P.G * SV_BLOCK && (P.G + VB - 1) / VB <= SM_GRID &&
+            cg_small(st, n, S, v, P, slots, sc, goal2, it, maxit) == 0) {
+            if ((rc = true_residual(norm))) return rc;
+            if (hsc[S_IT] < 0) return set_err(c, ELFEL_EHIP, "elfel_hip_pcg: the solve's workgroups lost each other");
+            it = (int)hsc[S_IT];
+            *rrec = hsc[S_RREC];
+            return 0;
+        }
+        for (;;) {
+            HIPCHK(c, hipStreamSynchronize(st));
+            *rrec = hsc[S_RR];
+            if (!(*rrec > goal2) || it >= maxit) break;
+            cg_group(st, n, S, v, P, sc, hsc);
+            HIPCHK(c, hipGetLastError());
+            it += CHECK;
+        }
+        return true_residual(norm);
+    };
+    double rrec = 0.0;  // recurrence residual norm^2 at the last check
     if (!mixed) {
         reset(v64, 1);
         nupd = 1;
         while (rn > target && it < maxit) {
-            // iterate until the recurrence residual reaches the target ...
-            double rrec = 0.0;
-            for (;;) {
-                if ((rc = read_sc(h))) return rc;
-                rrec = h[S_RR];
-                if (!(rrec > target * target) || it >= maxit) break;
-                cg_group(st, n, S, v64, P, sc);
-                HIPCHK(c, hipGetLastError());
-                it += CHECK;
-            }
-            // ... then check the true residual and continue from it if needed
-            if ((rc = true_residual(&rn))) return rc;
+            // iterate until the recurrence residual reaches the target, then
+            // check the true residual and continue from it if needed
+            if ((rc = solve_to(v64, target * target, &rrec, &rn))) return rc;
             if (rn > target && it < maxit) {
                 reset(v64, !(sqrt(std::max(rrec, 0.0)) >= RU_KEEP * rn));
                 nupd++;
@@ -816,17 +1112,8 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
         double rlast = rn;
         while (rn > target && it < maxit) {
             const double goal = std::max(target, RU_DROP * rlast);
-            double rrec = 0.0;  // recurrence residual norm^2 at the last check
-            for (;;) {
-                if ((rc = read_sc(h))) return rc;
-                rrec = h[S_RR];
-                if (!(rrec > goal * goal) || it >= maxit) break;
-                cg_group(st, n, S, v32, P, sc);
-                HIPCHK(c, hipGetLastError());
-                it += CHECK;
-            }
             // reliable update: the FP64 residual b - A x replaces the FP32 one
-            if ((rc = true_residual(&rn))) return rc;
+            if ((rc = solve_to(v32, goal * goal, &rrec, &rn))) return rc;
             nupd++;
             rlast = rn;
             // The search direction is kept while the recurrence still tracks the true residual; once
