@@ -10,9 +10,8 @@
 
 #include "common.h"
 
-int plain_coo_keys(elfel_hip_ctx *c, const int64_t *I, const int64_t *J, int64_t n, int64_t nrow, int64_t ncol,
-                   int minor_bits, int csc, uint64_t *keys);
-int plain_vec_keys(elfel_hip_ctx *c, const int64_t *I, int64_t n, int64_t ndofs, uint64_t *keys);
+int plain_coo_keys32(elfel_hip_ctx *c, const int32_t *I, const int32_t *J, int64_t n, int minor_bits, int csc, uint64_t *keys);
+int plain_vec_keys(elfel_hip_ctx *c, const int32_t *I, int64_t n, uint64_t *keys);
 int geometry_stats_run(elfel_hip_ctx *c, double *min_det, int64_t *nbad);
 int geometry_check(elfel_hip_ctx *c, int rule, double *min_det, int64_t *nbad, int64_t *nneg);
 int noalloc_init_device(int device);
@@ -201,14 +200,18 @@ void tm_collect(elfel_hip_ctx *c)
     c->tm.pending.clear();
 }
 
-// Reads and clears the device error flags.
-static int take_flags(elfel_hip_ctx *c, int *flags)
+int host_tables(elfel_hip_ctx *c, Field &f)
 {
-    int h = 0;
-    HIPCHK(c, hipMemcpyAsync(&h, (int *)c->dscal.p + 1, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    const size_t nc = (size_t)(f.E * f.nen), nd = f.has_dofs ? (size_t)(f.dof_Nn * f.ncomp) : 0;
+    if (f.h_conn.size() != nc) {
+        f.h_conn.resize(nc);
+        if (nc) HIPCHK(c, hipMemcpyAsync(f.h_conn.data(), f.conn.p, 4 * nc, hipMemcpyDeviceToHost, c->stream));
+    }
+    if (f.h_dof.size() != nd) {
+        f.h_dof.resize(nd);
+        if (nd) HIPCHK(c, hipMemcpyAsync(f.h_dof.data(), f.dof.p, 4 * nd, hipMemcpyDeviceToHost, c->stream));
+    }
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    if (h) HIPCHK(c, hipMemsetAsync((int *)c->dscal.p + 1, 0, sizeof(int), c->stream));
-    *flags = h;
     return 0;
 }
 
@@ -256,6 +259,7 @@ extern "C" int elfel_hip_init(int device, elfel_hip_ctx **out)
             delete c;
             return rc;
         }
+        transfer_user(true);
         *out = c;
         return ELFEL_OK;
     });
@@ -277,6 +281,9 @@ extern "C" int elfel_hip_free(elfel_hip_ctx *c)
                    &c->fpat.coo, &c->fpat.fcoo};
     for (Buf *b : bufs) release(*b);
     told_put(c->told);
+    for (auto &e : c->xfer_ev)
+        if (e) hipEventDestroy(e);
+    transfer_user(false);
     batch_free(c);
     for (auto &p : c->tm.pending) { hipEventDestroy(p.a); hipEventDestroy(p.b); }
     if (c->tm.r0) hipEventDestroy(c->tm.r0);
@@ -377,29 +384,24 @@ extern "C" int elfel_hip_sparse(elfel_hip_ctx *c, int64_t nrow, int64_t ncol, in
         const int minor_bits = bits_for(nmin), major_bits = bits_for(nmaj);
         int rc;
         const bool buckets = bucket_takes(n, nmaj, nmin);
-        if ((rc = ensure(c, c->vals[0], 8 * n)) || (rc = ensure(c, c->stage64, 16 * n)) ||
+        if ((rc = ensure(c, c->vals[0], 8 * n)) || (rc = ensure(c, c->stage64, 8 * n)) ||
             (rc = ensure(c, c->ptr, 4 * (nmaj + 1))) || (rc = ensure(c, c->ind, 4 * n)) || (rc = ensure(c, c->val, 8 * n)) ||
             (buckets && (rc = ensure(c, c->keys[0], bucket_scratch_bytes(n, nmaj)))))
             return rc;
         c->has_result = false;
-        int64_t *dI = (int64_t *)c->stage64.p, *dJ = dI + n;
-        if (n > 0) {
-            HIPCHK(c, hipMemcpyAsync(dI, row, 8 * n, hipMemcpyHostToDevice, c->stream));
-            HIPCHK(c, hipMemcpyAsync(dJ, col, 8 * n, hipMemcpyHostToDevice, c->stream));
-            HIPCHK(c, hipMemcpyAsync(c->vals[0].p, val, 8 * n, hipMemcpyHostToDevice, c->stream));
-        }
+        // the indices checked and narrowed on the way
+        int32_t *dI = (int32_t *)c->stage64.p, *dJ = dI + n;
+        const HostIn in[3] = {{row, dI, n, true, 1, nrow}, {col, dJ, n, true, 1, ncol}, {val, c->vals[0].p, n, false, 0, 0}};
+        bool bad = false;
+        if ((rc = to_device(c, in, 3, &bad))) return rc;
+        if (bad) return set_err(c, ELFEL_ERANGE, "row or column index out of range");
         int64_t h = 0;
         bool done = false;
         if (buckets) {
-            int flags = 0;
             bool toolong = false;
-            if ((rc = bucket_coo(c, c->keys[0].p, n, dI, dJ, (const double *)c->vals[0].p, nrow, ncol, csc,
-                                 (int32_t *)c->ptr.p, (int32_t *)c->ind.p, (double *)c->val.p, &flags, &toolong, &h)))
+            if ((rc = bucket_coo32(c, c->keys[0].p, n, dI, dJ, (const double *)c->vals[0].p, nrow, ncol, csc,
+                                   (int32_t *)c->ptr.p, (int32_t *)c->ind.p, (double *)c->val.p, &toolong, &h)))
                 return rc;
-            if (flags) {
-                HIPCHK(c, hipMemsetAsync((int *)c->dscal.p + 1, 0, sizeof(int), c->stream));
-                if (flags & DERR_RANGE) return set_err(c, ELFEL_ERANGE, "row or column index out of range");
-            }
             done = !toolong;
         }
         if (!done) {
@@ -407,10 +409,7 @@ extern "C" int elfel_hip_sparse(elfel_hip_ctx *c, int64_t nrow, int64_t ncol, in
                 return rc;
             uint64_t *k0 = (uint64_t *)c->keys[0].p, *k1 = (uint64_t *)c->keys[1].p;
             uint64_t *v0 = (uint64_t *)c->vals[0].p, *v1 = (uint64_t *)c->vals[1].p;
-            if ((rc = plain_coo_keys(c, dI, dJ, n, nrow, ncol, minor_bits, csc, k0))) return rc;
-            int flags = 0;
-            if ((rc = take_flags(c, &flags))) return rc;
-            if (flags & DERR_RANGE) return set_err(c, ELFEL_ERANGE, "row or column index out of range");
+            if ((rc = plain_coo_keys32(c, dI, dJ, n, minor_bits, csc, k0))) return rc;
             if ((rc = radix_sort_pairs(c, k0, v0, k1, v1, n, major_bits + minor_bits))) return rc;
             if ((rc = build_csr_from_sorted(c, k0, (const double *)v0, n, minor_bits, nmaj, (int32_t *)c->ptr.p,
                                             (int32_t *)c->ind.p, (double *)c->val.p, (int32_t *)c->dscal.p, true)))
@@ -430,12 +429,6 @@ extern "C" int elfel_hip_sparse(elfel_hip_ctx *c, int64_t nrow, int64_t ncol, in
         if (nnz) *nnz = h;
         return ELFEL_OK;
     });
-}
-
-__global__ void k_i32_to_i64(const int32_t *__restrict__ s, int64_t *__restrict__ d, int64_t n, int64_t base)
-{
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) d[i] = (int64_t)s[i] + base;
 }
 
 static int fetch_nnz(elfel_hip_ctx *c)
@@ -479,21 +472,8 @@ extern "C" int elfel_hip_copy_sparse(elfel_hip_ctx *c, int base, int64_t *ptr, i
         const int64_t nnz = c->nnz, np = c->nmaj + 1;
         const int32_t *dptr = result_ptr(c);
         const int32_t *dind = result_ind(c);
-        if ((rc = ensure(c, c->stage64, 8 * std::max(np, nnz)))) return rc;
-        int64_t *st = (int64_t *)c->stage64.p;
-        if (ptr) {
-            hipLaunchKernelGGL(k_i32_to_i64, dim3(ceil_div(np, 256)), dim3(256), 0, c->stream, dptr, st, np, (int64_t)base);
-            HIPCHK(c, hipMemcpyAsync(ptr, st, 8 * np, hipMemcpyDeviceToHost, c->stream));
-            HIPCHK(c, hipStreamSynchronize(c->stream));
-        }
-        if (ind && nnz > 0) {
-            hipLaunchKernelGGL(k_i32_to_i64, dim3(ceil_div(nnz, 256)), dim3(256), 0, c->stream, dind, st, nnz, (int64_t)base);
-            HIPCHK(c, hipMemcpyAsync(ind, st, 8 * nnz, hipMemcpyDeviceToHost, c->stream));
-            HIPCHK(c, hipStreamSynchronize(c->stream));
-        }
-        if (val && nnz > 0) HIPCHK(c, hipMemcpyAsync(val, c->val.p, 8 * nnz, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-        return ELFEL_OK;
+        const HostOut out[3] = {{ptr, dptr, np, true, base}, {ind, dind, nnz, true, base}, {val, c->val.p, nnz, false, 0}};
+        return to_host(c, out, 3);
     });
 }
 
@@ -511,23 +491,19 @@ extern "C" int elfel_hip_vector(elfel_hip_ctx *c, int64_t ndofs, int64_t n, cons
         int rc;
         if ((rc = ensure(c, c->fkeys[0], 8 * n)) || (rc = ensure(c, c->fkeys[1], 8 * n)) ||
             (rc = ensure(c, c->fvals[0], 8 * n)) || (rc = ensure(c, c->fvals[1], 8 * n)) ||
-            (rc = ensure(c, c->stage64, 8 * n)) || (rc = ensure(c, c->scal, 8 * ndofs)))
+            (rc = ensure(c, c->stage64, 4 * n)) || (rc = ensure(c, c->scal, 8 * ndofs)))
             return rc;
         uint64_t *k0 = (uint64_t *)c->fkeys[0].p, *k1 = (uint64_t *)c->fkeys[1].p;
         uint64_t *v0 = (uint64_t *)c->fvals[0].p, *v1 = (uint64_t *)c->fvals[1].p;
-        if (n > 0) {
-            HIPCHK(c, hipMemcpyAsync(c->stage64.p, idx, 8 * n, hipMemcpyHostToDevice, c->stream));
-            HIPCHK(c, hipMemcpyAsync(v0, v, 8 * n, hipMemcpyHostToDevice, c->stream));
-        }
-        if ((rc = plain_vec_keys(c, (const int64_t *)c->stage64.p, n, ndofs, k0))) return rc;
-        int flags = 0;
-        if ((rc = take_flags(c, &flags))) return rc;
-        if (flags & DERR_RANGE) return set_err(c, ELFEL_ERANGE, "dof number out of range (BoundsError)");
+        const HostIn in[2] = {{idx, c->stage64.p, n, true, 1, ndofs}, {v, v0, n, false, 0, 0}};
+        bool bad = false;
+        if ((rc = to_device(c, in, 2, &bad))) return rc;
+        if (bad) return set_err(c, ELFEL_ERANGE, "dof number out of range (BoundsError)");
+        if ((rc = plain_vec_keys(c, (const int32_t *)c->stage64.p, n, k0))) return rc;
         if ((rc = radix_sort_pairs(c, k0, v0, k1, v1, n, bits_for(ndofs)))) return rc;
         if ((rc = build_dense_from_sorted(c, k0, (const double *)v0, n, ndofs, (double *)c->scal.p))) return rc;
-        if (ndofs > 0) HIPCHK(c, hipMemcpyAsync(out, c->scal.p, 8 * ndofs, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-        return ELFEL_OK;
+        const HostOut o{out, c->scal.p, ndofs, false, 0};
+        return to_host(c, &o, 1);
     });
 }
 
@@ -545,20 +521,15 @@ extern "C" int elfel_hip_set_mesh_sdim(elfel_hip_ctx *c, int field, int32_t nen,
         if (E * nen >= INT32_MAX || Nn >= INT32_MAX) return set_err(c, ELFEL_ENOTSUP, "mesh beyond int32 indexing");
         Field &f = c->f[field];
         int rc;
-        if ((rc = ensure(c, f.conn, 4 * E * nen)) || (rc = ensure(c, f.xy, 8 * sdim * Nn)) ||
-            (rc = ensure(c, c->stage64, 8 * E * nen)))
-            return rc;
+        if ((rc = ensure(c, f.conn, 4 * E * nen)) || (rc = ensure(c, f.xy, 8 * sdim * Nn))) return rc;
         f.has_mesh = false;
-        if (E > 0) HIPCHK(c, hipMemcpyAsync(c->stage64.p, conn, 8 * E * nen, hipMemcpyHostToDevice, c->stream));
-        if (Nn > 0) HIPCHK(c, hipMemcpyAsync(f.xy.p, x, 8 * sdim * Nn, hipMemcpyHostToDevice, c->stream));
-        if ((rc = convert_indices(c, (const int64_t *)c->stage64.p, (int32_t *)f.conn.p, E * nen, 1, Nn))) return rc;
-        int flags = 0;
-        if ((rc = take_flags(c, &flags))) return rc;
-        if (flags & DERR_RANGE) return set_err(c, ELFEL_ERANGE, "connectivity refers to a node outside 1..Nn");
+        const HostIn in[2] = {{conn, f.conn.p, E * nen, true, 1, Nn}, {x, f.xy.p, sdim * Nn, false, 0, 0}};
+        bool bad = false;
+        if ((rc = to_device(c, in, 2, &bad))) return rc;
+        if (bad) return set_err(c, ELFEL_ERANGE, "connectivity refers to a node outside 1..Nn");
         field_mesh_changed(f, E, Nn);
         f.nen = nen; f.E = E; f.Nn = Nn; f.sdim = sdim;
-        f.h_conn.resize((size_t)(E * nen));
-        for (int64_t i = 0; i < E * nen; i++) f.h_conn[i] = (int32_t)(conn[i] - 1);
+        f.h_conn.clear();
         f.has_mesh = true;
         f.mesh_version++;
         c->pat.valid = false;
@@ -585,13 +556,12 @@ extern "C" int elfel_hip_set_element_dofs(elfel_hip_ctx *c, int field, int32_t n
         Field &f = c->f[field];
         const int64_t n = E * ncomp;
         int rc;
-        if ((rc = ensure(c, f.edof, 4 * n)) || (rc = ensure(c, c->stage64, 8 * n))) return rc;
+        if ((rc = ensure(c, f.edof, 4 * n))) return rc;
         f.has_edofs = false;
-        if (n > 0) HIPCHK(c, hipMemcpyAsync(c->stage64.p, dofnums, 8 * n, hipMemcpyHostToDevice, c->stream));
-        if ((rc = convert_indices(c, (const int64_t *)c->stage64.p, (int32_t *)f.edof.p, n, 1, ndofs))) return rc;
-        int flags = 0;
-        if ((rc = take_flags(c, &flags))) return rc;
-        if (flags & DERR_RANGE) return set_err(c, ELFEL_ERANGE, "cell dof number outside 1..ndofs (unnumbered dof 0?)");
+        const HostIn in{dofnums, f.edof.p, n, true, 1, ndofs};
+        bool bad = false;
+        if ((rc = to_device(c, &in, 1, &bad))) return rc;
+        if (bad) return set_err(c, ELFEL_ERANGE, "cell dof number outside 1..ndofs (unnumbered dof 0?)");
         f.edof_ncomp = ncomp; f.edof_E = E; f.edof_ndofs = ndofs;
         f.has_edofs = true;
         f.edof_version++;
@@ -610,18 +580,16 @@ extern "C" int elfel_hip_set_dofs(elfel_hip_ctx *c, int field, int32_t ncomp, in
         Field &f = c->f[field];
         const int64_t n = Nn * ncomp;
         int rc;
-        if ((rc = ensure(c, f.dof, 4 * n)) || (rc = ensure(c, c->stage64, 8 * n))) return rc;
+        if ((rc = ensure(c, f.dof, 4 * n))) return rc;
         f.has_dofs = false;
-        if (n > 0) HIPCHK(c, hipMemcpyAsync(c->stage64.p, dofnums, 8 * n, hipMemcpyHostToDevice, c->stream));
-        if ((rc = convert_indices(c, (const int64_t *)c->stage64.p, (int32_t *)f.dof.p, n, 1, ndofs))) return rc;
-        int flags = 0;
-        if ((rc = take_flags(c, &flags))) return rc;
-        if (flags & DERR_RANGE)
+        const HostIn in{dofnums, f.dof.p, n, true, 1, ndofs};
+        bool bad = false;
+        if ((rc = to_device(c, &in, 1, &bad))) return rc;
+        if (bad)
             return set_err(c, ELFEL_ERANGE, "dof number outside 1..ndofs (unnumbered dof 0?)");
         if (f.Nn != Nn && f.has_mesh) return set_err(c, ELFEL_EINVAL, "dof map size does not match the mesh");
         f.ncomp = ncomp; f.ndofs = ndofs; f.dof_Nn = Nn;
-        f.h_dof.resize((size_t)n);
-        for (int64_t i = 0; i < n; i++) f.h_dof[i] = (int32_t)(dofnums[i] - 1);
+        f.h_dof.clear();
         f.has_dofs = true;
         f.dof_version++;
         c->pat.valid = false;
@@ -646,7 +614,8 @@ extern "C" int elfel_hip_set_coefficients(elfel_hip_ctx *c, int64_t E, const dou
             if (!rc) rc = ensure(c, c->stage64, 8 * E);
             if (rc) return rc;
             if (E > 0) {
-                HIPCHK(c, hipMemcpyAsync(c->stage64.p, it.src, 8 * E, hipMemcpyHostToDevice, c->stream));
+                const HostIn in{it.src, c->stage64.p, E, false, 0, 0};
+                if ((rc = to_device(c, &in, 1, nullptr))) return rc;
                 if ((rc = copy_padded(c, it.dst->p, c->stage64.p, E, 8, COEF_GAP))) return rc;
             }
             *it.flag = true;
@@ -762,9 +731,8 @@ extern "C" int elfel_hip_copy_vector(elfel_hip_ctx *c, double *F, int64_t n)
         CHECK_CTX(c);
         if (!c->has_F) return set_err(c, ELFEL_ESTATE, "the last assembly produced no load vector");
         if (!F || n != c->nF) return set_err(c, ELFEL_EINVAL, "load vector size mismatch");
-        HIPCHK(c, hipMemcpyAsync(F, c->F.p, 8 * n, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-        return ELFEL_OK;
+        const HostOut o{F, c->F.p, n, false, 0};
+        return to_host(c, &o, 1);
     });
 }
 

@@ -731,12 +731,6 @@ extern "C" int elfel_hip_batch_info(elfel_hip_ctx *c, int32_t k, int64_t *ndofs,
     });
 }
 
-__global__ void k_ptr_i64(const int32_t *__restrict__ s, int64_t *__restrict__ d, int64_t n, int64_t base)
-{
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) d[i] = (int64_t)s[i] + base;
-}
-
 extern "C" int elfel_hip_batch_copy(elfel_hip_ctx *c, int32_t k, int base, int64_t *ptr, int64_t *ind, double *val,
                                     double *F)
 {
@@ -748,27 +742,11 @@ extern "C" int elfel_hip_batch_copy(elfel_hip_ctx *c, int32_t k, int base, int64
         if (!b || !b->built) return set_err(c, ELFEL_ESTATE, "build the batch first");
         if (k < 0 || k >= (int32_t)b->probs.size()) return set_err(c, ELFEL_EINVAL, "problem index out of range");
         const BatchProb &p = b->probs[k];
-        int rc = ensure(c, c->stage64, 8 * std::max<int64_t>(p.nnz, p.ndofs + 1));
-        if (rc) return rc;
-        int64_t *st = (int64_t *)c->stage64.p;
-        if (ptr) {
-            hipLaunchKernelGGL(k_ptr_i64, dim3(ceil_div(p.ndofs + 1, 256)), dim3(256), 0, c->stream,
-                               (const int32_t *)b->ptr.p + p.ptr_base, st, p.ndofs + 1, (int64_t)base);
-            HIPCHK(c, hipMemcpyAsync(ptr, st, 8 * (p.ndofs + 1), hipMemcpyDeviceToHost, c->stream));
-            HIPCHK(c, hipStreamSynchronize(c->stream));
-        }
-        if (ind && p.nnz) {
-            hipLaunchKernelGGL(k_ptr_i64, dim3(ceil_div(p.nnz, 256)), dim3(256), 0, c->stream,
-                               (const int32_t *)b->ind.p + p.val_base, st, p.nnz, (int64_t)base);
-            HIPCHK(c, hipMemcpyAsync(ind, st, 8 * p.nnz, hipMemcpyDeviceToHost, c->stream));
-            HIPCHK(c, hipStreamSynchronize(c->stream));
-        }
-        if (val && p.nnz)
-            HIPCHK(c, hipMemcpyAsync(val, (double *)b->val.p + p.val_base, 8 * p.nnz, hipMemcpyDeviceToHost, c->stream));
-        if (F && KS[p.kind].heat)
-            HIPCHK(c, hipMemcpyAsync(F, (double *)b->F.p + p.row_base, 8 * p.ndofs, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-        return ELFEL_OK;
+        const HostOut out[4] = {{ptr, (const int32_t *)b->ptr.p + p.ptr_base, p.ndofs + 1, true, base},
+                                {ind, (const int32_t *)b->ind.p + p.val_base, p.nnz, true, base},
+                                {val, (const double *)b->val.p + p.val_base, p.nnz, false, 0},
+                                {KS[p.kind].heat ? F : nullptr, (const double *)b->F.p + p.row_base, p.ndofs, false, 0}};
+        return to_host(c, out, 4);
     });
 }
 

@@ -124,6 +124,23 @@ struct CooSource {
     }
 };
 
+// The same with checked, 0-based indices.
+struct CooSource32 {
+    const int32_t *major, *minor;
+    __device__ __forceinline__ bool get(int64_t k, uint32_t &mj, uint32_t &mn) const
+    {
+        mj = (uint32_t)major[k];
+        mn = (uint32_t)minor[k];
+        return true;
+    }
+    __device__ __forceinline__ bool item(int64_t k, uint32_t &mj, uint32_t &wide) const
+    {
+        mj = (uint32_t)major[k];
+        wide = 1;
+        return true;
+    }
+};
+
 // The stream of an element loop: a local dof of an element is one item, as wide
 // as its row of the element block.
 template <int ND>
@@ -275,7 +292,8 @@ __global__ __launch_bounds__(BK_BLOCK) void k_bk_scan(uint32_t *__restrict__ cnt
 // The entries of a row side by side, each packed with its row's first entry in
 // the bits above `bits` = minor bits + kbits (those that overflow drop out: a
 // tile spans fewer than 2^11 entries), its minor index and its stream position.
-__global__ __launch_bounds__(BK_BLOCK) void k_bk_scatter(CooSource src, int64_t n, const uint32_t *__restrict__ start,
+template <typename Source>
+__global__ __launch_bounds__(BK_BLOCK) void k_bk_scatter(Source src, int64_t n, const uint32_t *__restrict__ start,
                                                          const uint32_t *__restrict__ place, int bits, int kbits,
                                                          uint64_t *__restrict__ packed)
 {
@@ -575,32 +593,51 @@ static void launch_zero_scan(elfel_hip_ctx *c, const Scratch &S, bool zero, int6
                            (uint32_t)S.nt, S.trow, S.tstart, S.st_scan, S.ctl);
 }
 
+template <typename Source>
+static int run_coo(elfel_hip_ctx *c, void *scratch, const Source &src, int64_t n, const double *val, int64_t nmaj,
+                   int64_t nmin, const BucketOut &o)
+{
+    const Scratch S = scratch_layout(scratch, n, nmaj);
+    const int kbits = bits_for(n), bits = kbits + bits_for(nmin);
+    int *err = (int *)c->dscal.p + 1;
+    launch_zero_scan(c, S, true, n, nmaj);
+    hipLaunchKernelGGL(k_bk_count<Source>, dim3(ceil_div(n, BK_BLOCK * BK_COUNT_ITEMS)), dim3(BK_BLOCK), 0, c->stream, src,
+                       n, S.cnt, S.place, err);
+    launch_zero_scan(c, S, false, n, nmaj);
+    hipLaunchKernelGGL(k_bk_scatter<Source>, dim3(ceil_div(n, BK_BLOCK)), dim3(BK_BLOCK), 0, c->stream, src, n, S.cnt,
+                       S.place, bits, kbits, S.packed);
+    // told: words 0-3 are the context's result's, these 4-7
+    hipLaunchKernelGGL((k_bk_tile<true, false>), dim3((unsigned)S.nt), dim3(BK_TB), 0, c->stream, S.packed, val,
+                       (const double *)nullptr, 1u, S.cnt, S.trow, S.tstart, (uint32_t)S.nt, nmaj, bits, kbits, S.st_tile,
+                       S.ctl, err, o, (int32_t *)c->dscal.p + 2, (int32_t *)c->told + 4);
+    HIPCHK(c, hipGetLastError());
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return 0;
+}
+
 int bucket_coo(elfel_hip_ctx *c, void *scratch, int64_t n, const int64_t *row, const int64_t *col, const double *val,
                int64_t nrow, int64_t ncol, int csc, int32_t *ptr, int32_t *ind, double *out, int *flags, bool *toolong,
                int64_t *nnz)
 {
-    const int64_t nmaj = csc ? ncol : nrow;
-    const Scratch S = scratch_layout(scratch, n, nmaj);
-    const CooSource src{row, col, nrow, ncol, csc};
-    const int kbits = bits_for(n), bits = kbits + bits_for(csc ? nrow : ncol);
-    int *err = (int *)c->dscal.p + 1;
-    int32_t *told = (int32_t *)c->told + 4;  // words 0-3: the context's result
     const BucketOut o{ptr, ind, out, nullptr, nullptr, nullptr, nullptr, nullptr};
-    launch_zero_scan(c, S, true, n, nmaj);
-    hipLaunchKernelGGL(k_bk_count<CooSource>, dim3(ceil_div(n, BK_BLOCK * BK_COUNT_ITEMS)), dim3(BK_BLOCK), 0, c->stream,
-                       src, n, S.cnt, S.place, err);
-    launch_zero_scan(c, S, false, n, nmaj);
-    hipLaunchKernelGGL(k_bk_scatter, dim3(ceil_div(n, BK_BLOCK)), dim3(BK_BLOCK), 0, c->stream, src, n, S.cnt, S.place,
-                       bits, kbits, S.packed);
-    hipLaunchKernelGGL((k_bk_tile<true, false>), dim3((unsigned)S.nt), dim3(BK_TB), 0, c->stream, S.packed, val,
-                       (const double *)nullptr, 1u, S.cnt, S.trow, S.tstart, (uint32_t)S.nt, nmaj, bits, kbits, S.st_tile,
-                       S.ctl, err, o, (int32_t *)c->dscal.p + 2, told);
-    HIPCHK(c, hipGetLastError());
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    const int rc = run_coo(c, scratch, CooSource{row, col, nrow, ncol, csc}, n, val, csc ? ncol : nrow, csc ? nrow : ncol, o);
+    const int32_t *told = (const int32_t *)c->told + 4;
     *nnz = told[0];
     *flags = told[1];
     *toolong = told[2] != 0;
-    return 0;
+    return rc;
+}
+
+int bucket_coo32(elfel_hip_ctx *c, void *scratch, int64_t n, const int32_t *row, const int32_t *col, const double *val,
+                 int64_t nrow, int64_t ncol, int csc, int32_t *ptr, int32_t *ind, double *out, bool *toolong, int64_t *nnz)
+{
+    const BucketOut o{ptr, ind, out, nullptr, nullptr, nullptr, nullptr, nullptr};
+    const int rc = run_coo(c, scratch, CooSource32{csc ? col : row, csc ? row : col}, n, val, csc ? ncol : nrow,
+                           csc ? nrow : ncol, o);
+    const int32_t *told = (const int32_t *)c->told + 4;
+    *nnz = told[0];
+    *toolong = told[2] != 0;
+    return rc;
 }
 
 // ---- the stream of an element loop ------------------------------------------------

@@ -73,7 +73,7 @@ struct Field {
     bool has_edofs = false;
     uint64_t edof_version = 0;
     Buf edof;
-    std::vector<int32_t> h_conn, h_dof;  // host copies (0-based) for the symbolic phase
+    std::vector<int32_t> h_conn, h_dof;  // host copies (0-based) for the host symbolic phase (host_tables); empty until then
     uint64_t mesh_version = 0, dof_version = 0;
 };
 
@@ -200,6 +200,7 @@ struct elfel_hip_ctx {
     } rows;
     // solver scratch: vectors, then the SELL-64 copy of the free block
     Buf pcg, pcg_sell;
+    hipEvent_t xfer_ev[8] = {};   // transfer.hip, made when first needed
     // batched problems (batch.hip)
     void *batch = nullptr;
 };
@@ -276,6 +277,34 @@ ThreadJoiner<F> join_on_exit(std::vector<std::thread> &ts, F before) { return Th
 int ensure(elfel_hip_ctx *c, Buf &b, size_t bytes);
 int copy_padded(elfel_hip_ctx *c, void *dst, const void *src, int64_t n, size_t esize, int gap);
 void release(Buf &b);
+
+// ---- transfer.hip -------------------------------------------------------------
+// A host array filled from the device: n 8-byte words, or (wide) the device's
+// int32 as int64 + base.  host null: left out.
+struct HostOut {
+    void *host;
+    const void *dev;
+    int64_t n;
+    bool wide;
+    int64_t base;
+};
+// A device array filled from the host: n 8-byte words, or (narrow) int64 in
+// lo..hi as 0-based int32.
+struct HostIn {
+    const void *host;
+    void *dev;
+    int64_t n;
+    bool narrow;
+    int64_t lo, hi;
+};
+// Both wait: for the stream's work before them and for the copies.
+int to_host(elfel_hip_ctx *c, const HostOut *segs, int nseg);
+// out_of_range: a narrowed value lay outside lo..hi (the device array is then
+// written all the same, with lo in its place).
+int to_device(elfel_hip_ctx *c, const HostIn *segs, int nseg, bool *out_of_range);
+void transfer_user(bool add);  // a context more or less that may transfer
+// The host copies of a field's connectivity and dof map.
+int host_tables(elfel_hip_ctx *c, Field &f);
 
 // ---- timing -----------------------------------------------------------------
 void tm_begin(elfel_hip_ctx *c, int phase, hipEvent_t *a);
@@ -354,11 +383,14 @@ bool bucket_form_takes(const FormMap &m, int64_t E, int64_t ndofs);
 int bucket_form(elfel_hip_ctx *c, void *scratch, const FormMap &m, int64_t E, const int32_t *edof, int64_t ndofs,
                 const double *vals, const double *fvals, const BucketOut &o);
 
-// COO stream (device arrays, 1-based indices) -> CSR/CSC by row buckets; waits.
+// COO stream (device arrays, 1-based int64 indices, or checked 0-based int32
+// ones) -> CSR/CSC by row buckets; waits.
 // flags: the range errors found (nothing is written then); toolong: a row is
 // longer than the tiles hold (nothing is written: use the sort).
 bool bucket_takes(int64_t n, int64_t nmaj, int64_t nmin);
 size_t bucket_scratch_bytes(int64_t n, int64_t nmaj);
+int bucket_coo32(elfel_hip_ctx *c, void *scratch, int64_t n, const int32_t *row, const int32_t *col, const double *val,
+                 int64_t nrow, int64_t ncol, int csc, int32_t *ptr, int32_t *ind, double *out, bool *toolong, int64_t *nnz);
 int bucket_coo(elfel_hip_ctx *c, void *scratch, int64_t n, const int64_t *row, const int64_t *col, const double *val,
                int64_t nrow, int64_t ncol, int csc, int32_t *ptr, int32_t *ind, double *out, int *flags, bool *toolong,
                int64_t *nnz);
@@ -394,8 +426,6 @@ int plain_stream_reuse(elfel_hip_ctx *c, const elfel_hip_problem *pb, const QTab
 bool family_problem(const elfel_hip_problem *pb);
 int family_validate(elfel_hip_ctx *c, const elfel_hip_problem *pb);  // sets c->nrow, c->ncol
 int family_assemble(elfel_hip_ctx *c, const elfel_hip_problem *pb);
-int convert_indices(elfel_hip_ctx *c, const int64_t *src_dev, int32_t *dst, int64_t n, int64_t lo,
-                    int64_t hi);
 
 // ---- reuse.hip ----------------------------------------------------------------
 int reuse_assemble(elfel_hip_ctx *c, const elfel_hip_problem *pb, const QTable &tab, const Coef &cf);

@@ -159,9 +159,7 @@ int finish_field_mesh(elfel_hip_ctx *c, Field &f, int nen, int64_t E, int64_t Nn
     f.sdim = 2;
     f.E = E;
     f.Nn = Nn;
-    f.h_conn.resize((size_t)(E * nen));
-    if (E > 0)
-        HIPCHK(c, hipMemcpyAsync(f.h_conn.data(), f.conn.p, 4 * (size_t)(E * nen), hipMemcpyDeviceToHost, c->stream));
+    f.h_conn.clear();
     HIPCHK(c, hipStreamSynchronize(c->stream));
     f.has_mesh = true;
     f.mesh_version++;
@@ -301,12 +299,8 @@ extern "C" int elfel_hip_copy_mesh(elfel_hip_ctx *c, int field, int64_t E, int64
         const Field &f = c->f[field];
         if (!f.has_mesh) return set_err(c, ELFEL_ESTATE, "elfel_hip_copy_mesh: no mesh");
         if (E != f.E || Nn != f.Nn) return set_err(c, ELFEL_EINVAL, "elfel_hip_copy_mesh: sizes differ from the mesh");
-        if (xy && Nn > 0)
-            HIPCHK(c, hipMemcpyAsync(xy, f.xy.p, 8 * (size_t)f.sdim * Nn, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-        if (conn)
-            for (int64_t i = 0; i < E * f.nen; i++) conn[i] = (int64_t)f.h_conn[i] + 1;
-        return ELFEL_OK;
+        const HostOut out[2] = {{conn, f.conn.p, E * f.nen, true, 1}, {xy, f.xy.p, (int64_t)f.sdim * Nn, false, 0}};
+        return to_host(c, out, 2);
     });
 }
 

@@ -160,7 +160,7 @@ static int sysvec_common(elfel_hip_ctx *c, int field, int64_t nvals, int64_t ndo
     if (field < 0 || field > 1) return set_err(c, ELFEL_EINVAL, "bad field");
     const Field &F = c->f[field];
     if (!F.has_dofs) return set_err(c, ELFEL_ESTATE, "set_dofs of this field first");
-    if (nvals != (int64_t)F.h_dof.size() || ndofs < 0) return set_err(c, ELFEL_EINVAL, "dof value array size mismatch");
+    if (nvals != F.dof_Nn * F.ncomp || ndofs < 0) return set_err(c, ELFEL_EINVAL, "dof value array size mismatch");
     return 0;
 }
 

@@ -14,29 +14,6 @@
 
 #include "elem.h"
 
-// ---- index conversion: 1-based int64 -> 0-based int32 with range check ----
-__global__ void k_convert(const int64_t *__restrict__ src, int32_t *__restrict__ dst, int64_t n, int64_t lo,
-                          int64_t hi, int *__restrict__ err)
-{
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    int64_t v = src[i];
-    if (v < lo || v > hi) {
-        atomicOr(err, DERR_RANGE);
-        v = lo;
-    }
-    dst[i] = (int32_t)(v - 1);
-}
-
-int convert_indices(elfel_hip_ctx *c, const int64_t *src_dev, int32_t *dst, int64_t n, int64_t lo, int64_t hi)
-{
-    if (n == 0) return 0;
-    int *err = (int *)c->dscal.p + 1;
-    hipLaunchKernelGGL(k_convert, dim3(ceil_div(n, 256)), dim3(256), 0, c->stream, src_dev, dst, n, lo, hi, err);
-    HIPCHK(c, hipGetLastError());
-    return 0;
-}
-
 // ---- element kernel: the values of the COO stream, in stream order ----------
 // A workgroup takes EB elements.  First a work-item per (element, point) leaves
 // the spatial gradients and JxW in LDS; then a work-item per (element, column of
@@ -212,20 +189,23 @@ __global__ void k_coo_keys(const int64_t *__restrict__ I, const int64_t *__restr
     keys[k] = (mj << minor_bits) | mn;
 }
 
-__global__ void k_vec_keys(const int64_t *__restrict__ I, int64_t n, int64_t ndofs, uint64_t *__restrict__ keys,
-                           int *__restrict__ err)
+// the same for checked 0-based indices
+__global__ void k_coo_keys32(const int32_t *__restrict__ I, const int32_t *__restrict__ J, int64_t n, int minor_bits, int csc,
+                             uint64_t *__restrict__ keys)
 {
-    int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
-    int64_t r = I[k];
-    if (r < 1 || r > ndofs) {
-        atomicOr(err, DERR_RANGE);
-        r = 1;
-    }
-    keys[k] = (uint64_t)(r - 1);
+    const uint64_t r = (uint64_t)I[k], cc = (uint64_t)J[k];
+    keys[k] = csc ? (cc << minor_bits) | r : (r << minor_bits) | cc;
 }
 
-// Host wrappers used by api.hip for the generic drop-in.
+__global__ void k_vec_keys(const int32_t *__restrict__ I, int64_t n, uint64_t *__restrict__ keys)
+{
+    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < n) keys[k] = (uint64_t)I[k];
+}
+
+// Host wrappers used for the generic drop-in.
 int plain_coo_keys(elfel_hip_ctx *c, const int64_t *I, const int64_t *J, int64_t n, int64_t nrow, int64_t ncol,
                    int minor_bits, int csc, uint64_t *keys)
 {
@@ -236,11 +216,18 @@ int plain_coo_keys(elfel_hip_ctx *c, const int64_t *I, const int64_t *J, int64_t
     return 0;
 }
 
-int plain_vec_keys(elfel_hip_ctx *c, const int64_t *I, int64_t n, int64_t ndofs, uint64_t *keys)
+int plain_coo_keys32(elfel_hip_ctx *c, const int32_t *I, const int32_t *J, int64_t n, int minor_bits, int csc, uint64_t *keys)
 {
     if (n == 0) return 0;
-    hipLaunchKernelGGL(k_vec_keys, dim3(ceil_div(n, 256)), dim3(256), 0, c->stream, I, n, ndofs, keys,
-                       (int *)c->dscal.p + 1);
+    hipLaunchKernelGGL(k_coo_keys32, dim3(ceil_div(n, 256)), dim3(256), 0, c->stream, I, J, n, minor_bits, csc, keys);
+    HIPCHK(c, hipGetLastError());
+    return 0;
+}
+
+int plain_vec_keys(elfel_hip_ctx *c, const int32_t *I, int64_t n, uint64_t *keys)
+{
+    if (n == 0) return 0;
+    hipLaunchKernelGGL(k_vec_keys, dim3(ceil_div(n, 256)), dim3(256), 0, c->stream, I, n, keys);
     HIPCHK(c, hipGetLastError());
     return 0;
 }

@@ -889,6 +889,7 @@ static int build_symbolic(elfel_hip_ctx *c, const elfel_hip_problem *pb, const Q
     ReuseTables T;
     const int cap = block * reuse_tpt(pb->kind);  // task slots per tile
     P.fallback = false;
+    if ((rc = host_tables(c, c->f[0])) || (F1 && (rc = host_tables(c, c->f[1])))) return rc;
     rc = tile_tables(c, stokes, F0, F1, n, hptr, hind, cap, block, T, env_int("ELFEL_HIP_PATCH_TILES", 1) != 0,
                      pb->kind == ELFEL_HEAT && env_int("ELFEL_HIP_HEAT_ROWS", 1) != 0);
     if (rc == ELFEL_ENOTSUP) {

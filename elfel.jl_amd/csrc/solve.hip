@@ -982,8 +982,8 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
     uint32_t *len = up; up += std::max<int64_t>(n, nslices);
     uint32_t *total = up;
 
-    HIPCHK(c, hipMemcpyAsync(xfull, x, 8 * N, hipMemcpyHostToDevice, st));
-    HIPCHK(c, hipMemcpyAsync(b, F, 8 * n, hipMemcpyHostToDevice, st));
+    const HostIn in[2] = {{x, xfull, N, false, 0, 0}, {F, b, n, false, 0, 0}};
+    if ((rc = to_device(c, in, 2, nullptr))) return rc;
 
     // ---- SELL-64 of the free block ------------------------------------------
     hipLaunchKernelGGL(k_fill<uint32_t>, dim3(1), dim3(64), 0, st, (int64_t)4, total, 0u);
@@ -1123,8 +1123,8 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
         }
     }
     HIPCHK(c, hipGetLastError());
-    HIPCHK(c, hipMemcpyAsync(x, xfull, 8 * n, hipMemcpyDeviceToHost, st));
-    HIPCHK(c, hipStreamSynchronize(st));
+    const HostOut o{x, xfull, n, false, 0};
+    if ((rc = to_host(c, &o, 1))) return rc;
     if (iters) *iters = it;
     if (outer) *outer = nupd;
     if (relres) *relres = rn / bnorm;
