@@ -134,7 +134,7 @@ __global__ void k_sell_width(int64_t nfree, int64_t nslices, const uint32_t *__r
     for (int d = 32; d > 0; d >>= 1) w = max(w, (uint32_t)__shfl_down((int)w, d, 64));
     if (lane == 0) {  // it holds the maximum
         size[s] = 64u * w;
-        if (w > SELL_UNROLL) *wide = 1u;
+        if (w > SELL_UNROLL) wide[0] = 1u;
     }
 }
 
@@ -190,6 +190,40 @@ __global__ void k_sell_uniform(int64_t nfree, int64_t nslices, const uint32_t *_
         if (lane == 0) uoff[sb + k] = d0;
     }
     if (lane == 0) uflag[s] = uniform ? 1u : 0u;
+}
+
+// A slice for the resident solve (k_cg_resident): the first offsets of (at
+// most) three runs of three neighbouring offsets that hold every entry of its
+// rows -- the three grid rows of a quadrilateral's or triangle's stencil; a row
+// may lack any of the nine.  nslow counts the slices that have no such runs.
+// One wave per slice.
+#define RES_W 9
+__global__ void k_sell_rec(int64_t nfree, int64_t nslices, const uint32_t *__restrict__ off,
+                           const int16_t *__restrict__ col, const uint32_t *__restrict__ len, uint4 *__restrict__ rec,
+                           uint32_t *__restrict__ nslow)
+{
+    const int64_t s = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    const int lane = threadIdx.x & 63;
+    if (s >= nslices) return;
+    const int64_t i = s * 64 + lane;
+    const uint32_t o = off[s], w = i < nfree ? len[i] : 0u;
+    const int32_t NONE = 1 << 20;
+    int32_t first[3], low = -NONE;
+    for (int g = 0; g < 4; g++) {
+        int32_t m = NONE;  // the smallest offset that the runs so far do not hold
+        for (uint32_t k = 0; k < w; k++) {
+            const int32_t d = col[(size_t)o + (size_t)k * 64 + lane];
+            if (d >= low && d < m) m = d;
+        }
+        for (int t = 32; t > 0; t >>= 1) m = min(m, __shfl_xor(m, t, 64));
+        if (g < 3) {
+            first[g] = m;  // NONE: no entry is there, and what is read for it meets zeros
+        } else if (m < NONE && lane == 0) {
+            atomicAdd(nslow, 1u);
+        }
+        low = m < NONE ? m + 3 : NONE;
+    }
+    if (lane == 0) rec[s] = make_uint4((uint32_t)first[0], (uint32_t)first[1], (uint32_t)first[2], 0);
 }
 
 struct SellU {
@@ -489,20 +523,24 @@ __global__ __launch_bounds__(SV_BLOCK) void k_cg_fin(int64_t n, const double *__
 // is through (everybody has read it then, and nobody looks at it before the
 // exchange after the next, which waits for this workgroup's next partial).
 // The launch is cooperative, so that all workgroups run and every wait ends;
-// a wait that lasts for seconds ends the solve with an error instead.
+// a wait of EX_LIMIT polls, near a second (another process's launch holds some
+// of the CUs, and waits too), ends the launch: what it has made of x is the
+// start of the two-launch iteration, as any x is.
 // VB: the registers of a row (its entries, the gathers in flight) leave 512
 // work-items of FP64 rows or 768 of FP32 rows; larger workgroups spill (1024
 // FP64: 14.9 us an iteration at 9801 rows), smaller ones are more pollers of the
 // same slots (256: 10.5 and 10.8 against 9.4 and 9.0 us at 62 000 rows).
 // SM_GRID: as many workgroups as measured faster than two launches (iteration
-// at 100^2, 250^2, 300^2 rows FP64 7.8, 9.4, 10.3 against 15.3, 15.2, 16.8 us;
-// mixed 100^2, 250^2, 400^2 8.8, 9.0, 11.3 against 15.5, 14.8, 17.0), with an
+// at 100^2, 250^2, 300^2 rows FP64 6.8, 8.3, 8.6 against 15.3, 15.2, 16.8 us;
+// mixed 100^2, 250^2, 400^2 6.8, 7.8, 9.0 against 15.5, 14.8, 17.0), with an
 // eighth of the CUs left free.
 #define SM_VB8 2
 #define SM_VB4 3
 #define SM_GRID 224
 #define EX_NONE 0xfff8dead5eedbeefull
-#define EX_LIMIT (1 << 23)
+#ifndef EX_LIMIT
+#define EX_LIMIT (1 << 20)
+#endif
 
 // z and p are written and gathered, and the slots filled and polled, with
 // relaxed agent-scope accesses: they bypass the XCDs' L2 (the compiler's
@@ -514,6 +552,17 @@ template <typename T>
 __device__ __forceinline__ T dev_load(const T *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 template <typename T>
 __device__ __forceinline__ void dev_store(T *p, T v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+// the same at 32-bit indexes (a scalar base and one offset register)
+template <typename T>
+__device__ __forceinline__ T dev_load_at(const T *p, int32_t i)
+{
+    return dev_load((const T *)((const char *)p + (uint32_t)i * (uint32_t)sizeof(T)));
+}
+template <typename T>
+__device__ __forceinline__ void dev_store_at(T *p, int32_t i, T v)
+{
+    dev_store((T *)((char *)p + (uint32_t)i * (uint32_t)sizeof(T)), v);
+}
 #define STORES_OUT() asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory")
 
 struct Exchange {
@@ -563,17 +612,30 @@ __device__ __forceinline__ bool exchange(const Exchange &X, uint32_t e, double &
     if (tid < SV_BLOCK) {
         a = 0.0;
         b = 0.0;
-        for (int i = tid; i < X.G; i += SV_BLOCK) {
-            uint64_t u, v = 0;
+        for (int i = tid; i < X.G; i += 4 * SV_BLOCK) {
+            uint64_t u[4], v[4];
             int spin = 0;
+            bool wait;
             do {
-                u = dev_load(set + i);
-                if (TWO) v = dev_load(set + X.G + i);
-                if (u != EX_NONE && v != EX_NONE) break;
-            } while (++spin < EX_LIMIT);
-            if (spin >= EX_LIMIT) *quit = 1u;
-            a += __builtin_bit_cast(double, u);
-            if (TWO) b += __builtin_bit_cast(double, v);
+                wait = false;
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    u[q] = v[q] = 0;
+                    if (i + q * SV_BLOCK < X.G) {
+                        u[q] = dev_load_at(set, i + q * SV_BLOCK);
+                        if (TWO) v[q] = dev_load_at(set, X.G + i + q * SV_BLOCK);
+                    }
+                }
+#pragma unroll
+                for (int q = 0; q < 4; q++) wait |= u[q] == EX_NONE || v[q] == EX_NONE;
+            } while (wait && ++spin < EX_LIMIT);
+            if (wait) *quit = 1u;
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                if (i + q * SV_BLOCK >= X.G) break;
+                a += __builtin_bit_cast(double, u[q]);
+                if (TWO) b += __builtin_bit_cast(double, v[q]);
+            }
         }
         for (int d = 32; d > 0; d >>= 1) {
             a += __shfl_down(a, d, 64);
@@ -606,7 +668,7 @@ __global__ void k_cg_slots(uint64_t *__restrict__ slots, int n)
 
 // Groups of CHECK iterations from the state that k_cg_reset or this kernel left
 // (r, z, p, r.z partials) until ||r||^2 <= goal2 or maxit; leaves the same state
-// as k_cg_fin, the iteration count in sc[S_IT] (-1 if a wait failed) and ||r||^2 in sc[S_RREC].
+// as k_cg_fin, the iteration count in sc[S_IT] (-1 - it if a wait failed) and ||r||^2 in sc[S_RREC].
 template <typename T, typename TX, typename C, int VB>
 __global__ __launch_bounds__(VB * SV_BLOCK) void k_cg_small(int64_t n, const uint32_t *__restrict__ off,
                                                        const C *__restrict__ col, const T *__restrict__ val,
@@ -706,7 +768,236 @@ __global__ __launch_bounds__(VB * SV_BLOCK) void k_cg_small(int64_t n, const uin
     // (every workgroup reads S_RR at its start: the result has its own word)
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         sc[S_RREC] = rr;
-        sc[S_IT] = ok ? (double)it : -1.0;
+        sc[S_IT] = ok ? (double)it : -1.0 - (double)it;
+    }
+}
+
+// ---- systems that the register file holds -----------------------------------------
+// The same one launch for larger systems on grid-like meshes (k_sell_rec): a
+// workgroup a CU, R rows a work-item, with their entries in registers (R x 9 of
+// them) and r, 1/diagonal, p and the iterate in LDS.  An iteration then reads
+// and writes z and p alone where the streaming kernels move 80 bytes a row.
+// Streaming -> resident, us an iteration: FP64 Q4 460x450 22.9 -> 9.4, T3
+// 700x690 29.4 -> 13.0; mixed Q4 500^2 19.1 -> 7.9, 1000^2 30.5 -> 14.4,
+// 1500x1300 (1.95 million rows) 44.3 -> 25.3.  Of the last, 8.5 are the two
+// exchanges and the wait for the slowest workgroup (the rest alone takes 16.7),
+// and loads through the L2 in place of device-scope ones would take as long.
+// The rows, blocks and sums are those of the streaming kernels (block b's rows
+// are b * 256 + t + k * 256 G): the same bits.
+//
+// A row's nine neighbours lie three by three: six loads of three words fetch
+// their z and p, past the caches that other workgroups' stores do not reach,
+// with bounds of their own (a word outside the vector reads zero, and the
+// entry for it is zero).  z, p and p2 lie between GUARD zeros, for runs that
+// begin just outside.
+#define RES_VB 4
+#define RES_BLOCK (RES_VB * SV_BLOCK)
+#define GUARD 4
+
+__global__ void k_cg_guards(double *__restrict__ a, float *__restrict__ b, int64_t n)
+{
+    const int t = threadIdx.x;
+    if (t >= 6 * GUARD) return;
+    const int64_t at = (t / (2 * GUARD)) * (n + 2 * GUARD) + (t % (2 * GUARD) < GUARD ? t % GUARD : n + GUARD + t % GUARD);
+    if (a) a[at] = 0.0;
+    if (b) b[at] = 0.f;
+}
+
+// a * b rounded, whatever it is added to
+template <typename T>
+__device__ __forceinline__ T product(T a, T b)
+{
+#pragma clang fp contract(off)
+    return a * b;
+}
+
+// Three neighbouring words of a guarded vector, device-coherent.
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+#define SC1 16  // cache policy: device scope
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t guarded_rsrc(const void *v, size_t word, int64_t n)
+{
+    return __builtin_amdgcn_make_buffer_rsrc((char *)const_cast<void *>(v) - GUARD * word, 0, (int)((n + 2 * GUARD) * word),
+                                             0x00020000);
+}
+__device__ __forceinline__ void load3(__amdgpu_buffer_rsrc_t r, int32_t i, float *o)
+{
+    const u32x3 v = __builtin_amdgcn_raw_buffer_load_b96(r, (i + GUARD) * 4, 0, SC1);
+#pragma unroll
+    for (int k = 0; k < 3; k++) o[k] = __builtin_bit_cast(float, (uint32_t)v[k]);
+}
+__device__ __forceinline__ void load3(__amdgpu_buffer_rsrc_t r, int32_t i, double *o)
+{
+    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, (i + GUARD) * 8, 0, SC1);
+    const u32x2 u = __builtin_amdgcn_raw_buffer_load_b64(r, (i + GUARD) * 8 + 16, 0, SC1);
+    o[0] = __builtin_bit_cast(double, ((uint64_t)v[1] << 32) | v[0]);
+    o[1] = __builtin_bit_cast(double, ((uint64_t)v[3] << 32) | v[2]);
+    o[2] = __builtin_bit_cast(double, ((uint64_t)u[1] << 32) | u[0]);
+}
+
+template <typename T, typename TX, int R>
+__global__ __launch_bounds__(RES_BLOCK) void k_cg_resident(int64_t n, const uint32_t *__restrict__ off,
+                                                           const int16_t *__restrict__ col, const T *__restrict__ val,
+                                                           const uint4 *__restrict__ rec, const T *__restrict__ dinv, T *r_,
+                                                           T *z_, T *pa, T *pb, TX *xs_, double *x_, const double *part_rz,
+                                                           Exchange X, double *sc, double goal2, int it, int maxit)
+{
+    __shared__ T sr[R][RES_BLOCK], sd[R][RES_BLOCK], sp[R][RES_BLOCK];
+    __shared__ TX sx[R][RES_BLOCK];
+    __shared__ double sh[2][RES_BLOCK / 64], sum[2][SV_BLOCK / 64];
+    __shared__ uint32_t quit;
+    const int tid = threadIdx.x, lane = tid & 63;
+    if (tid == 0) quit = 0;
+    const int32_t i0 = (int32_t)(blockIdx.x * RES_BLOCK + tid), stride = X.G * SV_BLOCK, nn = (int32_t)n;
+    const int32_t s0 = __builtin_amdgcn_readfirstlane(i0 >> 6), sstride = stride >> 6;
+    const int32_t slast = (nn - 1) >> 6;
+    // row k's number, formed anew (kept for all rows, with what follows from it,
+    // it would take the registers that hold the matrix)
+    auto row = [&](int k) -> int32_t {
+        int32_t i = i0 + k * stride;
+        asm volatile("" : "+v"(i));
+        return i;
+    };
+    T v[R][RES_W], qv[R];
+#pragma unroll
+    for (int k = 0; k < R; k++) {
+        const int32_t i = row(k), ic = min(i, nn - 1), s = s0 + k * sstride;
+        qv[k] = T(0);
+#pragma unroll
+        for (int q = 0; q < RES_W; q++) v[k][q] = T(0);
+        if (s <= slast) {
+            const uint4 m = rec[s];
+            const uint32_t o = off[s], w = (off[s + 1] - o) >> 6;
+            for (uint32_t q = 0; q < w; q++) {
+                const size_t at = (size_t)o + (size_t)q * 64 + lane;
+                const T x = val[at];  // zero in the padding of a short row, whose column is its own
+                const int32_t d = col[at];
+                if (x != T(0) || d != 0) {
+#pragma unroll
+                    for (int j = 0; j < RES_W; j++)
+                        if (d == (int32_t)(j < 3 ? m.x : j < 6 ? m.y : m.z) + j % 3) v[k][j] = x;
+                }
+            }
+        }
+        sr[k][tid] = r_[ic];
+        sd[k][tid] = dinv[ic];
+        sp[k][tid] = pa[ic];
+        sx[k][tid] = xs_[ic];
+        if (i >= nn) {
+#pragma unroll
+            for (int q = 0; q < RES_W; q++) v[k][q] = T(0);
+        }
+    }
+    double rz = 0.0, rz_old = 0.0, rr = 0.0, none = 0.0;
+    if (tid < SV_BLOCK) {
+        for (int k = tid; k < X.G; k += SV_BLOCK) rz += part_rz[k];
+        for (int d = 32; d > 0; d >>= 1) rz += __shfl_down(rz, d, 64);
+        if (lane == 0) sum[0][tid >> 6] = rz;
+    }
+    __syncthreads();
+    rz = 0.0;
+    for (int k = 0; k < SV_BLOCK / 64; k++) rz += sum[0][k];
+    const __amdgpu_buffer_rsrc_t bz = guarded_rsrc(z_, sizeof(T), n);
+    T *p_old = pa, *p_new = pb;
+    uint32_t e = 0;
+    bool dir = false, ok = true;
+    rr = sc[S_RR];
+    while (ok && rr > goal2 && it < maxit) {
+        for (int c = 0; c < CHECK && ok; c++) {
+            const T beta = dir ? (T)(rz_old != 0.0 ? rz / rz_old : 0.0) : T(0);
+            const __amdgpu_buffer_rsrc_t bp = guarded_rsrc(p_old, sizeof(T), n);
+            T zz[3][3], pp[3][3];
+            auto load = [&](int k) {
+                const uint4 m = rec[min(s0 + k * sstride, slast)];
+                const int32_t i = row(k);
+#pragma unroll
+                for (int g = 0; g < 3; g++) {
+                    const int32_t j = i + (int32_t)(g == 0 ? m.x : g == 1 ? m.y : m.z);
+                    load3(bp, j, pp[g]);
+                    load3(bz, j, zz[g]);
+                }
+            };
+            double pq = 0.0;
+            load(0);
+#pragma unroll
+            for (int k = 0; k < R; k++) {
+                T y[RES_W];
+#pragma unroll
+                for (int j = 0; j < RES_W; j++) y[j] = dir ? zz[j / 3][j % 3] + beta * pp[j / 3][j % 3] : pp[j / 3][j % 3];
+                __builtin_amdgcn_sched_barrier(0);
+                if (k + 1 < R) load(k + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                T acc = T(0);
+#pragma unroll
+                for (int j = 0; j < RES_W; j++) acc += v[k][j] * y[j];
+                qv[k] = acc;
+                const int32_t i = row(k);
+                if (i < nn) {
+                    T pk = sp[k][tid];
+                    if (dir) {
+                        pk = product(sd[k][tid], sr[k][tid]) + beta * pk;
+                        sp[k][tid] = pk;
+                        dev_store_at(p_new, i, pk);
+                    }
+                    pq += (double)pk * (double)acc;
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (dir) {
+                T *t = p_old;
+                p_old = p_new;
+                p_new = t;
+            }
+            dir = true;
+            if (!(ok = exchange<RES_VB, false>(X, e++, pq, none, sh, sum, &quit))) break;
+            const double alpha64 = pq != 0.0 ? rz / pq : 0.0;
+            const T alpha = (T)alpha64;
+            const TX alphax = (TX)alpha64;
+            double a = 0.0, b = 0.0;
+#pragma unroll
+            for (int k = 0; k < R; k++) {
+                const int32_t i = row(k);
+                if (i >= nn) break;
+                const T ri = sr[k][tid] - alpha * qv[k];
+                const T zi = sd[k][tid] * ri;
+                sr[k][tid] = ri;
+                dev_store_at(z_, i, zi);
+                a += (double)ri * (double)zi;
+                b += (double)ri * (double)ri;
+                sx[k][tid] += alphax * (TX)sp[k][tid];
+            }
+            if (!(ok = exchange<RES_VB, true>(X, e++, a, b, sh, sum, &quit))) break;
+            rz_old = rz;
+            rz = a;
+            rr = b;
+        }
+        if constexpr (sizeof(TX) == 4) {
+#pragma unroll
+            for (int k = 0; k < R; k++) {
+                const int32_t i = row(k);
+                if (i >= nn) break;
+                x_[i] += (double)sx[k][tid];
+                sx[k][tid] = TX(0);
+            }
+        }
+        it += CHECK;
+    }
+    // the state that the next reset continues from
+    if (dir) {
+        const T beta = (T)(rz_old != 0.0 ? rz / rz_old : 0.0);
+#pragma unroll
+        for (int k = 0; k < R; k++) {
+            const int32_t i = row(k);
+            if (i >= nn) break;
+            r_[i] = sr[k][tid];
+            pa[i] = product(sd[k][tid], sr[k][tid]) + beta * sp[k][tid];
+            xs_[i] = sx[k][tid];
+        }
+    }
+    if (blockIdx.x == 0 && tid == 0) {
+        sc[S_RREC] = rr;
+        sc[S_IT] = ok ? (double)it : -1.0 - (double)it;
     }
 }
 
@@ -833,6 +1124,7 @@ struct Sell {
     const double *v64;
     const float *v32;
     SellU U;
+    const uint4 *rec;  // per slice, for the resident solve (null: not made)
 };
 
 template <typename T>
@@ -917,6 +1209,48 @@ int cg_small(hipStream_t st, int64_t n, const Sell &S, Vecs<float> &v, const Par
                  : cg_small_as<float, float, int32_t>(st, n, S, v, v.xlo, P, slots, sc, goal2, it, maxit);
 }
 
+template <typename T, typename TX, int R>
+int cg_resident_as(hipStream_t st, int64_t n, const Sell &S, Vecs<T> &v, TX *xs, const Parts &P, uint64_t *slots, double *sc,
+                   double goal2, int it, int maxit)
+{
+    hipLaunchKernelGGL(k_cg_slots, dim3(ceil_div(6 * P.G, 256)), dim3(256), 0, st, slots, 6 * P.G);
+    Exchange X{slots, P.G};
+    const uint32_t *off = S.off;
+    const int16_t *col = (const int16_t *)S.col;
+    const T *val = sell_vals<T>(S);
+    const uint4 *rec = S.rec;
+    const T *dinv = v.dinv;
+    const double *prz = P.rz;
+    double *x = v.x;
+    void *args[] = {&n, &off, &col, &val, &rec, &dinv, &v.r, &v.z, &v.p, &v.p2, &xs, &x, &prz, &X, &sc, &goal2, &it, &maxit};
+    const hipError_t e = hipLaunchCooperativeKernel(reinterpret_cast<const void *>(&k_cg_resident<T, TX, R>),
+                                                    dim3((P.G + RES_VB - 1) / RES_VB), dim3(RES_BLOCK), args, 0, st);
+    if (e == hipSuccess) return 0;
+    (void)hipGetLastError();
+    return 1;
+}
+// Rows a work-item of the resident solve that n rows in G blocks need; most: 3
+// FP64 (786 000 rows on 256 CUs), 8 mixed (2.1 million).
+int cg_resident(hipStream_t st, int64_t n, const Sell &S, Vecs<double> &v, const Parts &P, uint64_t *slots, double *sc,
+                double goal2, int it, int maxit)
+{
+    const int64_t r = (n + (int64_t)P.G * SV_BLOCK - 1) / ((int64_t)P.G * SV_BLOCK);
+    if (r <= 1) return cg_resident_as<double, double, 1>(st, n, S, v, v.x, P, slots, sc, goal2, it, maxit);
+    if (r <= 2) return cg_resident_as<double, double, 2>(st, n, S, v, v.x, P, slots, sc, goal2, it, maxit);
+    if (r <= 3) return cg_resident_as<double, double, 3>(st, n, S, v, v.x, P, slots, sc, goal2, it, maxit);
+    return 1;
+}
+int cg_resident(hipStream_t st, int64_t n, const Sell &S, Vecs<float> &v, const Parts &P, uint64_t *slots, double *sc,
+                double goal2, int it, int maxit)
+{
+    const int64_t r = (n + (int64_t)P.G * SV_BLOCK - 1) / ((int64_t)P.G * SV_BLOCK);
+    if (r <= 1) return cg_resident_as<float, float, 1>(st, n, S, v, v.xlo, P, slots, sc, goal2, it, maxit);
+    if (r <= 2) return cg_resident_as<float, float, 2>(st, n, S, v, v.xlo, P, slots, sc, goal2, it, maxit);
+    if (r <= 4) return cg_resident_as<float, float, 4>(st, n, S, v, v.xlo, P, slots, sc, goal2, it, maxit);
+    if (r <= 8) return cg_resident_as<float, float, 8>(st, n, S, v, v.xlo, P, slots, sc, goal2, it, maxit);
+    return 1;
+}
+
 }  // namespace
 
 int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int precision, double tol, int maxit,
@@ -948,8 +1282,8 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
     //          FP64 vectors r z p p2 q [5n] (FP64 solve only)
     // floats:  r z p p2 q dinv xlo [7n] (mixed solve only; its iterate is the FP64 xfull + xlo)
     // uint32:  off[nslices + 1], len[max(n, nslices)], total[4]
-    const size_t nd = (size_t)N + 3 * (size_t)n + 10 * (size_t)G + S_NS + (mixed ? 0 : 5 * (size_t)n);
-    const size_t nf = mixed ? 7 * (size_t)n : 0;
+    const size_t nd = (size_t)N + 3 * (size_t)n + 10 * (size_t)G + S_NS + (mixed ? 0 : 5 * (size_t)n + 6 * GUARD);
+    const size_t nf = mixed ? 7 * (size_t)n + 6 * GUARD : 0;
     const size_t nu32 = (size_t)nslices + 1 + (size_t)std::max<int64_t>(n, nslices) + 4;
     int rc = ensure(c, c->pcg, 8 * nd + 4 * nf + 4 * nu32 + 256);
     if (rc) return rc;
@@ -963,17 +1297,22 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
     P.pq = dp; dp += G; P.rz = dp; dp += G; P.rr = dp; dp += G; P.aux = dp; dp += G;
     uint64_t *slots = (uint64_t *)dp; dp += 6 * G;
     double *sc = dp; dp += S_NS;
+    void *guarded = nullptr;  // z, p, p2, each between GUARD zeros
     Vecs<double> v64{};
     if (!mixed) {
         v64.x = xfull;  // the free part of the full vector is the iterate
-        v64.r = dp; dp += n; v64.z = dp; dp += n; v64.p = dp; dp += n; v64.p2 = dp; dp += n; v64.q = dp; dp += n;
+        v64.r = dp; dp += n; v64.q = dp; dp += n;
+        guarded = dp;
+        v64.z = dp + GUARD; dp += n + 2 * GUARD; v64.p = dp + GUARD; dp += n + 2 * GUARD; v64.p2 = dp + GUARD; dp += n + 2 * GUARD;
         v64.dinv = dinv64;
     }
     float *fp = (float *)dp;
     Vecs<float> v32{};
     if (mixed) {
         v32.x = xfull;  // the free part of the full vector is the iterate (FP64)
-        v32.r = fp; fp += n; v32.z = fp; fp += n; v32.p = fp; fp += n; v32.p2 = fp; fp += n; v32.q = fp; fp += n;
+        v32.r = fp; fp += n; v32.q = fp; fp += n;
+        guarded = fp;
+        v32.z = fp + GUARD; fp += n + 2 * GUARD; v32.p = fp + GUARD; fp += n + 2 * GUARD; v32.p2 = fp + GUARD; fp += n + 2 * GUARD;
         v32.dinv = fp; fp += n;
         v32.xlo = fp; fp += n;
     }
@@ -982,6 +1321,8 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
     uint32_t *len = up; up += std::max<int64_t>(n, nslices);
     uint32_t *total = up;
 
+    hipLaunchKernelGGL(k_cg_guards, dim3(1), dim3(64), 0, st, mixed ? nullptr : (double *)guarded,
+                       mixed ? (float *)guarded : nullptr, n);
     const HostIn in[2] = {{x, xfull, N, false, 0, 0}, {F, b, n, false, 0, 0}};
     if ((rc = to_device(c, in, 2, nullptr))) return rc;
 
@@ -1001,7 +1342,8 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
     const size_t cbytes = (size_t)nnzp * (c16 ? 2 : 4);
     const size_t nslots = (size_t)nnzp / 64;
     const size_t vbytes = (size_t)nnzp * (8 + (mixed ? 4 : 0));
-    const size_t sbytes = ((cbytes + 15) & ~(size_t)15) + vbytes + 4 * (size_t)(nslices + 1) + 4 * (nslots + SELL_UNROLL) + 256;
+    const size_t sbytes = ((cbytes + 15) & ~(size_t)15) + vbytes + 4 * (size_t)(nslices + 1) + 4 * (nslots + SELL_UNROLL) +
+                          16 * (size_t)(nslices + 1) + 256;
     if ((rc = ensure(c, c->pcg_sell, sbytes))) return rc;
     void *scol = c->pcg_sell.p;
     double *sv64 = (double *)((char *)c->pcg_sell.p + ((cbytes + 15) & ~(size_t)15));
@@ -1028,7 +1370,14 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
     hipLaunchKernelGGL(k_diag_inv, dim3(ceil_div(n, 256)), dim3(256), 0, st, n, ptr, ind, val, dinv64,
                        mixed ? v32.dinv : nullptr);
     HIPCHK(c, hipGetLastError());
-    const Sell S{off, scol, c16, sv64, sv32, SellU{uflag, uoff}};
+    // records for the resident solve where rows are narrow and columns near
+    const bool near9 = c16 && narrow;
+    uint4 *rec = (uint4 *)(((uintptr_t)(uoff + nslots + SELL_UNROLL) + 15) & ~(uintptr_t)15);
+    if (near9)
+        hipLaunchKernelGGL(k_sell_rec, dim3(ceil_div(nslices * 64, 256)), dim3(256), 0, st, n, nslices,
+                           (const uint32_t *)off, (const int16_t *)scol, (const uint32_t *)len, rec, total + 1);
+    hipLaunchKernelGGL(k_tell, dim3(1), dim3(64), 0, st, (const uint32_t *)total, (uint32_t *)c->told + 8);
+    const Sell S{off, scol, c16, sv64, sv32, SellU{uflag, uoff}, near9 ? rec : nullptr};
 
     // the scalars as the last reduction left them, in pinned memory
     double *hsc = (double *)c->told + 8;
@@ -1066,21 +1415,26 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
     int it = 0, nupd = 0;
     double rn = 0.0;
     if ((rc = true_residual(&rn))) return rc;
+    const bool resident = near9 && tot[1] == 0;
+    bool lost = false;  // a one-launch solve's workgroups did not all run: two launches from then on
     const double bnorm = hsc[S_BB] > 0 ? sqrt(hsc[S_BB]) : 1.0;
     const double target = tol * bnorm;
     // Iterations until ||r||^2 <= goal2 or maxit from the state of the last reset,
     // then the true residual (waits): *rrec the recurrence's ||r||^2, *norm the
     // true residual's norm.  One launch where every row has its own work-item,
-    // the rows fit its registers and there are few enough workgroups.
+    // the rows fit its registers and there are few enough workgroups, or where
+    // all slices have records and the rows fit the chip's registers.
     auto solve_to = [&](auto &v, double goal2, double *rrec, double *norm) -> int {
         using T = typename std::remove_pointer<decltype(v.r)>::type;
         constexpr int VB = sizeof(T) == 8 ? SM_VB8 : SM_VB4;
-        if (narrow && n <= (int64_t)P.G * SV_BLOCK && (P.G + VB - 1) / VB <= SM_GRID &&
-            cg_small(st, n, S, v, P, slots, sc, goal2, it, maxit) == 0) {
+        const bool small = narrow && n <= (int64_t)P.G * SV_BLOCK && (P.G + VB - 1) / VB <= SM_GRID;
+        const bool one = !lost && ((small && cg_small(st, n, S, v, P, slots, sc, goal2, it, maxit) == 0) ||
+                                   (resident && cg_resident(st, n, S, v, P, slots, sc, goal2, it, maxit) == 0));
+        if (one) {
             if ((rc = true_residual(norm))) return rc;
-            if (hsc[S_IT] < 0) return set_err(c, ELFEL_EHIP, "elfel_hip_pcg: the solve's workgroups lost each other");
-            it = (int)hsc[S_IT];
-            *rrec = hsc[S_RREC];
+            lost = hsc[S_IT] < 0;
+            it = lost ? -1 - (int)hsc[S_IT] : (int)hsc[S_IT];
+            *rrec = lost ? 0.0 : hsc[S_RREC];  // 0: the next reset restarts from p = z
             return 0;
         }
         for (;;) {

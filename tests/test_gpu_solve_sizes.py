@@ -1,8 +1,11 @@
 """elfel_hip_pcg at the sizes where its kernels change: rows either side of a
 wave, of a block of 256 rows, of a workgroup of the one-launch solve (512 rows
-FP64, 768 mixed), of the most rows that it takes (224 workgroups), a matrix
-whose rows are wider than its registers, and one whose columns are too far from
-the diagonal for 16-bit offsets.
+FP64, 768 mixed), of the most rows that it takes (224 workgroups), of each count
+of rows a work-item of the solve from registers (262144 rows each on 256 CUs; 1
+to 3 FP64, 1, 2, 4, 8 mixed) and past its last, grids with their boundary
+numbered last and ones whose slices it does not take, a matrix whose rows are
+wider than the registers, and one whose columns are too far from the diagonal
+for 16-bit offsets.
 
 The solve stops on its own FP64 residual, ||b - A x|| <= tol ||b||.  The same
 residual formed here differs by the rounding of its sums, at most about
@@ -21,13 +24,13 @@ pytestmark = pytest.mark.gpu
 TOL = 1e-8
 
 
-def _solve(ctx, fe, N, nfree, prec, seed=3, shuffle=False, kind=L.HEAT):
+def _solve(ctx, fe, N, nfree, prec, seed=3, shuffle=False, kind=L.HEAT, order=None):
     block = {L.Q4: eh.Q4block, L.T3: eh.T3block, L.T6: eh.T6block}[fe]
     mesh = block(1.0, 1.0, N, N)
     nc = 2 if kind == L.ELAST else 1
     n = mesh.nnodes * nc
     rng = np.random.default_rng(seed)
-    dn = (rng.permutation(n) if shuffle else np.arange(n)) + 1
+    dn = (rng.permutation(n) if shuffle else np.arange(n) if order is None else order) + 1
     ctx.set_mesh(0, mesh.conn, mesh.xy)
     ctx.set_dofs(0, dn.reshape(-1, nc), n)
     ctx.set_coefficients(mesh.nelements)
@@ -63,3 +66,29 @@ def test_wide_rows_and_far_columns(ctx, prec):
     _solve(ctx, L.T6, 12, 1100, prec, kind=L.ELAST)  # rows of up to 38 entries
     _solve(ctx, L.T3, 200, 39000, prec, shuffle=True)
     _solve(ctx, L.T3, 30, 900, prec, shuffle=True)
+
+
+@pytest.mark.parametrize("prec,fe,nfree,N", [
+    (L.FP64, L.Q4, 262144, 520), (L.FP64, L.T3, 262145, 520), (L.FP64, L.T3, 524288, 730), (L.FP64, L.Q4, 524289, 730),
+    (L.FP64, L.Q4, 786432, 890), (L.FP64, L.T3, 786433, 890),
+    (L.MIXED, L.T3, 262144, 520), (L.MIXED, L.Q4, 262145, 520), (L.MIXED, L.Q4, 524289, 730),
+    (L.MIXED, L.T3, 1048577, 1030), (L.MIXED, L.Q4, 2097152, 1449), (L.MIXED, L.T3, 2097153, 1449)])
+def test_rows_in_registers(ctx, prec, fe, nfree, N):
+    _solve(ctx, fe, N, nfree, prec)
+
+
+@pytest.mark.parametrize("prec", [L.FP64, L.MIXED])
+@pytest.mark.parametrize("fe", [L.T3, L.Q4])
+@pytest.mark.parametrize("held", ["boundary", "scattered", "swapped"])
+def test_held_nodes_and_numberings(ctx, held, fe, prec):
+    N = 560  # 561 x 561 nodes; the free ones first, in the mesh's order
+    fixed = np.zeros((N + 1, N + 1), bool)
+    fixed[[0, -1]] = fixed[:, [0, -1]] = True
+    if held == "scattered":
+        fixed |= np.random.default_rng(5).random(fixed.shape) < 0.01
+    fixed = fixed.ravel()
+    free = int((~fixed).sum())
+    order = np.where(fixed, free + np.cumsum(fixed) - 1, np.cumsum(~fixed) - 1)
+    if held == "swapped":  # free neighbours by twos: offsets of no three runs
+        order = np.where(order < free // 2 * 2, order ^ 1, order)
+    _solve(ctx, fe, N, free, prec, order=order)
