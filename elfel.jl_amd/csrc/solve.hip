@@ -62,7 +62,7 @@ int env_int(const char *name, int dflt);  // reuse.hip
 namespace {
 
 // Scalars (double) on the device, for the host's convergence checks.
-enum { S_RZ = 0, S_RR = 1, S_BB = 2, S_RR64 = 3, S_ALPHA = 4, S_RZS = 5 /* two words */, S_IT = 7, S_RREC = 8, S_NS = 10 };
+enum { S_RZ = 0, S_RR = 1, S_BB = 2, S_RR64 = 3, S_ALPHA = 4, S_RZS = 5 /* two words */, S_IT = 7, S_RREC = 8, S_LOST = 9, S_NS = 10 };
 
 __device__ __forceinline__ double block_sum(double v, double *sh)
 {
@@ -192,14 +192,14 @@ __global__ void k_sell_uniform(int64_t nfree, int64_t nslices, const uint32_t *_
     if (lane == 0) uflag[s] = uniform ? 1u : 0u;
 }
 
-// A slice for the resident solve (k_cg_resident): the first offsets of (at
-// most) three runs of three neighbouring offsets that hold every entry of its
-// rows -- the three grid rows of a quadrilateral's or triangle's stencil; a row
-// may lack any of the nine.  nslow counts the slices that have no such runs.
-// One wave per slice.
+// A slice for the resident solve (k_cg_resident): its rows' entries lie on the
+// diagonal and its two neighbours, in one run of three neighbouring offsets
+// below and one above -- the three grid rows of a quadrilateral's or triangle's
+// stencil; a row may lack any of the nine.  The record is the runs' first
+// offsets; nslow counts the slices that have no such runs.  One wave per slice.
 #define RES_W 9
 __global__ void k_sell_rec(int64_t nfree, int64_t nslices, const uint32_t *__restrict__ off,
-                           const int16_t *__restrict__ col, const uint32_t *__restrict__ len, uint4 *__restrict__ rec,
+                           const int16_t *__restrict__ col, const uint32_t *__restrict__ len, int2 *__restrict__ rec,
                            uint32_t *__restrict__ nslow)
 {
     const int64_t s = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
@@ -208,22 +208,27 @@ __global__ void k_sell_rec(int64_t nfree, int64_t nslices, const uint32_t *__res
     const int64_t i = s * 64 + lane;
     const uint32_t o = off[s], w = i < nfree ? len[i] : 0u;
     const int32_t NONE = 1 << 20;
-    int32_t first[3], low = -NONE;
-    for (int g = 0; g < 4; g++) {
-        int32_t m = NONE;  // the smallest offset that the runs so far do not hold
-        for (uint32_t k = 0; k < w; k++) {
-            const int32_t d = col[(size_t)o + (size_t)k * 64 + lane];
-            if (d >= low && d < m) m = d;
+    int32_t lo = NONE, lo_end = -NONE, hi = NONE, hi_end = -NONE;  // offsets below -1 and above 1
+    for (uint32_t k = 0; k < w; k++) {
+        const int32_t d = col[(size_t)o + (size_t)k * 64 + lane];
+        if (d < -1) {
+            lo = min(lo, d);
+            lo_end = max(lo_end, d);
+        } else if (d > 1) {
+            hi = min(hi, d);
+            hi_end = max(hi_end, d);
         }
-        for (int t = 32; t > 0; t >>= 1) m = min(m, __shfl_xor(m, t, 64));
-        if (g < 3) {
-            first[g] = m;  // NONE: no entry is there, and what is read for it meets zeros
-        } else if (m < NONE && lane == 0) {
-            atomicAdd(nslow, 1u);
-        }
-        low = m < NONE ? m + 3 : NONE;
     }
-    if (lane == 0) rec[s] = make_uint4((uint32_t)first[0], (uint32_t)first[1], (uint32_t)first[2], 0);
+    for (int t = 32; t > 0; t >>= 1) {
+        lo = min(lo, __shfl_xor(lo, t, 64));
+        hi = min(hi, __shfl_xor(hi, t, 64));
+        lo_end = max(lo_end, __shfl_xor(lo_end, t, 64));
+        hi_end = max(hi_end, __shfl_xor(hi_end, t, 64));
+    }
+    if (lane == 0) {
+        rec[s] = make_int2(lo, hi);  // NONE: no entry is there, and what is read for it meets zeros
+        if (lo_end - lo > 2 || hi_end - hi > 2) atomicAdd(nslow, 1u);
+    }
 }
 
 struct SellU {
@@ -531,8 +536,8 @@ __global__ __launch_bounds__(SV_BLOCK) void k_cg_fin(int64_t n, const double *__
 // FP64: 14.9 us an iteration at 9801 rows), smaller ones are more pollers of the
 // same slots (256: 10.5 and 10.8 against 9.4 and 9.0 us at 62 000 rows).
 // SM_GRID: as many workgroups as measured faster than two launches (iteration
-// at 100^2, 250^2, 300^2 rows FP64 6.8, 8.3, 8.6 against 15.3, 15.2, 16.8 us;
-// mixed 100^2, 250^2, 400^2 6.8, 7.8, 9.0 against 15.5, 14.8, 17.0), with an
+// at 100^2, 250^2, 300^2 rows FP64 5.8, 6.3, 6.5 against 15.3, 15.2, 16.8 us;
+// mixed 100^2, 250^2, 400^2 6.2, 6.0, 7.2 against 15.5, 14.8, 17.0), with an
 // eighth of the CUs left free.
 #define SM_VB8 2
 #define SM_VB4 3
@@ -552,22 +557,75 @@ template <typename T>
 __device__ __forceinline__ T dev_load(const T *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 template <typename T>
 __device__ __forceinline__ void dev_store(T *p, T v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-// the same at 32-bit indexes (a scalar base and one offset register)
-template <typename T>
-__device__ __forceinline__ T dev_load_at(const T *p, int32_t i)
-{
-    return dev_load((const T *)((const char *)p + (uint32_t)i * (uint32_t)sizeof(T)));
-}
-template <typename T>
-__device__ __forceinline__ void dev_store_at(T *p, int32_t i, T v)
-{
-    dev_store((T *)((char *)p + (uint32_t)i * (uint32_t)sizeof(T)), v);
-}
 #define STORES_OUT() asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory")
 
+// The value that lane l + D holds, for the lanes l that a tree of __shfl_down over
+// D = 32, 16, ... 1 needs (0 .. D - 1, and those that these need): register
+// moves of a few cycles in place of a round through LDS.
+template <int D>
+__device__ __forceinline__ uint32_t lane_down(uint32_t x)
+{
+    if constexpr (D == 32) return __builtin_amdgcn_permlane32_swap(x, x, false, false)[1];
+    else if constexpr (D == 16) return __builtin_amdgcn_permlane16_swap(x, x, false, false)[1];
+    else return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x100 | D, 0xf, 0xf, true);  // row_shl
+}
+template <int D>
+__device__ __forceinline__ double lane_down(double v)
+{
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    return __builtin_bit_cast(double, (uint64_t)lane_down<D>((uint32_t)(b >> 32)) << 32 | lane_down<D>((uint32_t)b));
+}
+// lane 0: the wave's sum in the order of the shuffle tree
+__device__ __forceinline__ double wave_sum(double v)
+{
+    v += lane_down<32>(v);
+    v += lane_down<16>(v);
+    v += lane_down<8>(v);
+    v += lane_down<4>(v);
+    v += lane_down<2>(v);
+    v += lane_down<1>(v);
+    return v;
+}
+
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+#define SC1 16               // cache policy of buffer accesses: device scope
+
+// Three sets of slots; a block's two partials lie side by side, four blocks to
+// 64 bytes, in EX_COPIES copies: every workgroup polls all slots, of the copy
+// of its number's remainder.  One copy in a few kilobytes is in the same few
+// channels for all of them (us an iteration, packed slots, 1, 4 and 8 copies:
+// FP64 300x290 8.6, 6.9, 6.6, 6.5; mixed 1000^2 15.4, 12.5, 12.4, 11.9).
+#define EX_COPIES 8
+#define EX_LINE (64 * EX_COPIES)
+#define EX_STRIDE(g) (((g) + 3) / 4 * EX_LINE)  // bytes of a set of g blocks
 struct Exchange {
-    uint64_t *slots;  // [3][2][G]
+    uint64_t *slots;
     int G;
+    int stride;  // bytes of a set
+    __device__ __forceinline__ uint32_t at(uint32_t e, int blk, int copy) const
+    {
+        return (e % 3) * (uint32_t)stride + (uint32_t)(blk >> 2) * EX_LINE + (uint32_t)copy * 64 + (uint32_t)(blk & 3) * 16;
+    }
+    __device__ __forceinline__ void put(uint32_t e, int blk, int copy, int two, uint64_t v) const
+    {
+        dev_store((uint64_t *)((char *)slots + at(e, blk, copy) + 8 * two), v);
+    }
+    template <bool TWO>
+    __device__ __forceinline__ void get(uint32_t e, int blk, uint64_t &u, uint64_t &v) const
+    {
+        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(slots, 0, 3 * stride, 0x00020000);
+        int o = (int)at(e, blk, blockIdx.x % EX_COPIES);
+        asm volatile("" : "+v"(o)::"memory");  // a load each time
+        if (TWO) {
+            const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(r, o, 0, SC1);
+            u = ((uint64_t)x[1] << 32) | x[0];
+            v = ((uint64_t)x[3] << 32) | x[2];
+        } else {
+            const u32x2 x = __builtin_amdgcn_raw_buffer_load_b64(r, o, 0, SC1);
+            u = ((uint64_t)x[1] << 32) | x[0];
+        }
+    }
 };
 
 __device__ __forceinline__ uint64_t ex_bits(double v)
@@ -586,28 +644,21 @@ __device__ __forceinline__ bool exchange(const Exchange &X, uint32_t e, double &
                                          double (*sum)[SV_BLOCK / 64], uint32_t *quit)
 {
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    uint64_t *set = X.slots + (size_t)(e % 3) * 2 * X.G, *old = X.slots + (size_t)((e + 2) % 3) * 2 * X.G;
-    const int blk = blockIdx.x * VB + tid;  // of the first VB work-items
     STORES_OUT();
-    for (int d = 32; d > 0; d >>= 1) {
-        a += __shfl_down(a, d, 64);
-        if (TWO) b += __shfl_down(b, d, 64);
-    }
+    a = wave_sum(a);
+    if (TWO) b = wave_sum(b);
     if (lane == 0) {
         sh[0][w] = a;
         if (TWO) sh[1][w] = b;
     }
     __syncthreads();
-    if (w == 0) {
-        if (tid < VB && blk < X.G) {
-            double s = 0.0, s2 = 0.0;
-            for (int k = 0; k < SV_BLOCK / 64; k++) {
-                s += sh[0][tid * (SV_BLOCK / 64) + k];
-                if (TWO) s2 += sh[1][tid * (SV_BLOCK / 64) + k];
-            }
-            dev_store(set + blk, ex_bits(s));
-            if (TWO) dev_store(set + X.G + blk, ex_bits(s2));
-        }
+    // lanes of the first wave: block, partial, copy
+    const int q = lane / (2 * EX_COPIES), two = lane / EX_COPIES % 2, copy = lane % EX_COPIES, blk = blockIdx.x * VB + q;
+    const bool mine = w == 0 && q < VB && blk < X.G;
+    if (mine && (TWO || two == 0)) {
+        double s = 0.0;
+        for (int k = 0; k < SV_BLOCK / 64; k++) s += sh[two][q * (SV_BLOCK / 64) + k];
+        X.put(e, blk, copy, two, ex_bits(s));
     }
     if (tid < SV_BLOCK) {
         a = 0.0;
@@ -621,10 +672,7 @@ __device__ __forceinline__ bool exchange(const Exchange &X, uint32_t e, double &
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
                     u[q] = v[q] = 0;
-                    if (i + q * SV_BLOCK < X.G) {
-                        u[q] = dev_load_at(set, i + q * SV_BLOCK);
-                        if (TWO) v[q] = dev_load_at(set, X.G + i + q * SV_BLOCK);
-                    }
+                    if (i + q * SV_BLOCK < X.G) X.get<TWO>(e, i + q * SV_BLOCK, u[q], v[q]);
                 }
 #pragma unroll
                 for (int q = 0; q < 4; q++) wait |= u[q] == EX_NONE || v[q] == EX_NONE;
@@ -637,10 +685,8 @@ __device__ __forceinline__ bool exchange(const Exchange &X, uint32_t e, double &
                 if (TWO) b += __builtin_bit_cast(double, v[q]);
             }
         }
-        for (int d = 32; d > 0; d >>= 1) {
-            a += __shfl_down(a, d, 64);
-            if (TWO) b += __shfl_down(b, d, 64);
-        }
+        a = wave_sum(a);
+        if (TWO) b = wave_sum(b);
         if (lane == 0) {
             sum[0][w] = a;
             if (TWO) sum[1][w] = b;
@@ -653,22 +699,21 @@ __device__ __forceinline__ bool exchange(const Exchange &X, uint32_t e, double &
         a += sum[0][k];
         if (TWO) b += sum[1][k];
     }
-    if (tid < VB && blk < X.G) {
-        dev_store(old + blk, (uint64_t)EX_NONE);
-        dev_store(old + X.G + blk, (uint64_t)EX_NONE);
-    }
+    if (mine) X.put(e + 2, blk, copy, two, EX_NONE);
     return *quit == 0u;  // set before the barrier by whoever gave up
 }
 
-__global__ void k_cg_slots(uint64_t *__restrict__ slots, int n)
+__global__ void k_cg_slots(uint64_t *__restrict__ slots, int n, double *__restrict__ sc)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0) sc[S_LOST] = 0.0;
     if (i < n) slots[i] = EX_NONE;
 }
 
 // Groups of CHECK iterations from the state that k_cg_reset or this kernel left
 // (r, z, p, r.z partials) until ||r||^2 <= goal2 or maxit; leaves the same state
-// as k_cg_fin, the iteration count in sc[S_IT] (-1 - it if a wait failed) and ||r||^2 in sc[S_RREC].
+// as k_cg_fin, the iteration count in sc[S_IT] and ||r||^2 in sc[S_RREC]; sc[S_LOST] is set by
+// every workgroup that gave up a wait (another may have been through it).
 template <typename T, typename TX, typename C, int VB>
 __global__ __launch_bounds__(VB * SV_BLOCK) void k_cg_small(int64_t n, const uint32_t *__restrict__ off,
                                                        const C *__restrict__ col, const T *__restrict__ val,
@@ -768,8 +813,9 @@ __global__ __launch_bounds__(VB * SV_BLOCK) void k_cg_small(int64_t n, const uin
     // (every workgroup reads S_RR at its start: the result has its own word)
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         sc[S_RREC] = rr;
-        sc[S_IT] = ok ? (double)it : -1.0 - (double)it;
+        sc[S_IT] = (double)it;
     }
+    if (!ok && threadIdx.x == 0) sc[S_LOST] = 1.0;
 }
 
 // ---- systems that the register file holds -----------------------------------------
@@ -777,32 +823,26 @@ __global__ __launch_bounds__(VB * SV_BLOCK) void k_cg_small(int64_t n, const uin
 // workgroup a CU, R rows a work-item, with their entries in registers (R x 9 of
 // them) and r, 1/diagonal, p and the iterate in LDS.  An iteration then reads
 // and writes z and p alone where the streaming kernels move 80 bytes a row.
-// Streaming -> resident, us an iteration: FP64 Q4 460x450 22.9 -> 9.4, T3
-// 700x690 29.4 -> 13.0; mixed Q4 500^2 19.1 -> 7.9, 1000^2 30.5 -> 14.4,
-// 1500x1300 (1.95 million rows) 44.3 -> 25.3.  Of the last, 8.5 are the two
-// exchanges and the wait for the slowest workgroup (the rest alone takes 16.7),
-// and loads through the L2 in place of device-scope ones would take as long.
+// Streaming -> resident, us an iteration: FP64 Q4 460x450 22.9 -> 8.7, T3
+// 700x690 29.4 -> 10.9; mixed Q4 500^2 19.1 -> 7.6, 1000^2 30.5 -> 10.7,
+// 1500x1300 (1.95 million rows) 44.3 -> 19.5.
 // The rows, blocks and sums are those of the streaming kernels (block b's rows
 // are b * 256 + t + k * 256 G): the same bits.
 //
-// A row's nine neighbours lie three by three: six loads of three words fetch
-// their z and p, past the caches that other workgroups' stores do not reach,
-// with bounds of their own (a word outside the vector reads zero, and the
-// entry for it is zero).  z, p and p2 lie between GUARD zeros, for runs that
-// begin just outside.
+// What bounds it: up to 1 million rows the two exchanges, 3 us each (a store
+// until it can be read, then a load of it, both past the L2s); beyond, z and p
+// through the Infinity Cache.  A row's nine neighbours lie three by three.  The
+// three on its own grid row come from p in LDS, with the two rows beside the
+// block read extra.  Of the runs above and below every lane reads one word of z
+// and of p, four lanes the two that follow the wave's 64, and the others come
+// from the next lanes: 13 % faster at 1 million rows than six loads of three
+// words (16 cycles each in the address unit, and a word fetched three times),
+// two full loads a run 5 % slower than one (twice the lines).  Loads are
+// device-scope, with bounds of their own: a word outside the vector reads zero,
+// and the entry for it is zero.
 #define RES_VB 4
 #define RES_BLOCK (RES_VB * SV_BLOCK)
-#define GUARD 4
-
-__global__ void k_cg_guards(double *__restrict__ a, float *__restrict__ b, int64_t n)
-{
-    const int t = threadIdx.x;
-    if (t >= 6 * GUARD) return;
-    const int64_t at = (t / (2 * GUARD)) * (n + 2 * GUARD) + (t % (2 * GUARD) < GUARD ? t % GUARD : n + GUARD + t % GUARD);
-    if (a) a[at] = 0.0;
-    if (b) b[at] = 0.f;
-}
-
+#define RES_GRID SV_BLOCK  // workgroups at most: block b's is b % RES_GRID
 // a * b rounded, whatever it is added to
 template <typename T>
 __device__ __forceinline__ T product(T a, T b)
@@ -811,45 +851,126 @@ __device__ __forceinline__ T product(T a, T b)
     return a * b;
 }
 
-// Three neighbouring words of a guarded vector, device-coherent.
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-#define SC1 16  // cache policy: device scope
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t guarded_rsrc(const void *v, size_t word, int64_t n)
+// A vector's n words, device-coherent: a word outside reads zero, a store there
+// is dropped (a negative number is one far past the end).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t words_rsrc(void *v, size_t word, int64_t n)
 {
-    return __builtin_amdgcn_make_buffer_rsrc((char *)const_cast<void *>(v) - GUARD * word, 0, (int)((n + 2 * GUARD) * word),
-                                             0x00020000);
+    return __builtin_amdgcn_make_buffer_rsrc(v, 0, (int)(n * word), 0x00020000);
 }
-__device__ __forceinline__ void load3(__amdgpu_buffer_rsrc_t r, int32_t i, float *o)
+__device__ __forceinline__ void load1(__amdgpu_buffer_rsrc_t r, int32_t i, float &o)
 {
-    const u32x3 v = __builtin_amdgcn_raw_buffer_load_b96(r, (i + GUARD) * 4, 0, SC1);
-#pragma unroll
-    for (int k = 0; k < 3; k++) o[k] = __builtin_bit_cast(float, (uint32_t)v[k]);
+    o = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, i * 4, 0, SC1));
 }
-__device__ __forceinline__ void load3(__amdgpu_buffer_rsrc_t r, int32_t i, double *o)
+__device__ __forceinline__ void load1(__amdgpu_buffer_rsrc_t r, int32_t i, double &o)
 {
-    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, (i + GUARD) * 8, 0, SC1);
-    const u32x2 u = __builtin_amdgcn_raw_buffer_load_b64(r, (i + GUARD) * 8 + 16, 0, SC1);
-    o[0] = __builtin_bit_cast(double, ((uint64_t)v[1] << 32) | v[0]);
-    o[1] = __builtin_bit_cast(double, ((uint64_t)v[3] << 32) | v[2]);
-    o[2] = __builtin_bit_cast(double, ((uint64_t)u[1] << 32) | u[0]);
+    const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, i * 8, 0, SC1);
+    o = __builtin_bit_cast(double, ((uint64_t)v[1] << 32) | v[0]);
+}
+__device__ __forceinline__ void store1(__amdgpu_buffer_rsrc_t r, int32_t i, float v)
+{
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, i * 4, 0, SC1);
+}
+__device__ __forceinline__ void store1(__amdgpu_buffer_rsrc_t r, int32_t i, double v)
+{
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    __builtin_amdgcn_raw_buffer_store_b64(u32x2{(uint32_t)b, (uint32_t)(b >> 32)}, r, i * 8, 0, SC1);
+}
+// Lane l: the next lane's x; lane 63: last.
+__device__ __forceinline__ float next_lane(float x, float last)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, last), __builtin_bit_cast(int, x), 0x130,
+                                                                 0xf, 0xf, false));  // wave_shl:1
+}
+__device__ __forceinline__ double next_lane(double x, double last)
+{
+    const uint64_t a = __builtin_bit_cast(uint64_t, x), b = __builtin_bit_cast(uint64_t, last);
+    const uint32_t l = (uint32_t)__builtin_amdgcn_update_dpp((int)b, (int)a, 0x130, 0xf, 0xf, false);
+    const uint32_t h = (uint32_t)__builtin_amdgcn_update_dpp((int)(b >> 32), (int)(a >> 32), 0x130, 0xf, 0xf, false);
+    return __builtin_bit_cast(double, (uint64_t)h << 32 | l);
+}
+__device__ __forceinline__ float of_lane(float x, int l)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), l));
+}
+__device__ __forceinline__ double of_lane(double x, int l)
+{
+    const uint64_t a = __builtin_bit_cast(uint64_t, x);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)a, l), hi = (uint32_t)__builtin_amdgcn_readlane((int)(a >> 32), l);
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+
+// exchange() for workgroups that hold the blocks w, w + RES_GRID, ...: these are
+// the ones that one work-item of the sum over all blocks adds up, so the
+// workgroup publishes what that work-item would have: a quarter of the slots.
+template <bool TWO>
+__device__ __forceinline__ bool exchange_res(const Exchange &X, uint32_t e, double &a, double &b,
+                                             double (*sh)[RES_BLOCK / 64], double (*sum)[SV_BLOCK / 64], uint32_t *quit)
+{
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, nw = gridDim.x;
+    STORES_OUT();
+    a = wave_sum(a);
+    if (TWO) b = wave_sum(b);
+    if (lane == 0) {
+        sh[0][w] = a;
+        if (TWO) sh[1][w] = b;
+    }
+    __syncthreads();
+    const int two = lane / EX_COPIES, copy = lane % EX_COPIES;  // lanes of the first wave: partial, copy
+    const bool mine = w == 0 && two < 2;
+    if (mine && (TWO || two == 0)) {
+        double t = 0.0;
+        for (int q = 0; q < RES_VB && (int)blockIdx.x + q * RES_GRID < X.G; q++) {
+            double s = 0.0;
+            for (int k = 0; k < SV_BLOCK / 64; k++) s += sh[two][q * (SV_BLOCK / 64) + k];
+            t += s;
+        }
+        X.put(e, blockIdx.x, copy, two, ex_bits(t));
+    }
+    if (tid < SV_BLOCK) {
+        uint64_t u = 0, v = 0;
+        if (tid < nw) {
+            int spin = 0;
+            do {
+                X.get<TWO>(e, tid, u, v);
+            } while ((u == EX_NONE || v == EX_NONE) && ++spin < EX_LIMIT);
+            if (u == EX_NONE || v == EX_NONE) *quit = 1u;
+        }
+        a = wave_sum(__builtin_bit_cast(double, u));
+        if (TWO) b = wave_sum(__builtin_bit_cast(double, v));
+        if (lane == 0) {
+            sum[0][w] = a;
+            if (TWO) sum[1][w] = b;
+        }
+    }
+    __syncthreads();
+    a = 0.0;
+    b = 0.0;
+    for (int k = 0; k < SV_BLOCK / 64; k++) {
+        a += sum[0][k];
+        if (TWO) b += sum[1][k];
+    }
+    if (mine) X.put(e + 2, blockIdx.x, copy, two, EX_NONE);
+    return *quit == 0u;
 }
 
 template <typename T, typename TX, int R>
 __global__ __launch_bounds__(RES_BLOCK) void k_cg_resident(int64_t n, const uint32_t *__restrict__ off,
                                                            const int16_t *__restrict__ col, const T *__restrict__ val,
-                                                           const uint4 *__restrict__ rec, const T *__restrict__ dinv, T *r_,
+                                                           const int2 *__restrict__ rec, const T *__restrict__ dinv, T *r_,
                                                            T *z_, T *pa, T *pb, TX *xs_, double *x_, const double *part_rz,
                                                            Exchange X, double *sc, double goal2, int it, int maxit)
 {
-    __shared__ T sr[R][RES_BLOCK], sd[R][RES_BLOCK], sp[R][RES_BLOCK];
+    constexpr int DEEP = R < 3 ? R : 3;  // rows in flight (1, 2, 3, 4, 6: 22.0, 20.5, 19.5, 19.8, 23.5 us at 1.95 million rows)
+    __shared__ T sr[R][RES_BLOCK], sd[R][RES_BLOCK];
+    __shared__ T sp[R][RES_VB][SV_BLOCK + 2];  // p, each block's between the two rows beside it
     __shared__ TX sx[R][RES_BLOCK];
     __shared__ double sh[2][RES_BLOCK / 64], sum[2][SV_BLOCK / 64];
     __shared__ uint32_t quit;
     const int tid = threadIdx.x, lane = tid & 63;
     if (tid == 0) quit = 0;
-    const int32_t i0 = (int32_t)(blockIdx.x * RES_BLOCK + tid), stride = X.G * SV_BLOCK, nn = (int32_t)n;
+    const int bq = tid / SV_BLOCK, bt = tid % SV_BLOCK, blk = blockIdx.x + bq * RES_GRID;
+    const int32_t stride = X.G * SV_BLOCK, nn = (int32_t)n;
+    const int32_t i0 = blk < X.G ? blk * SV_BLOCK + bt : ((nn + 63) & ~63) + bt;  // no such block: rows past the last
     const int32_t s0 = __builtin_amdgcn_readfirstlane(i0 >> 6), sstride = stride >> 6;
     const int32_t slast = (nn - 1) >> 6;
     // row k's number, formed anew (kept for all rows, with what follows from it,
@@ -860,14 +981,17 @@ __global__ __launch_bounds__(RES_BLOCK) void k_cg_resident(int64_t n, const uint
         return i;
     };
     T v[R][RES_W], qv[R];
+    int32_t lo[R], hi[R];  // of the wave's slices
 #pragma unroll
     for (int k = 0; k < R; k++) {
         const int32_t i = row(k), ic = min(i, nn - 1), s = s0 + k * sstride;
         qv[k] = T(0);
+        lo[k] = hi[k] = 0;
 #pragma unroll
         for (int q = 0; q < RES_W; q++) v[k][q] = T(0);
         if (s <= slast) {
-            const uint4 m = rec[s];
+            lo[k] = __builtin_amdgcn_readfirstlane(rec[s].x);
+            hi[k] = __builtin_amdgcn_readfirstlane(rec[s].y);
             const uint32_t o = off[s], w = (off[s + 1] - o) >> 6;
             for (uint32_t q = 0; q < w; q++) {
                 const size_t at = (size_t)o + (size_t)q * 64 + lane;
@@ -876,14 +1000,15 @@ __global__ __launch_bounds__(RES_BLOCK) void k_cg_resident(int64_t n, const uint
                 if (x != T(0) || d != 0) {
 #pragma unroll
                     for (int j = 0; j < RES_W; j++)
-                        if (d == (int32_t)(j < 3 ? m.x : j < 6 ? m.y : m.z) + j % 3) v[k][j] = x;
+                        if (d == (j < 3 ? lo[k] : j < 6 ? -1 : hi[k]) + j % 3) v[k][j] = x;
                 }
             }
         }
-        sr[k][tid] = r_[ic];
-        sd[k][tid] = dinv[ic];
-        sp[k][tid] = pa[ic];
-        sx[k][tid] = xs_[ic];
+        // zeros past the last row, and so all that follows from them
+        sr[k][tid] = i < nn ? r_[ic] : T(0);
+        sd[k][tid] = i < nn ? dinv[ic] : T(0);
+        sp[k][bq][bt + 1] = i < nn ? pa[ic] : T(0);
+        sx[k][tid] = i < nn ? xs_[ic] : TX(0);
         if (i >= nn) {
 #pragma unroll
             for (int q = 0; q < RES_W; q++) v[k][q] = T(0);
@@ -898,50 +1023,81 @@ __global__ __launch_bounds__(RES_BLOCK) void k_cg_resident(int64_t n, const uint
     __syncthreads();
     rz = 0.0;
     for (int k = 0; k < SV_BLOCK / 64; k++) rz += sum[0][k];
-    const __amdgpu_buffer_rsrc_t bz = guarded_rsrc(z_, sizeof(T), n);
+    const __amdgpu_buffer_rsrc_t bz = words_rsrc(z_, sizeof(T), n);
     T *p_old = pa, *p_new = pb;
     uint32_t e = 0;
     bool dir = false, ok = true;
     rr = sc[S_RR];
+    const int32_t past = lane < 4 ? 64 - (lane & 2) : 1 << 28;  // lanes 4 ..: outside the vector, nothing is fetched
     while (ok && rr > goal2 && it < maxit) {
         for (int c = 0; c < CHECK && ok; c++) {
             const T beta = dir ? (T)(rz_old != 0.0 ? rz / rz_old : 0.0) : T(0);
-            const __amdgpu_buffer_rsrc_t bp = guarded_rsrc(p_old, sizeof(T), n);
-            T zz[3][3], pp[3][3];
+            const __amdgpu_buffer_rsrc_t bp = words_rsrc(p_old, sizeof(T), n), bn = words_rsrc(p_new, sizeof(T), n);
+            // DEEP rows in flight: their lower and upper run's first words, and
+            // (lanes 0, 1 the lower's, 2, 3 the upper's) the two past the wave's
+            T zz[DEEP][3], pp[DEEP][3];
             auto load = [&](int k) {
-                const uint4 m = rec[min(s0 + k * sstride, slast)];
                 const int32_t i = row(k);
-#pragma unroll
-                for (int g = 0; g < 3; g++) {
-                    const int32_t j = i + (int32_t)(g == 0 ? m.x : g == 1 ? m.y : m.z);
-                    load3(bp, j, pp[g]);
-                    load3(bz, j, zz[g]);
-                }
+                int32_t l = lo[k], h = hi[k];
+                asm volatile("" : "+s"(l), "+s"(h));
+                load1(bp, i + l, pp[k % DEEP][0]);
+                load1(bz, i + l, zz[k % DEEP][0]);
+                load1(bp, i + h, pp[k % DEEP][1]);
+                load1(bz, i + h, zz[k % DEEP][1]);
+                const int32_t j = i + past + (lane < 2 ? l : h);
+                load1(bp, j, pp[k % DEEP][2]);
+                load1(bz, j, zz[k % DEEP][2]);
             };
+            if (tid < 2 * RES_VB * R) {  // the rows beside the blocks
+                const int k = tid / (2 * RES_VB), q = (tid >> 1) % RES_VB, right = tid & 1;
+                const int32_t i = (int32_t)(blockIdx.x + q * RES_GRID) * SV_BLOCK + k * stride + (right ? SV_BLOCK : -1);
+                T z1, p1;
+                load1(bp, i, p1);
+                load1(bz, i, z1);
+                sp[k][q][right ? SV_BLOCK + 1 : 0] = dir ? z1 + beta * p1 : p1;
+            }
+#pragma unroll
+            for (int k = 0; k < DEEP; k++) load(k);
+            __builtin_amdgcn_sched_barrier(0);
+            if (dir) {
+#pragma unroll
+                for (int k0 = 0; k0 < R; k0 += 4) {
+                    T pk[4];
+#pragma unroll
+                    for (int k = k0; k < k0 + 4 && k < R; k++)
+                        pk[k - k0] = product(sd[k][tid], sr[k][tid]) + beta * sp[k][bq][bt + 1];
+#pragma unroll
+                    for (int k = k0; k < k0 + 4 && k < R; k++) {
+                        sp[k][bq][bt + 1] = pk[k - k0];
+                        store1(bn, row(k), pk[k - k0]);
+                    }
+                }
+            }
+            __syncthreads();
             double pq = 0.0;
-            load(0);
 #pragma unroll
             for (int k = 0; k < R; k++) {
                 T y[RES_W];
 #pragma unroll
-                for (int j = 0; j < RES_W; j++) y[j] = dir ? zz[j / 3][j % 3] + beta * pp[j / 3][j % 3] : pp[j / 3][j % 3];
+                for (int g = 0; g < 3; g++) {
+                    const T zg = zz[k % DEEP][g], pg = pp[k % DEEP][g], yg = dir ? zg + beta * pg : pg;
+                    if (g < 2) y[6 * g] = yg;
+                    else y[4] = yg;
+                }
+                y[1] = next_lane(y[0], of_lane(y[4], 0));
+                y[2] = next_lane(y[1], of_lane(y[4], 1));
+                y[7] = next_lane(y[6], of_lane(y[4], 2));
+                y[8] = next_lane(y[7], of_lane(y[4], 3));
+#pragma unroll
+                for (int j = 0; j < 3; j++) y[3 + j] = sp[k][bq][bt + j];
                 __builtin_amdgcn_sched_barrier(0);
-                if (k + 1 < R) load(k + 1);
+                if (k + DEEP < R) load(k + DEEP);
                 __builtin_amdgcn_sched_barrier(0);
                 T acc = T(0);
 #pragma unroll
                 for (int j = 0; j < RES_W; j++) acc += v[k][j] * y[j];
                 qv[k] = acc;
-                const int32_t i = row(k);
-                if (i < nn) {
-                    T pk = sp[k][tid];
-                    if (dir) {
-                        pk = product(sd[k][tid], sr[k][tid]) + beta * pk;
-                        sp[k][tid] = pk;
-                        dev_store_at(p_new, i, pk);
-                    }
-                    pq += (double)pk * (double)acc;
-                }
+                pq += (double)y[4] * (double)acc;
                 __builtin_amdgcn_sched_barrier(0);
             }
             if (dir) {
@@ -950,24 +1106,31 @@ __global__ __launch_bounds__(RES_BLOCK) void k_cg_resident(int64_t n, const uint
                 p_new = t;
             }
             dir = true;
-            if (!(ok = exchange<RES_VB, false>(X, e++, pq, none, sh, sum, &quit))) break;
+            if (!(ok = exchange_res<false>(X, e++, pq, none, sh, sum, &quit))) break;
             const double alpha64 = pq != 0.0 ? rz / pq : 0.0;
             const T alpha = (T)alpha64;
             const TX alphax = (TX)alpha64;
             double a = 0.0, b = 0.0;
 #pragma unroll
-            for (int k = 0; k < R; k++) {
-                const int32_t i = row(k);
-                if (i >= nn) break;
-                const T ri = sr[k][tid] - alpha * qv[k];
-                const T zi = sd[k][tid] * ri;
-                sr[k][tid] = ri;
-                dev_store_at(z_, i, zi);
-                a += (double)ri * (double)zi;
-                b += (double)ri * (double)ri;
-                sx[k][tid] += alphax * (TX)sp[k][tid];
+            for (int k0 = 0; k0 < R; k0 += 4) {
+                T ri[4], zi[4];
+                TX xi[4];
+#pragma unroll
+                for (int k = k0; k < k0 + 4 && k < R; k++) {
+                    ri[k - k0] = sr[k][tid] - alpha * qv[k];
+                    zi[k - k0] = sd[k][tid] * ri[k - k0];
+                    xi[k - k0] = sx[k][tid] + alphax * (TX)sp[k][bq][bt + 1];
+                }
+#pragma unroll
+                for (int k = k0; k < k0 + 4 && k < R; k++) {
+                    store1(bz, row(k), zi[k - k0]);
+                    sr[k][tid] = ri[k - k0];
+                    sx[k][tid] = xi[k - k0];
+                    a += (double)ri[k - k0] * (double)zi[k - k0];
+                    b += (double)ri[k - k0] * (double)ri[k - k0];
+                }
             }
-            if (!(ok = exchange<RES_VB, true>(X, e++, a, b, sh, sum, &quit))) break;
+            if (!(ok = exchange_res<true>(X, e++, a, b, sh, sum, &quit))) break;
             rz_old = rz;
             rz = a;
             rr = b;
@@ -991,14 +1154,15 @@ __global__ __launch_bounds__(RES_BLOCK) void k_cg_resident(int64_t n, const uint
             const int32_t i = row(k);
             if (i >= nn) break;
             r_[i] = sr[k][tid];
-            pa[i] = product(sd[k][tid], sr[k][tid]) + beta * sp[k][tid];
+            pa[i] = product(sd[k][tid], sr[k][tid]) + beta * sp[k][bq][bt + 1];
             xs_[i] = sx[k][tid];
         }
     }
     if (blockIdx.x == 0 && tid == 0) {
         sc[S_RREC] = rr;
-        sc[S_IT] = ok ? (double)it : -1.0 - (double)it;
+        sc[S_IT] = (double)it;
     }
+    if (!ok && threadIdx.x == 0) sc[S_LOST] = 1.0;
 }
 
 // r = (T) r64, z = M r (p = z when `restart`); partials r.z (into rz_out) and r.r
@@ -1124,7 +1288,7 @@ struct Sell {
     const double *v64;
     const float *v32;
     SellU U;
-    const uint4 *rec;  // per slice, for the resident solve (null: not made)
+    const int2 *rec;  // per slice, for the resident solve (null: not made)
 };
 
 template <typename T>
@@ -1181,8 +1345,8 @@ int cg_small_as(hipStream_t st, int64_t n, const Sell &S, Vecs<T> &v, TX *xs, co
 {
     constexpr int VB = sizeof(T) == 8 ? SM_VB8 : SM_VB4;
     const int grid = (P.G + VB - 1) / VB;
-    hipLaunchKernelGGL(k_cg_slots, dim3(ceil_div(6 * P.G, 256)), dim3(256), 0, st, slots, 6 * P.G);
-    Exchange X{slots, P.G};
+    Exchange X{slots, P.G, EX_STRIDE(P.G)};
+    hipLaunchKernelGGL(k_cg_slots, dim3(ceil_div(3 * X.stride / 8, 256)), dim3(256), 0, st, slots, 3 * X.stride / 8, sc);
     const uint32_t *off = S.off;
     const C *col = (const C *)S.col;
     const T *val = sell_vals<T>(S);
@@ -1213,18 +1377,19 @@ template <typename T, typename TX, int R>
 int cg_resident_as(hipStream_t st, int64_t n, const Sell &S, Vecs<T> &v, TX *xs, const Parts &P, uint64_t *slots, double *sc,
                    double goal2, int it, int maxit)
 {
-    hipLaunchKernelGGL(k_cg_slots, dim3(ceil_div(6 * P.G, 256)), dim3(256), 0, st, slots, 6 * P.G);
-    Exchange X{slots, P.G};
+    if (P.G < RES_GRID || P.G > RES_VB * RES_GRID) return 1;  // every block's work-items
+    Exchange X{slots, P.G, EX_STRIDE(RES_GRID)};
+    hipLaunchKernelGGL(k_cg_slots, dim3(ceil_div(3 * X.stride / 8, 256)), dim3(256), 0, st, slots, 3 * X.stride / 8, sc);
     const uint32_t *off = S.off;
     const int16_t *col = (const int16_t *)S.col;
     const T *val = sell_vals<T>(S);
-    const uint4 *rec = S.rec;
+    const int2 *rec = S.rec;
     const T *dinv = v.dinv;
     const double *prz = P.rz;
     double *x = v.x;
     void *args[] = {&n, &off, &col, &val, &rec, &dinv, &v.r, &v.z, &v.p, &v.p2, &xs, &x, &prz, &X, &sc, &goal2, &it, &maxit};
     const hipError_t e = hipLaunchCooperativeKernel(reinterpret_cast<const void *>(&k_cg_resident<T, TX, R>),
-                                                    dim3((P.G + RES_VB - 1) / RES_VB), dim3(RES_BLOCK), args, 0, st);
+                                                    dim3(std::min(P.G, RES_GRID)), dim3(RES_BLOCK), args, 0, st);
     if (e == hipSuccess) return 0;
     (void)hipGetLastError();
     return 1;
@@ -1247,6 +1412,7 @@ int cg_resident(hipStream_t st, int64_t n, const Sell &S, Vecs<float> &v, const 
     if (r <= 1) return cg_resident_as<float, float, 1>(st, n, S, v, v.xlo, P, slots, sc, goal2, it, maxit);
     if (r <= 2) return cg_resident_as<float, float, 2>(st, n, S, v, v.xlo, P, slots, sc, goal2, it, maxit);
     if (r <= 4) return cg_resident_as<float, float, 4>(st, n, S, v, v.xlo, P, slots, sc, goal2, it, maxit);
+    if (r <= 6) return cg_resident_as<float, float, 6>(st, n, S, v, v.xlo, P, slots, sc, goal2, it, maxit);
     if (r <= 8) return cg_resident_as<float, float, 8>(st, n, S, v, v.xlo, P, slots, sc, goal2, it, maxit);
     return 1;
 }
@@ -1278,12 +1444,14 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
     const int G = (int)std::max<int64_t>(1, std::min<int64_t>(ceil_div(n, SV_BLOCK), 4 * (int64_t)cus));
 
     // ---- scratch layout (8-byte words first, then 4-byte) -----------------
-    // doubles: xfull[N], b[n], r64[n], dinv64[n], parts[4 G], slots[6 G], sc[S_NS],
-    //          FP64 vectors r z p p2 q [5n] (FP64 solve only)
-    // floats:  r z p p2 q dinv xlo [7n] (mixed solve only; its iterate is the FP64 xfull + xlo)
+    // doubles: xfull[N], b[n], r64[n], dinv64[n], parts[4 G], slots, sc[S_NS],
+    //          FP64 vectors r z p p2 q [5 m] (FP64 solve only)
+    // floats:  r z p p2 q dinv xlo [7 m] (mixed solve only; its iterate is the FP64 xfull + xlo)
     // uint32:  off[nslices + 1], len[max(n, nslices)], total[4]
-    const size_t nd = (size_t)N + 3 * (size_t)n + 10 * (size_t)G + S_NS + (mixed ? 0 : 5 * (size_t)n + 6 * GUARD);
-    const size_t nf = mixed ? 7 * (size_t)n + 6 * GUARD : 0;
+    // The vectors and the slots begin on 256 bytes: a wave's stores fill whole lines.
+    const size_t m = ((size_t)n + 63) & ~(size_t)63;
+    const size_t nd = (size_t)N + 3 * (size_t)n + 4 * (size_t)G + 3 * EX_STRIDE((size_t)G) / 8 + S_NS + 64 + (mixed ? 0 : 5 * m);
+    const size_t nf = mixed ? 7 * m : 0;
     const size_t nu32 = (size_t)nslices + 1 + (size_t)std::max<int64_t>(n, nslices) + 4;
     int rc = ensure(c, c->pcg, 8 * nd + 4 * nf + 4 * nu32 + 256);
     if (rc) return rc;
@@ -1295,34 +1463,29 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
     Parts P;
     P.G = G;
     P.pq = dp; dp += G; P.rz = dp; dp += G; P.rr = dp; dp += G; P.aux = dp; dp += G;
-    uint64_t *slots = (uint64_t *)dp; dp += 6 * G;
     double *sc = dp; dp += S_NS;
-    void *guarded = nullptr;  // z, p, p2, each between GUARD zeros
+    dp = (double *)(((uintptr_t)dp + 255) & ~(uintptr_t)255);
+    uint64_t *slots = (uint64_t *)dp; dp += 3 * EX_STRIDE((size_t)G) / 8;
+    dp = (double *)(((uintptr_t)dp + 255) & ~(uintptr_t)255);
     Vecs<double> v64{};
     if (!mixed) {
         v64.x = xfull;  // the free part of the full vector is the iterate
-        v64.r = dp; dp += n; v64.q = dp; dp += n;
-        guarded = dp;
-        v64.z = dp + GUARD; dp += n + 2 * GUARD; v64.p = dp + GUARD; dp += n + 2 * GUARD; v64.p2 = dp + GUARD; dp += n + 2 * GUARD;
+        v64.r = dp; dp += m; v64.z = dp; dp += m; v64.p = dp; dp += m; v64.p2 = dp; dp += m; v64.q = dp; dp += m;
         v64.dinv = dinv64;
     }
     float *fp = (float *)dp;
     Vecs<float> v32{};
     if (mixed) {
         v32.x = xfull;  // the free part of the full vector is the iterate (FP64)
-        v32.r = fp; fp += n; v32.q = fp; fp += n;
-        guarded = fp;
-        v32.z = fp + GUARD; fp += n + 2 * GUARD; v32.p = fp + GUARD; fp += n + 2 * GUARD; v32.p2 = fp + GUARD; fp += n + 2 * GUARD;
-        v32.dinv = fp; fp += n;
-        v32.xlo = fp; fp += n;
+        v32.r = fp; fp += m; v32.z = fp; fp += m; v32.p = fp; fp += m; v32.p2 = fp; fp += m; v32.q = fp; fp += m;
+        v32.dinv = fp; fp += m;
+        v32.xlo = fp; fp += m;
     }
     uint32_t *up = (uint32_t *)fp;
     uint32_t *off = up; up += nslices + 1;
     uint32_t *len = up; up += std::max<int64_t>(n, nslices);
     uint32_t *total = up;
 
-    hipLaunchKernelGGL(k_cg_guards, dim3(1), dim3(64), 0, st, mixed ? nullptr : (double *)guarded,
-                       mixed ? (float *)guarded : nullptr, n);
     const HostIn in[2] = {{x, xfull, N, false, 0, 0}, {F, b, n, false, 0, 0}};
     if ((rc = to_device(c, in, 2, nullptr))) return rc;
 
@@ -1372,7 +1535,7 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
     HIPCHK(c, hipGetLastError());
     // records for the resident solve where rows are narrow and columns near
     const bool near9 = c16 && narrow;
-    uint4 *rec = (uint4 *)(((uintptr_t)(uoff + nslots + SELL_UNROLL) + 15) & ~(uintptr_t)15);
+    int2 *rec = (int2 *)(((uintptr_t)(uoff + nslots + SELL_UNROLL) + 15) & ~(uintptr_t)15);
     if (near9)
         hipLaunchKernelGGL(k_sell_rec, dim3(ceil_div(nslices * 64, 256)), dim3(256), 0, st, n, nslices,
                            (const uint32_t *)off, (const int16_t *)scol, (const uint32_t *)len, rec, total + 1);
@@ -1432,8 +1595,8 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
                                    (resident && cg_resident(st, n, S, v, P, slots, sc, goal2, it, maxit) == 0));
         if (one) {
             if ((rc = true_residual(norm))) return rc;
-            lost = hsc[S_IT] < 0;
-            it = lost ? -1 - (int)hsc[S_IT] : (int)hsc[S_IT];
+            lost = hsc[S_LOST] != 0.0;
+            it = (int)hsc[S_IT];
             *rrec = lost ? 0.0 : hsc[S_RREC];  // 0: the next reset restarts from p = z
             return 0;
         }

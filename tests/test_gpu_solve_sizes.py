@@ -72,7 +72,7 @@ def test_wide_rows_and_far_columns(ctx, prec):
     (L.FP64, L.Q4, 262144, 520), (L.FP64, L.T3, 262145, 520), (L.FP64, L.T3, 524288, 730), (L.FP64, L.Q4, 524289, 730),
     (L.FP64, L.Q4, 786432, 890), (L.FP64, L.T3, 786433, 890),
     (L.MIXED, L.T3, 262144, 520), (L.MIXED, L.Q4, 262145, 520), (L.MIXED, L.Q4, 524289, 730),
-    (L.MIXED, L.T3, 1048577, 1030), (L.MIXED, L.Q4, 2097152, 1449), (L.MIXED, L.T3, 2097153, 1449)])
+    (L.MIXED, L.T3, 1048577, 1030), (L.MIXED, L.Q4, 1572865, 1260), (L.MIXED, L.Q4, 2097152, 1449), (L.MIXED, L.T3, 2097153, 1449)])
 def test_rows_in_registers(ctx, prec, fe, nfree, N):
     _solve(ctx, fe, N, nfree, prec)
 
