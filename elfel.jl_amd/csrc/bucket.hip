@@ -12,7 +12,7 @@
 //   k_bk_zero     the row counts, the look-back states and the counters
 //   k_bk_count    entries per major row; each entry's place in its row
 //   k_bk_scan     exclusive scan of the counts (one pass, decoupled look-back),
-//                 and the first row of every tile of BK_TILE entries
+//                 and the first row of every tile
 //   k_bk_scatter  (minor, stream position) of every entry into its row
 //   k_bk_tile     per tile: rank every entry within its row, find the runs,
 //                 sum them, and write the row pointers, indices and values at
@@ -22,25 +22,25 @@
 // its place written and read (8), the packed entry written and read (16), the
 // value (8, gathered), and 12 u/n of output -- against 40 a pass of the radix
 // sort and five to six passes.  Measured against it (whole calls): 1 045 458
-// entries of a T3 mesh on the device 249 -> 91 us, 4608 entries 148 -> 40 us.
+// entries of a T3 mesh on the device 249 -> 62 us, 4608 entries 148 -> 36 us.
 #include <algorithm>
 
 #include "common.h"
 
 #define BK_BLOCK 256
-#define BK_TB 512                   // work-items of a tile
+#define BK_TB 1024                  // work-items of a tile
 #define BK_ROWMAX 512               // longest row that a tile holds; a longer one goes to the sort
-#define BK_TILE 1536                // entries that start in a tile, its last row's overhang beyond
-#define BK_CAP (BK_TILE + BK_ROWMAX)
-#define BK_CAP_LOG2 11
-#define BK_ROUNDS (BK_CAP / BK_TB)
+#define BK_TILE 3584                // entries that start in a tile, its last row's overhang beyond
+#define BK_TILE_FEW 1536            // ... of a stream of at most BK_FEW entries
+#define BK_FEW (256 * 1536)
+#define BK_CAP_LOG2 12
 #define BK_COUNT_ITEMS 2            // entries per work-item of the counting pass
 #define BK_HASH_LOG2 10             // its LDS slots, twice its entries
 #define BK_HASH (1 << BK_HASH_LOG2)
 #define BK_SCAN_ITEMS 16
 #define BK_SCAN_CHUNK (BK_BLOCK * BK_SCAN_ITEMS)
 
-static_assert(BK_CAP == 1 << BK_CAP_LOG2 && BK_CAP % BK_TB == 0, "a tile is a whole number of rounds");
+static_assert(BK_TILE + BK_ROWMAX <= 1 << BK_CAP_LOG2, "a place in a tile has BK_CAP_LOG2 bits");
 static_assert(BK_HASH >= 2 * BK_BLOCK * BK_COUNT_ITEMS, "the hash of the counting pass is at most half full");
 
 // ---- decoupled look-back -------------------------------------------------------
@@ -49,7 +49,9 @@ static_assert(BK_HASH >= 2 * BK_BLOCK * BK_COUNT_ITEMS, "the hash of the countin
 // it.  Blocks take their numbers from a counter when they start, so every
 // block that one waits for has started and waits only for earlier ones: the
 // wait ends.  The word carries its own flag, so relaxed agent-scope accesses
-// are enough.
+// are enough.  (Words for groups of 64 blocks, counted up by atomics and read
+// back 64 at a time, took 181 us where this takes 119, and wider windows of
+// single blocks 139 to 193: what is waited on is the few lines that all read.)
 enum { LB_EMPTY = 0, LB_TOTAL = 1, LB_PREFIX = 2 };
 
 __device__ __forceinline__ void lb_store(uint64_t *st, uint32_t flag, uint32_t v)
@@ -212,11 +214,11 @@ __global__ __launch_bounds__(BK_BLOCK) void k_bk_count(Source src, int64_t n, ui
 }
 
 // cnt[0 .. nmaj] (cnt[nmaj] = 0) -> the rows' first entries, and for every tile
-// t the first row that starts at or after t * BK_TILE with that start (tile
+// t the first row that starts at or after t * tile with that start (tile
 // nt: nmaj and n).  A row's interval (s, s + len] holds the tile boundaries
 // that the next row is the first to reach.
 __global__ __launch_bounds__(BK_BLOCK) void k_bk_scan(uint32_t *__restrict__ cnt, int64_t nmaj, uint32_t n, uint32_t nt,
-                                                      uint32_t *__restrict__ trow, uint32_t *__restrict__ tstart,
+                                                      uint32_t tile, uint32_t *__restrict__ trow, uint32_t *__restrict__ tstart,
                                                       uint64_t *__restrict__ st, uint32_t *__restrict__ ctl)
 {
     __shared__ uint32_t wsum[BK_BLOCK / 64], sh_b, sh_base;
@@ -266,7 +268,7 @@ __global__ __launch_bounds__(BK_BLOCK) void k_bk_scan(uint32_t *__restrict__ cnt
     for (int i = 0; i < BK_SCAN_ITEMS; i++) {
         const uint32_t c = v[i];
         v[i] = s;
-        for (uint32_t t = s / BK_TILE + 1; t <= (s + c) / BK_TILE; t++) {  // c = 0 past the last row
+        for (uint32_t t = s / tile + 1; t <= (s + c) / tile; t++) {  // c = 0 past the last row
             trow[t] = (uint32_t)(r0 + i + 1);
             tstart[t] = s + c;
         }
@@ -291,7 +293,7 @@ __global__ __launch_bounds__(BK_BLOCK) void k_bk_scan(uint32_t *__restrict__ cnt
 
 // The entries of a row side by side, each packed with its row's first entry in
 // the bits above `bits` = minor bits + kbits (those that overflow drop out: a
-// tile spans fewer than 2^11 entries), its minor index and its stream position.
+// tile spans at most 2^12 entries, and starts no row that many after its first), its minor index and its stream position.
 template <typename Source>
 __global__ __launch_bounds__(BK_BLOCK) void k_bk_scatter(Source src, int64_t n, const uint32_t *__restrict__ start,
                                                          const uint32_t *__restrict__ place, int bits, int kbits,
@@ -323,21 +325,55 @@ __global__ __launch_bounds__(BK_BLOCK) void k_bk_scatter_form(FormMap map, int64
     packed[(int64_t)s + place[ea] + b] = ((uint64_t)s << bits) | ((uint64_t)(uint32_t)edof[e * ND + b] << kbits) | k;
 }
 
-// One workgroup per tile of whole rows, at most BK_CAP entries of rows of at
-// most BK_ROWMAX.  An entry less the tile's first entry (in the row field) is
-// (row begin, minor, stream position), so entries of a tile compare as plain
+// acc + v[j] + ... + v[e - 1], left to right; four loads at a time
+__device__ __forceinline__ double run_sum(const double *v, int j, int e, double acc)
+{
+    for (; j + 4 <= e; j += 4) {
+        const double a = v[j], b = v[j + 1], c = v[j + 2], d = v[j + 3];
+        acc += a;
+        acc += b;
+        acc += c;
+        acc += d;
+    }
+    for (; j < e; j++) acc += v[j];
+    return acc;
+}
+
+// the set bits of positions p .. e - 1
+__device__ __forceinline__ int bits_between(const uint64_t *m, int p, int e)
+{
+    int n = 0;
+    for (int x = p >> 6; x <= (e - 1) >> 6; x++) {
+        uint64_t g = m[x];
+        if (x == p >> 6) g &= ~0ull << (p & 63);
+        if (x == (e - 1) >> 6) g &= ~0ull >> (63 - ((e - 1) & 63));
+        n += __popcll(g);
+    }
+    return n;
+}
+
+// One workgroup per tile of whole rows: those that start in TILE entries, each
+// of at most BK_ROWMAX.  An entry less the tile's first entry (in the row field)
+// is (row begin, minor, stream position), so entries of a tile compare as plain
 // integers.  Each work-item counts, for four neighbouring entries at once, how
 // many entries of their rows are smaller: broadcast reads from LDS, for the 20
 // to 100 entries of a finite-element row as many steps as a sorting network
-// would take, without its exchanges.  512 work-items and 36 KiB of LDS fill a
-// CU with four workgroups; 256 work-items of the same tile left it half empty
-// (six million entries 137 against 83 us).
+// would take, without its exchanges.
+// What bounds it beyond the gathers: a tile takes its number from one counter
+// (11 ns each, in turn) and looks back over the tiles before it, so few large
+// tiles: 3584 entries by 1024 work-items, two workgroups a CU, against 1536 by
+// 512, four a CU, 139 -> 119 us (11.5 million entries), 81 -> 69 (6 million),
+// 1024 work-items on 1536 entries 165.  A stream that such small tiles put on
+// the CUs once (BK_FEW) is faster so: 4608 entries 11.4 -> 8.8 us, 394 000 whole
+// calls 49.9 -> 48.7, 551 000 53.2 -> 54.0.
 //
 // SUM: the values and (LOAD) the load vector; else the sort order.  LOAD: the
 // load-vector entries of a dof are those of the (element, local dof) pairs on
 // the diagonal of its row, which the run of the diagonal holds in stream
-// order.
-template <bool SUM, bool LOAD>
+// order; they are gathered with the values and summed by the work-item of that
+// run (one work-item a row that looked for the run and then loaded them one
+// after the other: 4.5 million entries 108 us, now 84).
+template <bool SUM, bool LOAD, int TILE>
 __global__ __launch_bounds__(BK_TB) void k_bk_tile(const uint64_t *__restrict__ packed, const double *__restrict__ vals,
                                                    const double *__restrict__ fvals, uint32_t nd,
                                                    const uint32_t *__restrict__ start, const uint32_t *__restrict__ trow,
@@ -346,10 +382,13 @@ __global__ __launch_bounds__(BK_TB) void k_bk_tile(const uint64_t *__restrict__ 
                                                    uint32_t *__restrict__ ctl, const int *__restrict__ err, BucketOut o,
                                                    int32_t *__restrict__ nnz_dev, int32_t *__restrict__ told)
 {
-    __shared__ __align__(16) uint64_t sk[BK_CAP + 4];  // the entries by row; then the values in sorted order
-    __shared__ uint64_t ss[BK_CAP];                    // the entries, sorted
-    __shared__ uint16_t se[BK_CAP + 1];                // end of a row, at its begin; then the runs before an entry
-    __shared__ uint64_t hm[BK_CAP / 64];               // one bit per entry that starts a run
+    constexpr int CAP = TILE + BK_ROWMAX, ROUNDS = CAP / BK_TB;
+    static_assert(CAP % BK_TB == 0, "a tile is a whole number of rounds");
+    __shared__ __align__(16) uint64_t sk[CAP + 4];  // the entries by row; then the values in sorted order
+    __shared__ uint64_t ss[CAP];                    // the entries, sorted
+    __shared__ uint16_t se[CAP + 1];                // end of a row, at its begin; then the runs before an entry
+    __shared__ uint64_t hm[CAP / 64];               // one bit per entry that starts a run
+    __shared__ uint64_t dm[LOAD ? CAP / 64 : 1];    // one bit per entry of a local dof with itself
     __shared__ uint32_t sh_t, sh_base;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     // nothing is written when an index was out of range or a row is too long
@@ -367,19 +406,19 @@ __global__ __launch_bounds__(BK_TB) void k_bk_tile(const uint64_t *__restrict__ 
     const uint32_t t = sh_t;
     const int64_t row0 = trow[t], row1 = trow[t + 1];
     const uint32_t s0 = tstart[t];
-    const int m = (int)(tstart[t + 1] - s0);  // <= BK_CAP
+    const int m = (int)(tstart[t + 1] - s0);  // <= CAP
     const uint64_t rebase = (uint64_t)s0 << bits;
-    uint64_t kr[BK_ROUNDS];
+    uint64_t kr[ROUNDS];
 #pragma unroll
-    for (int q = 0; q < BK_ROUNDS; q++) {
+    for (int q = 0; q < ROUNDS; q++) {
         const int p = q * BK_TB + tid;
         kr[q] = p < m ? packed[(int64_t)s0 + p] - rebase : ~0ull;
     }
 #pragma unroll
-    for (int q = 0; q < BK_ROUNDS; q++) sk[q * BK_TB + tid] = kr[q];
+    for (int q = 0; q < ROUNDS; q++) sk[q * BK_TB + tid] = kr[q];
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < BK_ROUNDS; q++) {
+    for (int q = 0; q < ROUNDS; q++) {
         const int p = q * BK_TB + tid;
         const uint32_t b = (uint32_t)(kr[q] >> bits);
         if (p < m && (p == m - 1 || (uint32_t)(sk[p + 1] >> bits) != b)) se[b] = (uint16_t)(p + 1);
@@ -413,61 +452,61 @@ __global__ __launch_bounds__(BK_TB) void k_bk_tile(const uint64_t *__restrict__ 
     // runs: entries that differ in more than the stream position start one
     const uint64_t kmask = (1ull << kbits) - 1;
     const uint32_t mmask = (uint32_t)((1ull << (bits - kbits)) - 1);
-    double vr[BK_ROUNDS];
+    double vr[ROUNDS], fr[ROUNDS];
 #pragma unroll
-    for (int q = 0; q < BK_ROUNDS; q++) {
+    for (int q = 0; q < ROUNDS; q++) {
         const int p = q * BK_TB + tid;
         kr[q] = p < m ? ss[p] : 0;
         if constexpr (SUM) vr[q] = p < m ? vals[kr[q] & kmask] : 0.0;
         else if (p < m) o.perm[(int64_t)s0 + p] = (int32_t)(kr[q] & kmask);
+        if constexpr (LOAD) {
+            const uint32_t k = (uint32_t)(kr[q] & kmask), el = k / (nd * nd), ab = k - el * (nd * nd), a = ab / nd;
+            const bool d = p < m && ab == a * (nd + 1);
+            fr[q] = d && SUM ? fvals[(int64_t)el * nd + a] : 0.0;
+            const uint64_t g = __ballot(d);
+            if (lane == 0) dm[q * (BK_TB / 64) + w] = g;
+        }
     }
 #pragma unroll
-    for (int q = 0; q < BK_ROUNDS; q++) {
+    for (int q = 0; q < ROUNDS; q++) {
         const int p = q * BK_TB + tid;
         const uint64_t h = __ballot(p < m && (p == 0 || (ss[p - 1] >> kbits) != (kr[q] >> kbits)));
         if (lane == 0) hm[q * (BK_TB / 64) + w] = h;
     }
     __syncthreads();
     // runs before each word of hm (every wave computes them, lanes as words)
-    static_assert(BK_CAP / 64 == 32, "one lane per word of the run mask, twice");
-    const uint32_t pc = (uint32_t)__popcll(hm[lane & 31]);
+    constexpr int WORDS = CAP / 64;
+    static_assert(WORDS == 32 || WORDS == 64, "one lane per word of the run mask");
+    const uint32_t pc = (uint32_t)__popcll(hm[lane % WORDS]);
     uint32_t inc = pc;
 #pragma unroll
-    for (int d = 1; d < 32; d <<= 1) {
-        const uint32_t o = (uint32_t)__shfl_up((int)inc, d, 32);
-        if ((lane & 31) >= d) inc += o;
+    for (int d = 1; d < WORDS; d <<= 1) {
+        const uint32_t o = (uint32_t)__shfl_up((int)inc, d, WORDS);
+        if (lane % WORDS >= d) inc += o;
     }
-    const uint32_t total = (uint32_t)__shfl((int)inc, 31, 64);
+    const uint32_t total = (uint32_t)__shfl((int)inc, WORDS - 1, 64);
     if (tid == 0) lb_publish(st, t, total);
-    double *sv = (double *)sk;
-    uint32_t un[BK_ROUNDS];
+    double *sv = (double *)sk, *sf = (double *)ss;
+    uint32_t un[ROUNDS];
     const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
 #pragma unroll
-    for (int q = 0; q < BK_ROUNDS; q++) {
+    for (int q = 0; q < ROUNDS; q++) {
         const int p = q * BK_TB + tid, word = q * (BK_TB / 64) + w;
         un[q] = (uint32_t)__shfl((int)(inc - pc), word, 64) + (uint32_t)__popcll(hm[word] & lt);
         if (p < m) {
             if constexpr (SUM) sv[p] = vr[q];
+            if constexpr (SUM && LOAD) sf[p] = fr[q];
             se[p] = (uint16_t)un[q];
         }
     }
     if (tid == 0) se[m] = (uint16_t)total;
-    if (w == 0) {
-        const uint32_t base = lb_wait(st, t, total);
-        if (lane == 0) sh_base = base;
-    }
     __syncthreads();
-    const uint32_t base = sh_base;
+    // the sums, while the tiles before this one finish theirs
 #pragma unroll
-    for (int q = 0; q < BK_ROUNDS; q++) {
+    for (int q = 0; q < ROUNDS; q++) {
         const int p = q * BK_TB + tid, word = q * (BK_TB / 64) + w;
         if (p >= m || !((hm[word] >> lane) & 1)) continue;
-        const int64_t u = (int64_t)base + un[q];
-        o.ind[u] = (int32_t)((uint32_t)(kr[q] >> kbits) & mmask);
-        if constexpr (!SUM) {
-            o.seg[u] = (int32_t)(s0 + p);
-            continue;
-        }
+        if constexpr (!SUM && !LOAD) continue;
         // the next run's start, or the tile's end
         const uint64_t above = lane == 63 ? 0ull : hm[word] >> (lane + 1);
         int e = above ? p + 1 + __builtin_ctzll(above) : -1;
@@ -475,38 +514,54 @@ __global__ __launch_bounds__(BK_TB) void k_bk_tile(const uint64_t *__restrict__ 
             if (x * 64 >= m) e = m;
             else if (hm[x]) e = x * 64 + __builtin_ctzll(hm[x]);
         }
-        double acc = vr[q];
-        for (int j = p + 1; j < e; j++) acc += sv[j];
-        o.val[u] = acc;
+        if constexpr (SUM) vr[q] = run_sum(sv, p + 1, e, vr[q]);
+        if constexpr (LOAD) {
+            // the diagonal's run, and no other, has entries of a local dof with itself
+            const int n = bits_between(dm, p, e);
+            if (n == 0) continue;
+            if constexpr (SUM) {
+                double f = 0.0;
+                if (n == e - p) {
+                    f = run_sum(sf, p + 1, e, fr[q]);
+                } else {  // an element with two local dofs of one number
+                    int cnt = 0;
+                    for (int j = p; j < e; j++)
+                        if ((dm[j >> 6] >> (j & 63)) & 1) f = cnt++ == 0 ? sf[j] : f + sf[j];
+                }
+                o.F[(uint32_t)(kr[q] >> kbits) & mmask] = 0.0 + f;  // start! zeros the vector, assemble! adds
+            } else {
+                const int64_t to = ((int64_t)s0 + (int64_t)(kr[q] >> bits)) / nd;
+                int cnt = 0;
+                for (int j = p; j < e; j++) {
+                    if (!((dm[j >> 6] >> (j & 63)) & 1)) continue;
+                    const uint32_t k = (uint32_t)(ss[j] & kmask), el = k / (nd * nd), ab = k - el * (nd * nd);
+                    o.fperm[to + cnt++] = (int32_t)(el * nd + ab / nd);
+                }
+            }
+        }
+    }
+    if (w == 0) {
+        const uint32_t base = lb_wait(st, t, total);
+        if (lane == 0) sh_base = base;
+    }
+    __syncthreads();
+    const uint32_t base = sh_base;
+#pragma unroll
+    for (int q = 0; q < ROUNDS; q++) {
+        const int p = q * BK_TB + tid, word = q * (BK_TB / 64) + w;
+        if (p >= m || !((hm[word] >> lane) & 1)) continue;
+        const int64_t u = (int64_t)base + un[q];
+        o.ind[u] = (int32_t)((uint32_t)(kr[q] >> kbits) & mmask);
+        if constexpr (SUM) o.val[u] = vr[q];
+        else o.seg[u] = (int32_t)(s0 + p);
     }
     for (int64_t r = row0 + tid; r < row1; r += BK_TB) {
-        const int b = (int)(start[r] - s0);
-        o.ptr[r] = (int32_t)(base + se[b]);
-        if constexpr (LOAD) {
-            int lo = b, hi = (int)(start[r + 1] - s0);
-            const int e = hi;
-            const uint64_t diag = ((uint64_t)b << bits) | ((uint64_t)r << kbits);
-            while (lo < hi) {
-                const int mid = (lo + hi) >> 1;
-                if (ss[mid] < diag) lo = mid + 1;
-                else hi = mid;
-            }
-            double acc = 0.0;
-            int cnt = 0;
-            if constexpr (!SUM) o.fbeg[r] = (int32_t)(start[r] / nd);
-            for (int p = lo; p < e && ((ss[p] ^ diag) >> kbits) == 0; p++) {
-                const uint32_t k = (uint32_t)(ss[p] & kmask), el = k / (nd * nd), ab = k - el * (nd * nd), a = ab / nd;
-                if (ab - a * nd != a) continue;  // two local dofs of an element with one number
-                if constexpr (SUM) {
-                    const double x = fvals[(int64_t)el * nd + a];
-                    acc = cnt == 0 ? x : acc + x;
-                } else {
-                    o.fperm[start[r] / nd + cnt] = (int32_t)(el * nd + a);
-                }
-                cnt++;
-            }
-            if constexpr (SUM) o.F[r] = cnt ? 0.0 + acc : 0.0;  // start! zeros the vector, assemble! adds
+        const uint32_t b = start[r];
+        o.ptr[r] = (int32_t)(base + se[b - s0]);
+        if constexpr (LOAD && SUM) {
+            if (start[r + 1] == b) o.F[r] = 0.0;  // a dof of no element
         }
+        if constexpr (LOAD && !SUM) o.fbeg[r] = (int32_t)(b / nd);
     }
     if (t == nt - 1 && tid == 0) {
         const int32_t nnz = (int32_t)(base + total);
@@ -523,7 +578,8 @@ __global__ __launch_bounds__(BK_TB) void k_bk_tile(const uint64_t *__restrict__ 
 }
 
 // ---- host -------------------------------------------------------------------------
-static int64_t bk_tiles(int64_t n) { return n / BK_TILE + 1; }
+static int bk_tile(int64_t n) { return n <= BK_FEW ? BK_TILE_FEW : BK_TILE; }
+static int64_t bk_tiles(int64_t n) { return n / bk_tile(n) + 1; }
 static int64_t bk_scan_blocks(int64_t nmaj) { return ceil_div(nmaj + 1, BK_SCAN_CHUNK); }
 // words zeroed before a build: control words, the look-back states, the counts
 static int64_t bk_zero_words(int64_t n, int64_t nmaj)
@@ -583,6 +639,12 @@ bool bucket_form_takes(const FormMap &m, int64_t E, int64_t ndofs)
     return E * m.nd < INT32_MAX && bucket_takes(E * m.nmat, ndofs, ndofs);
 }
 
+template <bool SUM, bool LOAD>
+static decltype(&k_bk_tile<SUM, LOAD, BK_TILE>) tile_kernel(int64_t n)
+{
+    return bk_tile(n) == BK_TILE ? k_bk_tile<SUM, LOAD, BK_TILE> : k_bk_tile<SUM, LOAD, BK_TILE_FEW>;
+}
+
 static void launch_zero_scan(elfel_hip_ctx *c, const Scratch &S, bool zero, int64_t n, int64_t nmaj)
 {
     if (zero)
@@ -590,7 +652,7 @@ static void launch_zero_scan(elfel_hip_ctx *c, const Scratch &S, bool zero, int6
                            S.zero_words / 4);
     else
         hipLaunchKernelGGL(k_bk_scan, dim3((unsigned)S.nsb), dim3(BK_BLOCK), 0, c->stream, S.cnt, nmaj, (uint32_t)n,
-                           (uint32_t)S.nt, S.trow, S.tstart, S.st_scan, S.ctl);
+                           (uint32_t)S.nt, (uint32_t)bk_tile(n), S.trow, S.tstart, S.st_scan, S.ctl);
 }
 
 template <typename Source>
@@ -607,7 +669,7 @@ static int run_coo(elfel_hip_ctx *c, void *scratch, const Source &src, int64_t n
     hipLaunchKernelGGL(k_bk_scatter<Source>, dim3(ceil_div(n, BK_BLOCK)), dim3(BK_BLOCK), 0, c->stream, src, n, S.cnt,
                        S.place, bits, kbits, S.packed);
     // told: words 0-3 are the context's result's, these 4-7
-    hipLaunchKernelGGL((k_bk_tile<true, false>), dim3((unsigned)S.nt), dim3(BK_TB), 0, c->stream, S.packed, val,
+    hipLaunchKernelGGL((tile_kernel<true, false>(n)), dim3((unsigned)S.nt), dim3(BK_TB), 0, c->stream, S.packed, val,
                        (const double *)nullptr, 1u, S.cnt, S.trow, S.tstart, (uint32_t)S.nt, nmaj, bits, kbits, S.st_tile,
                        S.ctl, err, o, (int32_t *)c->dscal.p + 2, (int32_t *)c->told + 4);
     HIPCHK(c, hipGetLastError());
@@ -742,8 +804,8 @@ int bucket_form(elfel_hip_ctx *c, void *scratch, const FormMap &m, int64_t E, co
     tm_end(c, ELFEL_PH_SORT, ev);
     tm_begin(c, ELFEL_PH_REDUCE, &ev);
     const bool sum = vals != nullptr, load = m.nvec > 0;
-    auto kern = sum ? (load ? k_bk_tile<true, true> : k_bk_tile<true, false>)
-                    : (load ? k_bk_tile<false, true> : k_bk_tile<false, false>);
+    auto kern = sum ? (load ? tile_kernel<true, true>(n) : tile_kernel<true, false>(n))
+                    : (load ? tile_kernel<false, true>(n) : tile_kernel<false, false>(n));
     hipLaunchKernelGGL(kern, dim3((unsigned)S.nt), dim3(BK_TB), 0, c->stream, S.packed, vals, fvals, (uint32_t)m.nd, S.cnt,
                        S.trow, S.tstart, (uint32_t)S.nt, ndofs, bits, kbits, S.st_tile, S.ctl, (int *)c->dscal.p + 1, o,
                        (int32_t *)c->dscal.p, (int32_t *)c->told);

@@ -1,11 +1,12 @@
 """The row-bucket COO build (elfel_hip_sparse, elfel_hip_sparse_noalloc) at the
 edges of its tiles, against the oracle's sparse(): pattern and values bit for
 bit (tolerance 0, the same sums in the same order).  1536 entries start in a
-tile, rows of up to 512 are held, longer ones and matrices of far more rows
-than entries take the sort."""
+tile, 3584 of a stream of more than 393216, rows of up to 512 are held, longer
+ones and matrices of far more rows than entries take the sort."""
 import numpy as np
 import pytest
 
+import elfel_hip as eh
 import oracle as O
 from elfel_hip import _lib as L
 from test_gpu_general_meshes import _oracle_heat, _same, fan_mesh
@@ -31,11 +32,16 @@ def _case(name, rng):
     if name.startswith("n="):
         n = int(name[2:])
         return (*_rows(rng.multinomial(n, np.full(40, 1 / 40)), 23, rng), 40, 23)
+    if name.startswith("many="):
+        n = int(name[5:])
+        return (*_rows(rng.multinomial(n, np.full(9000, 1 / 9000)), 60, rng), 9000, 60)
     if name.startswith("row="):  # one long row between short ones, and a tile that it straddles
         k = int(name[4:])
         return (*_rows([3] * 500 + [k] + [0] * 7 + [5] * 300, max(k // 2, 1), rng), 808, max(k // 2, 1))
     if name == "long rows side by side":  # every tile at its largest
         return (*_rows([511, 1024, 1, 512, 512, 512, 512, 511, 1][2:], 600, rng), 7, 600)
+    if name == "long rows, many":
+        return (*_rows([512] * 5 + [511, 1] + [512] * 830 + [3] * 20, 700, rng), 857, 700)
     if name == "empty ends":
         return (*_rows([0] * 9000 + [2] * 50 + [0] * 9000, 60, rng), 18050, 60)
     if name == "one entry":
@@ -52,7 +58,7 @@ def _case(name, rng):
     raise ValueError(name)
 
 
-CASES = ["n=1535", "n=1536", "n=1537", "n=2048", "n=3072", "n=9001", "row=511", "row=512", "row=513", "row=1600",
+CASES = ["many=393216", "many=393217", "many=401408", "long rows, many", "n=1535", "n=1536", "n=1537", "n=2048", "n=3072", "n=9001", "row=511", "row=512", "row=513", "row=1600",
          "long rows side by side", "empty ends", "one entry", "one row", "two rows, all duplicates",
          "more rows than entries", "last columns"]
 
@@ -119,3 +125,22 @@ def test_element_stream_at_the_longest_row(ctx, method, layout):
             ctx.assemble(L.HEAT, L.T3, 1, method=method, layout=layout, kappa=1.3, Q=-2.0, wait=wait)
             _same(ctx.copy_sparse(base=0), ref)
             assert np.array_equal(ctx.copy_vector(n), ref[3])
+
+
+@pytest.mark.parametrize("layout", [L.CSR, L.CSC])
+def test_element_stream_in_large_tiles(ctx, layout):
+    """460 800 entries: with a dof that two nodes of an element share, and one
+    that no element has (its load is zero)."""
+    mesh = eh.T3block(2.0, 1.0, 160, 160)
+    conn, xy = np.asarray(mesh.conn), np.asarray(mesh.xy)
+    n = xy.shape[0] + 1
+    dn = np.random.default_rng(8).permutation(n)[:-1] + 1
+    dn[2] = dn[1]
+    ref = _oracle_heat(conn, xy, dn, n, layout)
+    ctx.set_mesh(0, conn, xy)
+    ctx.set_dofs(0, dn, n)
+    ctx.set_coefficients(conn.shape[0])
+    for method in (L.SORT, L.REUSE):
+        ctx.assemble(L.HEAT, L.T3, 1, method=method, layout=layout, kappa=1.3, Q=-2.0)
+        _same(ctx.copy_sparse(base=0), ref)
+        assert np.array_equal(ctx.copy_vector(n), ref[3])
