@@ -17,12 +17,13 @@
 //   k_bk_tile     per tile: rank every entry within its row, find the runs,
 //                 sum them, and write the row pointers, indices and values at
 //                 the place that a second look-back over the tiles gives
+//   k_bk_one      all of it by one workgroup, for a few thousand entries
 //
 // Bytes per entry (n entries, u of them distinct): the two indices twice (32),
 // its place written and read (8), the packed entry written and read (16), the
 // value (8, gathered), and 12 u/n of output -- against 40 a pass of the radix
 // sort and five to six passes.  Measured against it (whole calls): 1 045 458
-// entries of a T3 mesh on the device 249 -> 62 us, 4608 entries 148 -> 36 us.
+// entries of a T3 mesh on the device 249 -> 62 us, 4608 entries 148 -> 32 us.
 #include <algorithm>
 
 #include "common.h"
@@ -373,50 +374,18 @@ __device__ __forceinline__ int bits_between(const uint64_t *m, int p, int e)
 // order; they are gathered with the values and summed by the work-item of that
 // run (one work-item a row that looked for the run and then loaded them one
 // after the other: 4.5 million entries 108 us, now 84).
-template <bool SUM, bool LOAD, int TILE>
-__global__ __launch_bounds__(BK_TB) void k_bk_tile(const uint64_t *__restrict__ packed, const double *__restrict__ vals,
-                                                   const double *__restrict__ fvals, uint32_t nd,
-                                                   const uint32_t *__restrict__ start, const uint32_t *__restrict__ trow,
-                                                   const uint32_t *__restrict__ tstart, uint32_t nt, int64_t nmaj,
-                                                   int bits, int kbits, uint64_t *__restrict__ st,
-                                                   uint32_t *__restrict__ ctl, const int *__restrict__ err, BucketOut o,
-                                                   int32_t *__restrict__ nnz_dev, int32_t *__restrict__ told)
+// A tile's rows, their entries in sk (and kr: entry q * BK_TB + tid); ~0 past m.
+// Gives back the runs up to the tile's end.  place: where the tile's runs begin.
+template <bool SUM, bool LOAD, int CAP, typename Place>
+__device__ __forceinline__ uint32_t tile_rows(uint64_t *sk, uint64_t *ss, uint16_t *se, uint64_t *hm, uint64_t *dm,
+                                              uint32_t *sh_base, uint64_t *kr, int m, uint32_t s0, int64_t row0, int64_t row1,
+                                              const uint32_t *start, const double *__restrict__ vals,
+                                              const double *__restrict__ fvals, uint32_t nd, int bits, int kbits,
+                                              const Place &place, const BucketOut &o)
 {
-    constexpr int CAP = TILE + BK_ROWMAX, ROUNDS = CAP / BK_TB;
+    constexpr int ROUNDS = CAP / BK_TB;
     static_assert(CAP % BK_TB == 0, "a tile is a whole number of rounds");
-    __shared__ __align__(16) uint64_t sk[CAP + 4];  // the entries by row; then the values in sorted order
-    __shared__ uint64_t ss[CAP];                    // the entries, sorted
-    __shared__ uint16_t se[CAP + 1];                // end of a row, at its begin; then the runs before an entry
-    __shared__ uint64_t hm[CAP / 64];               // one bit per entry that starts a run
-    __shared__ uint64_t dm[LOAD ? CAP / 64 : 1];    // one bit per entry of a local dof with itself
-    __shared__ uint32_t sh_t, sh_base;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    // nothing is written when an index was out of range or a row is too long
-    // (the flags were set by earlier kernels: the same for every workgroup)
-    if (*err != 0 || ctl[BK_LONG] != 0) {
-        if (blockIdx.x == 0 && tid == 0) {
-            told[0] = 0;
-            told[1] = *err;
-            told[2] = (int32_t)ctl[BK_LONG];
-        }
-        return;
-    }
-    if (tid == 0) sh_t = atomicAdd(&ctl[BK_T_TILE], 1u);
-    __syncthreads();
-    const uint32_t t = sh_t;
-    const int64_t row0 = trow[t], row1 = trow[t + 1];
-    const uint32_t s0 = tstart[t];
-    const int m = (int)(tstart[t + 1] - s0);  // <= CAP
-    const uint64_t rebase = (uint64_t)s0 << bits;
-    uint64_t kr[ROUNDS];
-#pragma unroll
-    for (int q = 0; q < ROUNDS; q++) {
-        const int p = q * BK_TB + tid;
-        kr[q] = p < m ? packed[(int64_t)s0 + p] - rebase : ~0ull;
-    }
-#pragma unroll
-    for (int q = 0; q < ROUNDS; q++) sk[q * BK_TB + tid] = kr[q];
-    __syncthreads();
 #pragma unroll
     for (int q = 0; q < ROUNDS; q++) {
         const int p = q * BK_TB + tid;
@@ -475,24 +444,27 @@ __global__ __launch_bounds__(BK_TB) void k_bk_tile(const uint64_t *__restrict__ 
     }
     __syncthreads();
     // runs before each word of hm (every wave computes them, lanes as words)
-    constexpr int WORDS = CAP / 64;
-    static_assert(WORDS == 32 || WORDS == 64, "one lane per word of the run mask");
-    const uint32_t pc = (uint32_t)__popcll(hm[lane % WORDS]);
+    constexpr int WORDS = CAP / 64, PER = (WORDS + 63) / 64;  // PER words a lane
+    uint32_t pc = 0;
+#pragma unroll
+    for (int i = 0; i < PER; i++) pc += PER * lane + i < WORDS ? (uint32_t)__popcll(hm[PER * lane + i]) : 0u;
     uint32_t inc = pc;
 #pragma unroll
-    for (int d = 1; d < WORDS; d <<= 1) {
-        const uint32_t o = (uint32_t)__shfl_up((int)inc, d, WORDS);
-        if (lane % WORDS >= d) inc += o;
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t o = (uint32_t)__shfl_up((int)inc, d, 64);
+        if (lane >= d) inc += o;
     }
-    const uint32_t total = (uint32_t)__shfl((int)inc, WORDS - 1, 64);
-    if (tid == 0) lb_publish(st, t, total);
+    const uint32_t total = (uint32_t)__shfl((int)inc, 63, 64);
+    if (tid == 0) place.publish(total);
     double *sv = (double *)sk, *sf = (double *)ss;
     uint32_t un[ROUNDS];
     const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
 #pragma unroll
     for (int q = 0; q < ROUNDS; q++) {
         const int p = q * BK_TB + tid, word = q * (BK_TB / 64) + w;
-        un[q] = (uint32_t)__shfl((int)(inc - pc), word, 64) + (uint32_t)__popcll(hm[word] & lt);
+        un[q] = (uint32_t)__shfl((int)(inc - pc), word / PER, 64) + (uint32_t)__popcll(hm[word] & lt);
+#pragma unroll
+        for (int i = 1; i < PER; i++) un[q] += word % PER >= i ? (uint32_t)__popcll(hm[word - i]) : 0u;
         if (p < m) {
             if constexpr (SUM) sv[p] = vr[q];
             if constexpr (SUM && LOAD) sf[p] = fr[q];
@@ -541,11 +513,11 @@ __global__ __launch_bounds__(BK_TB) void k_bk_tile(const uint64_t *__restrict__ 
         }
     }
     if (w == 0) {
-        const uint32_t base = lb_wait(st, t, total);
-        if (lane == 0) sh_base = base;
+        const uint32_t base = place.wait(total);
+        if (lane == 0) *sh_base = base;
     }
     __syncthreads();
-    const uint32_t base = sh_base;
+    const uint32_t base = *sh_base;
 #pragma unroll
     for (int q = 0; q < ROUNDS; q++) {
         const int p = q * BK_TB + tid, word = q * (BK_TB / 64) + w;
@@ -563,18 +535,211 @@ __global__ __launch_bounds__(BK_TB) void k_bk_tile(const uint64_t *__restrict__ 
         }
         if constexpr (LOAD && !SUM) o.fbeg[r] = (int32_t)(b / nd);
     }
-    if (t == nt - 1 && tid == 0) {
-        const int32_t nnz = (int32_t)(base + total);
-        o.ptr[nmaj] = nnz;
-        if constexpr (!SUM) {
-            o.seg[nnz] = (int32_t)start[nmaj];
-            if constexpr (LOAD) o.fbeg[nmaj] = (int32_t)(start[nmaj] / nd);
-        }
-        *nnz_dev = nnz;
-        told[0] = nnz;
-        told[1] = 0;
-        told[2] = 0;
+    return base + total;
+}
+
+__device__ __forceinline__ void tell_build(uint32_t nnz, const uint32_t *start, int64_t nmaj, uint32_t nd, bool sum, bool load,
+                                           const BucketOut &o, int32_t *nnz_dev, int32_t *told)
+{
+    o.ptr[nmaj] = (int32_t)nnz;
+    if (!sum) {
+        o.seg[nnz] = (int32_t)start[nmaj];
+        if (load) o.fbeg[nmaj] = (int32_t)(start[nmaj] / nd);
     }
+    *nnz_dev = (int32_t)nnz;
+    told[0] = (int32_t)nnz;
+    told[1] = 0;
+    told[2] = 0;
+}
+
+struct AfterTiles {
+    uint64_t *st;
+    uint32_t t;
+    __device__ __forceinline__ void publish(uint32_t total) const { lb_publish(st, t, total); }
+    __device__ __forceinline__ uint32_t wait(uint32_t total) const { return lb_wait(st, t, total); }
+};
+
+template <bool SUM, bool LOAD, int TILE>
+__global__ __launch_bounds__(BK_TB) void k_bk_tile(const uint64_t *__restrict__ packed, const double *__restrict__ vals,
+                                                   const double *__restrict__ fvals, uint32_t nd,
+                                                   const uint32_t *__restrict__ start, const uint32_t *__restrict__ trow,
+                                                   const uint32_t *__restrict__ tstart, uint32_t nt, int64_t nmaj,
+                                                   int bits, int kbits, uint64_t *__restrict__ st,
+                                                   uint32_t *__restrict__ ctl, const int *__restrict__ err, BucketOut o,
+                                                   int32_t *__restrict__ nnz_dev, int32_t *__restrict__ told)
+{
+    constexpr int CAP = TILE + BK_ROWMAX, ROUNDS = CAP / BK_TB;
+    __shared__ __align__(16) uint64_t sk[CAP + 4];  // the entries by row; then the values in sorted order
+    __shared__ uint64_t ss[CAP];                    // the entries, sorted
+    __shared__ uint16_t se[CAP + 1];                // end of a row, at its begin; then the runs before an entry
+    __shared__ uint64_t hm[CAP / 64];               // one bit per entry that starts a run
+    __shared__ uint64_t dm[LOAD ? CAP / 64 : 1];    // one bit per entry of a local dof with itself
+    __shared__ uint32_t sh_t, sh_base;
+    const int tid = threadIdx.x;
+    // nothing is written when an index was out of range or a row is too long
+    // (the flags were set by earlier kernels: the same for every workgroup)
+    if (*err != 0 || ctl[BK_LONG] != 0) {
+        if (blockIdx.x == 0 && tid == 0) {
+            told[0] = 0;
+            told[1] = *err;
+            told[2] = (int32_t)ctl[BK_LONG];
+        }
+        return;
+    }
+    if (tid == 0) sh_t = atomicAdd(&ctl[BK_T_TILE], 1u);
+    __syncthreads();
+    const uint32_t t = sh_t;
+    const int64_t row0 = trow[t], row1 = trow[t + 1];
+    const uint32_t s0 = tstart[t];
+    const int m = (int)(tstart[t + 1] - s0);  // <= CAP
+    const uint64_t rebase = (uint64_t)s0 << bits;
+    uint64_t kr[ROUNDS];
+#pragma unroll
+    for (int q = 0; q < ROUNDS; q++) {
+        const int p = q * BK_TB + tid;
+        kr[q] = p < m ? packed[(int64_t)s0 + p] - rebase : ~0ull;
+    }
+#pragma unroll
+    for (int q = 0; q < ROUNDS; q++) sk[q * BK_TB + tid] = kr[q];
+    __syncthreads();
+    const uint32_t nnz = tile_rows<SUM, LOAD, CAP>(sk, ss, se, hm, dm, &sh_base, kr, m, s0, row0, row1, start, vals, fvals, nd,
+                                                   bits, kbits, AfterTiles{st, t}, o);
+    if (t == nt - 1 && tid == 0) tell_build(nnz, start, nmaj, nd, SUM, LOAD, o, nnz_dev, told);
+}
+
+// ---- one workgroup for all ----------------------------------------------------------
+// The whole build of a stream of at most BK_ONE entries and BK_ONE_ROWS rows by
+// one workgroup, its counts and places in LDS (145 KB): one launch in place of
+// five, whose latencies are the time of so small a call (whole calls on the
+// device, five launches -> one: 72 entries 35 -> 25 us, 1152 37 -> 27, 4608 39
+// -> 34, 5832 39.6 -> 36.7).
+#define BK_ONE 6144
+#define BK_ONE_ROWS 8191
+
+// Item x of a stream: its row, column and stream position; false: none, or
+// (COO, *bad) an index out of range.
+template <typename Source>
+__device__ __forceinline__ bool one_item(const Source &src, uint32_t x, uint32_t &major, uint32_t &minor, uint32_t &k, bool &bad)
+{
+    k = x;
+    const bool ok = src.get(x, major, minor);
+    bad |= !ok;
+    return ok;
+}
+struct FormItems {
+    FormMap map;
+    const int32_t *edof;
+};
+__device__ __forceinline__ bool one_item(const FormItems &f, uint32_t x, uint32_t &major, uint32_t &minor, uint32_t &k, bool &bad)
+{
+    const uint32_t nd = (uint32_t)f.map.nd, ea = x / nd, b = x - ea * nd, e = ea / nd, a = ea - e * nd;
+    if ((int)b >= f.map.ncol[a]) return false;
+    major = (uint32_t)f.edof[ea];
+    minor = (uint32_t)f.edof[e * nd + b];
+    k = e * (uint32_t)f.map.nmat + (uint32_t)f.map.pos[a * nd + b];
+    return true;
+}
+
+struct FirstPlace {
+    __device__ __forceinline__ void publish(uint32_t) const {}
+    __device__ __forceinline__ uint32_t wait(uint32_t) const { return 0; }
+};
+
+template <bool SUM, bool LOAD, typename Source>
+__global__ __launch_bounds__(BK_TB) void k_bk_one(Source src, uint32_t items, int m, const double *__restrict__ vals,
+                                                  const double *__restrict__ fvals, uint32_t nd, int nmaj, int bits, int kbits,
+                                                  BucketOut o, int32_t *__restrict__ nnz_dev, int32_t *__restrict__ told)
+{
+    constexpr int ROUNDS = BK_ONE / BK_TB, PER = (BK_ONE_ROWS + 1) / BK_TB;
+    __shared__ __align__(16) uint64_t sk[BK_ONE + 4];
+    __shared__ uint64_t ss[BK_ONE];
+    __shared__ uint16_t se[BK_ONE + 1];
+    __shared__ uint64_t hm[BK_ONE / 64], dm[LOAD ? BK_ONE / 64 : 1];
+    __shared__ __align__(16) uint32_t first[BK_ONE_ROWS + 1];  // row r's entries at r + 1, then the end of its places so far
+    __shared__ uint32_t wsum[BK_TB / 64], sh_base, sh_bad, sh_long;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+#pragma unroll
+    for (int i = 0; i < PER; i += 4) *(uint4 *)(first + PER * tid + i) = make_uint4(0, 0, 0, 0);
+#pragma unroll
+    for (int q = 0; q < ROUNDS; q++) sk[q * BK_TB + tid] = ~0ull;
+    if (tid == 0) sh_bad = sh_long = 0;
+    __syncthreads();
+    uint32_t major[ROUNDS], minor[ROUNDS], k[ROUNDS];
+    bool bad = false, is[ROUNDS];
+    auto load = [&](uint32_t x0) {  // ROUNDS items a work-item at once
+#pragma unroll
+        for (int q = 0; q < ROUNDS; q++) {
+            const uint32_t x = x0 + q * BK_TB + tid;
+            is[q] = x < items && one_item(src, x, major[q], minor[q], k[q], bad);
+        }
+    };
+    for (uint32_t x0 = 0; x0 < items; x0 += ROUNDS * BK_TB) {
+        load(x0);
+#pragma unroll
+        for (int q = 0; q < ROUNDS; q++)
+            if (is[q]) atomicAdd(&first[major[q] + 1], 1u);
+    }
+    if (bad) sh_bad = 1;
+    __syncthreads();
+    // first[r + 1] = entries of the rows before r: where r's places begin
+    uint32_t v[PER], sum = 0, most = 0;
+#pragma unroll
+    for (int i = 0; i < PER; i++) {
+        v[i] = first[PER * tid + i];
+        most = max(most, v[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < PER; i++) sum += v[i];
+    uint32_t inc = sum;
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t u = (uint32_t)__shfl_up((int)inc, d, 64);
+        if (lane >= d) inc += u;
+    }
+    if (lane == 63) wsum[w] = inc;
+    if (most > BK_ROWMAX) sh_long = 1;
+    __syncthreads();
+    if (sh_bad || sh_long) {
+        if (tid == 0) {
+            told[0] = 0;
+            told[1] = sh_bad ? DERR_RANGE : 0;
+            told[2] = (int32_t)sh_long;
+        }
+        return;
+    }
+    uint32_t at = inc - sum;
+    for (int i = 0; i < w; i++) at += wsum[i];
+#pragma unroll
+    for (int i = 0; i < PER; i++) {
+        first[PER * tid + i] = at;
+        at += v[i];
+    }
+    __syncthreads();
+    // every entry to a place of its row; the row begin in its key is the row's
+    // first place, which the runs of smaller rows end at
+    for (uint32_t x0 = 0; x0 < items; x0 += ROUNDS * BK_TB) {
+        if (items > ROUNDS * BK_TB) load(x0);
+#pragma unroll
+        for (int q = 0; q < ROUNDS; q++)
+            if (is[q]) {
+                const uint32_t p = atomicAdd(&first[major[q] + 1], 1u);
+                sk[p] = ((uint64_t)major[q] << bits) | ((uint64_t)minor[q] << kbits) | k[q];
+            }
+    }
+    __syncthreads();
+    uint64_t kr[ROUNDS];
+#pragma unroll
+    for (int q = 0; q < ROUNDS; q++) {
+        const int p = q * BK_TB + tid;
+        kr[q] = sk[p];
+        if (p < m) kr[q] = (kr[q] & ((1ull << bits) - 1)) | ((uint64_t)first[kr[q] >> bits] << bits);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < ROUNDS; q++) sk[q * BK_TB + tid] = kr[q];
+    __syncthreads();
+    const uint32_t nnz = tile_rows<SUM, LOAD, BK_ONE>(sk, ss, se, hm, dm, &sh_base, kr, m, 0u, 0, nmaj, first, vals, fvals, nd,
+                                                      bits, kbits, FirstPlace{}, o);
+    if (tid == 0) tell_build(nnz, first, nmaj, nd, SUM, LOAD, o, nnz_dev, told);
 }
 
 // ---- host -------------------------------------------------------------------------
@@ -645,6 +810,8 @@ static decltype(&k_bk_tile<SUM, LOAD, BK_TILE>) tile_kernel(int64_t n)
     return bk_tile(n) == BK_TILE ? k_bk_tile<SUM, LOAD, BK_TILE> : k_bk_tile<SUM, LOAD, BK_TILE_FEW>;
 }
 
+static bool one_takes(int64_t n, int64_t nmaj) { return n <= BK_ONE && nmaj <= BK_ONE_ROWS; }
+
 static void launch_zero_scan(elfel_hip_ctx *c, const Scratch &S, bool zero, int64_t n, int64_t nmaj)
 {
     if (zero)
@@ -662,6 +829,14 @@ static int run_coo(elfel_hip_ctx *c, void *scratch, const Source &src, int64_t n
     const Scratch S = scratch_layout(scratch, n, nmaj);
     const int kbits = bits_for(n), bits = kbits + bits_for(nmin);
     int *err = (int *)c->dscal.p + 1;
+    if (one_takes(n, nmaj)) {
+        hipLaunchKernelGGL((k_bk_one<true, false, Source>), dim3(1), dim3(BK_TB), 0, c->stream, src, (uint32_t)n, (int)n, val,
+                           (const double *)nullptr, 1u, (int)nmaj, bits, kbits, o, (int32_t *)c->dscal.p + 2,
+                           (int32_t *)c->told + 4);
+        HIPCHK(c, hipGetLastError());
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        return 0;
+    }
     launch_zero_scan(c, S, true, n, nmaj);
     hipLaunchKernelGGL(k_bk_count<Source>, dim3(ceil_div(n, BK_BLOCK * BK_COUNT_ITEMS)), dim3(BK_BLOCK), 0, c->stream, src,
                        n, S.cnt, S.place, err);
@@ -792,8 +967,20 @@ int bucket_form(elfel_hip_ctx *c, void *scratch, const FormMap &m, int64_t E, co
     const int64_t n = E * m.nmat;
     const Scratch S = scratch_layout(scratch, n, ndofs);
     const int kbits = bits_for(n), bits = kbits + bits_for(ndofs);
+    const bool sum = vals != nullptr, load = m.nvec > 0;
     hipEvent_t ev = nullptr;
     tm_begin(c, ELFEL_PH_SORT, &ev);
+    if (one_takes(n, ndofs)) {
+        auto kern = sum ? (load ? k_bk_one<true, true, FormItems> : k_bk_one<true, false, FormItems>)
+                        : (load ? k_bk_one<false, true, FormItems> : k_bk_one<false, false, FormItems>);
+        hipLaunchKernelGGL(kern, dim3(1), dim3(BK_TB), 0, c->stream, FormItems{m, edof}, (uint32_t)(E * m.nd * m.nd), (int)n,
+                           vals, fvals, (uint32_t)m.nd, (int)ndofs, bits, kbits, o, (int32_t *)c->dscal.p, (int32_t *)c->told);
+        HIPCHK(c, hipGetLastError());
+        tm_end(c, ELFEL_PH_SORT, ev);
+        tm_begin(c, ELFEL_PH_REDUCE, &ev);  // nothing is left for it
+        tm_end(c, ELFEL_PH_REDUCE, ev);
+        return 0;
+    }
     switch (m.nd) {
 #define F(N) case N: launch_form<N>(c, S, m, E, edof, ndofs, bits, kbits); break
         F(2); F(3); F(4); F(6); F(8); F(9); F(11); F(12); F(15);
@@ -803,7 +990,6 @@ int bucket_form(elfel_hip_ctx *c, void *scratch, const FormMap &m, int64_t E, co
     HIPCHK(c, hipGetLastError());
     tm_end(c, ELFEL_PH_SORT, ev);
     tm_begin(c, ELFEL_PH_REDUCE, &ev);
-    const bool sum = vals != nullptr, load = m.nvec > 0;
     auto kern = sum ? (load ? tile_kernel<true, true>(n) : tile_kernel<true, false>(n))
                     : (load ? tile_kernel<false, true>(n) : tile_kernel<false, false>(n));
     hipLaunchKernelGGL(kern, dim3((unsigned)S.nt), dim3(BK_TB), 0, c->stream, S.packed, vals, fvals, (uint32_t)m.nd, S.cnt,

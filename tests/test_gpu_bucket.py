@@ -1,8 +1,9 @@
 """The row-bucket COO build (elfel_hip_sparse, elfel_hip_sparse_noalloc) at the
 edges of its tiles, against the oracle's sparse(): pattern and values bit for
-bit (tolerance 0, the same sums in the same order).  1536 entries start in a
-tile, 3584 of a stream of more than 393216, rows of up to 512 are held, longer
-ones and matrices of far more rows than entries take the sort."""
+bit (tolerance 0, the same sums in the same order).  Up to 6144 entries and 8191
+rows are one workgroup's; 1536 entries start in a tile, 3584 of a stream of more
+than 393216; rows of up to 512 are held, longer ones and matrices of far more
+rows than entries take the sort."""
 import numpy as np
 import pytest
 
@@ -35,11 +36,19 @@ def _case(name, rng):
     if name.startswith("many="):
         n = int(name[5:])
         return (*_rows(rng.multinomial(n, np.full(9000, 1 / 9000)), 60, rng), 9000, 60)
+    if name.startswith("rows="):
+        n = int(name[5:])
+        return (*_rows(rng.multinomial(6000, np.full(n, 1 / n)), 31, rng), n, 31)
+    if name.startswith("tiled row="):
+        k = int(name[10:])
+        return (*_rows([3] * 2500 + [k] + [0] * 7 + [5] * 300, max(k // 2, 1), rng), 2808, max(k // 2, 1))
     if name.startswith("row="):  # one long row between short ones, and a tile that it straddles
         k = int(name[4:])
         return (*_rows([3] * 500 + [k] + [0] * 7 + [5] * 300, max(k // 2, 1), rng), 808, max(k // 2, 1))
     if name == "long rows side by side":  # every tile at its largest
         return (*_rows([511, 1024, 1, 512, 512, 512, 512, 511, 1][2:], 600, rng), 7, 600)
+    if name == "long rows in tiles":
+        return (*_rows([512, 512, 512, 511, 1] * 4 + [512], 600, rng), 21, 600)
     if name == "long rows, many":
         return (*_rows([512] * 5 + [511, 1] + [512] * 830 + [3] * 20, 700, rng), 857, 700)
     if name == "empty ends":
@@ -58,7 +67,9 @@ def _case(name, rng):
     raise ValueError(name)
 
 
-CASES = ["many=393216", "many=393217", "many=401408", "long rows, many", "n=1535", "n=1536", "n=1537", "n=2048", "n=3072", "n=9001", "row=511", "row=512", "row=513", "row=1600",
+CASES = ["many=393216", "many=393217", "many=401408", "long rows, many", "n=1535", "n=1536", "n=1537", "n=2048", "n=3072", "n=6143", "n=6144", "n=6145", "n=7679",
+         "n=7680", "n=7681", "n=9001", "rows=8190", "rows=8191", "rows=8192", "tiled row=511", "tiled row=512",
+         "tiled row=513", "long rows in tiles", "row=511", "row=512", "row=513", "row=1600",
          "long rows side by side", "empty ends", "one entry", "one row", "two rows, all duplicates",
          "more rows than entries", "last columns"]
 
@@ -141,6 +152,25 @@ def test_element_stream_in_large_tiles(ctx, layout):
     ctx.set_dofs(0, dn, n)
     ctx.set_coefficients(conn.shape[0])
     for method in (L.SORT, L.REUSE):
+        ctx.assemble(L.HEAT, L.T3, 1, method=method, layout=layout, kappa=1.3, Q=-2.0)
+        _same(ctx.copy_sparse(base=0), ref)
+        assert np.array_equal(ctx.copy_vector(n), ref[3])
+
+
+@pytest.mark.parametrize("method", [L.SORT, L.REUSE])
+@pytest.mark.parametrize("ne", [2, 682, 683])
+def test_element_stream_of_one_workgroup(ctx, ne, method):
+    """6138 and 6147 entries lie either side of what one workgroup takes."""
+    mesh = eh.T3block(2.0, 1.0, 20, 20)
+    conn, xy = np.asarray(mesh.conn)[:ne], np.asarray(mesh.xy)
+    n = xy.shape[0] + 1
+    dn = np.random.default_rng(ne).permutation(n)[:-1] + 1
+    dn[conn[0][1]] = dn[conn[0][0]]  # one dof twice in an element
+    for layout in (L.CSR, L.CSC):
+        ref = _oracle_heat(conn, xy, dn, n, layout)
+        ctx.set_mesh(0, conn, xy)
+        ctx.set_dofs(0, dn, n)
+        ctx.set_coefficients(conn.shape[0])
         ctx.assemble(L.HEAT, L.T3, 1, method=method, layout=layout, kappa=1.3, Q=-2.0)
         _same(ctx.copy_sparse(base=0), ref)
         assert np.array_equal(ctx.copy_vector(n), ref[3])
