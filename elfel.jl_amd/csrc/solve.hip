@@ -953,6 +953,24 @@ __device__ __forceinline__ bool exchange_res(const Exchange &X, uint32_t e, doub
     return *quit == 0u;
 }
 
+// A row's nine entries out of its slice (v: zeros before).
+template <typename T>
+__device__ __forceinline__ void nine_entries(const uint32_t *__restrict__ off, const int16_t *__restrict__ col,
+                                             const T *__restrict__ val, int32_t s, int lane, int32_t lo, int32_t hi, T *v)
+{
+    const uint32_t o = off[s], w = (off[s + 1] - o) >> 6;
+    for (uint32_t q = 0; q < w; q++) {
+        const size_t at = (size_t)o + (size_t)q * 64 + lane;
+        const T x = val[at];  // zero in the padding of a short row, whose column is its own
+        const int32_t d = col[at];
+        if (x != T(0) || d != 0) {
+#pragma unroll
+            for (int j = 0; j < RES_W; j++)
+                if (d == (j < 3 ? lo : j < 6 ? -1 : hi) + j % 3) v[j] = x;
+        }
+    }
+}
+
 template <typename T, typename TX, int R>
 __global__ __launch_bounds__(RES_BLOCK) void k_cg_resident(int64_t n, const uint32_t *__restrict__ off,
                                                            const int16_t *__restrict__ col, const T *__restrict__ val,
@@ -992,17 +1010,7 @@ __global__ __launch_bounds__(RES_BLOCK) void k_cg_resident(int64_t n, const uint
         if (s <= slast) {
             lo[k] = __builtin_amdgcn_readfirstlane(rec[s].x);
             hi[k] = __builtin_amdgcn_readfirstlane(rec[s].y);
-            const uint32_t o = off[s], w = (off[s + 1] - o) >> 6;
-            for (uint32_t q = 0; q < w; q++) {
-                const size_t at = (size_t)o + (size_t)q * 64 + lane;
-                const T x = val[at];  // zero in the padding of a short row, whose column is its own
-                const int32_t d = col[at];
-                if (x != T(0) || d != 0) {
-#pragma unroll
-                    for (int j = 0; j < RES_W; j++)
-                        if (d == (j < 3 ? lo[k] : j < 6 ? -1 : hi[k]) + j % 3) v[k][j] = x;
-                }
-            }
+            nine_entries(off, col, val, s, lane, lo[k], hi[k], v[k]);
         }
         // zeros past the last row, and so all that follows from them
         sr[k][tid] = i < nn ? r_[ic] : T(0);
@@ -1163,6 +1171,140 @@ __global__ __launch_bounds__(RES_BLOCK) void k_cg_resident(int64_t n, const uint
         sc[S_IT] = (double)it;
     }
     if (!ok && threadIdx.x == 0) sc[S_LOST] = 1.0;
+}
+
+// The same for at most 2048 FP64 or 4096 FP32 rows, by one workgroup: p in LDS,
+// R rows a work-item (row tid + 1024 k: block 4 k + tid / 256), the sums over
+// waves in LDS and over the blocks by every wave for itself.  Three barriers are
+// left of the waits for other workgroups, which are most of an iteration of the
+// small systems above.  Whole solves, one launch of many workgroups -> of one:
+// FP64 T3 33x32 775 -> 421 us, T3 46x45 (1980 rows) 977 -> 642; mixed Q4 30^2
+// 959 -> 539, Q4 64^2 (3969) 1602 -> 1441.  Four FP64 rows a work-item spill
+// (Q4 64x63 1399 -> 1825).
+#define ONE_ROWS(T) (sizeof(T) == 8 ? 2 * RES_BLOCK : 4 * RES_BLOCK)
+template <typename T, typename TX, int R>
+__global__ __launch_bounds__(RES_BLOCK) void k_cg_one(int n, int G, const uint32_t *__restrict__ off,
+                                                      const int16_t *__restrict__ col, const T *__restrict__ val,
+                                                      const int2 *__restrict__ rec, const T *__restrict__ dinv, T *r_, T *pa,
+                                                      TX *xs_, double *x_, const double *part_rz, double *sc, double goal2,
+                                                      int it, int maxit)
+{
+    constexpr int N = R * RES_BLOCK, EDGE = 3;
+    __shared__ T sp[N + 2 * EDGE];  // p between zeros
+    __shared__ double sh[3][R * (RES_BLOCK / 64)];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    T v[R][RES_W], ri[R], di[R], pi[R], qi[R];
+    TX xi[R];
+    int lo[R], hi[R];  // where the row's runs begin in sp
+    if (tid < EDGE) sp[tid] = sp[N + EDGE + tid] = T(0);
+#pragma unroll
+    for (int k = 0; k < R; k++) {
+        const int i = k * RES_BLOCK + tid, s = i >> 6;
+#pragma unroll
+        for (int q = 0; q < RES_W; q++) v[k][q] = T(0);
+        lo[k] = hi[k] = 0;
+        if (i < n) {
+            const int2 m = rec[s];
+            nine_entries(off, col, val, s, lane, m.x, m.y, v[k]);
+            lo[k] = EDGE + min(max(i + m.x, -EDGE), N);  // beyond: entries of nothing but zeros
+            hi[k] = EDGE + min(max(i + m.y, -EDGE), N);
+        }
+        ri[k] = i < n ? r_[i] : T(0);
+        di[k] = i < n ? dinv[i] : T(0);
+        pi[k] = i < n ? pa[i] : T(0);
+        xi[k] = i < n ? xs_[i] : TX(0);
+    }
+    // sums over all blocks, the same in every lane; lane l adds up block l's waves
+    auto total = [&](const double *part) {
+        double s = 0.0;
+        if (lane < 4 * R)
+            for (int k = 0; k < SV_BLOCK / 64; k++) s += part[lane * (SV_BLOCK / 64) + k];
+        return 0.0 + of_lane(wave_sum(0.0 + s), 0);
+    };
+    double rz = 0.0 + of_lane(wave_sum(lane < G ? 0.0 + part_rz[lane] : 0.0), 0), rz_old = 0.0, rr = sc[S_RR];
+    bool dir = false;
+    while (rr > goal2 && it < maxit) {
+        for (int c = 0; c < CHECK; c++) {
+            const T beta = dir ? (T)(rz_old != 0.0 ? rz / rz_old : 0.0) : T(0);
+#pragma unroll
+            for (int k = 0; k < R; k++) {
+                if (dir) pi[k] = product(di[k], ri[k]) + beta * pi[k];
+                sp[EDGE + k * RES_BLOCK + tid] = pi[k];
+            }
+            dir = true;
+            __syncthreads();
+            double pq[R];
+#pragma unroll
+            for (int k = 0; k < R; k++) {
+                T acc = T(0);
+#pragma unroll
+                for (int j = 0; j < RES_W; j++)
+                    acc += v[k][j] * sp[j < 3 ? lo[k] + j : j < 6 ? EDGE - 4 + k * RES_BLOCK + tid + j : hi[k] + j - 6];
+                qi[k] = acc;
+                pq[k] = 0.0;
+                pq[k] += (double)pi[k] * (double)acc;
+                pq[k] = wave_sum(pq[k]);
+            }
+            if (lane == 0) {
+#pragma unroll
+                for (int k = 0; k < R; k++) sh[0][k * (RES_BLOCK / 64) + w] = pq[k];
+            }
+            __syncthreads();
+            const double pqs = total(sh[0]);
+            const double alpha64 = pqs != 0.0 ? rz / pqs : 0.0;
+            const T alpha = (T)alpha64;
+            const TX alphax = (TX)alpha64;
+            double a[R], b[R];
+#pragma unroll
+            for (int k = 0; k < R; k++) {
+                ri[k] = ri[k] - alpha * qi[k];
+                const T zi = product(di[k], ri[k]);
+                a[k] = b[k] = 0.0;
+                a[k] += (double)ri[k] * (double)zi;
+                b[k] += (double)ri[k] * (double)ri[k];
+                a[k] = wave_sum(a[k]);
+                b[k] = wave_sum(b[k]);
+                xi[k] += alphax * (TX)pi[k];
+            }
+            if (lane == 0) {
+#pragma unroll
+                for (int k = 0; k < R; k++) {
+                    sh[1][k * (RES_BLOCK / 64) + w] = a[k];
+                    sh[2][k * (RES_BLOCK / 64) + w] = b[k];
+                }
+            }
+            __syncthreads();
+            rz_old = rz;
+            rz = total(sh[1]);
+            rr = total(sh[2]);
+        }
+        if constexpr (sizeof(TX) == 4) {
+#pragma unroll
+            for (int k = 0; k < R; k++) {
+                const int i = k * RES_BLOCK + tid;
+                if (i < n) x_[i] += (double)xi[k];
+                xi[k] = TX(0);
+            }
+        }
+        it += CHECK;
+    }
+    // the state that the next reset continues from
+    if (dir) {
+        const T beta = (T)(rz_old != 0.0 ? rz / rz_old : 0.0);
+#pragma unroll
+        for (int k = 0; k < R; k++) {
+            const int i = k * RES_BLOCK + tid;
+            if (i >= n) break;
+            r_[i] = ri[k];
+            pa[i] = product(di[k], ri[k]) + beta * pi[k];
+            xs_[i] = xi[k];
+        }
+    }
+    if (tid == 0) {
+        sc[S_RREC] = rr;
+        sc[S_IT] = (double)it;
+        sc[S_LOST] = 0.0;
+    }
 }
 
 // r = (T) r64, z = M r (p = z when `restart`); partials r.z (into rz_out) and r.r
@@ -1394,6 +1536,22 @@ int cg_resident_as(hipStream_t st, int64_t n, const Sell &S, Vecs<T> &v, TX *xs,
     (void)hipGetLastError();
     return 1;
 }
+template <typename T, typename TX>
+void cg_one_as(hipStream_t st, int64_t n, const Sell &S, Vecs<T> &v, TX *xs, const Parts &P, double *sc, double goal2, int it,
+            int maxit)
+{
+    auto kern = n <= RES_BLOCK ? k_cg_one<T, TX, 1> : n <= 2 * RES_BLOCK ? k_cg_one<T, TX, 2> : k_cg_one<T, TX, ONE_ROWS(T) / RES_BLOCK>;
+    hipLaunchKernelGGL(kern, dim3(1), dim3(RES_BLOCK), 0, st, (int)n, P.G, S.off, (const int16_t *)S.col, sell_vals<T>(S), S.rec,
+                       (const T *)v.dinv, v.r, v.p, xs, v.x, (const double *)P.rz, sc, goal2, it, maxit);
+}
+void cg_one(hipStream_t st, int64_t n, const Sell &S, Vecs<double> &v, const Parts &P, double *sc, double goal2, int it, int maxit)
+{
+    cg_one_as(st, n, S, v, v.x, P, sc, goal2, it, maxit);
+}
+void cg_one(hipStream_t st, int64_t n, const Sell &S, Vecs<float> &v, const Parts &P, double *sc, double goal2, int it, int maxit)
+{
+    cg_one_as(st, n, S, v, v.xlo, P, sc, goal2, it, maxit);
+}
 // Rows a work-item of the resident solve that n rows in G blocks need; most: 3
 // FP64 (786 000 rows on 256 CUs), 8 mixed (2.1 million).
 int cg_resident(hipStream_t st, int64_t n, const Sell &S, Vecs<double> &v, const Parts &P, uint64_t *slots, double *sc,
@@ -1584,15 +1742,18 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
     const double target = tol * bnorm;
     // Iterations until ||r||^2 <= goal2 or maxit from the state of the last reset,
     // then the true residual (waits): *rrec the recurrence's ||r||^2, *norm the
-    // true residual's norm.  One launch where every row has its own work-item,
-    // the rows fit its registers and there are few enough workgroups, or where
-    // all slices have records and the rows fit the chip's registers.
+    // true residual's norm.  One launch of one workgroup where all slices have
+    // records and there are few rows; of many where every row has its own
+    // work-item, the rows fit its registers and there are few enough workgroups,
+    // or where all slices have records and the rows fit the chip's registers.
     auto solve_to = [&](auto &v, double goal2, double *rrec, double *norm) -> int {
         using T = typename std::remove_pointer<decltype(v.r)>::type;
         constexpr int VB = sizeof(T) == 8 ? SM_VB8 : SM_VB4;
         const bool small = narrow && n <= (int64_t)P.G * SV_BLOCK && (P.G + VB - 1) / VB <= SM_GRID;
-        const bool one = !lost && ((small && cg_small(st, n, S, v, P, slots, sc, goal2, it, maxit) == 0) ||
-                                   (resident && cg_resident(st, n, S, v, P, slots, sc, goal2, it, maxit) == 0));
+        bool one = resident && n <= ONE_ROWS(T);
+        if (one) cg_one(st, n, S, v, P, sc, goal2, it, maxit);
+        else one = !lost && ((small && cg_small(st, n, S, v, P, slots, sc, goal2, it, maxit) == 0) ||
+                             (resident && cg_resident(st, n, S, v, P, slots, sc, goal2, it, maxit) == 0));
         if (one) {
             if ((rc = true_residual(norm))) return rc;
             lost = hsc[S_LOST] != 0.0;

@@ -1,6 +1,7 @@
 """elfel_hip_pcg at the sizes where its kernels change: rows either side of a
-wave, of a block of 256 rows, of a workgroup of the one-launch solve (512 rows
-FP64, 768 mixed), of the most rows that it takes (224 workgroups), of each count
+wave, of a block of 256 rows, of what one workgroup solves (1024 rows each of a
+work-item's, 2048 FP64 and 4096 mixed at most; grids in their own order), of a
+workgroup of the one-launch solve (512 rows FP64, 768 mixed), of the most rows that it takes (224 workgroups), of each count
 of rows a work-item of the solve from registers (262144 rows each on 256 CUs; 1
 to 3 FP64, 1, 2, 4, 8 mixed) and past its last, grids with their boundary
 numbered last and ones whose slices it does not take, a matrix whose rows are
@@ -53,6 +54,15 @@ def _solve(ctx, fe, N, nfree, prec, seed=3, shuffle=False, kind=L.HEAT, order=No
 @pytest.mark.parametrize("nfree", [1, 2, 63, 64, 65, 255, 256, 257, 511, 512, 513, 767, 768, 769, 1535, 1536, 1537, 1600])
 def test_small(ctx, nfree, prec):
     _solve(ctx, L.Q4, 40, nfree, prec)
+    _solve(ctx, L.Q4, 40, nfree, prec, shuffle=True)
+
+
+@pytest.mark.parametrize("fe", [L.T3, L.Q4])
+@pytest.mark.parametrize("prec,nfree", [(L.FP64, 1023), (L.FP64, 1024), (L.FP64, 1025), (L.FP64, 2047), (L.FP64, 2048),
+                                        (L.FP64, 2049), (L.MIXED, 2049), (L.MIXED, 3072), (L.MIXED, 4095), (L.MIXED, 4096),
+                                        (L.MIXED, 4097)])
+def test_one_workgroup(ctx, nfree, prec, fe):
+    _solve(ctx, fe, 66, nfree, prec)
 
 
 @pytest.mark.parametrize("prec,nfree,N", [(L.FP64, 224 * 512, 340), (L.FP64, 224 * 512 + 1, 340),
