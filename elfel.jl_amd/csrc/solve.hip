@@ -589,7 +589,8 @@ __device__ __forceinline__ double wave_sum(double v)
 
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-#define SC1 16               // cache policy of buffer accesses: device scope
+#define SC1 16  // cache policy of buffer accesses: device scope
+#define NT 2    // ... read once
 
 // Three sets of slots; a block's two partials lie side by side, four blocks to
 // 64 bytes, in EX_COPIES copies: every workgroup polls all slots, of the copy
@@ -825,7 +826,7 @@ __global__ __launch_bounds__(VB * SV_BLOCK) void k_cg_small(int64_t n, const uin
 // and writes z and p alone where the streaming kernels move 80 bytes a row.
 // Streaming -> resident, us an iteration: FP64 Q4 460x450 22.9 -> 8.7, T3
 // 700x690 29.4 -> 10.9; mixed Q4 500^2 19.1 -> 7.6, 1000^2 30.5 -> 10.7,
-// 1500x1300 (1.95 million rows) 44.3 -> 19.5.
+// 1500x1300 (1.95 million rows) 44.3 -> 18.9.
 // The rows, blocks and sums are those of the streaming kernels (block b's rows
 // are b * 256 + t + k * 256 G): the same bits.
 //
@@ -857,13 +858,15 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t words_rsrc(void *v, size_t wor
 {
     return __builtin_amdgcn_make_buffer_rsrc(v, 0, (int)(n * word), 0x00020000);
 }
+template <int POLICY>
 __device__ __forceinline__ void load1(__amdgpu_buffer_rsrc_t r, int32_t i, float &o)
 {
-    o = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, i * 4, 0, SC1));
+    o = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, i * 4, 0, POLICY));
 }
+template <int POLICY>
 __device__ __forceinline__ void load1(__amdgpu_buffer_rsrc_t r, int32_t i, double &o)
 {
-    const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, i * 8, 0, SC1);
+    const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, i * 8, 0, POLICY);
     o = __builtin_bit_cast(double, ((uint64_t)v[1] << 32) | v[0]);
 }
 __device__ __forceinline__ void store1(__amdgpu_buffer_rsrc_t r, int32_t i, float v)
@@ -978,6 +981,9 @@ __global__ __launch_bounds__(RES_BLOCK) void k_cg_resident(int64_t n, const uint
                                                            T *z_, T *pa, T *pb, TX *xs_, double *x_, const double *part_rz,
                                                            Exchange X, double *sc, double goal2, int it, int maxit)
 {
+    // (z and p of more than a million rows are gone from an L2 before the next
+    // row of the grid reads them: 3 to 7 % faster past them; fewer rows 2 % slower)
+    constexpr int POLICY = R >= 6 ? SC1 | NT : SC1;
     constexpr int DEEP = R < 3 ? R : 3;  // rows in flight (1, 2, 3, 4, 6: 22.0, 20.5, 19.5, 19.8, 23.5 us at 1.95 million rows)
     __shared__ T sr[R][RES_BLOCK], sd[R][RES_BLOCK];
     __shared__ T sp[R][RES_VB][SV_BLOCK + 2];  // p, each block's between the two rows beside it
@@ -1048,20 +1054,20 @@ __global__ __launch_bounds__(RES_BLOCK) void k_cg_resident(int64_t n, const uint
                 const int32_t i = row(k);
                 int32_t l = lo[k], h = hi[k];
                 asm volatile("" : "+s"(l), "+s"(h));
-                load1(bp, i + l, pp[k % DEEP][0]);
-                load1(bz, i + l, zz[k % DEEP][0]);
-                load1(bp, i + h, pp[k % DEEP][1]);
-                load1(bz, i + h, zz[k % DEEP][1]);
+                load1<POLICY>(bp, i + l, pp[k % DEEP][0]);
+                load1<POLICY>(bz, i + l, zz[k % DEEP][0]);
+                load1<POLICY>(bp, i + h, pp[k % DEEP][1]);
+                load1<POLICY>(bz, i + h, zz[k % DEEP][1]);
                 const int32_t j = i + past + (lane < 2 ? l : h);
-                load1(bp, j, pp[k % DEEP][2]);
-                load1(bz, j, zz[k % DEEP][2]);
+                load1<POLICY>(bp, j, pp[k % DEEP][2]);
+                load1<POLICY>(bz, j, zz[k % DEEP][2]);
             };
             if (tid < 2 * RES_VB * R) {  // the rows beside the blocks
                 const int k = tid / (2 * RES_VB), q = (tid >> 1) % RES_VB, right = tid & 1;
                 const int32_t i = (int32_t)(blockIdx.x + q * RES_GRID) * SV_BLOCK + k * stride + (right ? SV_BLOCK : -1);
                 T z1, p1;
-                load1(bp, i, p1);
-                load1(bz, i, z1);
+                load1<POLICY>(bp, i, p1);
+                load1<POLICY>(bz, i, z1);
                 sp[k][q][right ? SV_BLOCK + 1 : 0] = dir ? z1 + beta * p1 : p1;
             }
 #pragma unroll
@@ -1567,6 +1573,7 @@ int cg_resident(hipStream_t st, int64_t n, const Sell &S, Vecs<float> &v, const 
                 double goal2, int it, int maxit)
 {
     const int64_t r = (n + (int64_t)P.G * SV_BLOCK - 1) / ((int64_t)P.G * SV_BLOCK);
+    // (5 and 7 of their own gain less than 1 % on the next)
     if (r <= 1) return cg_resident_as<float, float, 1>(st, n, S, v, v.xlo, P, slots, sc, goal2, it, maxit);
     if (r <= 2) return cg_resident_as<float, float, 2>(st, n, S, v, v.xlo, P, slots, sc, goal2, it, maxit);
     if (r <= 4) return cg_resident_as<float, float, 4>(st, n, S, v, v.xlo, P, slots, sc, goal2, it, maxit);

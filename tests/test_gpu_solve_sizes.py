@@ -1,9 +1,10 @@
 """elfel_hip_pcg at the sizes where its kernels change: rows either side of a
-wave, of a block of 256 rows, of what one workgroup solves (1024 rows each of a
-work-item's, 2048 FP64 and 4096 mixed at most; grids in their own order), of a
-workgroup of the one-launch solve (512 rows FP64, 768 mixed), of the most rows that it takes (224 workgroups), of each count
-of rows a work-item of the solve from registers (262144 rows each on 256 CUs; 1
-to 3 FP64, 1, 2, 4, 8 mixed) and past its last, grids with their boundary
+wave, of a block of 256 rows, of what one workgroup solves (1024 rows for each
+of a work-item's; 2048 FP64 and 4096 mixed at most, grids in their own order),
+of a workgroup of the one-launch solve (512 rows FP64, 768 mixed), of the most
+rows that it takes (224 workgroups), of each count of rows a work-item of the
+solve from registers (262144 rows each on 256 CUs; 1 to 3 FP64, 1 to 8 mixed)
+and past its last, grids with their boundary
 numbered last and ones whose slices it does not take, a matrix whose rows are
 wider than the registers, and one whose columns are too far from the diagonal
 for 16-bit offsets.
@@ -82,7 +83,8 @@ def test_wide_rows_and_far_columns(ctx, prec):
     (L.FP64, L.Q4, 262144, 520), (L.FP64, L.T3, 262145, 520), (L.FP64, L.T3, 524288, 730), (L.FP64, L.Q4, 524289, 730),
     (L.FP64, L.Q4, 786432, 890), (L.FP64, L.T3, 786433, 890),
     (L.MIXED, L.T3, 262144, 520), (L.MIXED, L.Q4, 262145, 520), (L.MIXED, L.Q4, 524289, 730),
-    (L.MIXED, L.T3, 1048577, 1030), (L.MIXED, L.Q4, 1572865, 1260), (L.MIXED, L.Q4, 2097152, 1449), (L.MIXED, L.T3, 2097153, 1449)])
+    (L.MIXED, L.Q4, 786433, 890), (L.MIXED, L.T3, 1048577, 1030), (L.MIXED, L.Q4, 1310721, 1150), (L.MIXED, L.Q4, 1572865, 1260),
+    (L.MIXED, L.T3, 1835009, 1360), (L.MIXED, L.Q4, 2097152, 1449), (L.MIXED, L.T3, 2097153, 1449)])
 def test_rows_in_registers(ctx, prec, fe, nfree, N):
     _solve(ctx, fe, N, nfree, prec)
 
