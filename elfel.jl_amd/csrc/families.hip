@@ -1,7 +1,7 @@
 // families.hip -- the element families beyond T3/T6/Q4 and the weak forms
-// that use them, on the plain FP64 method (COO in Elfel's stream order, then
-// the stable radix sort and in-order segmented reduce of plain.hip) and on the
-// REUSE method (that sort done once and kept as a permutation; each assembly
+// that use them, on the plain FP64 method (the values of the COO stream in
+// Elfel's order, then the row buckets or the sort of plain.hip) and on the
+// REUSE method (the order of that build found once and kept as a permutation; each assembly
 // sums the runs through it in the same order).
 // Compiled with -ffp-contract=off: every product and sum rounds as the
 // reference's unfused Julia arithmetic does.

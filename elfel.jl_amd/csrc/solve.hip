@@ -37,6 +37,10 @@
 // and no extra reduction launches; every run gives the same bits.  The CG
 // scalars stay on the device and the host reads the residual every CHECK
 // iterations.
+// Systems that fit on the chip run all of that in one launch, with the same
+// sums and bits: small ones, and on grid-like numberings up to 786 000 rows FP64
+// or 2.1 million mixed, with the matrix in registers (k_cg_small,
+// k_cg_resident; k_cg_one for a few thousand rows).
 #include <math.h>
 
 #include <algorithm>
@@ -519,7 +523,7 @@ __global__ __launch_bounds__(SV_BLOCK) void k_cg_fin(int64_t n, const double *__
 // A workgroup is VB blocks of SV_BLOCK rows, each with the partials that the
 // grid-wide kernels form for the same block, summed in the same order: the
 // same bits.  Heat T3 100^2 FP64, an iteration: 15 us in two launches (each
-// half launch and sums of partials) -> 7 us.
+// half launch and sums of partials) -> 5.8 us.
 //
 // An exchange of partials is also the barrier between an iteration's two halves:
 // a workgroup publishes after its stores of z and p are complete, and who has
@@ -534,7 +538,8 @@ __global__ __launch_bounds__(SV_BLOCK) void k_cg_fin(int64_t n, const double *__
 // VB: the registers of a row (its entries, the gathers in flight) leave 512
 // work-items of FP64 rows or 768 of FP32 rows; larger workgroups spill (1024
 // FP64: 14.9 us an iteration at 9801 rows), smaller ones are more pollers of the
-// same slots (256: 10.5 and 10.8 against 9.4 and 9.0 us at 62 000 rows).
+// same slots (256: 10.5 and 10.8 against 9.4 and 9.0 us at 62 000 rows, the
+// slots packed).
 // SM_GRID: as many workgroups as measured faster than two launches (iteration
 // at 100^2, 250^2, 300^2 rows FP64 5.8, 6.3, 6.5 against 15.3, 15.2, 16.8 us;
 // mixed 100^2, 250^2, 400^2 6.2, 6.0, 7.2 against 15.5, 14.8, 17.0), with an

@@ -3,7 +3,7 @@
 SysmatAssemblerHIP mirrors SysmatAssemblerSparse (src/Assemblers.jl:19-123):
 start(a, nrow, ncol), assemble(a, r, c, v), assemble(a, lma),
 assemble(a, lma.T) (transpose(lma)), finish(a) -> CSC sparse matrix.  The COO
-stream collected on the host is handed to the device, which sorts it stably and
+stream collected on the host is handed to the device, which orders it stably and
 sums duplicates in stream order (the semantics of SparseArrays.sparse).  The
 device-integrated weak forms of elfel_hip.integrate leave their matrix on the
 device instead; finish(a) then copies it out.

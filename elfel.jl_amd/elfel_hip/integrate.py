@@ -20,7 +20,7 @@ method.
 
 precision: "fp64" (the plain method: every operation as the reference does it)
 or "mixed" (FP32 element arithmetic, FP64 sums into the matrix).
-method: "sort" (COO -> stable radix sort -> segmented reduce, every call) or
+method: "sort" (COO -> stable order by row and column -> in-order sums, every call) or
 "reuse" (pattern built on the first call, then one fused kernel per call).
 """
 import numpy as np
