@@ -30,9 +30,10 @@
 
 #define BK_BLOCK 256
 #define BK_TB 1024                  // work-items of a tile
-#define BK_ROWMAX 512               // longest row that a tile holds; a longer one goes to the sort
-#define BK_TILE 3584                // entries that start in a tile, its last row's overhang beyond
-#define BK_TILE_FEW 1536            // ... of a stream of at most BK_FEW entries
+#define BK_CAP 4096                 // entries that a tile holds
+#define BK_CAP_FEW 2048             // ... of a stream of at most BK_FEW entries
+#define BK_ROWMAX 512               // room for the last row's overhang, the rest is for those that start in the tile;
+                                    // with a longer row, half and half; one longer than half goes to the sort
 #define BK_FEW (256 * 1536)
 #define BK_CAP_LOG2 12
 #define BK_COUNT_ITEMS 2            // entries per work-item of the counting pass
@@ -41,7 +42,7 @@
 #define BK_SCAN_ITEMS 16
 #define BK_SCAN_CHUNK (BK_BLOCK * BK_SCAN_ITEMS)
 
-static_assert(BK_TILE + BK_ROWMAX <= 1 << BK_CAP_LOG2, "a place in a tile has BK_CAP_LOG2 bits");
+static_assert(BK_CAP <= 1 << BK_CAP_LOG2, "a place in a tile has BK_CAP_LOG2 bits");
 static_assert(BK_HASH >= 2 * BK_BLOCK * BK_COUNT_ITEMS, "the hash of the counting pass is at most half full");
 
 // ---- decoupled look-back -------------------------------------------------------
@@ -95,9 +96,20 @@ __device__ __forceinline__ uint32_t lb_wait(uint64_t *st, uint32_t t, uint32_t t
 }
 
 // ---- control words ---------------------------------------------------------------
-// BK_LONG: a row longer than BK_ROWMAX exists and the tiles do not hold it; the
-// kernels after the scan then leave every output alone.
-enum { BK_T_SCAN = 0, BK_T_TILE = 1, BK_LONG = 2, BK_NCTL = 4 };
+// BK_LONG: a row longer than BK_ROWMAX exists: the tiles are those of the second
+// set.  BK_TOOLONG: one that no tile holds; the kernels after the scan then
+// leave every output alone.
+enum { BK_T_SCAN = 0, BK_T_TILE = 1, BK_LONG = 2, BK_TOOLONG = 3, BK_NCTL = 4 };
+
+// The first row and entry of every tile: for rows of at most BK_ROWMAX entries,
+// and of at most half a tile.
+struct Tiles {
+    uint32_t *row, *first;
+    uint32_t nt;
+};
+struct TileSets {
+    Tiles set[2];
+};
 
 __global__ void k_bk_zero(uint4 *__restrict__ p, int64_t n4)
 {
@@ -215,11 +227,11 @@ __global__ __launch_bounds__(BK_BLOCK) void k_bk_count(Source src, int64_t n, ui
 }
 
 // cnt[0 .. nmaj] (cnt[nmaj] = 0) -> the rows' first entries, and for every tile
-// t the first row that starts at or after t * tile with that start (tile
-// nt: nmaj and n).  A row's interval (s, s + len] holds the tile boundaries
+// t of both sets the first row that starts at or after t * tile with that start
+// (tile nt: nmaj and n).  A row's interval (s, s + len] holds the tile boundaries
 // that the next row is the first to reach.
-__global__ __launch_bounds__(BK_BLOCK) void k_bk_scan(uint32_t *__restrict__ cnt, int64_t nmaj, uint32_t n, uint32_t nt,
-                                                      uint32_t tile, uint32_t *__restrict__ trow, uint32_t *__restrict__ tstart,
+template <int CAP>
+__global__ __launch_bounds__(BK_BLOCK) void k_bk_scan(uint32_t *__restrict__ cnt, int64_t nmaj, uint32_t n, TileSets T,
                                                       uint64_t *__restrict__ st, uint32_t *__restrict__ ctl)
 {
     __shared__ uint32_t wsum[BK_BLOCK / 64], sh_b, sh_base;
@@ -265,13 +277,19 @@ __global__ __launch_bounds__(BK_BLOCK) void k_bk_scan(uint32_t *__restrict__ cnt
     __syncthreads();
     uint32_t s = sh_base + woff + inc - sum;
     if (most > BK_ROWMAX) ctl[BK_LONG] = 1u;
+    if (most > CAP / 2) ctl[BK_TOOLONG] = 1u;
 #pragma unroll
     for (int i = 0; i < BK_SCAN_ITEMS; i++) {
         const uint32_t c = v[i];
         v[i] = s;
-        for (uint32_t t = s / tile + 1; t <= (s + c) / tile; t++) {  // c = 0 past the last row
-            trow[t] = (uint32_t)(r0 + i + 1);
-            tstart[t] = s + c;
+        const uint32_t e = s + c;  // c = 0 past the last row
+        for (uint32_t t = s / (CAP - BK_ROWMAX) + 1; t <= e / (CAP - BK_ROWMAX); t++) {
+            T.set[0].row[t] = (uint32_t)(r0 + i + 1);
+            T.set[0].first[t] = e;
+        }
+        for (uint32_t t = s / (CAP / 2) + 1; t <= e / (CAP / 2); t++) {
+            T.set[1].row[t] = (uint32_t)(r0 + i + 1);
+            T.set[1].first[t] = e;
         }
         s += c;
     }
@@ -284,11 +302,12 @@ __global__ __launch_bounds__(BK_BLOCK) void k_bk_scan(uint32_t *__restrict__ cnt
             if (r0 + i + 2 <= nmaj) cnt[r0 + i + 2] = v[i + 2];
         }
     }
-    if (b == 0 && tid == 0) {
-        trow[0] = 0;
-        tstart[0] = 0;
-        trow[nt] = (uint32_t)nmaj;
-        tstart[nt] = n;
+    if (b == 0 && tid < 2) {
+        const Tiles &t = T.set[tid];
+        t.row[0] = 0;
+        t.first[0] = 0;
+        t.row[t.nt] = (uint32_t)nmaj;
+        t.first[t.nt] = n;
     }
 }
 
@@ -298,10 +317,10 @@ __global__ __launch_bounds__(BK_BLOCK) void k_bk_scan(uint32_t *__restrict__ cnt
 template <typename Source>
 __global__ __launch_bounds__(BK_BLOCK) void k_bk_scatter(Source src, int64_t n, const uint32_t *__restrict__ start,
                                                          const uint32_t *__restrict__ place, int bits, int kbits,
-                                                         uint64_t *__restrict__ packed)
+                                                         uint64_t *__restrict__ packed, const uint32_t *__restrict__ ctl)
 {
     const int64_t k = (int64_t)blockIdx.x * BK_BLOCK + threadIdx.x;
-    if (k >= n) return;
+    if (k >= n || ctl[BK_TOOLONG] != 0) return;
     uint32_t major, minor;
     src.get(k, major, minor);
     const uint32_t s = start[major];
@@ -353,8 +372,8 @@ __device__ __forceinline__ int bits_between(const uint64_t *m, int p, int e)
     return n;
 }
 
-// One workgroup per tile of whole rows: those that start in TILE entries, each
-// of at most BK_ROWMAX.  An entry less the tile's first entry (in the row field)
+// One workgroup per tile of whole rows: those that start in a tile's entries, each
+// of at most half of it.  An entry less the tile's first entry (in the row field)
 // is (row begin, minor, stream position), so entries of a tile compare as plain
 // integers.  Each work-item counts, for four neighbouring entries at once, how
 // many entries of their rows are smaller: broadcast reads from LDS, for the 20
@@ -559,16 +578,15 @@ struct AfterTiles {
     __device__ __forceinline__ uint32_t wait(uint32_t total) const { return lb_wait(st, t, total); }
 };
 
-template <bool SUM, bool LOAD, int TILE>
+template <bool SUM, bool LOAD, int CAP>
 __global__ __launch_bounds__(BK_TB) void k_bk_tile(const uint64_t *__restrict__ packed, const double *__restrict__ vals,
                                                    const double *__restrict__ fvals, uint32_t nd,
-                                                   const uint32_t *__restrict__ start, const uint32_t *__restrict__ trow,
-                                                   const uint32_t *__restrict__ tstart, uint32_t nt, int64_t nmaj,
+                                                   const uint32_t *__restrict__ start, TileSets T, int64_t nmaj,
                                                    int bits, int kbits, uint64_t *__restrict__ st,
                                                    uint32_t *__restrict__ ctl, const int *__restrict__ err, BucketOut o,
                                                    int32_t *__restrict__ nnz_dev, int32_t *__restrict__ told)
 {
-    constexpr int CAP = TILE + BK_ROWMAX, ROUNDS = CAP / BK_TB;
+    constexpr int ROUNDS = CAP / BK_TB;
     __shared__ __align__(16) uint64_t sk[CAP + 4];  // the entries by row; then the values in sorted order
     __shared__ uint64_t ss[CAP];                    // the entries, sorted
     __shared__ uint16_t se[CAP + 1];                // end of a row, at its begin; then the runs before an entry
@@ -578,14 +596,18 @@ __global__ __launch_bounds__(BK_TB) void k_bk_tile(const uint64_t *__restrict__ 
     const int tid = threadIdx.x;
     // nothing is written when an index was out of range or a row is too long
     // (the flags were set by earlier kernels: the same for every workgroup)
-    if (*err != 0 || ctl[BK_LONG] != 0) {
+    if (*err != 0 || ctl[BK_TOOLONG] != 0) {
         if (blockIdx.x == 0 && tid == 0) {
             told[0] = 0;
             told[1] = *err;
-            told[2] = (int32_t)ctl[BK_LONG];
+            told[2] = (int32_t)ctl[BK_TOOLONG];
         }
         return;
     }
+    const bool longrows = ctl[BK_LONG] != 0;
+    const uint32_t nt = longrows ? T.set[1].nt : T.set[0].nt;
+    const uint32_t *trow = longrows ? T.set[1].row : T.set[0].row, *tstart = longrows ? T.set[1].first : T.set[0].first;
+    if (blockIdx.x >= nt) return;  // launched for the larger of the two sets: nt numbers are taken
     if (tid == 0) sh_t = atomicAdd(&ctl[BK_T_TILE], 1u);
     __syncthreads();
     const uint32_t t = sh_t;
@@ -656,13 +678,13 @@ __global__ __launch_bounds__(BK_TB) void k_bk_one(Source src, uint32_t items, in
     __shared__ uint16_t se[BK_ONE + 1];
     __shared__ uint64_t hm[BK_ONE / 64], dm[LOAD ? BK_ONE / 64 : 1];
     __shared__ __align__(16) uint32_t first[BK_ONE_ROWS + 1];  // row r's entries at r + 1, then the end of its places so far
-    __shared__ uint32_t wsum[BK_TB / 64], sh_base, sh_bad, sh_long;
+    __shared__ uint32_t wsum[BK_TB / 64], sh_base, sh_bad;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
 #pragma unroll
     for (int i = 0; i < PER; i += 4) *(uint4 *)(first + PER * tid + i) = make_uint4(0, 0, 0, 0);
 #pragma unroll
     for (int q = 0; q < ROUNDS; q++) sk[q * BK_TB + tid] = ~0ull;
-    if (tid == 0) sh_bad = sh_long = 0;
+    if (tid == 0) sh_bad = 0;
     __syncthreads();
     uint32_t major[ROUNDS], minor[ROUNDS], k[ROUNDS];
     bool bad = false, is[ROUNDS];
@@ -682,27 +704,24 @@ __global__ __launch_bounds__(BK_TB) void k_bk_one(Source src, uint32_t items, in
     if (bad) sh_bad = 1;
     __syncthreads();
     // first[r + 1] = entries of the rows before r: where r's places begin
-    uint32_t v[PER], sum = 0, most = 0;
+    uint32_t v[PER], sum = 0;
 #pragma unroll
     for (int i = 0; i < PER; i++) {
         v[i] = first[PER * tid + i];
-        most = max(most, v[i]);
+        sum += v[i];
     }
-#pragma unroll
-    for (int i = 0; i < PER; i++) sum += v[i];
     uint32_t inc = sum;
     for (int d = 1; d < 64; d <<= 1) {
         const uint32_t u = (uint32_t)__shfl_up((int)inc, d, 64);
         if (lane >= d) inc += u;
     }
     if (lane == 63) wsum[w] = inc;
-    if (most > BK_ROWMAX) sh_long = 1;
     __syncthreads();
-    if (sh_bad || sh_long) {
+    if (sh_bad) {
         if (tid == 0) {
             told[0] = 0;
-            told[1] = sh_bad ? DERR_RANGE : 0;
-            told[2] = (int32_t)sh_long;
+            told[1] = DERR_RANGE;
+            told[2] = 0;
         }
         return;
     }
@@ -743,13 +762,13 @@ __global__ __launch_bounds__(BK_TB) void k_bk_one(Source src, uint32_t items, in
 }
 
 // ---- host -------------------------------------------------------------------------
-static int bk_tile(int64_t n) { return n <= BK_FEW ? BK_TILE_FEW : BK_TILE; }
-static int64_t bk_tiles(int64_t n) { return n / bk_tile(n) + 1; }
+static int bk_cap(int64_t n) { return n <= BK_FEW ? BK_CAP_FEW : BK_CAP; }
+static int64_t bk_tiles(int64_t n, bool longrows) { return n / (longrows ? bk_cap(n) / 2 : bk_cap(n) - BK_ROWMAX) + 1; }
 static int64_t bk_scan_blocks(int64_t nmaj) { return ceil_div(nmaj + 1, BK_SCAN_CHUNK); }
 // words zeroed before a build: control words, the look-back states, the counts
 static int64_t bk_zero_words(int64_t n, int64_t nmaj)
 {
-    return (BK_NCTL + 2 * bk_scan_blocks(nmaj) + 2 * bk_tiles(n) + nmaj + 1 + 7) & ~(int64_t)3;
+    return (BK_NCTL + 2 * bk_scan_blocks(nmaj) + 2 * bk_tiles(n, true) + nmaj + 1 + 7) & ~(int64_t)3;
 }
 
 // The scratch: the packed entries, what is zeroed (control words, look-back
@@ -757,20 +776,21 @@ static int64_t bk_zero_words(int64_t n, int64_t nmaj)
 namespace {
 struct Scratch {
     uint64_t *packed, *st_scan, *st_tile;
-    uint32_t *ctl, *cnt, *trow, *tstart, *place;
+    uint32_t *ctl, *cnt, *place;
+    TileSets T;
     int64_t zero_words, nt, nsb;
 };
 }  // namespace
 
 static size_t scratch_bytes(int64_t n, int64_t items, int64_t nmaj)
 {
-    return 8 * (size_t)n + 4 * (size_t)items + 4 * (size_t)bk_zero_words(n, nmaj) + 8 * (size_t)(bk_tiles(n) + 1) + 80;
+    return 8 * (size_t)n + 4 * (size_t)items + 4 * (size_t)bk_zero_words(n, nmaj) + 8 * (size_t)(bk_tiles(n, false) + bk_tiles(n, true) + 2) + 80;
 }
 
 static Scratch scratch_layout(void *p, int64_t n, int64_t nmaj)
 {
     Scratch S;
-    S.nt = bk_tiles(n);
+    S.nt = bk_tiles(n, true);
     S.nsb = bk_scan_blocks(nmaj);
     S.packed = (uint64_t *)p;
     S.ctl = (uint32_t *)(S.packed + n);
@@ -780,9 +800,14 @@ static Scratch scratch_layout(void *p, int64_t n, int64_t nmaj)
     S.cnt = (uint32_t *)(S.st_tile + S.nt);
     S.cnt += ((16 - ((uintptr_t)S.cnt & 15)) & 15) / 4;
     S.zero_words = bk_zero_words(n, nmaj);
-    S.trow = S.ctl + S.zero_words;
-    S.tstart = S.trow + S.nt + 1;
-    S.place = S.tstart + S.nt + 1;
+    S.place = S.ctl + S.zero_words;
+    for (int q = 0; q < 2; q++) {
+        Tiles &t = S.T.set[q];
+        t.nt = (uint32_t)bk_tiles(n, q);
+        t.row = S.place;
+        t.first = t.row + t.nt + 1;
+        S.place = t.first + t.nt + 1;
+    }
     return S;
 }
 
@@ -793,11 +818,17 @@ size_t bucket_form_bytes(const FormMap &m, int64_t E, int64_t ndofs)
 }
 
 // Where the buckets apply: the counts are zeroed, scanned and read over all
-// rows, so a matrix of far more rows than entries keeps the sort; and a minor
-// index, a stream position and a place in a tile have to fit one 64-bit word.
+// rows, so a matrix of far more rows than entries keeps the sort; so does one of
+// more than 128 entries a row on average, more than any element's mesh here has,
+// where the counting pass waits for few counters if the stream is in no order
+// (650 000 entries in random order, whole calls by the buckets and by the sort:
+// rows of 600 721 and 645 us, of 250 696 and 649, of 120 571 and 685); and a
+// minor index, a stream position and a place in a tile have to fit one 64-bit
+// word.
 bool bucket_takes(int64_t n, int64_t nmaj, int64_t nmin)
 {
-    return n > 0 && n < INT32_MAX && nmaj <= 16 * n + 65536 && bits_for(nmin) + bits_for(n) + BK_CAP_LOG2 <= 64;
+    return n > 0 && n < INT32_MAX && nmaj <= 16 * n + 65536 && (n <= BK_ONE || n <= 128 * nmaj) &&
+           bits_for(nmin) + bits_for(n) + BK_CAP_LOG2 <= 64;
 }
 bool bucket_form_takes(const FormMap &m, int64_t E, int64_t ndofs)
 {
@@ -805,9 +836,9 @@ bool bucket_form_takes(const FormMap &m, int64_t E, int64_t ndofs)
 }
 
 template <bool SUM, bool LOAD>
-static decltype(&k_bk_tile<SUM, LOAD, BK_TILE>) tile_kernel(int64_t n)
+static decltype(&k_bk_tile<SUM, LOAD, BK_CAP>) tile_kernel(int64_t n)
 {
-    return bk_tile(n) == BK_TILE ? k_bk_tile<SUM, LOAD, BK_TILE> : k_bk_tile<SUM, LOAD, BK_TILE_FEW>;
+    return n <= BK_FEW ? k_bk_tile<SUM, LOAD, BK_CAP_FEW> : k_bk_tile<SUM, LOAD, BK_CAP>;
 }
 
 static bool one_takes(int64_t n, int64_t nmaj) { return n <= BK_ONE && nmaj <= BK_ONE_ROWS; }
@@ -818,8 +849,8 @@ static void launch_zero_scan(elfel_hip_ctx *c, const Scratch &S, bool zero, int6
         hipLaunchKernelGGL(k_bk_zero, dim3(ceil_div(S.zero_words / 4, 256)), dim3(256), 0, c->stream, (uint4 *)S.ctl,
                            S.zero_words / 4);
     else
-        hipLaunchKernelGGL(k_bk_scan, dim3((unsigned)S.nsb), dim3(BK_BLOCK), 0, c->stream, S.cnt, nmaj, (uint32_t)n,
-                           (uint32_t)S.nt, (uint32_t)bk_tile(n), S.trow, S.tstart, S.st_scan, S.ctl);
+        hipLaunchKernelGGL((n <= BK_FEW ? k_bk_scan<BK_CAP_FEW> : k_bk_scan<BK_CAP>), dim3((unsigned)S.nsb), dim3(BK_BLOCK), 0, c->stream, S.cnt, nmaj, (uint32_t)n,
+                           S.T, S.st_scan, S.ctl);
 }
 
 template <typename Source>
@@ -842,10 +873,10 @@ static int run_coo(elfel_hip_ctx *c, void *scratch, const Source &src, int64_t n
                        n, S.cnt, S.place, err);
     launch_zero_scan(c, S, false, n, nmaj);
     hipLaunchKernelGGL(k_bk_scatter<Source>, dim3(ceil_div(n, BK_BLOCK)), dim3(BK_BLOCK), 0, c->stream, src, n, S.cnt,
-                       S.place, bits, kbits, S.packed);
+                       S.place, bits, kbits, S.packed, S.ctl);
     // told: words 0-3 are the context's result's, these 4-7
     hipLaunchKernelGGL((tile_kernel<true, false>(n)), dim3((unsigned)S.nt), dim3(BK_TB), 0, c->stream, S.packed, val,
-                       (const double *)nullptr, 1u, S.cnt, S.trow, S.tstart, (uint32_t)S.nt, nmaj, bits, kbits, S.st_tile,
+                       (const double *)nullptr, 1u, S.cnt, S.T, nmaj, bits, kbits, S.st_tile,
                        S.ctl, err, o, (int32_t *)c->dscal.p + 2, (int32_t *)c->told + 4);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -993,7 +1024,7 @@ int bucket_form(elfel_hip_ctx *c, void *scratch, const FormMap &m, int64_t E, co
     auto kern = sum ? (load ? tile_kernel<true, true>(n) : tile_kernel<true, false>(n))
                     : (load ? tile_kernel<false, true>(n) : tile_kernel<false, false>(n));
     hipLaunchKernelGGL(kern, dim3((unsigned)S.nt), dim3(BK_TB), 0, c->stream, S.packed, vals, fvals, (uint32_t)m.nd, S.cnt,
-                       S.trow, S.tstart, (uint32_t)S.nt, ndofs, bits, kbits, S.st_tile, S.ctl, (int *)c->dscal.p + 1, o,
+                       S.T, ndofs, bits, kbits, S.st_tile, S.ctl, (int *)c->dscal.p + 1, o,
                        (int32_t *)c->dscal.p, (int32_t *)c->told);
     HIPCHK(c, hipGetLastError());
     tm_end(c, ELFEL_PH_REDUCE, ev);

@@ -47,66 +47,106 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v, int lane)
     return v;
 }
 
-__global__ __launch_bounds__(SC_BLOCK) void k_scan_chunks(uint32_t *data, int64_t n, uint32_t *sums)
+// Sixteen neighbouring items a work-item, four at a time (an array that does
+// not begin on 16 bytes: one by one).
+__device__ __forceinline__ void scan_load(const uint32_t *data, int64_t n, int64_t i, uint32_t *v)
 {
-    __shared__ uint32_t s[SC_CHUNK];
-    __shared__ uint32_t wsum[SC_BLOCK / 64];
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int64_t base = (int64_t)blockIdx.x * SC_CHUNK;
-    for (int i = tid; i < SC_CHUNK; i += SC_BLOCK) {
-        int64_t g = base + i;
-        s[i] = g < n ? data[g] : 0u;
+    if (i + SC_ITEMS <= n && ((uintptr_t)data & 15) == 0) {
+#pragma unroll
+        for (int k = 0; k < SC_ITEMS; k += 4) {
+            const uint4 q = *(const uint4 *)(data + i + k);
+            v[k] = q.x; v[k + 1] = q.y; v[k + 2] = q.z; v[k + 3] = q.w;
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < SC_ITEMS; k++) v[k] = i + k < n ? data[i + k] : 0u;
     }
-    __syncthreads();
-    uint32_t loc[SC_ITEMS];
-    uint32_t tsum = 0;
-    for (int k = 0; k < SC_ITEMS; k++) {
-        loc[k] = tsum;
-        tsum += s[tid * SC_ITEMS + k];
-    }
-    uint32_t inc = wave_incl_scan(tsum, lane);
-    if (lane == 63) wsum[w] = inc;
-    __syncthreads();
-    uint32_t woff = 0;
-    for (int k = 0; k < w; k++) woff += wsum[k];
-    uint32_t excl = woff + inc - tsum;
-    for (int k = 0; k < SC_ITEMS; k++) s[tid * SC_ITEMS + k] = excl + loc[k];
-    if (tid == SC_BLOCK - 1) sums[blockIdx.x] = excl + tsum;
-    __syncthreads();
-    for (int i = tid; i < SC_CHUNK; i += SC_BLOCK) {
-        int64_t g = base + i;
-        if (g < n) data[g] = s[i];
+}
+__device__ __forceinline__ void scan_store(uint32_t *data, int64_t n, int64_t i, const uint32_t *v)
+{
+    if (i + SC_ITEMS <= n && ((uintptr_t)data & 15) == 0) {
+#pragma unroll
+        for (int k = 0; k < SC_ITEMS; k += 4) *(uint4 *)(data + i + k) = make_uint4(v[k], v[k + 1], v[k + 2], v[k + 3]);
+    } else {
+#pragma unroll
+        for (int k = 0; k < SC_ITEMS; k++)
+            if (i + k < n) data[i + k] = v[k];
     }
 }
 
-__global__ void k_scan_add(uint32_t *data, int64_t n, const uint32_t *sums)
+__global__ __launch_bounds__(SC_BLOCK) void k_scan_chunks(uint32_t *data, int64_t n, uint32_t *sums)
+{
+    __shared__ uint32_t wsum[SC_BLOCK / 64];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int64_t i = (int64_t)blockIdx.x * SC_CHUNK + tid * SC_ITEMS;
+    uint32_t v[SC_ITEMS], tsum = 0;
+    scan_load(data, n, i, v);
+#pragma unroll
+    for (int k = 0; k < SC_ITEMS; k++) {
+        const uint32_t x = v[k];
+        v[k] = tsum;
+        tsum += x;
+    }
+    const uint32_t inc = wave_incl_scan(tsum, lane);
+    if (lane == 63) wsum[w] = inc;
+    __syncthreads();
+    uint32_t before = inc - tsum;
+    for (int k = 0; k < w; k++) before += wsum[k];
+#pragma unroll
+    for (int k = 0; k < SC_ITEMS; k++) v[k] += before;
+    scan_store(data, n, i, v);
+    if (tid == SC_BLOCK - 1) sums[blockIdx.x] = before + tsum;
+}
+
+// The sums of the chunks before a chunk added to it; each workgroup sums them
+// for itself, up to SC_SUMS of them.
+#define SC_SUMS 4096
+__global__ __launch_bounds__(SC_BLOCK) void k_scan_add(uint32_t *data, int64_t n, const uint32_t *sums, uint32_t *total)
+{
+    __shared__ uint32_t wsum[SC_BLOCK / 64];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, b = blockIdx.x;
+    const int64_t i = (int64_t)b * SC_CHUNK + tid * SC_ITEMS;
+    uint32_t v[SC_ITEMS], s = 0;
+    scan_load(data, n, i, v);
+    for (int k = tid; k < b; k += SC_BLOCK) s += sums[k];
+    for (int d = 32; d > 0; d >>= 1) s += __shfl_xor(s, d, 64);
+    if (lane == 0) wsum[w] = s;
+    __syncthreads();
+    s = 0;
+    for (int k = 0; k < SC_BLOCK / 64; k++) s += wsum[k];
+#pragma unroll
+    for (int k = 0; k < SC_ITEMS; k++) v[k] += s;
+    if (b != 0) scan_store(data, n, i, v);
+    if (total && b == (int)gridDim.x - 1 && tid == 0) *total = s + sums[b];
+}
+
+// The same with the sums already scanned.
+__global__ void k_scan_add_scanned(uint32_t *data, int64_t n, const uint32_t *sums)
 {
     int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (g < n) data[g] += sums[g / SC_CHUNK];
 }
 
-__global__ void k_copy_u32(const uint32_t *src, uint32_t *dst) { *dst = *src; }
-
-// total_dev (optional) receives the sum of all n inputs.
+// total_dev (optional) receives the sum of all n inputs.  One launch up to a
+// chunk, two up to SC_SUMS chunks (16.8 million items): the chunk sums scanned
+// in a launch of their own took 6 us and its gap more at every size.
 static int scan_rec(elfel_hip_ctx *c, uint32_t *data, int64_t n, uint32_t *tmp, int64_t tmp_cap,
                     uint32_t *total_dev)
 {
     if (n <= 0) return 0;
     int64_t nb = (n + SC_CHUNK - 1) / SC_CHUNK;
     if (nb + 1 > tmp_cap) return set_err(c, ELFEL_EINVAL, "scan scratch too small");
-    uint32_t *sums = tmp;
+    uint32_t *sums = nb == 1 && total_dev ? total_dev : tmp;
     hipLaunchKernelGGL(k_scan_chunks, dim3((unsigned)nb), dim3(SC_BLOCK), 0, c->stream, data, n, sums);
     HIPCHK(c, hipGetLastError());
-    if (nb > 1) {
-        // sums[nb] receives the grand total via the recursive call.
+    if (nb > SC_SUMS) {
         int rc = scan_rec(c, sums, nb, tmp + nb + 1, tmp_cap - nb - 1, total_dev);
         if (rc) return rc;
-        hipLaunchKernelGGL(k_scan_add, dim3(ceil_div(n, 256)), dim3(256), 0, c->stream, data, n, sums);
-        HIPCHK(c, hipGetLastError());
-    } else if (total_dev) {
-        hipLaunchKernelGGL(k_copy_u32, dim3(1), dim3(1), 0, c->stream, sums, total_dev);
-        HIPCHK(c, hipGetLastError());
+        hipLaunchKernelGGL(k_scan_add_scanned, dim3(ceil_div(n, 256)), dim3(256), 0, c->stream, data, n, sums);
+    } else if (nb > 1) {
+        hipLaunchKernelGGL(k_scan_add, dim3((unsigned)nb), dim3(SC_BLOCK), 0, c->stream, data, n, sums, total_dev);
     }
+    HIPCHK(c, hipGetLastError());
     return 0;
 }
 

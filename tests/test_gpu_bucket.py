@@ -2,8 +2,8 @@
 edges of its tiles, against the oracle's sparse(): pattern and values bit for
 bit (tolerance 0, the same sums in the same order).  Up to 6144 entries and 8191
 rows are one workgroup's; 1536 entries start in a tile, 3584 of a stream of more
-than 393216; rows of up to 512 are held, longer ones and matrices of far more
-rows than entries take the sort."""
+than 393216, with rows of up to 512; with one of up to 1024, or 2048, as many;
+longer ones and matrices of far more rows than entries take the sort."""
 import numpy as np
 import pytest
 
@@ -42,15 +42,22 @@ def _case(name, rng):
     if name.startswith("tiled row="):
         k = int(name[10:])
         return (*_rows([3] * 2500 + [k] + [0] * 7 + [5] * 300, max(k // 2, 1), rng), 2808, max(k // 2, 1))
+    if name.startswith("large row="):
+        k = int(name[10:])
+        return (*_rows([40] * 5000 + [k] + [0] * 7 + [41] * 5000, max(k // 2, 1), rng), 10008, max(k // 2, 1))
     if name.startswith("row="):  # one long row between short ones, and a tile that it straddles
         k = int(name[4:])
         return (*_rows([3] * 500 + [k] + [0] * 7 + [5] * 300, max(k // 2, 1), rng), 808, max(k // 2, 1))
     if name == "long rows side by side":  # every tile at its largest
         return (*_rows([511, 1024, 1, 512, 512, 512, 512, 511, 1][2:], 600, rng), 7, 600)
     if name == "long rows in tiles":
-        return (*_rows([512, 512, 512, 511, 1] * 4 + [512], 600, rng), 21, 600)
+        return (*_rows([512, 512, 512, 511, 1] * 4 + [512] + [1] * 40, 600, rng), 61, 600)
+    if name == "longest rows":
+        return (*_rows([1024, 1023, 1] * 3 + [1024] * 4 + [1] * 40, 900, rng), 53, 900)
+    if name == "longest rows, many":
+        return (*_rows([2048, 2047, 1] * 30 + [2048] * 150 + [1] * 2000, 1500, rng), 2240, 1500)
     if name == "long rows, many":
-        return (*_rows([512] * 5 + [511, 1] + [512] * 830 + [3] * 20, 700, rng), 857, 700)
+        return (*_rows([512] * 5 + [511, 1] + [512] * 830 + [3] * 1020, 700, rng), 1857, 700)
     if name == "empty ends":
         return (*_rows([0] * 9000 + [2] * 50 + [0] * 9000, 60, rng), 18050, 60)
     if name == "one entry":
@@ -69,7 +76,8 @@ def _case(name, rng):
 
 CASES = ["many=393216", "many=393217", "many=401408", "long rows, many", "n=1535", "n=1536", "n=1537", "n=2048", "n=3072", "n=6143", "n=6144", "n=6145", "n=7679",
          "n=7680", "n=7681", "n=9001", "rows=8190", "rows=8191", "rows=8192", "tiled row=511", "tiled row=512",
-         "tiled row=513", "long rows in tiles", "row=511", "row=512", "row=513", "row=1600",
+         "tiled row=513", "tiled row=1023", "tiled row=1024", "tiled row=1025", "large row=513", "large row=2047", "large row=2048",
+         "large row=2049", "longest rows", "longest rows, many", "long rows in tiles", "row=511", "row=512", "row=513", "row=1600",
          "long rows side by side", "empty ends", "one entry", "one row", "two rows, all duplicates",
          "more rows than entries", "last columns"]
 
@@ -119,10 +127,11 @@ def test_bucket_build_refuses_then_works(ctx):
 @pytest.mark.parametrize("layout", [L.CSR, L.CSC])
 def test_element_stream_at_the_longest_row(ctx, method, layout):
     """A T3 fan's centre row has 3 K entries: 170 and 171 elements lie either
-    side of the 512 that a tile holds.  One context, so that the answer for one
+    side of 512 entries, 341 and 342 of the 1024 of a small tile.  One context, so that the answer for one
     mesh must not outlive it, with and without a wait, and a dof that two nodes
     (hence an element's two local dofs) share."""
-    for K, tie in ((170, False), (171, False), (40, True), (170, False), (171, True), (30, False)):
+    for K, tie in ((170, False), (171, False), (40, True), (170, False), (171, True), (30, False), (341, False), (342, True), (341, True),
+                   (342, False), (30, True)):
         conn, xy = fan_mesh(K, rings=2)
         dn = np.random.default_rng(K).permutation(xy.shape[0]) + 1
         if tie:

@@ -77,3 +77,10 @@ def test_number_dofs_c5_size(ctx):
     dt = time.perf_counter() - t0
     assert np.array_equal(dev, f.dofnums)
     print(f"number_dofs {f.isdatum.size} dofs: {dt * 1e3:.1f} ms (host round trip included)")
+
+
+@pytest.mark.parametrize("n", [1, 4094, 4095, 4096, 4097, 8191, 8192, 12289, 1 << 20])
+def test_number_dofs_at_the_chunks_of_the_scan(ctx, n):
+    flags = [_rng_flags(np.random.default_rng(n), n, 1, 0.3)]
+    for d, r in zip(ctx.number_dofs(flags), O.numberdofs(flags)):
+        assert np.array_equal(d, r)
