@@ -31,18 +31,19 @@
 #define BK_BLOCK 256
 #define BK_TB 1024                  // work-items of a tile
 #define BK_CAP 4096                 // entries that a tile holds
-#define BK_CAP_FEW 2048             // ... of a stream of at most BK_FEW entries
+#define BK_CAP_FEW 2048             // ... of a stream of at most BK_FEW entries, or of so many that a place in a tile has 11 bits
 #define BK_ROWMAX 512               // room for the last row's overhang, the rest is for those that start in the tile;
                                     // with a longer row, half and half; one longer than half goes to the sort
 #define BK_FEW (256 * 1536)
 #define BK_CAP_LOG2 12
+#define BK_CAP_FEW_LOG2 11
 #define BK_COUNT_ITEMS 2            // entries per work-item of the counting pass
 #define BK_HASH_LOG2 10             // its LDS slots, twice its entries
 #define BK_HASH (1 << BK_HASH_LOG2)
 #define BK_SCAN_ITEMS 16
 #define BK_SCAN_CHUNK (BK_BLOCK * BK_SCAN_ITEMS)
 
-static_assert(BK_CAP <= 1 << BK_CAP_LOG2, "a place in a tile has BK_CAP_LOG2 bits");
+static_assert(BK_CAP <= 1 << BK_CAP_LOG2 && BK_CAP_FEW <= 1 << BK_CAP_FEW_LOG2, "the bits of a place in a tile");
 static_assert(BK_HASH >= 2 * BK_BLOCK * BK_COUNT_ITEMS, "the hash of the counting pass is at most half full");
 
 // ---- decoupled look-back -------------------------------------------------------
@@ -762,13 +763,18 @@ __global__ __launch_bounds__(BK_TB) void k_bk_one(Source src, uint32_t items, in
 }
 
 // ---- host -------------------------------------------------------------------------
-static int bk_cap(int64_t n) { return n <= BK_FEW ? BK_CAP_FEW : BK_CAP; }
-static int64_t bk_tiles(int64_t n, bool longrows) { return n / (longrows ? bk_cap(n) / 2 : bk_cap(n) - BK_ROWMAX) + 1; }
+// (heat Q4 4096x4096, 268 million entries, is one bit over the larger tiles: the
+// plain assembly takes 30.0 ms by the sort, 8.7 with the smaller ones)
+static int bk_cap(int64_t n, int64_t nmin)
+{
+    return n <= BK_FEW || bits_for(nmin) + bits_for(n) + BK_CAP_LOG2 > 64 ? BK_CAP_FEW : BK_CAP;
+}
+static int64_t bk_tiles(int64_t n, int cap, bool longrows) { return n / (longrows ? cap / 2 : cap - BK_ROWMAX) + 1; }
 static int64_t bk_scan_blocks(int64_t nmaj) { return ceil_div(nmaj + 1, BK_SCAN_CHUNK); }
 // words zeroed before a build: control words, the look-back states, the counts
 static int64_t bk_zero_words(int64_t n, int64_t nmaj)
 {
-    return (BK_NCTL + 2 * bk_scan_blocks(nmaj) + 2 * bk_tiles(n, true) + nmaj + 1 + 7) & ~(int64_t)3;
+    return (BK_NCTL + 2 * bk_scan_blocks(nmaj) + 2 * bk_tiles(n, BK_CAP_FEW, true) + nmaj + 1 + 7) & ~(int64_t)3;
 }
 
 // The scratch: the packed entries, what is zeroed (control words, look-back
@@ -778,19 +784,22 @@ struct Scratch {
     uint64_t *packed, *st_scan, *st_tile;
     uint32_t *ctl, *cnt, *place;
     TileSets T;
+    int cap;
     int64_t zero_words, nt, nsb;
 };
 }  // namespace
 
 static size_t scratch_bytes(int64_t n, int64_t items, int64_t nmaj)
 {
-    return 8 * (size_t)n + 4 * (size_t)items + 4 * (size_t)bk_zero_words(n, nmaj) + 8 * (size_t)(bk_tiles(n, false) + bk_tiles(n, true) + 2) + 80;
+    return 8 * (size_t)n + 4 * (size_t)items + 4 * (size_t)bk_zero_words(n, nmaj) + 
+           8 * (size_t)(bk_tiles(n, BK_CAP_FEW, false) + bk_tiles(n, BK_CAP_FEW, true) + 2) + 80;
 }
 
-static Scratch scratch_layout(void *p, int64_t n, int64_t nmaj)
+static Scratch scratch_layout(void *p, int64_t n, int64_t nmaj, int64_t nmin)
 {
     Scratch S;
-    S.nt = bk_tiles(n, true);
+    S.cap = bk_cap(n, nmin);
+    S.nt = bk_tiles(n, S.cap, true);
     S.nsb = bk_scan_blocks(nmaj);
     S.packed = (uint64_t *)p;
     S.ctl = (uint32_t *)(S.packed + n);
@@ -803,7 +812,7 @@ static Scratch scratch_layout(void *p, int64_t n, int64_t nmaj)
     S.place = S.ctl + S.zero_words;
     for (int q = 0; q < 2; q++) {
         Tiles &t = S.T.set[q];
-        t.nt = (uint32_t)bk_tiles(n, q);
+        t.nt = (uint32_t)bk_tiles(n, S.cap, q);
         t.row = S.place;
         t.first = t.row + t.nt + 1;
         S.place = t.first + t.nt + 1;
@@ -828,7 +837,7 @@ size_t bucket_form_bytes(const FormMap &m, int64_t E, int64_t ndofs)
 bool bucket_takes(int64_t n, int64_t nmaj, int64_t nmin)
 {
     return n > 0 && n < INT32_MAX && nmaj <= 16 * n + 65536 && (n <= BK_ONE || n <= 128 * nmaj) &&
-           bits_for(nmin) + bits_for(n) + BK_CAP_LOG2 <= 64;
+           bits_for(nmin) + bits_for(n) + BK_CAP_FEW_LOG2 <= 64;
 }
 bool bucket_form_takes(const FormMap &m, int64_t E, int64_t ndofs)
 {
@@ -836,9 +845,9 @@ bool bucket_form_takes(const FormMap &m, int64_t E, int64_t ndofs)
 }
 
 template <bool SUM, bool LOAD>
-static decltype(&k_bk_tile<SUM, LOAD, BK_CAP>) tile_kernel(int64_t n)
+static decltype(&k_bk_tile<SUM, LOAD, BK_CAP>) tile_kernel(const Scratch &S)
 {
-    return n <= BK_FEW ? k_bk_tile<SUM, LOAD, BK_CAP_FEW> : k_bk_tile<SUM, LOAD, BK_CAP>;
+    return S.cap == BK_CAP ? k_bk_tile<SUM, LOAD, BK_CAP> : k_bk_tile<SUM, LOAD, BK_CAP_FEW>;
 }
 
 static bool one_takes(int64_t n, int64_t nmaj) { return n <= BK_ONE && nmaj <= BK_ONE_ROWS; }
@@ -849,7 +858,8 @@ static void launch_zero_scan(elfel_hip_ctx *c, const Scratch &S, bool zero, int6
         hipLaunchKernelGGL(k_bk_zero, dim3(ceil_div(S.zero_words / 4, 256)), dim3(256), 0, c->stream, (uint4 *)S.ctl,
                            S.zero_words / 4);
     else
-        hipLaunchKernelGGL((n <= BK_FEW ? k_bk_scan<BK_CAP_FEW> : k_bk_scan<BK_CAP>), dim3((unsigned)S.nsb), dim3(BK_BLOCK), 0, c->stream, S.cnt, nmaj, (uint32_t)n,
+        hipLaunchKernelGGL((S.cap == BK_CAP ? k_bk_scan<BK_CAP> : k_bk_scan<BK_CAP_FEW>), dim3((unsigned)S.nsb),
+                           dim3(BK_BLOCK), 0, c->stream, S.cnt, nmaj, (uint32_t)n,
                            S.T, S.st_scan, S.ctl);
 }
 
@@ -857,7 +867,7 @@ template <typename Source>
 static int run_coo(elfel_hip_ctx *c, void *scratch, const Source &src, int64_t n, const double *val, int64_t nmaj,
                    int64_t nmin, const BucketOut &o)
 {
-    const Scratch S = scratch_layout(scratch, n, nmaj);
+    const Scratch S = scratch_layout(scratch, n, nmaj, nmin);
     const int kbits = bits_for(n), bits = kbits + bits_for(nmin);
     int *err = (int *)c->dscal.p + 1;
     if (one_takes(n, nmaj)) {
@@ -875,7 +885,7 @@ static int run_coo(elfel_hip_ctx *c, void *scratch, const Source &src, int64_t n
     hipLaunchKernelGGL(k_bk_scatter<Source>, dim3(ceil_div(n, BK_BLOCK)), dim3(BK_BLOCK), 0, c->stream, src, n, S.cnt,
                        S.place, bits, kbits, S.packed, S.ctl);
     // told: words 0-3 are the context's result's, these 4-7
-    hipLaunchKernelGGL((tile_kernel<true, false>(n)), dim3((unsigned)S.nt), dim3(BK_TB), 0, c->stream, S.packed, val,
+    hipLaunchKernelGGL((tile_kernel<true, false>(S)), dim3((unsigned)S.nt), dim3(BK_TB), 0, c->stream, S.packed, val,
                        (const double *)nullptr, 1u, S.cnt, S.T, nmaj, bits, kbits, S.st_tile,
                        S.ctl, err, o, (int32_t *)c->dscal.p + 2, (int32_t *)c->told + 4);
     HIPCHK(c, hipGetLastError());
@@ -996,7 +1006,7 @@ int bucket_form(elfel_hip_ctx *c, void *scratch, const FormMap &m, int64_t E, co
                 const double *vals, const double *fvals, const BucketOut &o)
 {
     const int64_t n = E * m.nmat;
-    const Scratch S = scratch_layout(scratch, n, ndofs);
+    const Scratch S = scratch_layout(scratch, n, ndofs, ndofs);
     const int kbits = bits_for(n), bits = kbits + bits_for(ndofs);
     const bool sum = vals != nullptr, load = m.nvec > 0;
     hipEvent_t ev = nullptr;
@@ -1021,8 +1031,8 @@ int bucket_form(elfel_hip_ctx *c, void *scratch, const FormMap &m, int64_t E, co
     HIPCHK(c, hipGetLastError());
     tm_end(c, ELFEL_PH_SORT, ev);
     tm_begin(c, ELFEL_PH_REDUCE, &ev);
-    auto kern = sum ? (load ? tile_kernel<true, true>(n) : tile_kernel<true, false>(n))
-                    : (load ? tile_kernel<false, true>(n) : tile_kernel<false, false>(n));
+    auto kern = sum ? (load ? tile_kernel<true, true>(S) : tile_kernel<true, false>(S))
+                    : (load ? tile_kernel<false, true>(S) : tile_kernel<false, false>(S));
     hipLaunchKernelGGL(kern, dim3((unsigned)S.nt), dim3(BK_TB), 0, c->stream, S.packed, vals, fvals, (uint32_t)m.nd, S.cnt,
                        S.T, ndofs, bits, kbits, S.st_tile, S.ctl, (int *)c->dscal.p + 1, o,
                        (int32_t *)c->dscal.p, (int32_t *)c->told);
