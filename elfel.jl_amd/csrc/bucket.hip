@@ -14,6 +14,7 @@
 //   k_bk_scan     exclusive scan of the counts (one pass, decoupled look-back),
 //                 and the first row of every tile
 //   k_bk_scatter  (minor, stream position) of every entry into its row
+//   k_bk_items    for element blocks of equal rows, the items alone
 //   k_bk_tile     per tile: rank every entry within its row, find the runs,
 //                 sum them, and write the row pointers, indices and values at
 //                 the place that a second look-back over the tiles gives
@@ -346,6 +347,44 @@ __global__ __launch_bounds__(BK_BLOCK) void k_bk_scatter_form(FormMap map, int64
     packed[(int64_t)s + place[ea] + b] = ((uint64_t)s << bits) | ((uint64_t)(uint32_t)edof[e * ND + b] << kbits) | k;
 }
 
+// Where every item of an element stream is nd entries wide, the items alone go
+// into their rows, 4 bytes in place of 8 nd, and the tile forms the words from
+// them and the element dofs (scatter and tile: elasticity T6 200^2 152 -> 130
+// us, T4 36^3 97 -> 93; plain assembly of elasticity T6 400^2 0.89 -> 0.73 ms).
+__global__ __launch_bounds__(BK_BLOCK) void k_bk_items(int64_t items, uint32_t nd, const int32_t *__restrict__ edof,
+                                                       const uint32_t *__restrict__ start,
+                                                       const uint32_t *__restrict__ place, int32_t *__restrict__ list,
+                                                       const uint32_t *__restrict__ ctl)
+{
+    const int64_t x = (int64_t)blockIdx.x * BK_BLOCK + threadIdx.x;
+    if (x >= items || ctl[BK_TOOLONG] != 0) return;
+    list[(start[edof[x]] + place[x]) / nd] = (int32_t)x;
+}
+
+// Entry P of the rows, as a tile whose first entry is s0 compares it: the row
+// begin in the tile, the minor index, the stream position.
+struct PackedWords {
+    const uint64_t *packed;
+    __device__ __forceinline__ uint64_t get(uint32_t P, uint32_t s0, const uint32_t *, int bits, int) const
+    {
+        return packed[P] - ((uint64_t)s0 << bits);
+    }
+};
+struct ItemWords {
+    const int32_t *list, *edof;
+    double inv;  // 1 / nd
+    uint32_t nd;
+    int csc;
+    __device__ __forceinline__ uint32_t over(uint32_t x) const { return (uint32_t)(((double)x + 0.5) * inv); }  // x / nd
+    __device__ __forceinline__ uint64_t get(uint32_t P, uint32_t s0, const uint32_t *start, int bits, int kbits) const
+    {
+        const uint32_t slot = over(P), b = P - slot * nd, ea = (uint32_t)list[slot], e = over(ea), a = ea - e * nd;
+        const uint32_t minor = (uint32_t)edof[e * nd + b], row = start[edof[ea]];
+        const uint64_t k = (uint64_t)e * (nd * nd) + (csc ? b + nd * a : a + nd * b);
+        return ((uint64_t)(row - s0) << bits) | ((uint64_t)minor << kbits) | k;
+    }
+};
+
 // acc + v[j] + ... + v[e - 1], left to right; four loads at a time
 __device__ __forceinline__ double run_sum(const double *v, int j, int e, double acc)
 {
@@ -394,7 +433,8 @@ __device__ __forceinline__ int bits_between(const uint64_t *m, int p, int e)
 // order; they are gathered with the values and summed by the work-item of that
 // run (one work-item a row that looked for the run and then loaded them one
 // after the other: 4.5 million entries 108 us, now 84).
-// A tile's rows, their entries in sk (and kr: entry q * BK_TB + tid); ~0 past m.
+//
+// tile_rows: the rows of a tile, their entries in sk (and kr: entry q * BK_TB + tid); ~0 past m.
 // Gives back the runs up to the tile's end.  place: where the tile's runs begin.
 template <bool SUM, bool LOAD, int CAP, typename Place>
 __device__ __forceinline__ uint32_t tile_rows(uint64_t *sk, uint64_t *ss, uint16_t *se, uint64_t *hm, uint64_t *dm,
@@ -579,8 +619,8 @@ struct AfterTiles {
     __device__ __forceinline__ uint32_t wait(uint32_t total) const { return lb_wait(st, t, total); }
 };
 
-template <bool SUM, bool LOAD, int CAP>
-__global__ __launch_bounds__(BK_TB) void k_bk_tile(const uint64_t *__restrict__ packed, const double *__restrict__ vals,
+template <bool SUM, bool LOAD, int CAP, typename Words>
+__global__ __launch_bounds__(BK_TB) void k_bk_tile(Words words, const double *__restrict__ vals,
                                                    const double *__restrict__ fvals, uint32_t nd,
                                                    const uint32_t *__restrict__ start, TileSets T, int64_t nmaj,
                                                    int bits, int kbits, uint64_t *__restrict__ st,
@@ -615,12 +655,11 @@ __global__ __launch_bounds__(BK_TB) void k_bk_tile(const uint64_t *__restrict__ 
     const int64_t row0 = trow[t], row1 = trow[t + 1];
     const uint32_t s0 = tstart[t];
     const int m = (int)(tstart[t + 1] - s0);  // <= CAP
-    const uint64_t rebase = (uint64_t)s0 << bits;
     uint64_t kr[ROUNDS];
 #pragma unroll
     for (int q = 0; q < ROUNDS; q++) {
         const int p = q * BK_TB + tid;
-        kr[q] = p < m ? packed[(int64_t)s0 + p] - rebase : ~0ull;
+        kr[q] = p < m ? words.get(s0 + (uint32_t)p, s0, start, bits, kbits) : ~0ull;
     }
 #pragma unroll
     for (int q = 0; q < ROUNDS; q++) sk[q * BK_TB + tid] = kr[q];
@@ -764,7 +803,7 @@ __global__ __launch_bounds__(BK_TB) void k_bk_one(Source src, uint32_t items, in
 
 // ---- host -------------------------------------------------------------------------
 // (heat Q4 4096x4096, 268 million entries, is one bit over the larger tiles: the
-// plain assembly takes 30.0 ms by the sort, 8.7 with the smaller ones)
+// plain assembly takes 30.0 ms by the sort, 8.0 with the smaller ones)
 static int bk_cap(int64_t n, int64_t nmin)
 {
     return n <= BK_FEW || bits_for(nmin) + bits_for(n) + BK_CAP_LOG2 > 64 ? BK_CAP_FEW : BK_CAP;
@@ -844,10 +883,13 @@ bool bucket_form_takes(const FormMap &m, int64_t E, int64_t ndofs)
     return E * m.nd < INT32_MAX && bucket_takes(E * m.nmat, ndofs, ndofs);
 }
 
-template <bool SUM, bool LOAD>
-static decltype(&k_bk_tile<SUM, LOAD, BK_CAP>) tile_kernel(const Scratch &S)
+template <bool SUM, bool LOAD, typename Words>
+static void launch_tiles(elfel_hip_ctx *c, const Scratch &S, const Words &words, const double *vals, const double *fvals, int nd,
+                         int64_t nmaj, int bits, int kbits, const BucketOut &o, int32_t *nnz_dev, int32_t *told)
 {
-    return S.cap == BK_CAP ? k_bk_tile<SUM, LOAD, BK_CAP> : k_bk_tile<SUM, LOAD, BK_CAP_FEW>;
+    hipLaunchKernelGGL((S.cap == BK_CAP ? k_bk_tile<SUM, LOAD, BK_CAP, Words> : k_bk_tile<SUM, LOAD, BK_CAP_FEW, Words>),
+                       dim3((unsigned)S.nt), dim3(BK_TB), 0, c->stream, words, vals, fvals, (uint32_t)nd, S.cnt, S.T, nmaj, bits,
+                       kbits, S.st_tile, S.ctl, (const int *)c->dscal.p + 1, o, nnz_dev, told);
 }
 
 static bool one_takes(int64_t n, int64_t nmaj) { return n <= BK_ONE && nmaj <= BK_ONE_ROWS; }
@@ -885,9 +927,8 @@ static int run_coo(elfel_hip_ctx *c, void *scratch, const Source &src, int64_t n
     hipLaunchKernelGGL(k_bk_scatter<Source>, dim3(ceil_div(n, BK_BLOCK)), dim3(BK_BLOCK), 0, c->stream, src, n, S.cnt,
                        S.place, bits, kbits, S.packed, S.ctl);
     // told: words 0-3 are the context's result's, these 4-7
-    hipLaunchKernelGGL((tile_kernel<true, false>(S)), dim3((unsigned)S.nt), dim3(BK_TB), 0, c->stream, S.packed, val,
-                       (const double *)nullptr, 1u, S.cnt, S.T, nmaj, bits, kbits, S.st_tile,
-                       S.ctl, err, o, (int32_t *)c->dscal.p + 2, (int32_t *)c->told + 4);
+    launch_tiles<true, false>(c, S, PackedWords{S.packed}, val, nullptr, 1, nmaj, bits, kbits, o, (int32_t *)c->dscal.p + 2,
+                              (int32_t *)c->told + 4);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return 0;
@@ -989,7 +1030,7 @@ int form_keys(elfel_hip_ctx *c, const FormMap &m, int64_t E, const int32_t *edof
 
 template <int ND>
 static void launch_form(elfel_hip_ctx *c, const Scratch &S, const FormMap &m, int64_t E, const int32_t *edof,
-                        int64_t ndofs, int bits, int kbits)
+                        int64_t ndofs, int bits, int kbits, bool square)
 {
     FormSource<ND> src{edof, {m.ncol[0], m.ncol[ND - 1]}, ND};
     for (int a = ND - 1; a > 0 && m.ncol[a] != m.ncol[0]; a--) src.nfull = a;
@@ -998,8 +1039,12 @@ static void launch_form(elfel_hip_ctx *c, const Scratch &S, const FormMap &m, in
     hipLaunchKernelGGL(k_bk_count<FormSource<ND>>, dim3(ceil_div(items, BK_BLOCK * BK_COUNT_ITEMS)), dim3(BK_BLOCK), 0,
                        c->stream, src, items, S.cnt, S.place, (int *)c->dscal.p + 1);
     launch_zero_scan(c, S, false, E * m.nmat, ndofs);
-    hipLaunchKernelGGL(k_bk_scatter_form<ND>, dim3((unsigned)((n2 + BK_BLOCK - 1) / BK_BLOCK)), dim3(BK_BLOCK), 0,
-                       c->stream, m, n2, edof, S.cnt, S.place, bits, kbits, S.packed);
+    if (square)
+        hipLaunchKernelGGL(k_bk_items, dim3(ceil_div(items, BK_BLOCK)), dim3(BK_BLOCK), 0, c->stream, items, (uint32_t)ND, edof,
+                           S.cnt, S.place, (int32_t *)S.packed, S.ctl);
+    else
+        hipLaunchKernelGGL(k_bk_scatter_form<ND>, dim3((unsigned)((n2 + BK_BLOCK - 1) / BK_BLOCK)), dim3(BK_BLOCK), 0,
+                           c->stream, m, n2, edof, S.cnt, S.place, bits, kbits, S.packed);
 }
 
 int bucket_form(elfel_hip_ctx *c, void *scratch, const FormMap &m, int64_t E, const int32_t *edof, int64_t ndofs,
@@ -1022,8 +1067,13 @@ int bucket_form(elfel_hip_ctx *c, void *scratch, const FormMap &m, int64_t E, co
         tm_end(c, ELFEL_PH_REDUCE, ev);
         return 0;
     }
+    // (a block of nd x nd entries in either order: form_square's)
+    bool square = m.nmat == m.nd * m.nd;
+    const int csc = m.pos[1] == 1;
+    for (int a = 0; a < m.nd; a++)
+        for (int b = 0; square && b < m.nd; b++) square = m.pos[a * m.nd + b] == (csc ? b + m.nd * a : a + m.nd * b);
     switch (m.nd) {
-#define F(N) case N: launch_form<N>(c, S, m, E, edof, ndofs, bits, kbits); break
+#define F(N) case N: launch_form<N>(c, S, m, E, edof, ndofs, bits, kbits, square); break
         F(2); F(3); F(4); F(6); F(8); F(9); F(11); F(12); F(15);
 #undef F
     default: return set_err(c, ELFEL_ENOTSUP, "internal: element dof count without a bucket kernel");
@@ -1031,11 +1081,15 @@ int bucket_form(elfel_hip_ctx *c, void *scratch, const FormMap &m, int64_t E, co
     HIPCHK(c, hipGetLastError());
     tm_end(c, ELFEL_PH_SORT, ev);
     tm_begin(c, ELFEL_PH_REDUCE, &ev);
-    auto kern = sum ? (load ? tile_kernel<true, true>(S) : tile_kernel<true, false>(S))
-                    : (load ? tile_kernel<false, true>(S) : tile_kernel<false, false>(S));
-    hipLaunchKernelGGL(kern, dim3((unsigned)S.nt), dim3(BK_TB), 0, c->stream, S.packed, vals, fvals, (uint32_t)m.nd, S.cnt,
-                       S.T, ndofs, bits, kbits, S.st_tile, S.ctl, (int *)c->dscal.p + 1, o,
-                       (int32_t *)c->dscal.p, (int32_t *)c->told);
+    int32_t *nnz_dev = (int32_t *)c->dscal.p, *told = (int32_t *)c->told;
+    const ItemWords items{(const int32_t *)S.packed, edof, 1.0 / m.nd, (uint32_t)m.nd, csc};
+    const PackedWords packed{S.packed};
+#define TILES(SUM, LOAD, W) launch_tiles<SUM, LOAD>(c, S, W, vals, fvals, m.nd, ndofs, bits, kbits, o, nnz_dev, told)
+    if (load && !square) return set_err(c, ELFEL_ENOTSUP, "internal: a load vector without a square element block");
+    if (load) sum ? TILES(true, true, items) : TILES(false, true, items);
+    else if (square) sum ? TILES(true, false, items) : TILES(false, false, items);
+    else sum ? TILES(true, false, packed) : TILES(false, false, packed);
+#undef TILES
     HIPCHK(c, hipGetLastError());
     tm_end(c, ELFEL_PH_REDUCE, ev);
     return 0;
