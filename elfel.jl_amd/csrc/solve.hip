@@ -47,6 +47,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "nine.h"
 
 int env_int(const char *name, int dflt);  // reuse.hip
 
@@ -201,7 +202,6 @@ __global__ void k_sell_uniform(int64_t nfree, int64_t nslices, const uint32_t *_
 // below and one above -- the three grid rows of a quadrilateral's or triangle's
 // stencil; a row may lack any of the nine.  The record is the runs' first
 // offsets; nslow counts the slices that have no such runs.  One wave per slice.
-#define RES_W 9
 __global__ void k_sell_rec(int64_t nfree, int64_t nslices, const uint32_t *__restrict__ off,
                            const int16_t *__restrict__ col, const uint32_t *__restrict__ len, int2 *__restrict__ rec,
                            uint32_t *__restrict__ nslow)
@@ -211,27 +211,17 @@ __global__ void k_sell_rec(int64_t nfree, int64_t nslices, const uint32_t *__res
     if (s >= nslices) return;
     const int64_t i = s * 64 + lane;
     const uint32_t o = off[s], w = i < nfree ? len[i] : 0u;
-    const int32_t NONE = 1 << 20;
-    int32_t lo = NONE, lo_end = -NONE, hi = NONE, hi_end = -NONE;  // offsets below -1 and above 1
-    for (uint32_t k = 0; k < w; k++) {
-        const int32_t d = col[(size_t)o + (size_t)k * 64 + lane];
-        if (d < -1) {
-            lo = min(lo, d);
-            lo_end = max(lo_end, d);
-        } else if (d > 1) {
-            hi = min(hi, d);
-            hi_end = max(hi_end, d);
-        }
-    }
+    NineRuns R;
+    for (uint32_t k = 0; k < w; k++) R.add(col[(size_t)o + (size_t)k * 64 + lane]);
     for (int t = 32; t > 0; t >>= 1) {
-        lo = min(lo, __shfl_xor(lo, t, 64));
-        hi = min(hi, __shfl_xor(hi, t, 64));
-        lo_end = max(lo_end, __shfl_xor(lo_end, t, 64));
-        hi_end = max(hi_end, __shfl_xor(hi_end, t, 64));
+        R.lo = min(R.lo, __shfl_xor(R.lo, t, 64));
+        R.hi = min(R.hi, __shfl_xor(R.hi, t, 64));
+        R.lo_end = max(R.lo_end, __shfl_xor(R.lo_end, t, 64));
+        R.hi_end = max(R.hi_end, __shfl_xor(R.hi_end, t, 64));
     }
     if (lane == 0) {
-        rec[s] = make_int2(lo, hi);  // NONE: no entry is there, and what is read for it meets zeros
-        if (lo_end - lo > 2 || hi_end - hi > 2) atomicAdd(nslow, 1u);
+        rec[s] = make_int2(R.lo, R.hi);  // NINE_NONE: no entry is there, and what is read for it meets zeros
+        if (!R.fit()) atomicAdd(nslow, 1u);
     }
 }
 
@@ -971,11 +961,7 @@ __device__ __forceinline__ void nine_entries(const uint32_t *__restrict__ off, c
         const size_t at = (size_t)o + (size_t)q * 64 + lane;
         const T x = val[at];  // zero in the padding of a short row, whose column is its own
         const int32_t d = col[at];
-        if (x != T(0) || d != 0) {
-#pragma unroll
-            for (int j = 0; j < RES_W; j++)
-                if (d == (j < 3 ? lo : j < 6 ? -1 : hi) + j % 3) v[j] = x;
-        }
+        if (x != T(0) || d != 0) nine_put(x, d, lo, hi, v);
     }
 }
 
@@ -1758,14 +1744,15 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
     // records and there are few rows; of many where every row has its own
     // work-item, the rows fit its registers and there are few enough workgroups,
     // or where all slices have records and the rows fit the chip's registers.
+    const bool one_launch = env_int("ELFEL_HIP_PCG_ONE_LAUNCH", 1) != 0;
     auto solve_to = [&](auto &v, double goal2, double *rrec, double *norm) -> int {
         using T = typename std::remove_pointer<decltype(v.r)>::type;
         constexpr int VB = sizeof(T) == 8 ? SM_VB8 : SM_VB4;
         const bool small = narrow && n <= (int64_t)P.G * SV_BLOCK && (P.G + VB - 1) / VB <= SM_GRID;
-        bool one = resident && n <= ONE_ROWS(T);
+        bool one = one_launch && resident && n <= ONE_ROWS(T);
         if (one) cg_one(st, n, S, v, P, sc, goal2, it, maxit);
-        else one = !lost && ((small && cg_small(st, n, S, v, P, slots, sc, goal2, it, maxit) == 0) ||
-                             (resident && cg_resident(st, n, S, v, P, slots, sc, goal2, it, maxit) == 0));
+        else one = one_launch && !lost && ((small && cg_small(st, n, S, v, P, slots, sc, goal2, it, maxit) == 0) ||
+                                            (resident && cg_resident(st, n, S, v, P, slots, sc, goal2, it, maxit) == 0));
         if (one) {
             if ((rc = true_residual(norm))) return rc;
             lost = hsc[S_LOST] != 0.0;

@@ -1,0 +1,86 @@
+"""elfel_hip_pcg gives the same iterations and the same bits whether a solve runs
+in one launch or in two launches an iteration (ELFEL_HIP_PCG_ONE_LAUNCH=0), and
+its solution has the residual that it claims, formed here in float64: tol plus
+the rounding of the sums, 2^-52 * 256 * nfree (test_gpu_solve_sizes.py)."""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+import elfel_hip as eh
+from elfel_hip import _lib as L
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-10
+
+
+def _both(ctx, monkeypatch, nfree, prec, seed=3):
+    """Solves the context's CSR matrix for a random right-hand side both ways."""
+    ptr, ind, val = ctx.copy_sparse(base=0)[:3]
+    n = ptr.size - 1
+    K = sp.csr_matrix((val, ind, ptr), shape=(n, n))
+    rng = np.random.default_rng(seed)
+    F, x0 = rng.standard_normal(n), rng.standard_normal(n)
+    monkeypatch.setenv("ELFEL_HIP_PCG_ONE_LAUNCH", "0")
+    x2, it2, _, rel2 = ctx.pcg(nfree, F, x0, precision=prec, tol=TOL, maxit=20000)
+    monkeypatch.delenv("ELFEL_HIP_PCG_ONE_LAUNCH")
+    x, it, _, rel = ctx.pcg(nfree, F, x0, precision=prec, tol=TOL, maxit=20000)
+    assert it == it2 and rel == rel2 <= TOL, (it, it2, rel, rel2)
+    assert np.array_equal(x, x2)
+    b = F[:nfree] - K[:nfree, nfree:] @ x0[nfree:]
+    r = b - K[:nfree, :nfree] @ x[:nfree]
+    assert np.linalg.norm(r) <= (TOL + 2.0 ** -52 * 256 * nfree) * np.linalg.norm(b)
+
+
+def _heat(ctx, fe, nx, ny, fixed):
+    """Heat on nx x ny cells, the fixed nodes' dofs last; the free dofs' number."""
+    mesh = {L.T3: eh.T3block, L.Q4: eh.Q4block}[fe](float(nx), float(ny), nx, ny)
+    x, y = np.rint(mesh.xy).astype(int).T
+    fixed = fixed(x, y)
+    free = int((~fixed).sum())
+    order = np.where(fixed, free + np.cumsum(fixed) - 1, np.cumsum(~fixed) - 1)
+    ctx.set_mesh(0, mesh.conn, mesh.xy)
+    ctx.set_dofs(0, order.reshape(-1, 1) + 1, mesh.nnodes)
+    ctx.set_coefficients(mesh.nelements)
+    ctx.assemble(L.HEAT, fe, 2 if fe == L.Q4 else 1, precision=L.FP64, method=L.REUSE, layout=L.CSR)
+    return free
+
+
+@pytest.mark.parametrize("prec", [L.FP64, L.MIXED])
+@pytest.mark.parametrize("fe,across", [(L.T3, 1), (L.T3, 2), (L.T3, 3), (L.T3, 4), (L.Q4, 2), (L.Q4, 3), (L.Q4, 4)])
+@pytest.mark.parametrize("along", [2, 60, 1000, 30000, 100000])
+def test_strips_with_held_sides(ctx, monkeypatch, along, fe, across, prec):
+    """`across` free nodes between two held sides, numbered first along the short
+    side.  (Quadrilaterals with one free node across have few distinct
+    eigenvalues: the mixed iteration, by either way, runs past its end there.)"""
+    nx, ny = across + 1, along + 1
+    free = _heat(ctx, fe, nx, ny, lambda x, y: (x == 0) | (x == nx) | (y == 0) | (y == ny))
+    assert free == across * along
+    _both(ctx, monkeypatch, free, prec)
+
+
+@pytest.mark.parametrize("prec", [L.FP64, L.MIXED])
+@pytest.mark.parametrize("fe", [L.T3, L.Q4])
+@pytest.mark.parametrize("cells", [1, 2, 3])
+def test_strips_with_free_sides(ctx, monkeypatch, cells, fe, prec):
+    free = _heat(ctx, fe, cells, 61, lambda x, y: (y == 0) | (y == 61))
+    assert free == 60 * (cells + 1)
+    _both(ctx, monkeypatch, free, prec)
+
+
+@pytest.mark.parametrize("prec", [L.FP64, L.MIXED])
+@pytest.mark.parametrize("n", [5, 300, 2500, 120000, 180000])
+@pytest.mark.parametrize("offsets", [(1,), (2,), (1, 2), (1, 3), (1, 2, 3), (2, 3, 4), (1, 2, 3, 4)])
+def test_bands(ctx, monkeypatch, offsets, n, prec):
+    """Diagonally dominant bands of a COO stream: the diagonal 2.5 times the sum of its row."""
+    rng = np.random.default_rng(n)
+    i = np.arange(1, n + 1)
+    I, J, V, diag = [], [], [], np.full(n, 0.5)
+    for d in offsets:
+        v = rng.uniform(0.5, 1.0, max(n - d, 0))
+        I += [i[:-d], i[d:]]
+        J += [i[d:], i[:-d]]
+        V += [-v, -v]
+        diag[: n - d] += 2.5 * v
+        diag[d:] += 2.5 * v
+    ctx.sparse(np.concatenate(I + [i]), np.concatenate(J + [i]), np.concatenate(V + [diag]), n, n, layout=L.CSR)
+    _both(ctx, monkeypatch, n, prec)
