@@ -1,5 +1,7 @@
-// nine.h -- the nine-entry rows of the one-launch solves (solve.hip): which
-// slices of 64 rows have them, and which slot an entry takes.
+// nine.h -- how the one-launch solves (solve.hip) take the rows of a slice of 64
+// into registers: the slots that a row of any narrow slice reads, and, for rows
+// of nine entries in three runs, which slices have them and which register an
+// entry takes.
 //
 // Slots 0-2 are the entries at lo, lo + 1, lo + 2 from the diagonal, 3-5 those at
 // -1, 0, 1, and 6-8 those at hi, hi + 1, hi + 2, with lo the slice's smallest
@@ -13,6 +15,14 @@
 
 #define RES_W 9
 #define NINE_NONE (1 << 20)  // a run without entries: no offset is so large
+
+// Where entry k of lane's row is read in a slice that begins at o and is w
+// entries wide: past its width the first once more (it adds nothing), and in a
+// slice of no entries (64 rows of dofs of no element) nowhere: -1.
+__host__ __device__ __forceinline__ int64_t sell_slot(uint32_t o, uint32_t w, uint32_t k, int lane)
+{
+    return w == 0 ? -1 : (int64_t)o + (int64_t)(k < w ? k : 0) * 64 + lane;
+}
 
 // The ends of a slice's lower and upper runs.
 struct NineRuns {

@@ -197,6 +197,14 @@ __global__ void k_sell_uniform(int64_t nfree, int64_t nslices, const uint32_t *_
     if (lane == 0) uflag[s] = uniform ? 1u : 0u;
 }
 
+// Without them: a slice of no entries alone is flagged (there is no slot that its
+// rows could read).
+__global__ void k_sell_empty(int64_t nslices, const uint32_t *__restrict__ off, uint32_t *__restrict__ uflag)
+{
+    const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (s < nslices) uflag[s] = off[s] == off[s + 1] ? 1u : 0u;
+}
+
 // A slice for the resident solve (k_cg_resident): its rows' entries lie on the
 // diagonal and its two neighbours, in one run of three neighbouring offsets
 // below and one above -- the three grid rows of a quadrilateral's or triangle's
@@ -729,9 +737,13 @@ __global__ __launch_bounds__(VB * SV_BLOCK) void k_cg_small(int64_t n, const uin
     int32_t cj[SELL_UNROLL];
 #pragma unroll
     for (int k = 0; k < SELL_UNROLL; k++) {
-        const size_t at = (size_t)o + (size_t)(k < (int)w ? k : 0) * 64 + (size_t)(ic & 63);
-        v[k] = val[at];
-        cj[k] = sell_col<C>(col[at], ic);
+        const int64_t at = sell_slot(o, w, k, (int)(ic & 63));
+        v[k] = T(0);
+        cj[k] = (int32_t)ic;
+        if (at >= 0) {
+            v[k] = val[at];
+            cj[k] = sell_col<C>(col[at], ic);
+        }
     }
     const T di = dinv[ic];
     T ri = r_[ic], zi = z_[ic], pi = pa[ic];
@@ -1684,7 +1696,7 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
             hipLaunchKernelGGL((k_sell_uniform<int32_t>), dim3(ceil_div(nslices * 64, 256)), dim3(256), 0, st, n,
                                nslices, (const uint32_t *)off, (const int32_t *)scol, uflag, uoff);
     } else {
-        hipLaunchKernelGGL(k_fill<uint32_t>, dim3(ceil_div(nslices, 256)), dim3(256), 0, st, nslices, uflag, 0u);
+        hipLaunchKernelGGL(k_sell_empty, dim3(ceil_div(nslices, 256)), dim3(256), 0, st, nslices, (const uint32_t *)off, uflag);
     }
     hipLaunchKernelGGL(k_diag_inv, dim3(ceil_div(n, 256)), dim3(256), 0, st, n, ptr, ind, val, dinv64,
                        mixed ? v32.dinv : nullptr);

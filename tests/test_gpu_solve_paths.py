@@ -84,3 +84,42 @@ def test_bands(ctx, monkeypatch, offsets, n, prec):
         diag[d:] += 2.5 * v
     ctx.sparse(np.concatenate(I + [i]), np.concatenate(J + [i]), np.concatenate(V + [diag]), n, n, layout=L.CSR)
     _both(ctx, monkeypatch, n, prec)
+
+
+@pytest.mark.parametrize("prec", [L.FP64, L.MIXED])
+@pytest.mark.parametrize("N,shuffle", [(20, False), (70, False), (40, True), (200, False), (200, True)])
+@pytest.mark.parametrize("where", ["last", "between", "both"])
+def test_free_dofs_of_no_element(ctx, monkeypatch, where, N, shuffle, prec):
+    """Free dofs that no element has, whole slices of 64 rows of them: their rows
+    have no entries and their load is zero, so they keep their values.  N = 200
+    shuffled has columns beyond 16-bit offsets."""
+    mesh = eh.Q4block(1.0, 1.0, N, N)
+    n, held = mesh.nnodes, mesh.nnodes // 10
+    rng = np.random.default_rng(N)
+    dof = rng.permutation(n) if shuffle else np.arange(n)
+    half = (n - held) // 2
+    between, last = {"last": (0, 333), "between": (200, 0), "both": (200, 333)}[where]
+    dof = dof + np.where(dof >= half, between, 0) + np.where(dof >= n - held, last, 0)
+    total, free = n + between + last, n - held + between + last
+    ctx.set_mesh(0, mesh.conn, mesh.xy)
+    ctx.set_dofs(0, dof.reshape(-1, 1) + 1, total)
+    ctx.set_coefficients(mesh.nelements)
+    ctx.assemble(L.HEAT, L.Q4, 2, precision=L.FP64, method=L.SORT, layout=L.CSR)
+    ptr, ind, val = ctx.copy_sparse(base=0)[:3]
+    K = sp.csr_matrix((val, ind, ptr), shape=(total, total))
+    none = np.diff(ptr) == 0
+    assert none.sum() == between + last
+    F, x0 = rng.standard_normal(total), rng.standard_normal(total)
+    F[none] = 0.0
+    monkeypatch.setenv("ELFEL_HIP_PCG_ONE_LAUNCH", "0")
+    x2, it2, _, rel2 = ctx.pcg(free, F, x0, precision=prec, tol=TOL, maxit=20000)
+    monkeypatch.setenv("ELFEL_HIP_SELL_UNIFORM", "0")
+    x3, it3, _, rel3 = ctx.pcg(free, F, x0, precision=prec, tol=TOL, maxit=20000)
+    monkeypatch.delenv("ELFEL_HIP_PCG_ONE_LAUNCH")
+    monkeypatch.delenv("ELFEL_HIP_SELL_UNIFORM")
+    x, it, _, rel = ctx.pcg(free, F, x0, precision=prec, tol=TOL, maxit=20000)
+    assert it == it2 == it3 and rel == rel2 == rel3 <= TOL
+    assert np.array_equal(x, x2) and np.array_equal(x, x3)
+    assert np.array_equal(x[none], x0[none])
+    b = F[:free] - K[:free, free:] @ x0[free:]
+    assert np.linalg.norm(b - K[:free, :free] @ x[:free]) <= (TOL + 2.0 ** -52 * 256 * free) * np.linalg.norm(b)
