@@ -60,6 +60,13 @@ int noalloc_init_device(int device)
     return 0;
 }
 
+// Whether two ranges of memory have a byte in common.
+static bool overlap(const void *a, int64_t na, const void *b, int64_t nb)
+{
+    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+    return na > 0 && nb > 0 && x < y + (uintptr_t)nb && y < x + (uintptr_t)na;
+}
+
 static void *noalloc_scratch(int device)
 {
     if (device < 0 || device >= MAXDEV) return nullptr;
@@ -104,11 +111,21 @@ extern "C" int elfel_hip_sparse_noalloc(elfel_hip_ctx *c, int64_t nrow, int64_t 
         int32_t *nnz_dev = (int32_t *)(base + O_NNZ);
         int rc;
         // row buckets where their scratch fits in the array (up to some seven
-        // million rows at the largest n); the sort for the rest and for long rows
-        if (bucket_takes(n, nmaj, nmin) && bucket_scratch_bytes(n, nmaj) <= SCRATCH_BYTES) {
+        // million rows at the largest n); the sort for the rest and for long rows.
+        // The buckets' tiles read values while others write their results: values
+        // that lie in an output's memory are read from a copy, as the sort does
+        // (the indices are all read before the first result).
+        const bool shared = overlap(val, 8 * n, out, 8 * n) || overlap(val, 8 * n, ind, 4 * n) || overlap(val, 8 * n, ptr, 4 * (nmaj + 1));
+        const size_t bytes = bucket_takes(n, nmaj, nmin) ? align256(bucket_scratch_bytes(n, nmaj)) : 0;
+        if (bytes && bytes + (shared ? 8 * (size_t)n : 0) <= SCRATCH_BYTES) {
             int bad = 0;
             bool toolong = false;
-            if ((rc = bucket_coo(c, base, n, row, col, val, nrow, ncol, csc, ptr, ind, out, &bad, &toolong, nnz))) return rc;
+            const double *v = val;
+            if (shared) {
+                HIPCHK(c, hipMemcpyAsync(base + bytes, val, 8 * (size_t)n, hipMemcpyDeviceToDevice, c->stream));
+                v = (const double *)(base + bytes);
+            }
+            if ((rc = bucket_coo(c, base, n, row, col, v, nrow, ncol, csc, ptr, ind, out, &bad, &toolong, nnz))) return rc;
             if (bad) {
                 HIPCHK(c, hipMemsetAsync((int *)c->dscal.p + 1, 0, sizeof(int), c->stream));
                 if (bad & DERR_RANGE) return set_err(c, ELFEL_ERANGE, "row or column index out of range");

@@ -98,7 +98,8 @@ int elfel_hip_sparse(elfel_hip_ctx *ctx, int64_t nrow, int64_t ncol, int64_t n,
  * array, so calls that overlap on one GPU (two contexts, two threads) race;
  * the context's own calls are serialised on its stream.  Same order and
  * semantics as elfel_hip_sparse (stable order, structural zeros kept,
- * ELFEL_ERANGE for indices out of range); the call waits for the result. */
+ * ELFEL_ERANGE for indices out of range); the call waits for the result.
+ * The outputs may lie in the inputs' memory (not in each other's). */
 #define ELFEL_NOALLOC_MAX_COO (1 << 20)
 int elfel_hip_sparse_noalloc(elfel_hip_ctx *ctx, int64_t nrow, int64_t ncol, int64_t n, const int64_t *row,
                              const int64_t *col, const double *val, int layout, int32_t *ptr, int32_t *ind,
