@@ -120,17 +120,21 @@ extern "C" int elfel_hip_sparse_noalloc(elfel_hip_ctx *c, int64_t nrow, int64_t 
         if (bytes && bytes + (shared ? 8 * (size_t)n : 0) <= SCRATCH_BYTES) {
             int bad = 0;
             bool toolong = false;
+            int64_t count = 0;  // *nnz changes with a result only
             const double *v = val;
             if (shared) {
                 HIPCHK(c, hipMemcpyAsync(base + bytes, val, 8 * (size_t)n, hipMemcpyDeviceToDevice, c->stream));
                 v = (const double *)(base + bytes);
             }
-            if ((rc = bucket_coo(c, base, n, row, col, v, nrow, ncol, csc, ptr, ind, out, &bad, &toolong, nnz))) return rc;
+            if ((rc = bucket_coo(c, base, n, row, col, v, nrow, ncol, csc, ptr, ind, out, &bad, &toolong, &count))) return rc;
             if (bad) {
                 HIPCHK(c, hipMemsetAsync((int *)c->dscal.p + 1, 0, sizeof(int), c->stream));
                 if (bad & DERR_RANGE) return set_err(c, ELFEL_ERANGE, "row or column index out of range");
             }
-            if (!toolong) return ELFEL_OK;
+            if (!toolong) {
+                *nnz = count;
+                return ELFEL_OK;
+            }
         }
         if (n > 0) HIPCHK(c, hipMemcpyAsync(v0, val, 8 * (size_t)n, hipMemcpyDeviceToDevice, c->stream));
         if ((rc = plain_coo_keys(c, row, col, n, nrow, ncol, minor_bits, csc, k0))) return rc;

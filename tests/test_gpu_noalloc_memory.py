@@ -2,6 +2,8 @@
 same pattern and values, bit for bit, as into memory of their own.  4600 entries
 are one workgroup's, 300 000 and 900 000 small and large tiles, and a row of
 5000 goes to the sort."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -52,3 +54,17 @@ def test_results_in_the_inputs_memory(ctx, hip, n, nrow, long_row, layout):
     row, col = hip.put(I), hip.put(J)
     shifted = hip.put(np.concatenate([np.zeros(100), V]))
     build(row, col, shifted + 800, ptr, ind, shifted)  # the values 100 words earlier
+
+
+@pytest.mark.parametrize("n,nrow", [(50, 20), (20000, 3000)])
+def test_refused_call_changes_nothing(ctx, hip, n, nrow):
+    """An index out of range: the count and the result arrays keep what they hold."""
+    I, J, V = _stream(n, nrow, 0, n)
+    J[n // 2] = nrow + 1
+    ptr, ind, out = hip.put(np.full(nrow + 1, -7, np.int32)), hip.put(np.full(n, -7, np.int32)), hip.put(np.full(n, -7.0))
+    nnz = ctypes.c_int64(-7)
+    rc = ctx.lib.elfel_hip_sparse_noalloc(ctx.h, nrow, nrow, n, hip.put(I), hip.put(J), hip.put(V), L.CSR, ptr, ind, out,
+                                          ctypes.byref(nnz))
+    assert rc == L.ERANGE and nnz.value == -7
+    assert np.all(hip.get(ptr, nrow + 1, np.int32) == -7) and np.all(hip.get(ind, n, np.int32) == -7)
+    assert np.all(hip.get(out, n, np.float64) == -7.0)
