@@ -546,9 +546,7 @@ __global__ __launch_bounds__(SV_BLOCK) void k_cg_fin(int64_t n, const double *__
 #define SM_VB4 3
 #define SM_GRID 224
 #define EX_NONE 0xfff8dead5eedbeefull
-#ifndef EX_LIMIT
 #define EX_LIMIT (1 << 20)
-#endif
 
 // z and p are written and gathered, and the slots filled and polled, with
 // relaxed agent-scope accesses: they bypass the XCDs' L2 (the compiler's
@@ -606,10 +604,11 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 struct Exchange {
     uint64_t *slots;
     int G;
-    int stride;  // bytes of a set
+    int limit;  // polls of a wait
+    __host__ __device__ __forceinline__ int stride() const { return EX_STRIDE(G); }  // bytes of a set
     __device__ __forceinline__ uint32_t at(uint32_t e, int blk, int copy) const
     {
-        return (e % 3) * (uint32_t)stride + (uint32_t)(blk >> 2) * EX_LINE + (uint32_t)copy * 64 + (uint32_t)(blk & 3) * 16;
+        return (e % 3) * (uint32_t)stride() + (uint32_t)(blk >> 2) * EX_LINE + (uint32_t)copy * 64 + (uint32_t)(blk & 3) * 16;
     }
     __device__ __forceinline__ void put(uint32_t e, int blk, int copy, int two, uint64_t v) const
     {
@@ -618,7 +617,7 @@ struct Exchange {
     template <bool TWO>
     __device__ __forceinline__ void get(uint32_t e, int blk, uint64_t &u, uint64_t &v) const
     {
-        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(slots, 0, 3 * stride, 0x00020000);
+        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(slots, 0, 3 * stride(), 0x00020000);
         int o = (int)at(e, blk, blockIdx.x % EX_COPIES);
         asm volatile("" : "+v"(o)::"memory");  // a load each time
         if (TWO) {
@@ -669,7 +668,7 @@ __device__ __forceinline__ bool exchange(const Exchange &X, uint32_t e, double &
         b = 0.0;
         for (int i = tid; i < X.G; i += 4 * SV_BLOCK) {
             uint64_t u[4], v[4];
-            int spin = 0;
+            int spin = X.limit;
             bool wait;
             do {
                 wait = false;
@@ -680,7 +679,7 @@ __device__ __forceinline__ bool exchange(const Exchange &X, uint32_t e, double &
                 }
 #pragma unroll
                 for (int q = 0; q < 4; q++) wait |= u[q] == EX_NONE || v[q] == EX_NONE;
-            } while (wait && ++spin < EX_LIMIT);
+            } while (wait && --spin > 0);
             if (wait) *quit = 1u;
 #pragma unroll
             for (int q = 0; q < 4; q++) {
@@ -939,10 +938,10 @@ __device__ __forceinline__ bool exchange_res(const Exchange &X, uint32_t e, doub
     if (tid < SV_BLOCK) {
         uint64_t u = 0, v = 0;
         if (tid < nw) {
-            int spin = 0;
+            int spin = X.limit;
             do {
                 X.get<TWO>(e, tid, u, v);
-            } while ((u == EX_NONE || v == EX_NONE) && ++spin < EX_LIMIT);
+            } while ((u == EX_NONE || v == EX_NONE) && --spin > 0);
             if (u == EX_NONE || v == EX_NONE) *quit = 1u;
         }
         a = wave_sum(__builtin_bit_cast(double, u));
@@ -1488,6 +1487,9 @@ void cg_group(hipStream_t st, int64_t n, const Sell &S, Vecs<float> &v, const Pa
     else cg_group_as<float, float, int32_t>(st, n, S, v, v.xlo, P, sc, hsc);
 }
 
+// (a small number makes waits give up, for the tests of what follows then)
+int ex_limit() { return std::max(1, env_int("ELFEL_HIP_PCG_POLLS", EX_LIMIT)); }
+
 // Groups of iterations until ||r||^2 <= goal2 or maxit, in one launch; *it is
 // carried on.  1: the device cannot run the launch (nothing has run).
 template <typename T, typename TX, typename C>
@@ -1496,8 +1498,8 @@ int cg_small_as(hipStream_t st, int64_t n, const Sell &S, Vecs<T> &v, TX *xs, co
 {
     constexpr int VB = sizeof(T) == 8 ? SM_VB8 : SM_VB4;
     const int grid = (P.G + VB - 1) / VB;
-    Exchange X{slots, P.G, EX_STRIDE(P.G)};
-    hipLaunchKernelGGL(k_cg_slots, dim3(ceil_div(3 * X.stride / 8, 256)), dim3(256), 0, st, slots, 3 * X.stride / 8, sc);
+    Exchange X{slots, P.G, ex_limit()};
+    hipLaunchKernelGGL(k_cg_slots, dim3(ceil_div(3 * X.stride() / 8, 256)), dim3(256), 0, st, slots, 3 * X.stride() / 8, sc);
     const uint32_t *off = S.off;
     const C *col = (const C *)S.col;
     const T *val = sell_vals<T>(S);
@@ -1529,8 +1531,8 @@ int cg_resident_as(hipStream_t st, int64_t n, const Sell &S, Vecs<T> &v, TX *xs,
                    double goal2, int it, int maxit)
 {
     if (P.G < RES_GRID || P.G > RES_VB * RES_GRID) return 1;  // every block's work-items
-    Exchange X{slots, P.G, EX_STRIDE(RES_GRID)};
-    hipLaunchKernelGGL(k_cg_slots, dim3(ceil_div(3 * X.stride / 8, 256)), dim3(256), 0, st, slots, 3 * X.stride / 8, sc);
+    Exchange X{slots, P.G, ex_limit()};
+    hipLaunchKernelGGL(k_cg_slots, dim3(ceil_div(3 * X.stride() / 8, 256)), dim3(256), 0, st, slots, 3 * X.stride() / 8, sc);
     const uint32_t *off = S.off;
     const int16_t *col = (const int16_t *)S.col;
     const T *val = sell_vals<T>(S);
