@@ -13,22 +13,25 @@ pytestmark = pytest.mark.gpu
 TOL = 1e-10
 
 
-def _both(ctx, monkeypatch, nfree, prec, seed=3):
-    """Solves the context's CSR matrix for a random right-hand side both ways."""
+def _both(ctx, monkeypatch, nfree, prec, seed=3, tol=TOL, ends=True):
+    """Solves the context's CSR matrix for a random right-hand side both ways.
+    ends: the iteration reaches the tolerance."""
     ptr, ind, val = ctx.copy_sparse(base=0)[:3]
     n = ptr.size - 1
     K = sp.csr_matrix((val, ind, ptr), shape=(n, n))
     rng = np.random.default_rng(seed)
     F, x0 = rng.standard_normal(n), rng.standard_normal(n)
     monkeypatch.setenv("ELFEL_HIP_PCG_ONE_LAUNCH", "0")
-    x2, it2, _, rel2 = ctx.pcg(nfree, F, x0, precision=prec, tol=TOL, maxit=20000)
+    x2, it2, _, rel2 = ctx.pcg(nfree, F, x0, precision=prec, tol=tol, maxit=100000)
     monkeypatch.delenv("ELFEL_HIP_PCG_ONE_LAUNCH")
-    x, it, _, rel = ctx.pcg(nfree, F, x0, precision=prec, tol=TOL, maxit=20000)
-    assert it == it2 and rel == rel2 <= TOL, (it, it2, rel, rel2)
-    assert np.array_equal(x, x2)
+    x, it, _, rel = ctx.pcg(nfree, F, x0, precision=prec, tol=tol, maxit=100000)
+    assert it == it2 and np.array_equal(x, x2, equal_nan=True) and np.array_equal(rel, rel2, equal_nan=True), (it, it2, rel, rel2)
+    if not ends:
+        return
+    assert rel <= tol
     b = F[:nfree] - K[:nfree, nfree:] @ x0[nfree:]
     r = b - K[:nfree, :nfree] @ x[:nfree]
-    assert np.linalg.norm(r) <= (TOL + 2.0 ** -52 * 256 * nfree) * np.linalg.norm(b)
+    assert np.linalg.norm(r) <= (tol + 2.0 ** -52 * 256 * nfree) * np.linalg.norm(b)
 
 
 def _heat(ctx, fe, nx, ny, fixed):
@@ -123,3 +126,21 @@ def test_free_dofs_of_no_element(ctx, monkeypatch, where, N, shuffle, prec):
     assert np.array_equal(x[none], x0[none])
     b = F[:free] - K[:free, free:] @ x0[free:]
     assert np.linalg.norm(b - K[:free, :free] @ x[:free]) <= (TOL + 2.0 ** -52 * 256 * free) * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("fe", [L.T3, L.Q4])
+@pytest.mark.parametrize("N,prec,sizes", [
+    (70, L.FP64, (1, 64, 65, 255, 257, 1023, 1024, 1025, 2047, 2048, 2049, 3071)),
+    (70, L.MIXED, (1, 64, 65, 255, 257, 1023, 1024, 1025, 2048, 2049, 3072, 4095, 4096, 4097, 4609)),
+    (340, L.FP64, (224 * 512, 224 * 512 + 1)), (416, L.MIXED, (224 * 768, 224 * 768 + 1)),
+    (730, L.FP64, (262144, 262145, 524288, 524289)), (890, L.FP64, (786432, 786433)),
+    (730, L.MIXED, (262144, 262145, 524289)), (1030, L.MIXED, (786433, 1048577)), (1449, L.MIXED, (1572865, 2097152, 2097153))])
+def test_both_ways_where_the_kernels_change(ctx, monkeypatch, N, prec, sizes, fe):
+    """Rows either side of what each one-launch kernel and each number of rows a
+    work-item takes (test_gpu_solve_sizes.py), grids in their own order."""
+    n = (N + 1) ** 2
+    for nfree in sizes:
+        free = _heat(ctx, fe, N, N, lambda x, y: x + (N + 1) * y >= nfree)
+        assert free == nfree < n
+        # (one grid row of quadrilaterals: the strips of one free node across, above)
+        _both(ctx, monkeypatch, nfree, prec, tol=1e-8, ends=prec == L.FP64 or fe == L.T3 or nfree > N + 1)
