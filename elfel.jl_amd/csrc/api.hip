@@ -281,6 +281,7 @@ extern "C" int elfel_hip_free(elfel_hip_ctx *c)
                    &c->fpat.coo, &c->fpat.fcoo};
     for (Buf *b : bufs) release(*b);
     told_put(c->told);
+    if (c->xs) hipHostFree(c->xs);
     for (auto &e : c->xfer_ev)
         if (e) hipEventDestroy(e);
     transfer_user(false);
@@ -605,23 +606,18 @@ extern "C" int elfel_hip_set_coefficients(elfel_hip_ctx *c, int64_t E, const dou
         if (E < 0) return set_err(c, ELFEL_EINVAL, "elfel_hip_set_coefficients: bad E");
         struct { const double *src; Buf *dst; bool *flag; } items[3] = {
             {kappa_e, &c->kappa_e, &c->has_kappa_e}, {Q_e, &c->Q_e, &c->has_Q_e}, {scale_e, &c->scale_e, &c->has_scale_e}};
+        // padded storage: blocks of 4096 entries + COEF_GAP
+        HostIn in[3];
+        int n = 0, rc;
         for (auto &it : items) {
             *it.flag = false;
             if (!it.src) continue;
-            // padded storage: one host-to-device copy into the staging buffer,
-            // then a strided device copy into blocks of 4096 entries + COEF_GAP
-            int rc = ensure(c, *it.dst, 8 * padded_len(E, COEF_GAP));
-            if (!rc) rc = ensure(c, c->stage64, 8 * E);
-            if (rc) return rc;
-            if (E > 0) {
-                const HostIn in{it.src, c->stage64.p, E, false, 0, 0};
-                if ((rc = to_device(c, &in, 1, nullptr))) return rc;
-                if ((rc = copy_padded(c, it.dst->p, c->stage64.p, E, 8, COEF_GAP))) return rc;
-            }
-            *it.flag = true;
+            if ((rc = ensure(c, *it.dst, 8 * padded_len(E, COEF_GAP)))) return rc;
+            in[n++] = HostIn{it.src, it.dst->p, E, false, 0, 0, COEF_GAP};
         }
+        if ((rc = to_device(c, in, n, nullptr))) return rc;
+        for (auto &it : items) *it.flag = it.src != nullptr;
         c->coef_E = E;
-        HIPCHK(c, hipStreamSynchronize(c->stream));
         return ELFEL_OK;
     });
 }

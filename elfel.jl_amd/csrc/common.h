@@ -201,6 +201,8 @@ struct elfel_hip_ctx {
     // solver scratch: vectors, then the SELL-64 copy of the free block
     Buf pcg, pcg_sell;
     hipEvent_t xfer_ev[8] = {};   // transfer.hip, made when first needed
+    void *xs = nullptr;           // pinned memory of the small transfers, likewise
+    int64_t xs_at = 0;            // what uploads under way still read of it
     // batched problems (batch.hip)
     void *batch = nullptr;
 };
@@ -288,16 +290,19 @@ struct HostOut {
     bool wide;
     int64_t base;
 };
-// A device array filled from the host: n 8-byte words, or (narrow) int64 in
-// lo..hi as 0-based int32.
+// A device array filled from the host: n 8-byte words (gap: stored as padded()
+// says), or (narrow) int64 in lo..hi as 0-based int32.
 struct HostIn {
     const void *host;
     void *dev;
     int64_t n;
     bool narrow;
     int64_t lo, hi;
+    int gap = 0;
 };
-// Both wait: for the stream's work before them and for the copies.
+// to_host waits for the stream's work before it and for the copies; after
+// to_device the host array may change, and the stream's work that follows sees
+// the device's.
 int to_host(elfel_hip_ctx *c, const HostOut *segs, int nseg);
 // out_of_range: a narrowed value lay outside lo..hi (the device array is then
 // written all the same, with lo in its place).
