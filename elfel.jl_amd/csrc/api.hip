@@ -259,7 +259,7 @@ extern "C" int elfel_hip_init(int device, elfel_hip_ctx **out)
             delete c;
             return rc;
         }
-        transfer_user(true);
+        transfer_user(device, true);
         *out = c;
         return ELFEL_OK;
     });
@@ -284,7 +284,7 @@ extern "C" int elfel_hip_free(elfel_hip_ctx *c)
     if (c->xs) hipHostFree(c->xs);
     for (auto &e : c->xfer_ev)
         if (e) hipEventDestroy(e);
-    transfer_user(false);
+    transfer_user(c->device, false);
     batch_free(c);
     for (auto &p : c->tm.pending) { hipEventDestroy(p.a); hipEventDestroy(p.b); }
     if (c->tm.r0) hipEventDestroy(c->tm.r0);

@@ -280,6 +280,8 @@ int ensure(elfel_hip_ctx *c, Buf &b, size_t bytes);
 int copy_padded(elfel_hip_ctx *c, void *dst, const void *src, int64_t n, size_t esize, int gap);
 void release(Buf &b);
 
+#define ELFEL_MAXDEV 64  // devices of a process
+
 // ---- transfer.hip -------------------------------------------------------------
 // A host array filled from the device: n 8-byte words, or (wide) the device's
 // int32 as int64 + base.  host null: left out.
@@ -307,7 +309,7 @@ int to_host(elfel_hip_ctx *c, const HostOut *segs, int nseg);
 // out_of_range: a narrowed value lay outside lo..hi (the device array is then
 // written all the same, with lo in its place).
 int to_device(elfel_hip_ctx *c, const HostIn *segs, int nseg, bool *out_of_range);
-void transfer_user(bool add);  // a context more or less that may transfer
+void transfer_user(int device, bool add);  // a context of the device more or less that may transfer
 // The host copies of a field's connectivity and dof map.
 int host_tables(elfel_hip_ctx *c, Field &f);
 

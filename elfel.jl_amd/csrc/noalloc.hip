@@ -39,15 +39,14 @@ constexpr size_t SCRATCH_BYTES = O_NNZ + 256;
 static __device__ __align__(256) unsigned char scratch[SCRATCH_BYTES];
 
 namespace {
-constexpr int MAXDEV = 64;
 std::mutex noalloc_mu;
-void *noalloc_base[MAXDEV] = {};
+void *noalloc_base[ELFEL_MAXDEV] = {};
 }  // namespace
 
 // Called by elfel_hip_init with `device` current.
 int noalloc_init_device(int device)
 {
-    if (device < 0 || device >= MAXDEV) return ELFEL_ENOTSUP;
+    if (device < 0 || device >= ELFEL_MAXDEV) return ELFEL_ENOTSUP;
     std::lock_guard<std::mutex> g(noalloc_mu);
     if (noalloc_base[device]) return 0;
     void *p = nullptr;
@@ -69,7 +68,7 @@ static bool overlap(const void *a, int64_t na, const void *b, int64_t nb)
 
 static void *noalloc_scratch(int device)
 {
-    if (device < 0 || device >= MAXDEV) return nullptr;
+    if (device < 0 || device >= ELFEL_MAXDEV) return nullptr;
     std::lock_guard<std::mutex> g(noalloc_mu);
     return noalloc_base[device];
 }

@@ -11,8 +11,10 @@
 // six million COO entries in and 2.4 million out 8.0 -> 3.8 ms.
 //
 // A ring of pinned memory, XF_SLOTS batches of XF_BATCH bytes, is shared by all
-// contexts (one transfer holds it at a time, with its device work already
-// done), allocated by the first that needs it and freed with the last context.
+// contexts of a device (one transfer holds it at a time, with its device work
+// already done: a second would halve the link's share of both), allocated by the
+// first that needs it (0.2 ms; its pages are mapped as they are used) and freed
+// with the device's last context.
 //
 // Up to XF_SMALL bytes the fixed costs are the time: a copy, an event and a wait
 // an array.  Such a transfer goes through pinned memory of the context's own,
@@ -42,19 +44,22 @@ constexpr int64_t XF_PER_THREAD = 1 << 20;  // bytes of the caller's memory that
 constexpr int64_t XF_SMALL = 1 << 20;
 constexpr int XF_MOVES = 4;            // arrays of a small transfer
 
-std::mutex ring_mu;       // held during a transfer
-std::mutex ring_life_mu;  // guards the two below
-char *ring = nullptr;
-int ring_users = 0;
+struct Ring {
+    std::mutex hold;  // during a transfer
+    std::mutex life;  // guards what follows
+    char *mem = nullptr;
+    int users = 0;
+};
+Ring rings[ELFEL_MAXDEV];
 
-char *ring_get()
+char *ring_get(Ring &R)
 {
-    std::lock_guard<std::mutex> g(ring_life_mu);
-    if (!ring && hipHostMalloc((void **)&ring, XF_BATCH * XF_SLOTS, hipHostMallocPortable) != hipSuccess) {
+    std::lock_guard<std::mutex> g(R.life);
+    if (!R.mem && hipHostMalloc((void **)&R.mem, XF_BATCH * XF_SLOTS, hipHostMallocPortable) != hipSuccess) {
         (void)hipGetLastError();
-        ring = nullptr;
+        R.mem = nullptr;
     }
-    return ring;
+    return R.mem;
 }
 
 // One thread's share of a batch: `n` words of the caller's array.
@@ -234,13 +239,14 @@ int launch_moves(elfel_hip_ctx *c, const Moves &M, int n)
 
 }  // namespace
 
-void transfer_user(bool add)
+void transfer_user(int device, bool add)
 {
-    std::lock_guard<std::mutex> g(ring_life_mu);
-    ring_users += add ? 1 : -1;
-    if (ring_users == 0 && ring) {
-        hipHostFree(ring);
-        ring = nullptr;
+    Ring &R = rings[device];
+    std::lock_guard<std::mutex> g(R.life);
+    R.users += add ? 1 : -1;
+    if (R.users == 0 && R.mem) {
+        hipHostFree(R.mem);
+        R.mem = nullptr;
     }
 }
 
@@ -286,8 +292,9 @@ int to_host(elfel_hip_ctx *c, const HostOut *segs, int nseg)
     // the device's own work is done before the ring is taken
     HIPCHK(c, hipStreamSynchronize(c->stream));
     c->xs_at = 0;
-    std::lock_guard<std::mutex> hold(ring_mu);
-    char *base = ring_get();
+    Ring &R = rings[c->device];
+    std::lock_guard<std::mutex> hold(R.hold);
+    char *base = ring_get(R);
     if (!base) return set_err(c, ELFEL_ENOMEM, "pinned host memory for a transfer");
     const int nb = (int)J.batches.size();
     std::atomic<int> issued{0};
@@ -419,8 +426,9 @@ int to_device(elfel_hip_ctx *c, const HostIn *segs, int nseg, bool *out_of_range
     }
     HIPCHK(c, hipStreamSynchronize(c->stream));
     c->xs_at = 0;
-    std::lock_guard<std::mutex> hold(ring_mu);
-    char *base = ring_get();
+    Ring &R = rings[c->device];
+    std::lock_guard<std::mutex> hold(R.hold);
+    char *base = ring_get(R);
     if (!base) return set_err(c, ELFEL_ENOMEM, "pinned host memory for a transfer");
     const int nb = (int)J.batches.size();
     std::atomic<int> open{std::min(nb, XF_SLOTS)};  // batches whose slot may be filled
