@@ -14,7 +14,8 @@
 // contexts of a device (one transfer holds it at a time, with its device work
 // already done: a second would halve the link's share of both), allocated by the
 // first that needs it (0.2 ms; its pages are mapped as they are used) and freed
-// with the device's last context.
+// with the device's last context.  Where it cannot be pinned it is ordinary
+// memory, which the runtime copies through buffers of its own.
 //
 // Up to XF_SMALL bytes the fixed costs are the time: a copy, an event and a wait
 // an array.  Such a transfer goes through pinned memory of the context's own,
@@ -24,6 +25,7 @@
 // REUSE step with new coefficients, matrix and load read back, heat Q4 48x48:
 // the runtime's copies 133 us, through the ring 163, so 65; 100x100 192, 204, 137.
 #include <emmintrin.h>
+#include <stdlib.h>
 #include <string.h>
 
 #include <algorithm>
@@ -31,6 +33,8 @@
 #include <mutex>
 
 #include "common.h"
+
+int env_int(const char *name, int dflt);  // reuse.hip
 
 namespace {
 
@@ -44,10 +48,20 @@ constexpr int64_t XF_PER_THREAD = 1 << 20;  // bytes of the caller's memory that
 constexpr int64_t XF_SMALL = 1 << 20;
 constexpr int XF_MOVES = 4;            // arrays of a small transfer
 
+// Pinned memory; null: there is none (ELFEL_HIP_PINNED=0: as if there were none).
+void *pin(size_t bytes)
+{
+    void *p = nullptr;
+    if (env_int("ELFEL_HIP_PINNED", 1) != 0 && hipHostMalloc(&p, bytes, hipHostMallocPortable) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
+}
+
 struct Ring {
     std::mutex hold;  // during a transfer
     std::mutex life;  // guards what follows
     char *mem = nullptr;
+    bool pinned = false;
     int users = 0;
 };
 Ring rings[ELFEL_MAXDEV];
@@ -55,9 +69,10 @@ Ring rings[ELFEL_MAXDEV];
 char *ring_get(Ring &R)
 {
     std::lock_guard<std::mutex> g(R.life);
-    if (!R.mem && hipHostMalloc((void **)&R.mem, XF_BATCH * XF_SLOTS, hipHostMallocPortable) != hipSuccess) {
-        (void)hipGetLastError();
-        R.mem = nullptr;
+    if (!R.mem) {
+        R.mem = (char *)pin(XF_BATCH * XF_SLOTS);
+        R.pinned = R.mem != nullptr;
+        if (!R.mem) R.mem = (char *)aligned_alloc(XF_PAGE, XF_BATCH * XF_SLOTS);
     }
     return R.mem;
 }
@@ -225,11 +240,7 @@ int64_t round64(int64_t n) { return (n + 63) & ~(int64_t)63; }
 char *small_room(elfel_hip_ctx *c, int64_t need)
 {
     if (need > XF_SMALL) return nullptr;
-    if (!c->xs && hipHostMalloc(&c->xs, XF_SMALL, hipHostMallocPortable) != hipSuccess) {
-        (void)hipGetLastError();
-        c->xs = nullptr;
-        return nullptr;
-    }
+    if (!c->xs && !(c->xs = pin(XF_SMALL))) return nullptr;
     if (c->xs_at + need > XF_SMALL) {
         if (hipStreamSynchronize(c->stream) != hipSuccess) return nullptr;
         c->xs_at = 0;
@@ -254,7 +265,8 @@ void transfer_user(int device, bool add)
     std::lock_guard<std::mutex> g(R.life);
     R.users += add ? 1 : -1;
     if (R.users == 0 && R.mem) {
-        hipHostFree(R.mem);
+        if (R.pinned) hipHostFree(R.mem);
+        else free(R.mem);
         R.mem = nullptr;
     }
 }
@@ -304,7 +316,7 @@ int to_host(elfel_hip_ctx *c, const HostOut *segs, int nseg)
     Ring &R = rings[c->device];
     std::lock_guard<std::mutex> hold(R.hold);
     char *base = ring_get(R);
-    if (!base) return set_err(c, ELFEL_ENOMEM, "pinned host memory for a transfer");
+    if (!base) return set_err(c, ELFEL_ENOMEM, "host memory for a transfer");
     const int nb = (int)J.batches.size();
     std::atomic<int> issued{0};
     std::vector<std::atomic<int>> here(nb);  // 0: not known, 1: a thread waits for it, 2: in the slot
@@ -437,7 +449,7 @@ int to_device(elfel_hip_ctx *c, const HostIn *segs, int nseg, bool *out_of_range
     Ring &R = rings[c->device];
     std::lock_guard<std::mutex> hold(R.hold);
     char *base = ring_get(R);
-    if (!base) return set_err(c, ELFEL_ENOMEM, "pinned host memory for a transfer");
+    if (!base) return set_err(c, ELFEL_ENOMEM, "host memory for a transfer");
     const int nb = (int)J.batches.size();
     std::atomic<int> open{std::min(nb, XF_SLOTS)};  // batches whose slot may be filled
     std::atomic<bool> bad{false};
