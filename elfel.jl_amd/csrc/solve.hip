@@ -30,10 +30,11 @@
 // the CSR matrix).  When every free column lies within a 16-bit offset of its
 // row (banded numberings: structured grids, RCM-ordered meshes) the columns
 // are stored as int16 offsets, 2 bytes per entry instead of 4.
-// Per iteration two kernels on a fixed grid of 4 workgroups per CU (grid-stride
-// loops): q = A p with the new direction formed on the way, one partial of p.q
-// per workgroup; and the r / z update (every workgroup first sums the p.q
-// partials itself, in the same order) with partials of r.z and r.r.  No atomics
+// Per iteration two or three kernels on a fixed grid of 4 workgroups per CU
+// (grid-stride loops): q = A p, one partial of p.q per workgroup, with the new
+// direction formed on the way or by a kernel of its own before it; and the r / z
+// update (every workgroup first sums the p.q partials itself, in the same order)
+// with partials of r.z and r.r.  No atomics
 // and no extra reduction launches; every run gives the same bits.  The CG
 // scalars stay on the device and the host reads the residual every CHECK
 // iterations.
@@ -176,11 +177,13 @@ __global__ void k_sell_fill(int64_t nfree, const int32_t *__restrict__ ptr, cons
 // Slices whose every slot holds one column offset for all its rows (each row
 // of the slice has its k-th entry at row + d_k: the stencil of a structured
 // grid away from its boundary) are flagged, and their offsets d_k are kept
-// once per slot; such a slice reads no per-entry column at all.  One wave per
-// slice.
+// once per slot; such a slice reads no per-entry column at all.  many: how many
+// of every UNI_STEP-th slice are.  One wave per slice.
+#define UNI_STEP 16
 template <typename C>
 __global__ void k_sell_uniform(int64_t nfree, int64_t nslices, const uint32_t *__restrict__ off,
-                               const C *__restrict__ col, uint32_t *__restrict__ uflag, int32_t *__restrict__ uoff)
+                               const C *__restrict__ col, uint32_t *__restrict__ uflag, int32_t *__restrict__ uoff,
+                               uint32_t *__restrict__ many)
 {
     const int64_t s = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const int lane = threadIdx.x & 63;
@@ -194,7 +197,10 @@ __global__ void k_sell_uniform(int64_t nfree, int64_t nslices, const uint32_t *_
         if (__ballot((i < nfree) && (d != d0)) != 0ull) uniform = false;
         if (lane == 0) uoff[sb + k] = d0;
     }
-    if (lane == 0) uflag[s] = uniform ? 1u : 0u;
+    if (lane == 0) {
+        uflag[s] = uniform ? 1u : 0u;
+        if (uniform && s % UNI_STEP == 0) atomicAdd(many, 1u);
+    }
 }
 
 // Without them: a slice of no entries alone is flagged (there is no slot that its
@@ -353,23 +359,27 @@ __device__ __forceinline__ T sell_row(int64_t i, const C *__restrict__ col, cons
 // over the rows; each writes one partial per workgroup per dot product.
 //   parts layout: pq[G], rz[G], rr[G], aux[G]
 //
-// Two kernels an iteration.  The product forms the new direction itself,
-// p = z + beta p, for its own row (stored, in the other of two buffers) and for
-// each entry it gathers, and adds the previous step to the iterate while it
-// holds the previous direction: a pass over z, p and p' and a launch less than
-// a direction kernel, and the update does not read p.  k_cg_fin closes a group
-// of CHECK iterations.  The dot products are summed as ever, so the bits are
-// those of the three-kernel iteration.  Mixed heat Q4 1500x1300, an iteration:
-// 55.7 -> 44.8 us (rows of the neighbouring blocks on one XCD: 5 us of it);
-// bytes a row (nine entries) 88 -> 80.  Two rows of loads in flight per
-// work-item measured slower than one (57 us: 144 registers, three waves a SIMD
-// where the grid has four), and so did taking the grid neighbours' values from
-// the next lane in place of two thirds of the gathers (46.6 us: L1 is not the
-// bound).
+// Three kernels an iteration: the new direction with the last step of the
+// iterate (k_cg_dir), the product, the update.  Or two: the product forms the new
+// direction itself, p = z + beta p, for its own row (stored, in the other of two
+// buffers) and for each entry it gathers, and adds the last step while it holds
+// the last direction, a pass over z, p and p' and a launch less, but every
+// gather is of two vectors.  All sums are the same, so the bits are.  Measured,
+// three kernels against two, us an iteration: mixed heat Q4 1300^2 36.9, 36.2, T3
+// 1000^2 26.7, 25.2, T4 60^3 19.7, 18.7, Q4 4096^2 284, 279; FP64 the same 62.2,
+// 66.1; 38.5, 39.9; 23.7, 25.0; 538, 588; rows in random order, T3 1000^2, mixed
+// 67, 134, FP64 98, 198; wide rows of two dofs a node, elasticity T6 250^2, 34,
+// 41 and 42, 63.  So two kernels for FP32 vectors where most slices are uniform,
+// three for the rest.
+// Neighbouring blocks' rows on one XCD take 5 us off mixed heat Q4 1500x1300.
+// Two rows of loads in flight per work-item measured slower than one (57 us
+// against 45: 144 registers, three waves a SIMD where the grid has four), and so
+// did taking the grid neighbours' values from the next lane in place of two
+// thirds of the gathers (46.6 us: L1 is not the bound).
 
 // The iterate's last step, x += alpha p: the FP64 solve updates its FP64
 // iterate (TX = double).  The mixed solve adds alpha p to an FP32 accumulator
-// of the last few iterations' steps (TX = float), which k_cg_fin folds into the
+// of the last few iterations' steps (TX = float), which k_cg_dir folds into the
 // FP64 iterate every CHECK iterations: an FP32 iterate itself absorbs the late,
 // small corrections (x + alpha p rounds back to x; the mixed solve then needed
 // 69 % more iterations than FP64 PCG on heat Q4 1024^2 against 9 % with an FP64
@@ -377,10 +387,10 @@ __device__ __forceinline__ T sell_row(int64_t i, const C *__restrict__ col, cons
 // corrections, so each keeps its FP32 relative precision.
 //
 // DIR: p = z + beta p_old into p, x += alpha p_old; else the product with p_old
-// as it is (the first iteration of a group).  q = A p; partial p.q.  Workgroup 0
-// leaves this iteration's r.z in rzs[par].
-template <typename T, typename TX, typename C, bool DIR>
-__global__ __launch_bounds__(SV_BLOCK, 4) void k_cg_spmv(int64_t n, const uint32_t *__restrict__ off,
+// as it is.  q = A p; partial p.q.  SUMS: workgroup 0 leaves this iteration's r.z
+// in rzs[par] (else k_cg_dir has).
+template <typename T, typename TX, typename C, bool DIR, bool SUMS>
+__global__ __launch_bounds__(SV_BLOCK, DIR ? 4 : 1) void k_cg_spmv(int64_t n, const uint32_t *__restrict__ off,
                                                       const C *__restrict__ col, const T *__restrict__ val,
                                                       SellU U, const T *__restrict__ z, const T *__restrict__ p_old,
                                                       T *__restrict__ p, T *__restrict__ q, TX *__restrict__ x,
@@ -390,7 +400,9 @@ __global__ __launch_bounds__(SV_BLOCK, 4) void k_cg_spmv(int64_t n, const uint32
     __shared__ double sh[SV_BLOCK / 64];
     using V = typename std::conditional<DIR, DirGather<T>, VecGather<T>>::type;
     const int64_t stride = (int64_t)gridDim.x * SV_BLOCK;
-    const uint32_t blk = row_block();
+    // (columns beyond 16 bits are not neighbours: there the blocks in order are
+    // up to 10 % faster)
+    const uint32_t blk = sizeof(C) == 2 ? row_block() : blockIdx.x;
     int64_t i = (int64_t)blk * SV_BLOCK + threadIdx.x;
     V g;
     if constexpr (DIR) { g.z = z; g.p = p_old; } else g.x = p_old;
@@ -400,8 +412,11 @@ __global__ __launch_bounds__(SV_BLOCK, 4) void k_cg_spmv(int64_t n, const uint32
         m0 = slice_meta(i, off, U);
         if (m0.w <= SELL_UNROLL) R0.load(i, col, val, g, U, m0);
     }
-    const double rz = sum_partials(part_rz, gridDim.x, sh);
-    if (blockIdx.x == 0 && threadIdx.x == 0) sc[S_RZS + par] = rz;
+    double rz = 0.0;
+    if constexpr (SUMS) {
+        rz = sum_partials(part_rz, gridDim.x, sh);
+        if (blockIdx.x == 0 && threadIdx.x == 0) sc[S_RZS + par] = rz;
+    }
     TX alphax = TX(0);
     if constexpr (DIR) {
         const double rz_old = sc[S_RZS + (par ^ 1)];
@@ -480,11 +495,12 @@ __global__ __launch_bounds__(SV_BLOCK) void k_cg_update(int64_t n, const T *__re
     if (threadIdx.x == 0) { part_rz[blockIdx.x] = a; part_rr[blockIdx.x] = b; }
 }
 
-// The end of a group of iterations: x += alpha p (and, mixed, the accumulated
-// steps xlo into the FP64 iterate), p = z + beta p.  Workgroup 0 also leaves rz
-// and ||r||^2 for the host.
-template <typename T, typename TX>
-__global__ __launch_bounds__(SV_BLOCK) void k_cg_fin(int64_t n, const double *__restrict__ part_rz,
+// x += alpha p, p = z + beta p; par: the iteration's parity whose update came
+// last.  Workgroup 0 leaves the r.z that beta was formed with in rzs[par ^ 1].
+// END, the end of a group of iterations: the accumulated steps xlo go into the
+// FP64 iterate too (mixed), and workgroup 0 leaves rz and ||r||^2 for the host.
+template <typename T, typename TX, bool END>
+__global__ __launch_bounds__(SV_BLOCK) void k_cg_dir(int64_t n, const double *__restrict__ part_rz,
                                                      const double *__restrict__ part_rr, const T *__restrict__ z,
                                                      T *__restrict__ p, TX *__restrict__ xs, double *__restrict__ x,
                                                      double *__restrict__ sc, int par, double *__restrict__ hsc)
@@ -499,7 +515,7 @@ __global__ __launch_bounds__(SV_BLOCK) void k_cg_fin(int64_t n, const double *__
         const T pr = p[i];
         TX t = xs[i];
         t += alphax * (TX)pr;
-        if constexpr (sizeof(TX) == 4) {
+        if constexpr (END && sizeof(TX) == 4) {
             x[i] += (double)t;
             xs[i] = TX(0);
         } else {
@@ -507,7 +523,8 @@ __global__ __launch_bounds__(SV_BLOCK) void k_cg_fin(int64_t n, const double *__
         }
         p[i] = z[i] + beta * pr;
     }
-    if (blockIdx.x == 0) {
+    if (!END && blockIdx.x == 0 && threadIdx.x == 0) sc[S_RZS + (par ^ 1)] = rz;
+    if (END && blockIdx.x == 0) {
         const double rr = sum_partials(part_rr, G, sh);
         if (threadIdx.x == 0) { sc[S_RZ] = rz; sc[S_RR] = rr; hsc[S_RR] = rr; }
     }
@@ -532,7 +549,7 @@ __global__ __launch_bounds__(SV_BLOCK) void k_cg_fin(int64_t n, const double *__
 // The launch is cooperative, so that all workgroups run and every wait ends;
 // a wait of EX_LIMIT polls, near a second (another process's launch holds some
 // of the CUs, and waits too), ends the launch: what it has made of x is the
-// start of the two-launch iteration, as any x is.
+// start of the iteration of several launches, as any x is.
 // VB: the registers of a row (its entries, the gathers in flight) leave 512
 // work-items of FP64 rows or 768 of FP32 rows; larger workgroups spill (1024
 // FP64: 14.9 us an iteration at 9801 rows), smaller ones are more pollers of the
@@ -715,7 +732,7 @@ __global__ void k_cg_slots(uint64_t *__restrict__ slots, int n, double *__restri
 
 // Groups of CHECK iterations from the state that k_cg_reset or this kernel left
 // (r, z, p, r.z partials) until ||r||^2 <= goal2 or maxit; leaves the same state
-// as k_cg_fin, the iteration count in sc[S_IT] and ||r||^2 in sc[S_RREC]; sc[S_LOST] is set by
+// as k_cg_dir, the iteration count in sc[S_IT] and ||r||^2 in sc[S_RREC]; sc[S_LOST] is set by
 // every workgroup that gave up a wait (another may have been through it).
 template <typename T, typename TX, typename C, int VB>
 __global__ __launch_bounds__(VB * SV_BLOCK) void k_cg_small(int64_t n, const uint32_t *__restrict__ off,
@@ -1428,7 +1445,7 @@ template <typename T>
 struct Vecs {
     double *x;  // the iterate: FP64 in both solves
     T *r, *z, *p, *p2, *q, *dinv;
-    float *xlo;  // mixed solve: the steps since the last k_cg_fin (null: x updated directly)
+    float *xlo;  // mixed solve: the steps since the last k_cg_dir (null: x updated directly)
 };
 
 struct Sell {
@@ -1439,6 +1456,7 @@ struct Sell {
     const float *v32;
     SellU U;
     const int2 *rec;  // per slice, for the resident solve (null: not made)
+    bool fused;       // the mixed solve's product forms the direction
 };
 
 template <typename T>
@@ -1460,18 +1478,19 @@ void cg_group_as(hipStream_t st, int64_t n, const Sell &S, Vecs<T> &v, TX *xs, c
     const C *col = (const C *)S.col;
     const T *val = sell_vals<T>(S);
     for (int k = 0; k < CHECK; k++) {
-        if (k == 0) {
-            hipLaunchKernelGGL((k_cg_spmv<T, TX, C, false>), g, b, 0, st, n, S.off, col, val, S.U, (const T *)v.z,
-                               (const T *)v.p, v.p2, v.q, xs, P.rz, sc, k & 1, P.pq);
-        } else {
-            hipLaunchKernelGGL((k_cg_spmv<T, TX, C, true>), g, b, 0, st, n, S.off, col, val, S.U, (const T *)v.z,
-                               (const T *)v.p, v.p2, v.q, xs, P.rz, sc, k & 1, P.pq);
-            std::swap(v.p, v.p2);
-        }
+        const bool form = k > 0 && S.fused && sizeof(T) == 4;
+        if (k > 0 && !form)
+            hipLaunchKernelGGL((k_cg_dir<T, TX, false>), g, b, 0, st, n, P.rz, P.rr, (const T *)v.z, v.p, xs, v.x, sc,
+                               (k - 1) & 1, hsc);
+        hipLaunchKernelGGL((form ? k_cg_spmv<T, TX, C, sizeof(T) == 4, true>
+                                 : k > 0 ? k_cg_spmv<T, TX, C, false, false> : k_cg_spmv<T, TX, C, false, true>),
+                           g, b, 0, st, n, S.off, col, val, S.U, (const T *)v.z, (const T *)v.p, v.p2, v.q, xs, P.rz, sc, k & 1,
+                           P.pq);
+        if (form) std::swap(v.p, v.p2);
         hipLaunchKernelGGL((k_cg_update<T>), g, b, 0, st, n, (const T *)v.dinv, v.r, v.z, (const T *)v.q, P.pq, sc, k & 1,
                            P.rz, P.rr);
     }
-    hipLaunchKernelGGL((k_cg_fin<T, TX>), g, b, 0, st, n, P.rz, P.rr, (const T *)v.z, v.p, xs, v.x, sc,
+    hipLaunchKernelGGL((k_cg_dir<T, TX, true>), g, b, 0, st, n, P.rz, P.rr, (const T *)v.z, v.p, xs, v.x, sc,
                        (CHECK - 1) & 1, hsc);
 }
 
@@ -1693,10 +1712,10 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
     if (uniform_slots) {
         if (c16)
             hipLaunchKernelGGL((k_sell_uniform<int16_t>), dim3(ceil_div(nslices * 64, 256)), dim3(256), 0, st, n,
-                               nslices, (const uint32_t *)off, (const int16_t *)scol, uflag, uoff);
+                               nslices, (const uint32_t *)off, (const int16_t *)scol, uflag, uoff, total + 3);
         else
             hipLaunchKernelGGL((k_sell_uniform<int32_t>), dim3(ceil_div(nslices * 64, 256)), dim3(256), 0, st, n,
-                               nslices, (const uint32_t *)off, (const int32_t *)scol, uflag, uoff);
+                               nslices, (const uint32_t *)off, (const int32_t *)scol, uflag, uoff, total + 3);
     } else {
         hipLaunchKernelGGL(k_sell_empty, dim3(ceil_div(nslices, 256)), dim3(256), 0, st, nslices, (const uint32_t *)off, uflag);
     }
@@ -1710,7 +1729,7 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
         hipLaunchKernelGGL(k_sell_rec, dim3(ceil_div(nslices * 64, 256)), dim3(256), 0, st, n, nslices,
                            (const uint32_t *)off, (const int16_t *)scol, (const uint32_t *)len, rec, total + 1);
     hipLaunchKernelGGL(k_tell, dim3(1), dim3(64), 0, st, (const uint32_t *)total, (uint32_t *)c->told + 8);
-    const Sell S{off, scol, c16, sv64, sv32, SellU{uflag, uoff}, near9 ? rec : nullptr};
+    Sell S{off, scol, c16, sv64, sv32, SellU{uflag, uoff}, near9 ? rec : nullptr, false};
 
     // the scalars as the last reduction left them, in pinned memory
     double *hsc = (double *)c->told + 8;
@@ -1749,7 +1768,8 @@ int pcg_solve(elfel_hip_ctx *c, int64_t nfree, const double *F, double *x, int p
     double rn = 0.0;
     if ((rc = true_residual(&rn))) return rc;
     const bool resident = near9 && tot[1] == 0;
-    bool lost = false;  // a one-launch solve's workgroups did not all run: two launches from then on
+    S.fused = env_int("ELFEL_HIP_PCG_FUSED", 2 * tot[3] >= (nslices + UNI_STEP - 1) / UNI_STEP) != 0;
+    bool lost = false;  // a one-launch solve's workgroups did not all run: several launches an iteration from then on
     const double bnorm = hsc[S_BB] > 0 ? sqrt(hsc[S_BB]) : 1.0;
     const double target = tol * bnorm;
     // Iterations until ||r||^2 <= goal2 or maxit from the state of the last reset,

@@ -144,3 +144,34 @@ def test_both_ways_where_the_kernels_change(ctx, monkeypatch, N, prec, sizes, fe
         assert free == nfree < n
         # (one grid row of quadrilaterals: the strips of one free node across, above)
         _both(ctx, monkeypatch, nfree, prec, tol=1e-8, ends=prec == L.FP64 or fe == L.T3 or nfree > N + 1)
+
+
+@pytest.mark.parametrize("prec", [L.FP64, L.MIXED])
+@pytest.mark.parametrize("fe,N,shuffle", [(L.T3, 40, False), (L.Q4, 300, False), (L.T3, 300, True), (L.Q4, 700, False), (L.T6, 60, False),
+                                          (L.T6, 60, True)])
+def test_direction_in_the_product_or_before_it(ctx, monkeypatch, fe, N, shuffle, prec):
+    """Two and three kernels an iteration (ELFEL_HIP_PCG_FUSED), heat and, on T6,
+    elasticity, whose rows are wider than the registers; in a random order the
+    columns lie beyond 16-bit offsets."""
+    mesh = {L.T3: eh.T3block, L.Q4: eh.Q4block, L.T6: eh.T6block}[fe](1.0, 1.0, N, N)
+    nc = 2 if fe == L.T6 else 1
+    n = mesh.nnodes * nc
+    nfree = n - 3 * N * nc
+    dof = np.random.default_rng(N).permutation(n) if shuffle else np.arange(n)
+    ctx.set_mesh(0, mesh.conn, mesh.xy)
+    ctx.set_dofs(0, dof.reshape(-1, nc) + 1, n)
+    ctx.set_coefficients(mesh.nelements)
+    ctx.assemble(L.ELAST if nc == 2 else L.HEAT, fe, {L.T3: 1, L.Q4: 2, L.T6: 3}[fe], precision=L.FP64, method=L.REUSE,
+                 layout=L.CSR, D=eh.plane_strain_D(1.0, 0.3))
+    rng = np.random.default_rng(7)
+    F, x0 = rng.standard_normal(n), rng.standard_normal(n)
+    monkeypatch.setenv("ELFEL_HIP_PCG_ONE_LAUNCH", "0")
+    got = []
+    for fused in ("0", "1", None):
+        if fused is None:
+            monkeypatch.delenv("ELFEL_HIP_PCG_FUSED")
+        else:
+            monkeypatch.setenv("ELFEL_HIP_PCG_FUSED", fused)
+        got.append(ctx.pcg(nfree, F, x0, precision=prec, tol=1e-8, maxit=20000))
+    for x, it, _, rel in got:
+        assert rel <= 1e-8 and it == got[0][1] and np.array_equal(x, got[0][0])
