@@ -1,7 +1,7 @@
-"""Small transfers (arrays of a call up to 1 MiB together, transfer.hip): uploads
+"""Small transfers (arrays of a call up to 2 MiB on the device, transfer.hip): uploads
 that nothing waits for, one after another through more memory than a context
 keeps for them, from host arrays that change right after the call; coefficients
-at the edges of the padded blocks (4096) and of what counts as small (65536 of
+at the edges of the padded blocks (4096) and of what counts as small (131072 of
 two coefficients), read back exactly: a matrix and a load of powers of two."""
 import numpy as np
 import pytest
@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("nx,ny", [(1, 1), (45, 45), (63, 65), (64, 64), (241, 17), (128, 128), (256, 250), (256, 256), (65537, 1),
-                                   (300, 300)])
+                                   (300, 300), (512, 256), (43691, 3)])
 def test_uploads_without_waits(ctx, nx, ny):
     mesh = eh.Q4block(float(nx), float(ny), nx, ny)
     n, E = mesh.nnodes, mesh.nelements
