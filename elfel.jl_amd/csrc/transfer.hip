@@ -297,7 +297,9 @@ int to_host(elfel_hip_ctx *c, const HostOut *segs, int nseg)
             M.m[k++] = Move{segs[s].dev, at, segs[s].n, segs[s].wide ? 4 : 8, 0};
             at += round64((segs[s].wide ? 4 : 8) * segs[s].n);
         }
-        if (int rc = launch_moves(c, M, k)) return rc;
+        // (one array: a copy is 3 us faster than the kernel at 64 KB, 9 at 1 MB)
+        if (k == 1) HIPCHK(c, hipMemcpyAsync(M.m[0].dst, M.m[0].src, (size_t)(M.m[0].word * M.m[0].n), hipMemcpyDeviceToHost, c->stream));
+        else if (int rc = launch_moves(c, M, k)) return rc;
         HIPCHK(c, hipStreamSynchronize(c->stream));
         c->xs_at = 0;
         k = 0;

@@ -3,6 +3,8 @@ that nothing waits for, one after another through more memory than a context
 keeps for them, from host arrays that change right after the call; coefficients
 at the edges of the padded blocks (4096) and of what counts as small (131072 of
 two coefficients), read back exactly: a matrix and a load of powers of two."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -10,6 +12,7 @@ import elfel_hip as eh
 from elfel_hip import _lib as L
 
 pytestmark = pytest.mark.gpu
+I64, F64 = ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_double)
 
 
 @pytest.mark.parametrize("nx,ny", [(1, 1), (45, 45), (63, 65), (64, 64), (241, 17), (128, 128), (256, 250), (256, 256), (65537, 1),
@@ -72,3 +75,16 @@ def test_refused_upload_then_the_next(ctx):
         with pytest.raises(L.ElfelRangeError):
             ctx.vector(np.array([1, 2, bad], np.int64), np.ones(3), mesh.nnodes)
     assert np.array_equal(ctx.vector(np.array([3, 1, 3], np.int64), np.array([1.0, 2.0, 4.0]), 3), [2.0, 0.0, 5.0])
+
+
+@pytest.mark.parametrize("n", [1, 8191, 8192, 8193, 8200, 131071, 131072, 131073, 262144, 262145])
+@pytest.mark.parametrize("off", [0, 1])
+def test_one_array_out(ctx, n, off):
+    """Words as they are, one array of a call: either side of 64 KB, 1 MB and 2 MB, new memory and kept."""
+    idx, val = np.arange(1, n + 1, dtype=np.int64), np.random.default_rng(n).standard_normal(n)
+    for _ in range(3):
+        buf = np.full(n + 2, -7.0)
+        out = buf[off:off + n]
+        rc = ctx.lib.elfel_hip_vector(ctx.h, n, n, idx.ctypes.data_as(I64), val.ctypes.data_as(F64), out.ctypes.data_as(F64))
+        assert rc == L.OK and np.array_equal(out, val) and np.all(buf[off + n:] == -7.0) and np.all(buf[:off] == -7.0)
+        val = -2.0 * val
