@@ -48,7 +48,8 @@ static_assert(BK_CAP <= 1 << BK_CAP_LOG2 && BK_CAP_FEW <= 1 << BK_CAP_FEW_LOG2, 
 static_assert(BK_HASH >= 2 * BK_BLOCK * BK_COUNT_ITEMS, "the hash of the counting pass is at most half full");
 
 // ---- decoupled look-back -------------------------------------------------------
-// One 64-bit word per block of the scan: the upper half says whether the lower
+// (Merrill and Garland, Single-pass Parallel Prefix Scan with Decoupled
+// Look-back, NVIDIA Technical Report NVR-2016-002.)  One 64-bit word per block of the scan: the upper half says whether the lower
 // holds nothing yet, the block's own total or the total up to and including
 // it.  Blocks take their numbers from a counter when they start, so every
 // block that one waits for has started and waits only for earlier ones: the
